@@ -83,18 +83,22 @@ typedef struct {
 /* Intersection strategy knobs (bin thresholds and list walk); the package's
  * autotuner (katric_amd.tune) chooses them per graph class.  Counts never
  * depend on them. */
-#define KT_STRATEGY_STREAMED 0u  /* the wave walks one T list at a time, 256 ids per step (128 for lists of <= 128) */
-#define KT_STRATEGY_GROUPED16 1u /* groups of 16 lanes walk 4 T lists at a time (short lists) */
-#define KT_STRATEGY_GROUPED8 2u  /* groups of 8 lanes walk 8 T lists at a time (very short lists) */
-#define KT_STRATEGY_GROUPED32 3u /* groups of 32 lanes walk 2 T lists at a time */
-#define KT_STRATEGY_GROUPED4 4u  /* groups of 4 lanes walk 16 T lists at a time */
-#define KT_STRATEGY_GROUPED2 5u  /* groups of 2 lanes walk 32 T lists at a time */
+/* List-walk hints; accepted for callers that set them.  Every value takes the
+ * same walk: the T lists of up to 64 neighbours are streamed as one sequence
+ * of 16-byte blocks, one block per lane, so that short and long lists fill a
+ * wave alike. */
+#define KT_STRATEGY_STREAMED 0u
+#define KT_STRATEGY_GROUPED16 1u
+#define KT_STRATEGY_GROUPED8 2u
+#define KT_STRATEGY_GROUPED32 3u
+#define KT_STRATEGY_GROUPED4 4u
+#define KT_STRATEGY_GROUPED2 5u
 #define KT_ORDER_DEGREE 0u      /* work queues by degree bucket, largest first */
 #define KT_ORDER_VERTEX 1u      /* work queues by vertex id (locality across a batch's graphs) */
 typedef struct {
     uint32_t wave_max_deg;  /* |N+(v)| <= this: one wave per tail, LDS hash (<= 256) */
     uint32_t group_max_deg; /* |N+(v)| <= this: one workgroup per tail, LDS hash (<= 2048) */
-    uint32_t grid_per_cu;   /* persistent 512-thread workgroups per compute unit (1..4 fill the CU) */
+    uint32_t grid_per_cu;   /* persistent 512-thread workgroups per compute unit (3 fill the CU; more are taken as 3) */
     uint32_t strategy;      /* KT_STRATEGY_* */
     uint32_t order;         /* KT_ORDER_* */
     /* |N+(v)| above this: the tail's set is probed by binary search in global

@@ -303,11 +303,12 @@ struct PlainBufs {
     uint64_t* ws_radix;
     uint64_t* pv;
     uint64_t* small;  // [0] = err flags (u32), [1] = total, [2..] = tc stats
+    uint64_t entries;  // walk entries ws_tc's part list is sized for (0: none)
 };
 
 // Lays out every buffer of the plain path; with base == nullptr only sizes.
-uint64_t plain_layout(void* base, uint32_t n, uint64_t nnz, bool host_in, bool want_pv_dev, bool unsorted,
-                      PlainBufs& B) {
+uint64_t plain_layout(void* base, uint32_t n, uint64_t nnz, uint64_t entries, int num_cus, bool host_in,
+                      bool want_pv_dev, bool unsorted, PlainBufs& B) {
     Carver cv{base, 0};
     const uint64_t m = nnz / 2;
     B.small = static_cast<uint64_t*>(cv.take(64 * sizeof(uint64_t)));
@@ -322,7 +323,7 @@ uint64_t plain_layout(void* base, uint32_t n, uint64_t nnz, bool host_in, bool w
     B.oheads = static_cast<uint32_t*>(cv.take((m + 4) * 4));  // +4: 16-byte block reads past the end
     B.ws_orient = static_cast<uint64_t*>(cv.take(orient_ws_words(n, nnz) * 8));
     // also the scratch of the longest-list reduction of unsorted input
-    B.ws_tc = static_cast<uint64_t*>(cv.take(std::max(tc_ws_words(n), segsort_tmp_words()) * 8));
+    B.ws_tc = static_cast<uint64_t*>(cv.take(std::max(tc_ws_words(n, entries, num_cus), segsort_tmp_words()) * 8));
     B.pv = want_pv_dev ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(n, 1) * 8)) : nullptr;
     B.keys = B.alt = B.ws_radix = nullptr;
     if (unsorted) {
@@ -395,11 +396,17 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
                     bool host_in, bool pv_dev_needed, PlainBufs& B, bool& unsorted, const Workspace& ws = {}) {
     hipStream_t st = c->stream;
     unsorted = false;
-    uint64_t need = plain_layout(nullptr, n, nnz, host_in, pv_dev_needed, false, B);
+    // part list of the intersection: left out where only it does not fit a
+    // fixed workspace
+    uint64_t entries = nnz;
+    if (ws.fixed_base && plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, false, B) > ws.fixed_cap)
+        entries = 0;
+    uint64_t need = plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, false, B);
     trace("orientation: n=%u nnz=%llu workspace=%llu", n, (unsigned long long)nnz, (unsigned long long)need);
     int rc = ws.ensure(c, need);
     if (rc) return rc;
-    plain_layout(ws.base(c), n, nnz, host_in, pv_dev_needed, false, B);
+    plain_layout(ws.base(c), n, nnz, entries, c->num_cus, host_in, pv_dev_needed, false, B);
+    B.entries = entries;
     trace("workspace=%p bytes=%llu", ws.base(c), (unsigned long long)ws.cap(c));
     (void)hipEventRecord(c->ev[EV_START], st);
     rc = upload_and_count(c, n, nnz, user_off, user_heads, host_in, B);
@@ -445,16 +452,20 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
         if (flags & KT_ERR_MASK) return c->fail(KT_EINVAL, "malformed CSR: duplicate edge");
     } else if (flags & KT_FLAG_UNSORTED) {
         unsorted = true;
-        need = plain_layout(nullptr, n, nnz, host_in, pv_dev_needed, true, B);
+        if (ws.fixed_base &&
+            plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B) > ws.fixed_cap)
+            entries = 0;
+        need = plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B);
+        B.entries = entries;
         if (need > ws.cap(c)) {
             // growing the arena drops its contents: upload and count again
             rc = ws.ensure(c, need);
             if (rc) return rc;
-            plain_layout(ws.base(c), n, nnz, host_in, pv_dev_needed, true, B);
+            plain_layout(ws.base(c), n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B);
             rc = upload_and_count(c, n, nnz, user_off, user_heads, host_in, B);
             if (rc) return rc;
         } else {
-            plain_layout(ws.base(c), n, nnz, host_in, pv_dev_needed, true, B);
+            plain_layout(ws.base(c), n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B);
             if (!host_in) {
                 B.off = user_off;
                 B.heads = user_heads;
@@ -535,6 +546,7 @@ int kt::count_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, const uint3
         view.in_heads = B.heads;
         view.in_keep = orient_keep_bits(n, nnz, B.ws_orient);
     }
+    view.entries = B.entries;
     TcOut out{pv, totals};
     trace("intersection: X=%u pv=%p", n, (void*)pv);
     // wave-bin tails per queue access for one graph: each grab costs a queue

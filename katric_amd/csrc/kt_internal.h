@@ -74,20 +74,21 @@ struct TcParams {
     uint32_t wave_max_deg;    // d+(v) <= this: one wave per tail vertex (LDS hash)
     uint32_t group_max_deg;   // d+(v) <= this: one workgroup (8 waves) per tail vertex (LDS hash)
     uint32_t team_chunk;      // neighbours per work grab inside a workgroup team (1..64)
-    uint32_t grid_per_cu;     // persistent workgroups per CU
-    uint32_t strategy;        // TC_STREAMED or TC_GROUPED* (hash-probe tails)
+    uint32_t grid_per_cu;     // persistent workgroups per CU (at most three fit)
+    uint32_t strategy;        // TC_STREAMED or TC_GROUPED*
     uint32_t order;           // TC_BY_DEGREE or TC_BY_VERTEX (work-queue order)
     uint32_t table_shift = 3; // hash tables hold >= 2^table_shift slots per key where they fit (8: smaller
                               // tables to clear and flush per tail; 16 gave the same RMAT-22 time, batches 1 % slower)
+    uint32_t wave_split = 0xffffffffu;  // walk entries per part of a wave / workgroup tail (set by the launch)
+    uint32_t team_split = 0xffffffffu;
     uint32_t wave_grab = 32;  // wave-bin tails a wave takes per queue access (1..64), vertex order
     uint32_t bsearch_min_deg = 8192;  // |S(x)| above this: binary-search probes in global memory (<= 8192)
     uint32_t pseudo2core = 0; // skip tails with |S(x)| < 2 and count them (Config::pseudo2core)
     uint32_t min_side = 1;    // plain counting: intersect every edge from the side with the shorter T list
 };
 
-// How a team walks the T lists of a chunk of neighbours: the whole wave on
-// one list at a time, 256 ids per step (TC_STREAMED, long lists), or groups
-// of G lanes on 64 / G lists at a time (TC_GROUPED<G>, short lists).
+// List-walk hints of kt_params: every value takes the same walk, which fills
+// a wave whatever the lists' lengths are (walk_lists in kt_tc.hip).
 enum : uint32_t {
     TC_STREAMED = 0,
     TC_GROUPED16 = 1,
@@ -121,7 +122,6 @@ struct TcView {
     const uint64_t* t_end;      // per u (nullptr: t_end[u] = t_beg[u+1])
     const uint32_t* theads;
     const uint32_t* tail_id;    // X (nullptr: identity) -> per-vertex index of the tail
-    const uint32_t* tail_graph; // X (nullptr: all graph 0) -> index into per-graph totals
     // work counters of a message phase: stat_off (X+1, nullable) gives the
     // length each tail's message adds to intersection_size per receiver (the
     // whole received message, not only its ghost part S); with
@@ -136,6 +136,13 @@ struct TcView {
     const uint32_t* in_heads = nullptr;
     const uint64_t* in_keep = nullptr;
     uint64_t in_hash_max = 0;
+    // upper bound of all tails' walk entries, as given to tc_ws_words (0: the
+    // workspace has no part list, every tail is walked by one team)
+    uint64_t entries = 0;
+    // device flag word (nullable): with any of these bits set no tail is
+    // queued, so input that failed its checks is never walked
+    const uint32_t* gate = nullptr;
+    uint32_t gate_bits = 0;
 };
 
 struct TcOut {
@@ -172,8 +179,8 @@ struct BatchBufs {
 // in place per list (every list at most segsort_max_len() ids), or by the
 // global radix sort (its scratch is in the layout).
 enum BatchSort : uint32_t { SORT_NONE = 0, SORT_SEGMENTED = 1, SORT_RADIX = 2 };
-uint64_t batch_layout(void* base, uint32_t G, uint64_t N, uint64_t nnz, bool host_in, bool own_pv, bool unsorted,
-                      BatchBufs& B);
+uint64_t batch_layout(void* base, uint32_t G, uint64_t N, uint64_t nnz, int num_cus, bool host_in, bool own_pv,
+                      bool unsorted, BatchBufs& B);
 hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, const BatchBufs& B, uint32_t G, uint64_t N,
                           uint64_t nnz, uint64_t* pv, uint64_t* h_totals, uint64_t* h_small, uint32_t sort,
                           const uint64_t sym_key[2]);
@@ -181,7 +188,9 @@ hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, cons
 // longest oriented list of that run (B as it ran; synchronises st).
 hipError_t batch_sort_mode(hipStream_t st, const BatchBufs& B, uint64_t N, uint64_t* h_small, uint32_t& mode);
 
-uint64_t tc_ws_words(uint32_t X);
+// Words of the launch workspace for X tails whose walks hold at most `entries`
+// entries in all (0: no part list).
+uint64_t tc_ws_words(uint32_t X, uint64_t entries, int num_cus);
 // Enqueues binning and the intersection kernels; returns the launch status.
 hipError_t tc_launch(const TcView& view, const TcOut& out, const TcParams& prm, uint64_t* ws, int num_cus,
                      hipStream_t st, hipEvent_t ev_begin, hipEvent_t ev_end);

@@ -142,12 +142,12 @@ struct ServeState {
 // Device bytes of a slot's batch: the batch pipeline's buffers (with the
 // radix-sort scratch for a relaunch of unsorted lists that needs it) and the
 // gather descriptors after them.
-static uint64_t slot_bytes(uint32_t G, uint64_t N, uint64_t nnz, bool radix) {
+static uint64_t slot_bytes(const ServeState* S, uint32_t G, uint64_t N, uint64_t nnz, bool radix) {
     BatchBufs B;
-    return ((batch_layout(nullptr, G, N, nnz, true, true, radix, B) + 255) & ~255ull) + (uint64_t)G * sizeof(GatherDesc);
+    return ((batch_layout(nullptr, G, N, nnz, S->num_cus, true, true, radix, B) + 255) & ~255ull) + (uint64_t)G * sizeof(GatherDesc);
 }
 
-static uint64_t req_bytes(const ServeReq* r) { return slot_bytes(1, r->n, r->nnz, false); }
+static uint64_t req_bytes(const ServeState* S, const ServeReq* r) { return slot_bytes(S, 1, r->n, r->nnz, false); }
 
 static int slot_grow(ServeSlot& s, uint64_t bytes, uint32_t G) {
     if (bytes > s.arena_bytes) {
@@ -188,13 +188,13 @@ static int launch(ServeState* S, ServeSlot& sl, uint32_t sort) {
     }
     BatchBufs B;
     const bool radix = sort == SORT_RADIX;
-    const uint64_t used = (batch_layout(nullptr, G, N, nnz, true, true, radix, B) + 255) & ~255ull;
+    const uint64_t used = (batch_layout(nullptr, G, N, nnz, S->num_cus, true, true, radix, B) + 255) & ~255ull;
     // a slot never holds more than its share of the budget (a relaunch with
     // the radix-sort scratch can need more than admission counted)
-    if (slot_bytes(G, N, nnz, radix) > S->slot_cap) return KT_ENOMEM;
+    if (slot_bytes(S, G, N, nnz, radix) > S->slot_cap) return KT_ENOMEM;
     int rc = slot_grow(sl, used + (uint64_t)G * sizeof(GatherDesc), G);
     if (rc) return rc;
-    batch_layout(sl.arena, G, N, nnz, true, true, radix, B);
+    batch_layout(sl.arena, G, N, nnz, S->num_cus, true, true, radix, B);
     GatherDesc* d_desc = reinterpret_cast<GatherDesc*>(static_cast<char*>(sl.arena) + used);
     uint64_t* vb = sl.h_meta;
     GatherDesc* desc = reinterpret_cast<GatherDesc*>(sl.h_meta + (sl.meta_cap + 1));
@@ -321,7 +321,7 @@ static void worker_main(ServeState* S) {
                 // same requests, with the oriented lists sorted (the sort
                 // chosen from the longest list of the run that found them)
                 BatchBufs B0;
-                batch_layout(sl.arena, (uint32_t)sl.reqs.size(), sl.N, sl.nnz, true, true, false, B0);
+                batch_layout(sl.arena, (uint32_t)sl.reqs.size(), sl.N, sl.nnz, S->num_cus, true, true, false, B0);
                 uint32_t mode = SORT_RADIX;
                 int rc = batch_sort_mode(sl.stream, B0, sl.N, sl.h_small, mode) == hipSuccess ? KT_OK : KT_EHIP;
                 if (rc == KT_OK) rc = launch(S, sl, mode);
@@ -371,7 +371,7 @@ static void worker_main(ServeState* S) {
                 if (large || r->isolate) {
                     if (batch.empty() && !(large && other_large)) {
                         S->pending.erase(S->pending.begin() + (ptrdiff_t)i);
-                        if (req_bytes(r) > S->slot_cap) {
+                        if (req_bytes(S, r) > S->slot_cap) {
                             r->status = KT_ENOMEM;
                             r->done = true;
                             S->cv_done.notify_all();
@@ -384,7 +384,7 @@ static void worker_main(ServeState* S) {
                     ++i;  // keeps its place; smaller requests behind it go ahead
                     continue;
                 }
-                const uint64_t bytes = slot_bytes((uint32_t)batch.size() + 1, N + r->n, nnz + r->nnz, false);
+                const uint64_t bytes = slot_bytes(S, (uint32_t)batch.size() + 1, N + r->n, nnz + r->nnz, false);
                 const bool limits = batch.size() + 1 <= S->cfg.max_batch_graphs &&
                                     (nnz + r->nnz) / 2 <= S->cfg.max_batch_edges;
                 if (!batch.empty() && (bytes > S->slot_cap || !limits)) break;
@@ -533,7 +533,7 @@ extern "C" int kt_serve_submit(kt_ctx* c, uint32_t n, const uint64_t* offsets, c
         }
         r->ticket = S->next_ticket++;
         S->all[r->ticket] = r;
-        if (req_bytes(r) > S->slot_cap) {
+        if (req_bytes(S, r) > S->slot_cap) {
             r->status = KT_ENOMEM;
             r->done = true;
         } else {

@@ -386,8 +386,8 @@ struct ShardBufs {
 };
 
 
-uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t mtot, bool host_in, bool pv_dev,
-                      ShardBufs& B) {
+uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t mtot, int num_cus, bool host_in,
+                      bool pv_dev, ShardBufs& B) {
     Carver cv{base, 0};
     const uint64_t nloc = in->range_bounds[in->rank + 1] - in->range_bounds[in->rank];
     const uint64_t X = nloc + in->n_ghost;
@@ -419,7 +419,9 @@ uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t 
     const uint64_t rs_words = (n_all + 31) / 32;
     B.scan_tmp = static_cast<uint64_t*>(
         cv.take(scan_tmp_words(std::max(std::max<uint64_t>(X, in->n_msg), rs_words) + 1) * 8));
-    B.tc_ws = static_cast<uint64_t*>(cv.take(tc_ws_words((uint32_t)std::max<uint64_t>(X, in->n_msg)) * 8));
+    // both phases use it: the list of the larger set of tails, the parts of the longer walk
+    B.tc_ws = static_cast<uint64_t*>(cv.take(
+        tc_ws_words((uint32_t)std::max<uint64_t>(X, in->n_msg), std::max(nnz, mtot), num_cus) * 8));
     B.pv = pv_dev ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(X, 1) * 8)) : nullptr;
     B.rs = static_cast<uint2*>(cv.take((rs_words + 1) * 8));
     B.rs_cnt = static_cast<uint64_t*>(cv.take((rs_words + 1) * 8));
@@ -472,10 +474,10 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
         (in->n_msg && (!in->msg_src || !in->msg_offsets || (mtot && !in->msg_heads))))
         return c->fail(KT_EINVAL, "null shard array");
     ShardBufs B;
-    const uint64_t need = shard_layout(nullptr, in, nnz, mtot, host_in, want_pv && !pv_dev, B);
+    const uint64_t need = shard_layout(nullptr, in, nnz, mtot, c->num_cus, host_in, want_pv && !pv_dev, B);
     rc = c->reserve(need);
     if (rc) return rc;
-    shard_layout(c->arena, in, nnz, mtot, host_in, want_pv && !pv_dev, B);
+    shard_layout(c->arena, in, nnz, mtot, c->num_cus, host_in, want_pv && !pv_dev, B);
     hipStream_t st = c->stream;
     (void)hipEventRecord(c->ev[EV_START], st);
     if (host_in) {
@@ -586,6 +588,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
             v.t_end = B.coff + 1;
             v.theads = B.cheads;
         }
+        v.entries = std::max(nnz, mtot);
         TcOut o{pv, totals};
         rc = c->hip_check(tc_launch(v, o, c->prm, B.tc_ws, c->num_cus, st, c->ev[EV_TC0], c->ev[EV_TC1]),
                           "intersection launch");
@@ -617,6 +620,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
         // intersected ids; a CeTriC receiver without cut edges was compacted away
         v.stat_off = B.msg_off;
         v.stat_skip_empty = cetric ? 1u : 0u;
+        v.entries = std::max(nnz, mtot);
         TcOut o{pv, totals + 1};
         // message tails have short owned parts: a whole workgroup on one of
         // them idles, so tails up to the largest wave table stay with one

@@ -5,19 +5,21 @@
 // hash-probe design for CDNA (wave64, LDS):
 //
 //   * a "team" -- one wave, or all eight waves of a 512-thread workgroup for
-//     heavier tails -- takes a tail x and builds a linear-probing hash of
-//     S(x) = N+(x) in LDS (load factor <= 1/16 where the table allows, <= 1/2
+//     heavier tails -- takes a tail x and builds a bucketed hash of
+//     S(x) = N+(x) in LDS (load <= 1/8 where the table allows, <= 1/2
 //     at the bins' largest sets): few buckets are full, so a probe rarely
-//     has to continue into the next bucket;
-//   * the team walks R(x) = N+(x) one neighbour u per wave at a time (u, and
-//     the bounds of T(u) = N+(u), are wave-uniform scalar loads); the wave
-//     streams T(u) with coalesced 16-byte loads, four ids per lane, the next
-//     block prefetched while the current one is probed;
+//     has to continue into the next bucket; tails of at most 64 ids and 64
+//     walk entries share a wave, several at a time (pack_process);
+//   * a wave takes up to 64 walk entries of R(x) at once and streams their T
+//     lists as one sequence of 16-byte blocks, a block per lane and step
+//     (walk_lists), the next step's blocks loaded while the current ones are
+//     probed;
 //   * every hit w is one emitted Triangle{x, u, w}; per-vertex counts are
-//     privatised -- per-slot LDS counters for w, a wave sum for u, a team sum
-//     for x -- and flushed with one global atomic per non-zero counter;
-//   * tails are bucketed by ceil(log2 |S(x)|) and taken largest first from
-//     per-bucket work queues (dynamic, LPT-like balance across the grid);
+//     privatised -- per-slot LDS counters for w, a count per list for u, a
+//     team sum for x -- and flushed with one global atomic per non-zero counter;
+//   * tails are bucketed by ceil(log2 |S(x)|), largest first; walks longer than
+//     a team's share are split into parts (split_rule); workgroups take fixed
+//     shares first and pull the rest from queues (Shares);
 //   * tails above the workgroup bin go to 16-wave teams whose table fills a
 //     workgroup's LDS (16384 slots, |S| <= 8192); only larger S(x) are probed
 //     by binary search in the sorted S(x) in global memory.
@@ -44,21 +46,26 @@ constexpr uint32_t MIN_LOGS = 6;
 // XCD, each in vertex order.  Bucket 17 holds the tails above the workgroup
 // bin whose table still fits a workgroup's whole LDS (k_tc_big), bucket 16
 // those beyond (binary search, k_tc_huge).
-constexpr int NBUCKET = 18;
+// Buckets 18 and 19 hold parts of tails whose walk is too long for one team
+// (see split_rule): entries (part << 32 | tail) in a list of their own, taken
+// by workgroup teams (18) and by waves (19) before everything else.
+constexpr int NBUCKET = 20;
 constexpr int BUCKET_HUGE = 16;
 constexpr int BUCKET_BIG = 17;
+constexpr int BUCKET_TEAM_PARTS = 18;
+constexpr int BUCKET_WAVE_PARTS = 19;
+constexpr int NLIST = 18;  // buckets whose tails share the u32 list
 // k_tc_big: one 1024-thread workgroup per CU with a 16384-slot table (128 KB
 // of LDS for keys and counters), for |S| <= 8192
 constexpr int BIG_THREADS = 1024;
 constexpr int BIG_WAVES = BIG_THREADS / KT_WAVE;
 constexpr uint32_t BIG_SLOTS = 16384;
 constexpr int NXCD = 8;  // MI355X: workgroup i runs on XCD i % 8
-constexpr uint32_t WAVE_GRAB = 8;  // wave-phase tails taken per queue access
 
 // work-queue header (u32 words at the start of the workspace); every counter
 // that waves update concurrently sits on its own 128-byte line so that the
 // queues of different buckets land on different L2 channels:
-//   [0, 18)               tails per bucket (written by binning, then read-only)
+//   [0, 20)               tails (parts) per bucket (written by binning, then read-only)
 //   Q_PULL + 32 * b       pull cursor of bucket b
 //   Q_FILL + 32 * b       fill cursor of bucket b (binning pass 2)
 enum : int { Q_CNT = 0, Q_PULL = 32, Q_FILL = 32 * (NBUCKET + 1), Q_STRIDE = 32, Q_WORDS = 32 * (2 * NBUCKET + 2) };
@@ -149,13 +156,12 @@ struct View {
     __device__ __forceinline__ uint32_t tail_pv(uint32_t x) const {
         return (PLAIN || v.tail_id == nullptr) ? x : v.tail_id[x];
     }
-    __device__ __forceinline__ uint32_t tail_graph(uint32_t x) const {
-        return v.tail_graph ? v.tail_graph[x] : 0u;
-    }
     // length tail x charges to intersection_size per receiver (ns = |S(x)|)
     __device__ __forceinline__ uint64_t stat_len(uint32_t x, uint64_t ns) const {
         return (!PLAIN && v.stat_off) ? v.stat_off[x + 1] - v.stat_off[x] : ns;
     }
+    // the input failed its checks (read after the kernels that check it)
+    __device__ __forceinline__ bool gated() const { return v.gate && (*v.gate & v.gate_bits); }
     __device__ __forceinline__ bool stat_skip_empty() const { return !PLAIN && v.stat_skip_empty; }
 };
 
@@ -173,8 +179,9 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 // ---------------------------------------------------------------------------
 template <bool PLAIN>
 __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams& prm, uint32_t x, uint64_t& s,
-                                           uint64_t& r) {
+                                           uint64_t& r, uint32_t& parts) {
     uint64_t sb, se, rb, re;
+    parts = 1;
     V.s_range(x, sb, se);
     V.r_range(x, rb, re);
     s = se - sb;
@@ -186,9 +193,15 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
     // a min-side walk covers the whole input row: a long row goes to a
     // bigger bucket (a workgroup team beyond 512 entries), whatever |S(x)|
     if (V.min_side()) b = max(b, min((int)ceil_log2(r) - 2, (int)ceil_log2(prm.group_max_deg)));
+    const bool wave = b <= (int)ceil_log2(prm.wave_max_deg);
+    const uint32_t split = wave ? prm.wave_split : prm.team_split;
+    if (r > split) {
+        parts = (uint32_t)((r + split - 1) / split);
+        return wave ? BUCKET_WAVE_PARTS : BUCKET_TEAM_PARTS;
+    }
     if (prm.order == TC_BY_VERTEX) {  // two classes per XCD, each in vertex order
         const int xcd = (int)(((uint64_t)x * NXCD) / V.v.X);
-        return b <= (int)ceil_log2(prm.wave_max_deg) ? NXCD + xcd : xcd;
+        return wave ? NXCD + xcd : xcd;
     }
     return b;
 }
@@ -200,13 +213,15 @@ __global__ void __launch_bounds__(256) k_tc_bin_count(View<PLAIN> V, TcParams pr
                                                       uint64_t* __restrict__ stats) {
     __shared__ uint32_t cnt[NBUCKET];
     __shared__ uint64_t red[3][4];
+    if (V.gated()) return;
     if (threadIdx.x < NBUCKET) cnt[threadIdx.x] = 0;
     __syncthreads();
     uint64_t wedge = 0, isz = 0, skipped = 0;
     for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < V.v.X; x += gridDim.x * blockDim.x) {
         uint64_t s, r;
-        int b = tail_bucket(V, prm, x, s, r);
-        if (b >= 0) atomicAdd(&cnt[b], 1u);
+        uint32_t parts;
+        int b = tail_bucket(V, prm, x, s, r, parts);
+        if (b >= 0) atomicAdd(&cnt[b], parts);
         // pseudo2core: tails with fewer than two out-neighbours are skipped
         // and counted (cetric_edge_iterator.h:239-242)
         if (prm.pseudo2core && s < 2) ++skipped;
@@ -256,10 +271,15 @@ __global__ void __launch_bounds__(256) k_tc_bin_count(View<PLAIN> V, TcParams pr
     if (threadIdx.x < NBUCKET && cnt[threadIdx.x]) atomicAdd(&q[Q_CNT + threadIdx.x], cnt[threadIdx.x]);
 }
 
-// Bucket regions in one list: bucket b starts at sum of counts of b' < b.
+// Bucket regions in one list, the highest bucket first, so that by degree the
+// workgroup tails and the wave tails are each one run, largest first (the part
+// buckets: in the part list, in order).
 __device__ __forceinline__ uint32_t bucket_base(const uint32_t* q, int b) {
     uint32_t s = 0;
-    for (int i = 0; i < b; ++i) s += q[Q_CNT + i];
+    if (b < NLIST)
+        for (int i = b + 1; i < NLIST; ++i) s += q[Q_CNT + i];
+    else
+        for (int i = NLIST; i < b; ++i) s += q[Q_CNT + i];
     return s;
 }
 
@@ -268,9 +288,10 @@ __device__ __forceinline__ uint32_t bucket_base(const uint32_t* q, int b) {
 // writes its tails into the reserved ranges.
 template <bool PLAIN>
 __global__ void __launch_bounds__(256) k_tc_bin_fill(View<PLAIN> V, TcParams prm, uint32_t* __restrict__ q,
-                                                     uint32_t* __restrict__ list) {
+                                                     uint32_t* __restrict__ list, uint64_t* __restrict__ plist) {
     __shared__ uint32_t cnt[NBUCKET];
     __shared__ uint32_t pos[NBUCKET];
+    if (V.gated()) return;
     const uint32_t X = V.v.X;
     const uint32_t per = (X + gridDim.x - 1) / gridDim.x;
     const uint32_t x0 = min(X, blockIdx.x * per), x1 = min(X, x0 + per);
@@ -278,8 +299,9 @@ __global__ void __launch_bounds__(256) k_tc_bin_fill(View<PLAIN> V, TcParams prm
     __syncthreads();
     for (uint32_t x = x0 + threadIdx.x; x < x1; x += blockDim.x) {
         uint64_t s, r;
-        int b = tail_bucket(V, prm, x, s, r);
-        if (b >= 0) atomicAdd(&cnt[b], 1u);
+        uint32_t parts;
+        int b = tail_bucket(V, prm, x, s, r, parts);
+        if (b >= 0) atomicAdd(&cnt[b], parts);
     }
     __syncthreads();
     if (threadIdx.x < NBUCKET) {
@@ -289,37 +311,54 @@ __global__ void __launch_bounds__(256) k_tc_bin_fill(View<PLAIN> V, TcParams prm
     __syncthreads();
     for (uint32_t x = x0 + threadIdx.x; x < x1; x += blockDim.x) {
         uint64_t s, r;
-        int b = tail_bucket(V, prm, x, s, r);
-        if (b >= 0) list[atomicAdd(&pos[b], 1u)] = x;
+        uint32_t parts;
+        int b = tail_bucket(V, prm, x, s, r, parts);
+        if (b < 0) continue;
+        const uint32_t at = atomicAdd(&pos[b], parts);
+        if (b < NLIST) {
+            list[at] = x;
+        } else {
+            for (uint32_t k = 0; k < parts; ++k) plist[at + k] = ((uint64_t)k << 32) | x;
+        }
     }
 }
 
 // ---------------------------------------------------------------------------
 // the team worker
 // ---------------------------------------------------------------------------
-// Per-wave scratch of the grouped scan: the lanes of the chunk's non-empty
-// lists in order, and the hit counters of the chunk's (up to 64) neighbours.
+__device__ __forceinline__ uint32_t readlane32(uint32_t x, int j) { return __builtin_amdgcn_readlane(x, j); }
+__device__ __forceinline__ uint64_t readlane64(uint64_t x, int j) {
+    uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, j);
+    uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), j);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Per-wave scratch of the list walk: the boundary bits of a window of blocks,
+// where each list's blocks are, and the lists' hit counts.
 struct PackLds {
-    uint32_t marks[KT_WAVE / 4];
+    uint32_t bits[KT_WAVE];
+    uint4 rec[KT_WAVE];
     uint32_t ucnt[KT_WAVE];
 };
 
 struct Lds {
     uint32_t keys[GROUP_SLOTS];
     uint32_t cnt[GROUP_SLOTS];
-    uint32_t ovf[GROUP_SLOTS / 128];  // a bit per bucket (the team's table, or 4 words per wave table)
     PackLds pk[TC_WAVES];
+    uint32_t ovf[GROUP_SLOTS / 128];  // a bit per bucket (the team's table, or 4 words per wave table)
     uint64_t red[TC_WAVES];
     unsigned long long list_ctr[TC_WAVES];  // listing: triangles of the current tail written so far
     uint32_t next_u;
     uint32_t bcast;
     uint32_t full;  // the team table has a full bucket
+    uint32_t qcnt[NBUCKET], qbase[NBUCKET];  // the queue's buckets
+    uint32_t qctr[NBUCKET];                  // wave grabs handed out of this workgroup's shares
 };
 
 // Team control words of k_tc_big (its table is dynamic LDS).
 struct LdsBig {
-    uint32_t ovf[BIG_SLOTS / 128];  // a bit per bucket of the dynamic-LDS table
     PackLds pk[BIG_WAVES];
+    uint32_t ovf[BIG_SLOTS / 128];  // a bit per bucket of the dynamic-LDS table
     uint64_t red[BIG_WAVES];
     unsigned long long list_ctr[BIG_WAVES];
     uint32_t next_u;
@@ -339,7 +378,9 @@ __device__ __forceinline__ void team_sync() {
 // ds_read_b128), filled left to right; a key lives in its home bucket
 // hash(w) or, when that was full at insertion, in a later bucket (linear
 // probing over buckets).  A lookup therefore ends at the first bucket that
-// holds w or has an empty last slot.
+// holds w or has an empty last slot.  A table is empty (keys KT_EMPTY, counters
+// and bucket bits zero) whenever no tail uses it: the thread that inserted an
+// id empties its slot again, so no pass over all slots is needed.
 // Home bucket of id w as a byte offset into the table: w xor w rotated right
 // by 12, masked with boff_mask = (buckets - 1) << 4 -- two full-rate
 // instructions (one v_bitop3 after the rotation) that give the LDS address
@@ -357,54 +398,57 @@ __device__ __forceinline__ const uint4* bucket_at(const uint32_t* keys, uint32_t
     return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(keys) + off);
 }
 
-// Inserts w; returns true when w went past its home bucket (which then gets
+// Inserts w into the table at byte offset toff and returns the byte offset of
+// its slot; `moved` is set when w went past its home bucket (which then gets
 // its bit in `ovf`, one bit per bucket).  A lookup continues past its home
 // bucket only when that bucket is full and has the bit; in a table where no
 // insertion went past its home bucket, every lookup ends there.
-__device__ __forceinline__ bool table_insert(uint32_t* keys, uint32_t* ovf, uint32_t boff_mask, uint32_t w) {
+__device__ __forceinline__ uint32_t table_insert(uint32_t* keys, uint32_t* ovf, uint32_t toff, uint32_t boff_mask,
+                                                 uint32_t w, bool& moved) {
     const uint32_t home = bucket_off(w, boff_mask);
     uint32_t b = home;
-    bool moved = false;
+    bool first = true;
     while (true) {
-        uint32_t* bk = at_byte(keys, b);
+        uint32_t* bk = at_byte(keys, toff + b);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            uint32_t old = atomicCAS(&bk[s], KT_EMPTY, w);
-            if (old == KT_EMPTY || old == w) return moved;
+            const uint32_t old = atomicCAS(&bk[s], KT_EMPTY, w);
+            if (old == KT_EMPTY || old == w) return toff + b + 4 * s;
         }
-        if (!moved) atomicOr(&ovf[home >> 9], 1u << ((home >> 4) & 31));
+        if (first) atomicOr(&ovf[(toff + home) >> 9], 1u << (((toff + home) >> 4) & 31));
         b = (b + 16) & boff_mask;
+        first = false;
         moved = true;
     }
 }
 
-// Probes the first N (2 or 4) ids of this lane (id e valid iff valid[e]) and
-// returns this lane's number of hits.  Each hit bumps the w-counter of its slot and calls
+// Probes this lane's four ids (id e valid iff e < lim) and returns its number
+// of hits.  Each hit bumps the w-counter of its slot and calls
 // on_hit(e).  The four slot compares of a probe stay lane masks; hits are
 // counted per lane (one add), so the scalar unit only sees the branch masks.
 // Lookups continue past a full home bucket only in a table where some key
 // went past its home bucket (moved, wave-uniform), and only from a bucket
 // with its `ovf` bit.
-template <int N, class OnHit>
-__device__ __forceinline__ uint32_t probe_ids(const uint32_t* keys, uint32_t* cnt, const uint32_t* ovf,
-                                           uint32_t boff_mask, bool moved, const uint32_t (&w)[4],
-                                           const bool (&valid)[4], OnHit on_hit) {
+template <class OnHit>
+__device__ __forceinline__ uint32_t probe_ids(const uint32_t* keys, uint32_t* cnt, const uint32_t* ovf, uint32_t toff,
+                                              uint32_t boff_mask, bool moved, const uint32_t (&w)[4], int lim,
+                                              OnHit on_hit) {
     uint32_t bo[4];
     uint4 kk[4];
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
+    for (int e = 0; e < 4; ++e) {
         bo[e] = bucket_off(w[e], boff_mask);
-        kk[e] = *bucket_at(keys, bo[e]);
+        kk[e] = *bucket_at(keys, toff + bo[e]);
     }
     uint32_t nh = 0;
     bool hit[4];
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
+    for (int e = 0; e < 4; ++e) {
         const bool m0 = kk[e].x == w[e], m1 = kk[e].y == w[e], m2 = kk[e].z == w[e], m3 = kk[e].w == w[e];
-        hit[e] = valid[e] && (m0 || m1 || m2 || m3);
+        hit[e] = e < lim && (m0 || m1 || m2 || m3);
         nh += hit[e] ? 1u : 0u;
         if (hit[e]) {
-            atomicAdd(at_byte(cnt, bo[e]) + (m0 ? 0u : m1 ? 1u : m2 ? 2u : 3u), 1u);
+            atomicAdd(at_byte(cnt, toff + bo[e]) + (m0 ? 0u : m1 ? 1u : m2 ? 2u : 3u), 1u);
             on_hit(e);
         }
     }
@@ -412,24 +456,22 @@ __device__ __forceinline__ uint32_t probe_ids(const uint32_t* keys, uint32_t* cn
     // a full home bucket without w: w may sit in a later bucket
     bool need[4];
 #pragma unroll
-    for (int e = 0; e < N; ++e) need[e] = valid[e] && !hit[e] && kk[e].w != KT_EMPTY;
-    // one branch for the N ids, skipped as a whole when no lane needs it
-    bool any = false;
+    for (int e = 0; e < 4; ++e) need[e] = e < lim && !hit[e] && kk[e].w != KT_EMPTY;
+    // one branch for the four ids, skipped as a whole when no lane needs it
+    if (need[0] || need[1] || need[2] || need[3]) {
 #pragma unroll
-    for (int e = 0; e < N; ++e) any = any || need[e];
-    if (any) {
-#pragma unroll
-        for (int e = 0; e < N; ++e) {
+        for (int e = 0; e < 4; ++e) {
             if (!need[e]) continue;
             // nothing went past w's home bucket: w is not in the table
-            if (!((ovf[bo[e] >> 9] >> ((bo[e] >> 4) & 31)) & 1u)) continue;
+            const uint32_t home = toff + bo[e];
+            if (!((ovf[home >> 9] >> ((home >> 4) & 31)) & 1u)) continue;
             uint32_t b = bo[e];
             while (true) {
                 b = (b + 16) & boff_mask;
-                const uint4 k = *bucket_at(keys, b);
+                const uint4 k = *bucket_at(keys, toff + b);
                 const bool n0 = k.x == w[e], n1 = k.y == w[e], n2 = k.z == w[e], n3 = k.w == w[e];
                 if (n0 || n1 || n2 || n3) {
-                    atomicAdd(at_byte(cnt, b) + (n0 ? 0u : n1 ? 1u : n2 ? 2u : 3u), 1u);
+                    atomicAdd(at_byte(cnt, toff + b) + (n0 ? 0u : n1 ? 1u : n2 ? 2u : 3u), 1u);
                     on_hit(e);
                     ++nh;
                     break;
@@ -451,18 +493,12 @@ struct __attribute__((packed, aligned(4))) Ids4 {
 };
 __device__ __forceinline__ Ids4 load_ids4(const uint32_t* p) { return *reinterpret_cast<const Ids4*>(p); }
 
-// A T list of n ids is walked 64 << sh ids per step, 1 << sh per lane: two
-// ids per lane up to 128 ids (one step, half the probes of four per lane),
-// four beyond.  One id per lane for lists up to 64 was slower: a step's four
-// (or two) independent bucket reads per lane are what hide its latency.
-__device__ __forceinline__ uint32_t lane_shift(uint32_t n) { return n <= 2 * KT_WAVE ? 1u : 2u; }
-
 // Binary-search probe of the sorted S(x) in global memory (huge tails).
-__device__ __forceinline__ uint32_t probe_bsearch(const uint32_t* __restrict__ s, uint64_t ns, uint64_t* pv,
+__device__ __forceinline__ uint32_t probe_bsearch(const uint32_t* __restrict__ s, uint32_t ns, uint64_t* pv,
                                                   uint32_t w) {
-    uint64_t lo = 0, hi = ns;
+    uint32_t lo = 0, hi = ns;
     while (lo < hi) {
-        uint64_t mid = (lo + hi) >> 1;
+        const uint32_t mid = lo + ((hi - lo) >> 1);
         if (s[mid] < w)
             lo = mid + 1;
         else
@@ -473,13 +509,6 @@ __device__ __forceinline__ uint32_t probe_bsearch(const uint32_t* __restrict__ s
         return 1;
     }
     return 0;
-}
-
-__device__ __forceinline__ uint32_t readlane32(uint32_t x, int j) { return __builtin_amdgcn_readlane(x, j); }
-__device__ __forceinline__ uint64_t readlane64(uint64_t x, int j) {
-    uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, j);
-    uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), j);
-    return ((uint64_t)hi << 32) | lo;
 }
 
 // Triangle listing: the calling lanes (exactly those that hit) write their
@@ -510,279 +539,218 @@ struct Emitter {
 
 // Per-wave work counters: the reference's wedge_checks and
 // intersection_size, and the T-list ids this design streams through probes.
+// Kept per lane, summed over the wave once at the end.
 struct WorkStats {
-    uint64_t wedge = 0, isz = 0, stream = 0;
-    uint64_t stream_lane = 0;  // per lane, summed into stream once per wave at the end (grouped walks)
-    // the wave's total of stream and stream_lane (every lane calls this)
-    __device__ __forceinline__ uint64_t streamed() const { return stream + uniform64(wave_sum(stream_lane)); }
+    uint64_t wedge_lane = 0, stream_lane = 0;
+    uint64_t recv_lane = 0;  // what the receivers add to intersection_size beside their lists
+    __device__ __forceinline__ uint64_t wedge() const { return uniform64(wave_sum(wedge_lane)); }
+    __device__ __forceinline__ uint64_t recv() const { return uniform64(wave_sum(recv_lane)); }
+    __device__ __forceinline__ uint64_t streamed() const { return uniform64(wave_sum(stream_lane)); }
 };
 
+// What the walk probes: a hash table in LDS, or (huge tails) the sorted S(x).
 struct ProbeCtx {
     Emitter em;  // listing launches only
     uint32_t* keys;
     uint32_t* cnt;
-    uint32_t* ovf;   // one bit per bucket: some key went past it
-    uint32_t boff;   // (buckets - 1) << 4: bucket byte-offset mask
-    bool full;       // some key went past its home bucket (wave-uniform)
+    uint32_t* ovf;      // one bit per bucket: some key went past it
+    uint32_t boff;      // (buckets - 1) << 4: bucket byte-offset mask
+    bool full;          // some key went past its home bucket (wave-uniform)
     const uint32_t* s;  // sorted S(x) (binary-search probes)
-    uint64_t ns;
+    uint32_t ns;
     uint64_t* pv;
 };
 
-// Streams the T lists of up to 64 neighbours R[k0, k0+cnt) through the probe.
-// Lane j first loads u_j and the bounds of T(u_j) (one coalesced load plus two
-// gathers for the whole chunk); the wave then walks the non-empty lists in
-// order, four ids per lane per step (two for lists of at most 128 ids; one
-// 16-byte load per lane either way, which needs only 4-byte alignment: a load
-// whose width followed the list would have to complete before the branches
-// join), prefetching the next block -- of the same list or the next one --
-// before probing the current block.  Positions
-// and list bounds are wave-uniform 32-bit values; hits are counted per lane
-// and summed across the wave once per list.  Returns the chunk's hits.
-template <bool HASH, bool PLAIN, bool LIST>
-__device__ __forceinline__ uint64_t scan_chunk(const View<PLAIN>& V, uint64_t k0, uint32_t cnt, uint32_t uj,
-                                               uint32_t kw, const ProbeCtx& P, uint64_t nstat, WorkStats& wk) {
-    const uint32_t lane = lane_id();
-    uint64_t tbj = 0, tej = 0;
-    uint64_t stl = 0;
-    bool stc = false;
-    if (lane < cnt) {
-        V.entry_bounds(k0 + lane, uj, kw, P.ns, tbj, tej, stl, stc);
-    }
-    uint64_t pending = __ballot(lane < cnt && tej > tbj);
-    {
-        const uint64_t cw = uniform64(wave_sum(stl));
-        const uint32_t nrecv = (uint32_t)__popcll(__ballot(stc));
-        wk.wedge += cw;
-        wk.isz += cw + (uint64_t)nrecv * nstat;
-    }
-    if (pending == 0) return 0;
-    const uint32_t* __restrict__ T = V.t_heads();
-
-    int j = __ffsll((unsigned long long)pending) - 1;
-    pending &= pending - 1;
-    uint32_t u = readlane32(uj, j);
-    const uint32_t* base = T + readlane64(tbj, j);  // list start (uniform)
-    // |T(u)| < 2^32: an out-list holds distinct 32-bit ids
-    uint32_t len = (uint32_t)(readlane64(tej, j) - readlane64(tbj, j));
-    wk.stream += len;
-    uint32_t pos = 0;               // block start within the list (uniform)
-    uint32_t sh = lane_shift(len);  // 1 << sh ids per lane (uniform)
-    // Every lane loads (lanes past the list end re-read its start; their ids
-    // are masked by `valid`): an unconditional load keeps the number of
-    // loads in flight static, so the prefetch below is not waited for early.
-    // Addresses are a wave-uniform base plus a 32-bit lane offset; at most
-    // three ids past a list's end are read.
-    Ids4 q = load_ids4(base + ((lane << sh) < len ? (lane << sh) : 0u));
-    uint32_t nh = 0;    // this lane's hits on the current list
-    uint32_t uacc = 0;  // hits on this lane's own list (T(uj)), added at the list's end
-    uint64_t total = 0;
-    while (true) {
-        // next block: same list, or the first block of the next non-empty list
-        const uint32_t* nbase = base;
-        uint32_t npos = pos + (KT_WAVE << sh), nlen = len, nu = u, nsh = sh;
-        int nj = j;
-        bool more = true, switch_u = false;
-        if (npos >= len) {
-            switch_u = true;
-            if (pending) {
-                nj = __ffsll((unsigned long long)pending) - 1;
-                pending &= pending - 1;
-                nu = readlane32(uj, nj);
-                const uint64_t ntb = readlane64(tbj, nj);
-                nbase = T + ntb;
-                nlen = (uint32_t)(readlane64(tej, nj) - ntb);
-                wk.stream += nlen;
-                nsh = lane_shift(nlen);
-                npos = 0;
-            } else {
-                more = false;
-            }
-        }
-        const uint32_t noff = npos + (lane << nsh);
-        const Ids4 qn = load_ids4(nbase + (noff < nlen ? noff : 0u));
-        // probe the current block: id e < (1 << sh) of this lane is list
-        // entry pos + (lane << sh) + e
-        const int lim = (int)(len - pos) - (int)(lane << sh);
-        const bool valid[4] = {0 < lim, 1 < lim, 2 < lim, 3 < lim};  // ids 2, 3 only when sh == 2
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-        if (HASH) {
-            if constexpr (LIST) {
-                auto hit = [&](int e) { P.em(u, w[e]); };
-                if (sh == 2)
-                    nh += probe_ids<4>(P.keys, P.cnt, P.ovf, P.boff, P.full, w, valid, hit);
-                else
-                    nh += probe_ids<2>(P.keys, P.cnt, P.ovf, P.boff, P.full, w, valid, hit);
-            } else {
-                if (sh == 2)
-                    nh += probe_ids<4>(P.keys, P.cnt, P.ovf, P.boff, P.full, w, valid, NoHitAction{});
-                else
-                    nh += probe_ids<2>(P.keys, P.cnt, P.ovf, P.boff, P.full, w, valid, NoHitAction{});
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (e >= (1 << sh) || !valid[e]) continue;
-                const uint32_t h = probe_bsearch(P.s, P.ns, P.pv, w[e]);
-                nh += h;
-                if (LIST && h) P.em(u, w[e]);
-            }
-        }
-        if (switch_u) {
-            const uint32_t h = wave_total_dpp(nh);
-            total += h;
-            uacc += (lane == (uint32_t)j) ? h : 0u;
-            nh = 0;
-        }
-        if (!more) break;
-        u = nu;
-        j = nj;
-        base = nbase;
-        len = nlen;
-        pos = npos;
-        sh = nsh;
-        q = qn;
-    }
-    // one atomic per neighbour with hits, issued once for the chunk
-    if (P.pv && uacc) atomic_add_u64(&P.pv[uj], uacc);
-    return total;
+// Inclusive prefix sum over the wave (row shifts and row broadcasts, as wave_total_dpp).
+__device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);   // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);   // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);   // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
 }
 
-// Grouped variant of scan_chunk for the hash probe: the wave splits into
-// 64 / G groups of G lanes, and group q streams the chunk's non-empty T lists
-// of rank q, q + 64/G, q + 2*64/G, ... -- four ids per lane per step, G * 4
-// contiguous ids per group (one coalesced run per group), the next block of
-// the same list or the first block of the group's next list prefetched.  A
-// step therefore covers 64/G lists at once: short lists no longer leave most
-// of the wave idle.  Group state (list start, length, position) lives in
-// vector registers, uniform within the group; the next list's start and
-// length are read from the lane that loaded them (ds_bpermute, every lane
-// active).  Hits are added to the neighbour's LDS counter as they occur and
-// flushed with one global atomic per neighbour.
-template <int G, bool PLAIN>
-__device__ __forceinline__ uint64_t scan_chunk_grouped(const View<PLAIN>& V, uint64_t k0, uint32_t cnt, uint32_t uj,
-                                                       uint32_t kw, const ProbeCtx& P, uint64_t nstat,
-                                                       WorkStats& wk, PackLds& pk) {
-    constexpr uint32_t NQ = KT_WAVE / G;
+__device__ __forceinline__ uint32_t rank_below(uint64_t mask, uint32_t base) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, base));
+}
+__device__ __forceinline__ uint32_t from_lane(uint32_t x, uint32_t l) {
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4 * l), (int)x);
+}
+__device__ __forceinline__ uint64_t from_lane64(uint64_t x, uint32_t l) {
+    return ((uint64_t)from_lane((uint32_t)(x >> 32), l) << 32) | from_lane((uint32_t)x, l);
+}
+
+// Ids of one list walked per round (its rest follows in further rounds), so
+// that a chunk's ids are counted in 32 bits.
+constexpr uint32_t ROUND_IDS = 1u << 18;
+constexpr uint32_t WINDOW = 2048;  // blocks whose boundary bits fit one word per lane
+
+// Streams the T lists of up to 64 walk entries through the probe: lane j's
+// list is T[tb, tb + rem) (empty: rem == 0), its neighbour uj, its table the
+// one at byte offset ttab >> 16 with bucket mask ttab & 0xffff (TAILS, the
+// entries of several tails, each with its own table; else P.boff).  The lists
+// are cut into blocks of four ids (16 bytes) and the blocks of all lists
+// numbered through; a step takes 64 consecutive blocks, one per lane,
+// whichever lists they belong to.  A lane finds its list from the bits that
+// mark each list's last block: their number below the lane (two mbcnt) is the
+// list's rank, under which its start and end lie in LDS.  So a step is full
+// whatever the lists' lengths are -- a wave that walked one list at a time
+// left most of its lanes idle on the short lists that most edges have (60 ids
+// on average at R-MAT n = 300,007, 4 M pairs) -- and costs one list's worth
+// of address work.  The next step's blocks are loaded before the current ones
+// are probed.  Hits are counted per lane; a wave scan gives every list's
+// share, which the lanes at the lists' ends add to the list's count in LDS.
+// Returns the hits on lane j's list; `total` receives all of them.
+template <bool HASH, bool TAILS, bool LIST>
+__device__ __forceinline__ uint32_t walk_lists(const uint32_t* __restrict__ T, uint64_t tb, uint64_t rem, uint32_t uj,
+                                               uint32_t ttab, const ProbeCtx& P, PackLds& pk, uint32_t* uid,
+                                               uint64_t& total) {
     const uint32_t lane = lane_id();
-    uint64_t tbj = 0, tej = 0, stl = 0;
-    bool stc = false;
-    if (lane < cnt) {
-        V.entry_bounds(k0 + lane, uj, kw, P.ns, tbj, tej, stl, stc);
-    }
-    const bool nonempty = lane < cnt && tej > tbj;
-    const uint64_t nem = __builtin_amdgcn_ballot_w64(nonempty);
-    const uint32_t nne = (uint32_t)__popcll(nem);
-    {
-        const uint64_t cw = uniform64(wave_sum(stl));
-        wk.wedge += cw;
-        wk.isz += cw + (uint64_t)__popcll(__builtin_amdgcn_ballot_w64(stc)) * nstat;
-        wk.stream_lane += nonempty ? tej - tbj : 0ull;
-    }
-    if (nne == 0) return 0;
-    // order[r] = lane of the r-th non-empty list
-    uint8_t* order = reinterpret_cast<uint8_t*>(pk.marks);
-    if (nonempty) order[__builtin_amdgcn_mbcnt_hi((uint32_t)(nem >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)nem, 0))] =
-        (uint8_t)lane;
-    pk.ucnt[lane] = 0;
-    wave_sync();
-    const uint32_t tb_lo = (uint32_t)tbj, tb_hi = (uint32_t)(tbj >> 32);
-    const uint32_t len32 = (uint32_t)(tej - tbj);  // distinct 32-bit ids: < 2^32
-    const uint32_t* __restrict__ T = V.t_heads();
-    const uint32_t q = lane / G, s4 = 4 * (lane % G);
-    // state of list rank r: source lane, start, length (every lane calls this)
-    auto fetch = [&](uint32_t r, uint32_t& src, const uint32_t*& base, uint32_t& len) {
-        const bool ok = r < nne;
-        src = order[ok ? r : 0];
-        const int a = (int)(src * 4);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(a, (int)tb_lo);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(a, (int)tb_hi);
-        const uint32_t l = (uint32_t)__builtin_amdgcn_ds_bpermute(a, (int)len32);
-        base = T + (((uint64_t)hi << 32) | lo);
-        len = ok ? l : 0u;
-    };
-    uint32_t k = q;  // rank of the group's current list
-    uint32_t csrc, nsrc, clen, nlen;
-    const uint32_t *cbase, *nbase;
-    fetch(k, csrc, cbase, clen);
-    fetch(k + NQ, nsrc, nbase, nlen);
-    uint32_t pos = 0;
-    // every lane loads (lanes past their list's end re-read its start, masked
-    // by `valid`): a static number of loads in flight keeps the prefetch from
-    // being waited for early
-    Ids4 cur = load_ids4(s4 < clen ? cbase + s4 : cbase);
-    uint32_t nh = 0;
-    while (__builtin_amdgcn_ballot_w64(clen != 0)) {
-        // the next block of this group: same list, or its next list
-        const bool same = pos + 4 * G < clen;
-        const uint32_t npos = same ? pos + 4 * G : 0u;
-        const uint32_t* bb = same ? cbase : nbase;
-        const uint32_t bl = same ? clen : nlen;
-        const Ids4 nxt = load_ids4(npos + s4 < bl ? bb + npos + s4 : (bl ? bb : cbase));
-        const int lim = (int)clen - (int)(pos + s4);
-        const bool valid[4] = {0 < lim, 1 < lim, 2 < lim, 3 < lim};
-        const uint32_t w[4] = {cur.x, cur.y, cur.z, cur.w};
-        nh += probe_ids<4>(P.keys, P.cnt, P.ovf, P.boff, P.full, w, valid,
-                           [&](int) { atomicAdd(&pk.ucnt[csrc], 1u); });
-        // advance; a group that switched lists fetches its list after next
-        uint32_t fsrc, flen;
-        const uint32_t* fbase;
-        fetch(same ? k + NQ : k + 2 * NQ, fsrc, fbase, flen);
-        if (!same) {
-            k += NQ;
-            csrc = nsrc;
-            cbase = nbase;
-            clen = nlen;
-            nsrc = fsrc;
-            nbase = fbase;
-            nlen = flen;
+    uint32_t mine = 0;
+    total = 0;
+    while (true) {
+        const uint32_t len = (uint32_t)min<uint64_t>(rem, ROUND_IDS);
+        const uint64_t nem = __builtin_amdgcn_ballot_w64(len != 0);
+        if (nem == 0) break;
+        const uint32_t nb = (len + 3) >> 2;
+        const uint32_t incl = wave_scan_dpp(nb);
+        const uint32_t first = incl - nb;  // the list's first block
+        const uint32_t blocks = readlane32(incl, KT_WAVE - 1);
+        const uint32_t rank = rank_below(nem, 0);
+        const bool bounded = len != 0 && rank != 0;  // a list whose first block ends another's
+        pk.ucnt[lane] = 0;
+        if (len) {
+            const uint64_t t0 = tb - 4ull * first;  // modulo 2^64: + 4 * block is inside the list
+            pk.rec[rank] = uint4{(uint32_t)t0, (uint32_t)(t0 >> 32), len + 4 * first, ttab};
+            if (LIST) uid[rank] = uj;
         }
-        pos = npos;
-        cur = nxt;
+        for (uint32_t w0 = 0; w0 < blocks; w0 += WINDOW) {
+            pk.bits[lane] = 0;
+            wave_sync();
+            const uint32_t at = first - 1 - w0;
+            if (bounded && at < WINDOW) atomicOr(&pk.bits[at >> 5], 1u << (at & 31));
+            wave_sync();
+            const uint32_t bits = pk.bits[lane];
+            uint32_t base = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(bounded && first <= w0));
+            wave_sync();
+            const uint32_t steps = min((blocks - w0 + KT_WAVE - 1) / KT_WAVE, WINDOW / KT_WAVE);
+            // step s: this lane's block, its list's rank and table, its ids'
+            // number (<= 0 past the end)
+            uint64_t ends = 0;
+            uint32_t rk = 0, tt = 0;
+            int lim = 0;
+            Ids4 q;
+            // (s == steps, loaded but not probed: every lane takes the step's
+            // first block, which is in list `base`, or the last block there is)
+            auto load = [&](uint32_t s) {
+                const bool over = s == steps;
+                const int l0 = over ? 0 : (int)(2 * s);
+                ends = over ? 0 : (uint64_t)readlane32(bits, l0) | ((uint64_t)readlane32(bits, l0 + 1) << 32);
+                rk = rank_below(ends, base);
+                base += (uint32_t)__popcll(ends);
+                const uint4 r = pk.rec[rk];
+                const uint32_t p = w0 + s * KT_WAVE + (over ? 0 : lane);
+                lim = (int)r.z - (int)(4 * p);
+                tt = r.w;
+                q = load_ids4(T + ((((uint64_t)r.y << 32) | r.x) + 4ull * min(p, blocks - 1)));
+            };
+            load(0);
+            for (uint32_t s = 0; s < steps; ++s) {
+                const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+                const uint64_t c_ends = ends;
+                const uint32_t c_rk = rk;
+                const uint32_t c_off = TAILS ? tt >> 16 : 0u, c_mask = TAILS ? tt & 0xffffu : P.boff;
+                const int c_lim = s * KT_WAVE + w0 + lane < blocks ? lim : 0;
+                load(s + 1);
+                uint32_t nh = 0;
+                if (HASH) {
+                    if constexpr (LIST) {
+                        const uint32_t u = uid[c_rk];
+                        nh = probe_ids(P.keys, P.cnt, P.ovf, c_off, c_mask, P.full, w, c_lim,
+                                       [&](int e) { P.em(u, w[e]); });
+                    } else {
+                        nh = probe_ids(P.keys, P.cnt, P.ovf, c_off, c_mask, P.full, w, c_lim, NoHitAction{});
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (e >= c_lim) continue;
+                        const uint32_t h = probe_bsearch(P.s, P.ns, P.pv, w[e]);
+                        nh += h;
+                        if (LIST && h) P.em(uid[c_rk], w[e]);
+                    }
+                }
+                if (__builtin_amdgcn_ballot_w64(nh != 0)) {
+                    const uint32_t sum = wave_scan_dpp(nh);
+                    total += readlane32(sum, KT_WAVE - 1);
+                    const bool end = (c_ends >> lane) & 1;
+                    if (end || lane == KT_WAVE - 1) atomicAdd(&pk.ucnt[c_rk], sum);
+                    if (end && lane != KT_WAVE - 1) atomicSub(&pk.ucnt[c_rk + 1], sum);
+                }
+            }
+            wave_sync();
+        }
+        if (len) mine += pk.ucnt[rank];
+        wave_sync();
+        tb += len;
+        rem -= len;
     }
-    wave_sync();
-    const uint32_t h = lane < cnt ? pk.ucnt[lane] : 0u;
-    if (h && P.pv) atomic_add_u64(&P.pv[uj], h);
-    return wave_total_dpp(nh);
+    return mine;
 }
 
 // Bounds of a tail's S and R ranges and its counter length.
 struct TailBounds {
-    uint64_t sb, se, rb, re, nstat;
+    uint64_t sb, rb;
+    uint32_t ns, nr;  // lists hold distinct 32-bit ids
+    uint32_t nstat;
 };
 
 template <bool PLAIN>
 __device__ __forceinline__ TailBounds tail_bounds(const View<PLAIN>& V, uint32_t x) {
     TailBounds t;
-    V.s_range(x, t.sb, t.se);
-    V.r_range(x, t.rb, t.re);
-    t.nstat = V.stat_len(x, t.se - t.sb);
+    uint64_t e;
+    V.s_range(x, t.sb, e);
+    t.ns = (uint32_t)(e - t.sb);
+    V.r_range(x, t.rb, e);
+    t.nr = (uint32_t)(e - t.rb);
+    t.nstat = (uint32_t)V.stat_len(x, t.ns);
+    return t;
+}
+
+// Bounds of part `part` (of `split` walk entries) of tail x.
+template <bool PLAIN>
+__device__ __forceinline__ TailBounds part_bounds(const View<PLAIN>& V, uint32_t x, uint32_t part, uint32_t split) {
+    TailBounds t = tail_bounds(V, x);
+    t.rb += (uint64_t)part * split;
+    t.nr = min(split, t.nr - part * split);
     return t;
 }
 
 // Process tail x, whose bounds are tb, with a team of NW waves (NW == 1:
-// this wave alone).
-template <int NW, bool HASH, bool PLAIN, int GL, bool LIST, class LdsT>
+// this wave alone); KS: the most ids of S(x) per thread.
+template <int NW, int KS, bool HASH, bool PLAIN, bool LIST, class LdsT>
 __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, const TailBounds& tb, LdsT& L,
                                              uint32_t* keys, uint32_t* cnt, uint32_t* ovf, uint32_t cap_slots,
                                              uint32_t shift, uint32_t chunk, const TcOut& out,
-                                             uint64_t& my_total, WorkStats& wk) {
+                                             uint64_t& my_total, WorkStats& wk, uint32_t* uid) {
     const unsigned lane = lane_id();
     const unsigned wave = threadIdx.x / KT_WAVE;
     const unsigned twave = NW > 1 ? wave : 0;
     const unsigned tid = twave * KT_WAVE + lane;
 
-    const uint64_t sb = uniform64(tb.sb), se = uniform64(tb.se);
-    const uint64_t rb = uniform64(tb.rb), re = uniform64(tb.re);
-    const uint64_t ns = se - sb, nr = re - rb;
-    const uint64_t nstat = uniform64(tb.nstat);
+    const uint64_t sb = uniform64(tb.sb), rb = uniform64(tb.rb);
+    const uint32_t ns = uniform(tb.ns), nr = uniform(tb.nr), nstat = uniform(tb.nstat);
+    // every wave of the team gets at least two grabs where the walk allows
+    if (NW > 1) chunk = min(chunk, max(1u, (nr + 2 * NW - 1) / (2 * NW)));
     // The first chunk's neighbours are loaded before the tail's table is
-    // built (clearing it and inserting S(x) hide the round trip); every later
-    // chunk's neighbours are loaded while the chunk before it is scanned (the
-    // bounds of their T lists depend on them).
-    uint64_t k = (uint64_t)twave * chunk;
+    // built (inserting S(x) hides the round trip); every later chunk's
+    // neighbours are loaded while the chunk before it is scanned (the bounds
+    // of their T lists depend on them).
+    uint32_t k = twave * chunk;
     uint32_t u_nx = 0, kw_nx = 0;
-    if (k < nr && lane < min<uint64_t>(chunk, nr - k)) V.entry_head(rb + k + lane, u_nx, kw_nx);
+    if (k < nr && lane < min(chunk, nr - k)) V.entry_head(rb + k + lane, u_nx, kw_nx);
 
     ProbeCtx P;
     P.keys = keys;
@@ -793,31 +761,19 @@ __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, c
     P.s = V.v.sheads + sb;
     P.ns = ns;
     P.pv = out.per_vertex;
-    uint32_t slots = 0;
+    uint32_t slot[(KS + 1) / 2] = {};  // where this thread's ids of S(x) are (byte offsets, two per word)
     if (HASH) {
-        uint32_t logS = ceil_log2(ns << shift);  // load <= 2^-shift unless capped
-        if (logS < MIN_LOGS) logS = MIN_LOGS;
-        slots = 1u << logS;
-        if (slots > cap_slots) {  // bins guarantee cap_slots >= 2 * ns
-            slots = cap_slots;
-            logS = ceil_log2(cap_slots);
-        }
-        P.boff = ((slots >> 2) - 1) << 4;
-        for (uint32_t i = tid; i < slots; i += NW * KT_WAVE) {
-            keys[i] = KT_EMPTY;
-            cnt[i] = 0;
-        }
-        for (uint32_t i = tid; i < (slots + 127) / 128; i += NW * KT_WAVE) ovf[i] = 0;  // one bit per 4-slot bucket
-        team_sync<NW>();
+        uint32_t logS = max(ceil_log2((uint64_t)ns << shift), MIN_LOGS);  // load <= 2^-shift unless capped
+        logS = min(logS, 31u - (uint32_t)__clz(cap_slots));               // bins guarantee cap_slots >= 2 * ns
+        P.boff = ((1u << logS >> 2) - 1) << 4;
         bool full = false;
-        for (uint64_t i = tid; i < ns; i += NW * KT_WAVE)
-            full |= table_insert(keys, ovf, P.boff, V.v.sheads[sb + i]);
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            const uint32_t i = tid + j * NW * KT_WAVE;
+            if (i < ns) slot[j / 2] |= table_insert(keys, ovf, 0, P.boff, P.s[i], full) << (16 * (j & 1));
+        }
         if (NW > 1) {
-            if (tid == 0) L.full = 0;
-            team_sync<NW>();
-            if (__builtin_amdgcn_ballot_w64(full) && lane == 0) atomicOr(&L.full, 1u);
-            team_sync<NW>();
-            P.full = uniform(L.full) != 0;
+            if (full) L.full = 1;
         } else {
             P.full = __builtin_amdgcn_ballot_w64(full) != 0;
         }
@@ -828,12 +784,13 @@ __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, c
         if (tid == 0) *P.em.ctr = 0;
     }
     team_sync<NW>();
+    if (HASH && NW > 1) P.full = uniform(L.full) != 0;
 
-    uint64_t tail_hits = 0;
+    uint64_t hsum = 0;  // wave-uniform
     while (k < nr) {
-        const uint32_t c = (uint32_t)min<uint64_t>(chunk, nr - k);
-        const uint32_t u_cur = u_nx, kw_cur = kw_nx;
-        uint64_t nk;
+        const uint32_t c = min(chunk, nr - k);
+        const uint32_t u = u_nx, kw = kw_nx;
+        uint32_t nk;
         if (NW > 1) {
             uint32_t g = 0;
             if (lane == 0) g = atomicAdd(&L.next_u, chunk);
@@ -841,16 +798,22 @@ __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, c
         } else {
             nk = k + chunk;
         }
-        if (nk < nr && lane < min<uint64_t>(chunk, nr - nk)) V.entry_head(rb + nk + lane, u_nx, kw_nx);
-        if (GL < KT_WAVE && HASH)
-            tail_hits += scan_chunk_grouped<GL, PLAIN>(V, rb + k, c, u_cur, kw_cur, P, nstat, wk, L.pk[wave]);
-        else
-            tail_hits += scan_chunk<HASH, PLAIN, LIST>(V, rb + k, c, u_cur, kw_cur, P, nstat, wk);
+        if (nk < nr && lane < min(chunk, nr - nk)) V.entry_head(rb + nk + lane, u_nx, kw_nx);
+        uint64_t b = 0, e = 0, stl = 0;
+        bool stc = false;
+        if (lane < c) V.entry_bounds(rb + k + lane, u, kw, ns, b, e, stl, stc);
+        const uint64_t len = e > b ? e - b : 0;
+        wk.wedge_lane += stl;
+        wk.recv_lane += stc ? nstat : 0u;
+        wk.stream_lane += len;
+        uint64_t hits;
+        const uint32_t h = walk_lists<HASH, false, LIST>(V.t_heads(), b, len, u, 0, P, L.pk[wave], uid, hits);
+        if (h && P.pv) atomic_add_u64(&P.pv[u], h);
+        hsum += hits;
         k = nk;
     }
 
     // team reduction of the tail's hits
-    uint64_t hsum = tail_hits;  // wave-uniform
     if (NW > 1) {
         if (lane == 0) L.red[wave] = hsum;
         __syncthreads();
@@ -859,119 +822,316 @@ __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, c
         for (int i = 0; i < NW; ++i) hsum += L.red[i];
     }
     if (HASH) {
-        team_sync<NW>();
-        if (out.per_vertex) {
-            for (uint32_t i = tid; i < slots; i += NW * KT_WAVE) {
-                uint32_t c = cnt[i];
-                if (c) atomic_add_u64(&out.per_vertex[keys[i]], c);
+        if (NW == 1) wave_sync();
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            if (tid + j * NW * KT_WAVE >= ns) break;
+            const uint32_t o = (slot[j / 2] >> (16 * (j & 1))) & 0xffffu;
+            const uint32_t c = *at_byte(cnt, o);
+            if (c) {
+                if (P.pv) atomic_add_u64(&P.pv[*at_byte(keys, o)], c);
+                *at_byte(cnt, o) = 0;
             }
+            *at_byte(keys, o) = KT_EMPTY;
         }
+        if (P.full)
+            for (uint32_t i = tid; i < (P.boff >> 9) + 1; i += NW * KT_WAVE) ovf[i] = 0;
+        if (NW > 1 && tid == 0) L.full = 0;  // read by every wave before the walk
     }
     if (tid == 0 && out.tail_count) out.tail_count[x] = hsum;
     if (tid == 0 && hsum) {
-        if (out.per_vertex) atomic_add_u64(&out.per_vertex[V.tail_pv(x)], hsum);
-        if (V.v.tail_graph)
-            atomic_add_u64(&out.totals[V.tail_graph(x)], hsum);
-        else
-            my_total += hsum;
+        if (P.pv) atomic_add_u64(&P.pv[V.tail_pv(x)], hsum);
+        my_total += hsum;
     }
     team_sync<NW>();  // table reuse by the next tail
 }
 
-// Streamed walks fit 64 VGPRs (8 waves per SIMD, four workgroups per CU);
-// grouped walks keep more list state per lane and get 80 VGPRs (6 waves per
-// SIMD), which keeps their step loop free of register spills.
-template <bool PLAIN, int GL, bool LIST>
-__global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu(GL < KT_WAVE ? 6 : 8, 8))) k_tc_main(View<PLAIN> V, TcOut out, TcParams prm,
+// Tails that a wave takes several at a time: at most 64 ids in S(x) and 64
+// walk entries, so that the entries and set members of a few such tails fill
+// one wave.  (One by one, each tail of R-MAT or G(n, m) -- 16 to 36 entries on
+// average -- cost the wave a chain of six dependent round trips with most of
+// its lanes idle: 12-19 us.)
+constexpr uint32_t PACK_MAX = KT_WAVE;
+
+__device__ __forceinline__ uint32_t pack_slots(uint32_t ns) {  // load 1/8 to 1/4
+    return 1u << max(ceil_log2(4ull * ns), 4u);
+}
+
+// Tails of lanes [j0, j0 + n) of a grab (tail xl with bounds bl; er / es / et
+// = its walk entries, set members and table slots below the pack's first).
+template <bool PLAIN>
+__device__ __forceinline__ void pack_process(const View<PLAIN>& V, uint32_t xl, const TailBounds& bl, uint32_t er,
+                                             uint32_t es, uint32_t et, uint32_t j0, uint32_t n, uint32_t nR,
+                                             uint32_t nS, PackLds& pk, uint32_t* keys, uint32_t* cnt, uint32_t* ovf,
+                                             const TcOut& out, uint64_t& my_total, WorkStats& wk) {
+    const uint32_t lane = lane_id();
+    // which tail a lane's entry / set member belongs to, from the bits at the
+    // tails' last ones
+    pk.bits[lane] = 0;
+    wave_sync();
+    if (lane > j0 && lane < j0 + n) {
+        atomicOr(&pk.bits[(er - 1) >> 5], 1u << ((er - 1) & 31));
+        atomicOr(&pk.bits[2 + ((es - 1) >> 5)], 1u << ((es - 1) & 31));
+    }
+    wave_sync();
+    const uint32_t word = pk.bits[lane];
+    wave_sync();
+    const uint64_t mr = (uint64_t)readlane32(word, 0) | ((uint64_t)readlane32(word, 1) << 32);
+    const uint64_t ms = (uint64_t)readlane32(word, 2) | ((uint64_t)readlane32(word, 3) << 32);
+    const uint32_t tr = j0 + rank_below(mr, 0), ts = j0 + rank_below(ms, 0);
+    const uint32_t tab = (4 * et << 16) | (((pack_slots(bl.ns) >> 2) - 1) << 4);
+    // set members and walk entries
+    const uint64_t si = from_lane64(bl.sb - es, ts) + lane;
+    const uint64_t ri = from_lane64(bl.rb - er, tr) + lane;
+    const uint32_t stab = from_lane(tab, ts), rtab = from_lane(tab, tr);
+    const uint32_t rns = from_lane(bl.ns, tr), rstat = PLAIN ? rns : from_lane(bl.nstat, tr);
+    uint32_t id = 0, u = 0, kw = 0;
+    if (lane < nS) id = V.v.sheads[si];
+    if (lane < nR) V.entry_head(ri, u, kw);
+    uint32_t slot = 0;
+    bool moved = false;
+    if (lane < nS) slot = table_insert(keys, ovf, stab >> 16, stab & 0xffffu, id, moved);
+    ProbeCtx P;
+    P.keys = keys;
+    P.cnt = cnt;
+    P.ovf = ovf;
+    P.boff = 0;
+    P.full = __builtin_amdgcn_ballot_w64(moved) != 0;
+    P.pv = out.per_vertex;
+    uint64_t b = 0, e = 0, stl = 0;
+    bool stc = false;
+    if (lane < nR) V.entry_bounds(ri, u, kw, rns, b, e, stl, stc);
+    const uint64_t len = e > b ? e - b : 0;
+    wk.wedge_lane += stl;
+    wk.recv_lane += stc ? rstat : 0u;
+    wk.stream_lane += len;
+    uint64_t hits;
+    const uint32_t h = walk_lists<true, true, false>(V.t_heads(), b, len, u, rtab, P, pk, nullptr, hits);
+    if (hits) {
+        my_total += hits;
+        if (P.pv) {
+            if (h) atomic_add_u64(&P.pv[u], h);
+            const uint32_t sum = wave_scan_dpp(h);
+            const uint32_t last = from_lane(sum, er + bl.nr - 1), before = from_lane(sum, er - 1);
+            const uint32_t th = last - (lane > j0 ? before : 0u);
+            if (lane >= j0 && lane < j0 + n && th) atomic_add_u64(&P.pv[V.tail_pv(xl)], th);
+        }
+    }
+    if (lane < nS) {
+        const uint32_t c = *at_byte(cnt, slot);
+        if (c) {
+            if (P.pv) atomic_add_u64(&P.pv[id], c);
+            *at_byte(cnt, slot) = 0;
+        }
+        *at_byte(keys, slot) = KT_EMPTY;
+    }
+    if (P.full && lane < WAVE_SLOTS / 128) ovf[lane] = 0;
+    wave_sync();
+}
+
+// A run of the tail list.
+struct Segment {
+    uint32_t base, cnt;
+};
+
+// How a segment is shared out without a queue access: an atomic on one word
+// that many XCDs update costs 50-100 ns, one after the other (with every tail
+// taken from a queue, R-MAT n = 300,007 with 4 M pairs spent 1.2 of its
+// 1.4 ms on them), so the first items go to the workgroups in turn.  `whole`:
+// the segment is shared by the grid, starting at workgroup rot, else by the
+// workgroups of XCD sx.
+struct Shares {
+    uint32_t first, blocks;
+    bool mine;
+    __device__ __forceinline__ Shares(uint32_t cnt, bool whole, uint32_t sx, uint32_t rot) {
+        whole = whole || cnt < 4 * gridDim.x;  // too few for the XCD's own caches to matter
+        if (whole) {
+            blocks = gridDim.x;
+            first = (blockIdx.x + blocks - rot % blocks) % blocks;
+            mine = true;
+        } else {
+            blocks = (gridDim.x + NXCD - 1 - sx) / NXCD;
+            first = blockIdx.x / NXCD;
+            mine = blockIdx.x % NXCD == sx;
+        }
+    }
+};
+
+// 80 VGPRs and 43 KB of LDS: three workgroups per CU, 6 waves per SIMD.
+template <bool PLAIN, bool LIST>
+__global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) k_tc_main(View<PLAIN> V, TcOut out, TcParams prm,
                                                          uint32_t* __restrict__ q,
                                                          const uint32_t* __restrict__ list,
+                                                         const uint64_t* __restrict__ plist,
                                                          uint64_t* __restrict__ stats) {
     __shared__ Lds L;
+    __shared__ uint32_t uids[LIST ? TC_THREADS : 1];  // a listing's neighbours, per wave
     const unsigned wave = threadIdx.x / KT_WAVE;
     const unsigned lane = lane_id();
+    uint32_t* uid = uids + (LIST ? wave * KT_WAVE : 0);
     uint64_t my_total = 0;
     WorkStats wk;
     const int wave_bucket_max = (int)ceil_log2(prm.wave_max_deg);
 
+    // Every bucket's count and place in the list, read once.
+    if (wave == 0) {
+        const uint32_t c = lane < (unsigned)NBUCKET ? q[Q_CNT + lane] : 0u;
+        if (lane < (unsigned)NBUCKET) {
+            L.qcnt[lane] = c;
+            L.qctr[lane] = 0;
+        }
+        uint32_t base = 0;
+        for (int i = 0; i < NBUCKET; ++i) {
+            const uint32_t ci = readlane32(c, i);
+            const bool same = (i < NLIST) == (lane < (unsigned)NLIST);
+            base += (same && (i < NLIST ? i > (int)lane : i < (int)lane)) ? ci : 0u;
+        }
+        if (lane < (unsigned)NBUCKET) L.qbase[lane] = base;
+    }
+    for (uint32_t i = threadIdx.x; i < GROUP_SLOTS; i += TC_THREADS) {
+        L.keys[i] = KT_EMPTY;
+        L.cnt[i] = 0;
+    }
+    if (threadIdx.x < GROUP_SLOTS / 128) L.ovf[threadIdx.x] = 0;
+    if (threadIdx.x == 0) L.full = 0;
+    __syncthreads();
     const bool by_vertex = prm.order == TC_BY_VERTEX;
-    const int xcd = (int)(blockIdx.x % NXCD);
-    // team phase: by degree, the workgroup-bin buckets from the largest down;
-    // by vertex, this XCD's workgroup tails first, then the other XCDs'
-    const int team_hi = by_vertex ? NXCD - 1 : BUCKET_HUGE - 1;
-    const int team_lo = by_vertex ? 0 : wave_bucket_max + 1;
-    for (int k = team_hi; k >= team_lo; --k) {
-        const int b = by_vertex ? (xcd + NXCD - 1 - k) % NXCD : k;
-        const uint32_t cnt = q[Q_CNT + b];
-        if (cnt == 0) continue;
-        const uint32_t base = bucket_base(q, b);
-        uint32_t* pull = &q[Q_PULL + Q_STRIDE * b];
+    const uint32_t xcd = blockIdx.x % NXCD;
+    // Shares of a segment start where those of the one before ended (by
+    // vertex, where the order of the segments differs per XCD: an eighth of the
+    // grid further per XCD), so that every workgroup gets as many.
+    const uint32_t team_parts = L.qcnt[BUCKET_TEAM_PARTS], wave_parts = L.qcnt[BUCKET_WAVE_PARTS];
+    // team phase: the parts of long walks, then, by degree, the workgroup
+    // tails from the largest down (one segment); by vertex, this XCD's
+    // workgroup tails first, then the other XCDs'
+    for (uint32_t k = 0; k <= (by_vertex ? NXCD : 1u); ++k) {
+        const bool parts = k == 0;
+        const uint32_t sx = (xcd + k - 1) % NXCD;  // by vertex: the segment's XCD
+        const Segment sg = parts       ? Segment{L.qbase[BUCKET_TEAM_PARTS], L.qcnt[BUCKET_TEAM_PARTS]}
+                           : by_vertex ? Segment{L.qbase[sx], L.qcnt[sx]}
+                                       : Segment{L.qbase[BUCKET_HUGE - 1],
+                                                 L.qbase[wave_bucket_max] - L.qbase[BUCKET_HUGE - 1]};
+        if (sg.cnt == 0) continue;
+        const Shares sh(sg.cnt, parts || !by_vertex, sx, parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : team_parts);
+        uint32_t* pull = &q[Q_PULL + Q_STRIDE * (parts ? BUCKET_TEAM_PARTS : by_vertex ? (int)sx : 0)];
+        const uint32_t fixed = sg.cnt <= 4 * sh.blocks ? sg.cnt : sh.blocks;
+        uint32_t i = sh.mine ? sh.first : fixed;
         while (true) {
-            if (threadIdx.x == 0)
-                L.bcast = (__hip_atomic_load(pull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= cnt)
-                              ? cnt
-                              : atomicAdd(pull, 1u);
-            __syncthreads();
-            const uint32_t i = L.bcast;
-            __syncthreads();
-            if (i >= cnt) break;
-            const uint32_t x = list[base + i];
-            team_process<TC_WAVES, true, PLAIN, GL, LIST>(V, x, tail_bounds(V, x), L, L.keys, L.cnt, L.ovf, GROUP_SLOTS,
-                                                          prm.table_shift, prm.team_chunk, out, my_total, wk);
+            if (i >= fixed) {
+                if (fixed == sg.cnt) break;
+                if (threadIdx.x == 0)
+                    L.bcast = (__hip_atomic_load(pull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= sg.cnt - fixed)
+                                  ? sg.cnt
+                                  : fixed + atomicAdd(pull, 1u);
+                __syncthreads();
+                i = L.bcast;
+                __syncthreads();
+                if (i >= sg.cnt) break;
+            }
+            const uint64_t xp = parts ? plist[sg.base + i] : list[sg.base + i];
+            const uint32_t x = (uint32_t)xp;
+            const TailBounds tb =
+                parts ? part_bounds(V, x, (uint32_t)(xp >> 32), prm.team_split) : tail_bounds(V, x);
+            team_process<TC_WAVES, GROUP_SLOTS / 2 / TC_THREADS, true, PLAIN, LIST>(V, x, tb, L, L.keys, L.cnt, L.ovf, GROUP_SLOTS,
+                                                          prm.table_shift, prm.team_chunk, out, my_total, wk, uid);
+            i = i < fixed ? i + sh.blocks : fixed;
         }
     }
-    // wave phase: independent waves with private tables; by degree, largest
-    // buckets first; by vertex, this XCD's wave tails first
+    // wave phase: independent waves with private tables, the same segments.
+    // A wave takes `grab` tails at a time: first the blocks of its
+    // workgroup's share (handed out by an LDS counter), then, where a wave
+    // gets many, the second half of the segment from its queue.
     {
         uint32_t* keys = L.keys + wave * WAVE_SLOTS;
         uint32_t* tcnt = L.cnt + wave * WAVE_SLOTS;
-        const int wave_hi = by_vertex ? NXCD - 1 : wave_bucket_max;
-        for (int k = wave_hi; k >= 0; --k) {
-            const int b = by_vertex ? NXCD + (xcd + NXCD - 1 - k) % NXCD : k;
-            const uint32_t cnt = q[Q_CNT + b];
-            if (cnt == 0) continue;
-            const uint32_t base = bucket_base(q, b);
-            uint32_t* pull = &q[Q_PULL + Q_STRIDE * b];
-            // more tails per grab for the small buckets (less queue traffic);
-            // in vertex order, the grab set per launch
-            const uint32_t grab = by_vertex ? min(max(prm.wave_grab, 1u), (uint32_t)KT_WAVE)
-                                            : (b <= 3 ? 4 * WAVE_GRAB : (b <= 5 ? 2 * WAVE_GRAB : WAVE_GRAB));
+        uint32_t* wovf = L.ovf + wave * (WAVE_SLOTS / 128);
+        for (uint32_t k = 0; k <= (by_vertex ? NXCD : 1u); ++k) {
+            const bool parts = k == 0;
+            const uint32_t sx = (xcd + k - 1) % NXCD;
+            const Segment sg = parts       ? Segment{L.qbase[BUCKET_WAVE_PARTS], L.qcnt[BUCKET_WAVE_PARTS]}
+                               : by_vertex ? Segment{L.qbase[NXCD + sx], L.qcnt[NXCD + sx]}
+                                           : Segment{L.qbase[wave_bucket_max],
+                                                     L.qbase[0] + L.qcnt[0] - L.qbase[wave_bucket_max]};
+            if (sg.cnt == 0) continue;
+            const Shares sh(sg.cnt, parts || !by_vertex, sx,
+                            parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : wave_parts);
+            const uint32_t most = parts ? 4u : min(max(prm.wave_grab, 1u), (uint32_t)KT_WAVE);
+            const uint32_t grab = max(1u, min(most, sg.cnt / (2 * TC_WAVES * sh.blocks)));
+            const uint32_t grabs = (sg.cnt + grab - 1) / grab;
+            const uint32_t fixed = grabs <= 8 * TC_WAVES * sh.blocks ? grabs : grabs / 2;
+            uint32_t* pull = &q[Q_PULL + Q_STRIDE * (parts ? BUCKET_WAVE_PARTS : by_vertex ? (int)(NXCD + sx) : 1)];
+            uint32_t* ctr = &L.qctr[parts ? BUCKET_WAVE_PARTS : by_vertex ? NXCD + sx : 1];
+            bool own = sh.mine;
             while (true) {
-                uint32_t i = 0;
-                if (lane == 0)
-                    i = (__hip_atomic_load(pull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= cnt)
-                            ? cnt
-                            : atomicAdd(pull, grab);
-                i = uniform(i);
-                if (i >= cnt) break;
+                uint32_t g = 0;
+                if (own) {
+                    if (lane == 0) g = sh.first + atomicAdd(ctr, 1u) * sh.blocks;
+                    g = uniform(g);
+                    own = g < fixed;
+                }
+                if (!own) {
+                    if (fixed == grabs) break;
+                    if (lane == 0)
+                        g = (__hip_atomic_load(pull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= grabs - fixed)
+                                ? grabs
+                                : fixed + atomicAdd(pull, 1u);
+                    g = uniform(g);
+                    if (g >= grabs) break;
+                }
                 // the grabbed tails (grab <= 64) and their bounds, loaded by
                 // one lane each before the first is processed: one round
                 // trip for the batch instead of two per tail
-                const uint32_t ng = min(cnt, i + grab) - i;
+                const uint32_t i = g * grab;
+                const uint32_t ng = min(sg.cnt, i + grab) - i;
                 uint32_t xl = 0;
                 TailBounds bl{0, 0, 0, 0, 0};
                 if (lane < ng) {
-                    xl = list[base + i + lane];
-                    bl = tail_bounds(V, xl);
+                    if (parts) {
+                        const uint64_t xp = plist[sg.base + i + lane];
+                        xl = (uint32_t)xp;
+                        bl = part_bounds(V, xl, (uint32_t)(xp >> 32), prm.wave_split);
+                    } else {
+                        xl = list[sg.base + i + lane];
+                        bl = tail_bounds(V, xl);
+                    }
                 }
-                for (uint32_t j = 0; j < ng; ++j) {
-                    const TailBounds tb{readlane64(bl.sb, j), readlane64(bl.se, j), readlane64(bl.rb, j),
-                                        readlane64(bl.re, j), readlane64(bl.nstat, j)};
-                    team_process<1, true, PLAIN, GL, LIST>(V, readlane32(xl, j), tb, L, keys, tcnt,
-                                                           L.ovf + wave * (WAVE_SLOTS / 128), WAVE_SLOTS,
-                                                           prm.table_shift, KT_WAVE, out, my_total, wk);
+                // Consecutive small tails are taken together while their
+                // entries, set members and tables fit the wave.
+                const bool small = !LIST && !out.tail_count && lane < ng && bl.nr <= PACK_MAX && bl.ns <= PACK_MAX;
+                const uint32_t sr = wave_scan_dpp(small ? bl.nr : 0u), ss = wave_scan_dpp(small ? bl.ns : 0u),
+                               st = wave_scan_dpp(small ? pack_slots(bl.ns) : 0u);
+                for (uint32_t j = 0; j < ng;) {
+                    const uint32_t br = j ? readlane32(sr, j - 1) : 0u, bs = j ? readlane32(ss, j - 1) : 0u,
+                                   bt = j ? readlane32(st, j - 1) : 0u;
+                    const bool fits = small && sr - br <= KT_WAVE && ss - bs <= KT_WAVE && st - bt <= WAVE_SLOTS;
+                    const uint64_t run = __builtin_amdgcn_ballot_w64(fits) >> j;
+                    if (run & 1) {
+                        const uint32_t n = run == ~0ull ? KT_WAVE : (uint32_t)__builtin_ctzll(~run);
+                        pack_process(V, xl, bl, sr - bl.nr - br, ss - bl.ns - bs, st - pack_slots(bl.ns) - bt, j, n,
+                                     readlane32(sr, j + n - 1) - br, readlane32(ss, j + n - 1) - bs, L.pk[wave], keys,
+                                     tcnt, wovf, out, my_total, wk);
+                        j += n;
+                    } else {
+                        const TailBounds tb{readlane64(bl.sb, j), readlane64(bl.rb, j), readlane32(bl.ns, j),
+                                            readlane32(bl.nr, j), readlane32(bl.nstat, j)};
+                        team_process<1, WAVE_SLOTS / 2 / KT_WAVE, true, PLAIN, LIST>(
+                            V, readlane32(xl, j), tb, L, keys, tcnt, wovf, WAVE_SLOTS, prm.table_shift, KT_WAVE, out,
+                            my_total, wk, uid);
+                        ++j;
+                    }
                 }
             }
         }
     }
     // flush the wave-uniform accumulators: one atomic per workgroup and counter
-    const uint64_t streamed = wk.streamed();
+    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), isz = wedge + wk.recv();
     __syncthreads();
     if (lane == 0) {
         L.red[wave] = my_total;
-        L.keys[wave] = (uint32_t)wk.wedge;
-        L.keys[TC_WAVES + wave] = (uint32_t)(wk.wedge >> 32);
-        L.cnt[wave] = (uint32_t)wk.isz;
-        L.cnt[TC_WAVES + wave] = (uint32_t)(wk.isz >> 32);
+        L.keys[wave] = (uint32_t)wedge;
+        L.keys[TC_WAVES + wave] = (uint32_t)(wedge >> 32);
+        L.cnt[wave] = (uint32_t)isz;
+        L.cnt[TC_WAVES + wave] = (uint32_t)(isz >> 32);
         L.keys[2 * TC_WAVES + wave] = (uint32_t)streamed;
         L.keys[3 * TC_WAVES + wave] = (uint32_t)(streamed >> 32);
     }
@@ -999,6 +1159,8 @@ __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out
                                                          const uint32_t* __restrict__ list,
                                                          uint64_t* __restrict__ stats) {
     __shared__ Lds L;
+    __shared__ uint32_t uids[LIST ? TC_THREADS : 1];
+    uint32_t* uid = uids + (LIST ? threadIdx.x / KT_WAVE * KT_WAVE : 0);
     uint64_t my_total = 0;
     WorkStats wk;
     const uint32_t cnt = q[Q_CNT + BUCKET_HUGE];
@@ -1014,14 +1176,14 @@ __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out
         __syncthreads();
         if (i >= cnt) break;
         const uint32_t x = list[base + i];
-        team_process<TC_WAVES, false, PLAIN, KT_WAVE, LIST>(V, x, tail_bounds(V, x), L, nullptr, nullptr, nullptr, 0, 0,
-                                                            prm.team_chunk, out, my_total, wk);
+        team_process<TC_WAVES, 1, false, PLAIN, LIST>(V, x, tail_bounds(V, x), L, nullptr, nullptr, nullptr, 0, 0,
+                                                            prm.team_chunk, out, my_total, wk, uid);
     }
-    const uint64_t streamed = wk.streamed();
+    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), isz = wedge + wk.recv();
     if (lane_id() == 0) {
         if (my_total) atomic_add_u64(&out.totals[0], my_total);
-        if (wk.wedge) atomic_add_u64(&stats[ST_WEDGE], wk.wedge);
-        if (wk.isz) atomic_add_u64(&stats[ST_ISZ], wk.isz);
+        if (wedge) atomic_add_u64(&stats[ST_WEDGE], wedge);
+        if (isz) atomic_add_u64(&stats[ST_ISZ], isz);
         if (streamed) atomic_add_u64(&stats[ST_STREAM], streamed);
     }
 }
@@ -1034,7 +1196,16 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
                                                         uint32_t* __restrict__ q, const uint32_t* __restrict__ list,
                                                         uint64_t* __restrict__ stats) {
     __shared__ LdsBig L;
+    __shared__ uint32_t uids[LIST ? BIG_THREADS : 1];
+    uint32_t* uid = uids + (LIST ? threadIdx.x / KT_WAVE * KT_WAVE : 0);
     extern __shared__ uint32_t big_table[];  // keys[BIG_SLOTS], then cnt[BIG_SLOTS]
+    if (q[Q_CNT + BUCKET_BIG] == 0) return;
+    for (uint32_t i = threadIdx.x; i < BIG_SLOTS; i += BIG_THREADS) {
+        big_table[i] = KT_EMPTY;
+        big_table[BIG_SLOTS + i] = 0;
+    }
+    if (threadIdx.x < BIG_SLOTS / 128) L.ovf[threadIdx.x] = 0;
+    if (threadIdx.x == 0) L.full = 0;
     uint64_t my_total = 0;
     WorkStats wk;
     const uint32_t cnt = q[Q_CNT + BUCKET_BIG];
@@ -1050,15 +1221,15 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
         __syncthreads();
         if (i >= cnt) break;
         const uint32_t x = list[base + i];
-        team_process<BIG_WAVES, true, PLAIN, KT_WAVE, LIST>(V, x, tail_bounds(V, x), L, big_table,
+        team_process<BIG_WAVES, BIG_SLOTS / 2 / BIG_THREADS, true, PLAIN, LIST>(V, x, tail_bounds(V, x), L, big_table,
                                                             big_table + BIG_SLOTS, L.ovf, BIG_SLOTS, prm.table_shift,
-                                                            prm.team_chunk, out, my_total, wk);
+                                                            prm.team_chunk, out, my_total, wk, uid);
     }
-    const uint64_t streamed = wk.streamed();
+    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), isz = wedge + wk.recv();
     if (lane_id() == 0) {
         if (my_total) atomic_add_u64(&out.totals[0], my_total);
-        if (wk.wedge) atomic_add_u64(&stats[ST_WEDGE], wk.wedge);
-        if (wk.isz) atomic_add_u64(&stats[ST_ISZ], wk.isz);
+        if (wedge) atomic_add_u64(&stats[ST_WEDGE], wedge);
+        if (isz) atomic_add_u64(&stats[ST_ISZ], isz);
         if (streamed) atomic_add_u64(&stats[ST_STREAM], streamed);
     }
 }
@@ -1066,9 +1237,32 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-uint64_t tc_ws_words(uint32_t X) {
-    // queue header (u32) + stats (u64) + one u32 list of X
-    return Q_WORDS / 2 + ST_WORDS + (uint64_t(X) + 1) / 2 + 1;
+// Walk entries per part: tails with longer walks are split, so that a few
+// long rows (an R-MAT hub's row has a large share of all entries) do not
+// leave the rest of the chip waiting for the team that drew them.
+struct Split {
+    uint32_t wave, team;
+};
+
+static Split split_rule(uint64_t entries, int num_cus) {
+    const uint64_t teams = (uint64_t)num_cus * 3, waves = teams * TC_WAVES;
+    auto size = [](uint64_t want, uint64_t lo, uint64_t hi) {
+        uint64_t p = lo;
+        while (p < want && p < hi) p <<= 1;
+        return (uint32_t)p;
+    };
+    return {size(entries / (2 * waves), 16, 1024), size(entries / (4 * teams), 128, 4096)};
+}
+
+// A walk of r > split entries becomes ceil(r / split) <= 2 r / split parts.
+static uint64_t max_parts(uint64_t entries, const Split& s) {
+    return 2 * entries / s.team + (s.wave < 1024 ? 2 * entries / s.wave : 0);
+}
+
+uint64_t tc_ws_words(uint32_t X, uint64_t entries, int num_cus) {
+    // queue header (u32) + stats (u64) + one u32 list of X + the part list
+    return Q_WORDS / 2 + ST_WORDS + (uint64_t(X) + 1) / 2 + 1 +
+           (entries ? max_parts(entries, split_rule(entries, num_cus)) : 0);
 }
 
 uint64_t* tc_stats_ptr(uint64_t* ws) { return ws + Q_WORDS / 2; }
@@ -1085,6 +1279,7 @@ static hipError_t launch_impl(const TcView& view, const TcOut& out, const TcPara
     uint32_t* q = reinterpret_cast<uint32_t*>(ws);
     uint64_t* stats = ws + Q_WORDS / 2;
     uint32_t* list = reinterpret_cast<uint32_t*>(stats + ST_WORDS);
+    uint64_t* plist = stats + ST_WORDS + (uint64_t(view.X) + 1) / 2 + 1;
     fill_u64(ws, Q_WORDS / 2 + ST_WORDS, 0, st);
     TcParams p = prm;
     if (p.wave_max_deg > WAVE_SLOTS / 2) p.wave_max_deg = WAVE_SLOTS / 2;
@@ -1096,15 +1291,25 @@ static hipError_t launch_impl(const TcView& view, const TcOut& out, const TcPara
     p.wave_max_deg = wm;
     // |S| up to this is probed in an LDS table (k_tc_main or k_tc_big)
     V.v.in_hash_max = p.bsearch_min_deg;
+    // parts: the workspace holds the part list of view.entries entries; a
+    // listing writes whole tails
+    p.wave_split = p.team_split = 0xffffffffu;
+    if (view.entries && !out.tri && !out.tail_count) {
+        const Split sp = split_rule(view.entries, num_cus);
+        p.team_split = sp.team;
+        if (sp.wave < 1024) p.wave_split = sp.wave;
+    }
     // a min-side walk covers in- and out-neighbours and streams from only
     // some of them: four times the entries per team grab
     if (V.v.in_off) p.team_chunk = std::min<uint32_t>(4 * std::max<uint32_t>(p.team_chunk, 1), KT_WAVE);
     if (view.X > 0) {
         const unsigned g = std::min<unsigned>((view.X + 255) / 256, (unsigned)num_cus * 8);
         k_tc_bin_count<PLAIN><<<g, 256, 0, st>>>(V, p, q, stats);
-        k_tc_bin_fill<PLAIN><<<g, 256, 0, st>>>(V, p, q, list);
+        k_tc_bin_fill<PLAIN><<<g, 256, 0, st>>>(V, p, q, list, plist);
     }
-    unsigned grid = (unsigned)num_cus * (p.grid_per_cu ? p.grid_per_cu : 4);
+    // no more workgroups than fit at once (three per CU): shares are fixed per
+    // workgroup, and one that starts late would hold its share back
+    const unsigned grid = (unsigned)num_cus * std::clamp<unsigned>(p.grid_per_cu, 1, 3);
     constexpr uint32_t big_lds = 2 * BIG_SLOTS * sizeof(uint32_t);
     if constexpr (PLAIN) {
         if (out.tri) {  // listing: streamed walks only
@@ -1115,7 +1320,7 @@ static hipError_t launch_impl(const TcView& view, const TcOut& out, const TcPara
             if (big_list_ok != hipSuccess) return big_list_ok;
             k_tc_big<PLAIN, true><<<(unsigned)num_cus, BIG_THREADS, big_lds, st>>>(V, out, p, q, list, stats);
             if (ev_begin) (void)hipEventRecord(ev_begin, st);
-            k_tc_main<PLAIN, KT_WAVE, true><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats);
+            k_tc_main<PLAIN, true><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, plist, stats);
             if (ev_end) (void)hipEventRecord(ev_end, st);
             return hipGetLastError();
         }
@@ -1129,15 +1334,7 @@ static hipError_t launch_impl(const TcView& view, const TcOut& out, const TcPara
     if (big_ok != hipSuccess) return big_ok;
     k_tc_big<PLAIN, false><<<(unsigned)num_cus, BIG_THREADS, big_lds, st>>>(V, out, p, q, list, stats);
     if (ev_begin) (void)hipEventRecord(ev_begin, st);
-    // lanes per list: the whole wave (streamed) or groups of 32, 16 or 8
-    switch (p.strategy) {
-        case TC_GROUPED32: k_tc_main<PLAIN, 32, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats); break;
-        case TC_GROUPED16: k_tc_main<PLAIN, 16, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats); break;
-        case TC_GROUPED8: k_tc_main<PLAIN, 8, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats); break;
-        case TC_GROUPED4: k_tc_main<PLAIN, 4, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats); break;
-        case TC_GROUPED2: k_tc_main<PLAIN, 2, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats); break;
-        default: k_tc_main<PLAIN, KT_WAVE, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, stats); break;
-    }
+    k_tc_main<PLAIN, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, plist, stats);
     if (ev_end) (void)hipEventRecord(ev_end, st);
     return hipGetLastError();  // a launch that did not start (e.g. LDS beyond the device's limit)
 }
