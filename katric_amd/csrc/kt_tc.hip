@@ -40,21 +40,24 @@ constexpr int TC_WAVES = TC_THREADS / KT_WAVE;           // 8
 constexpr uint32_t GROUP_SLOTS = 4096;                   // shared table of the 8-wave team
 constexpr uint32_t WAVE_SLOTS = GROUP_SLOTS / TC_WAVES;  // private table of a 1-wave team (512)
 constexpr uint32_t MIN_LOGS = 6;
-// Work-queue buckets.  By degree: bucket b < 12 holds tails with |S| in
-// (2^(b-1), 2^b].  By vertex: buckets 0..7 hold the workgroup tails and 8..15
-// the wave tails of the eight contiguous eighths of the tail range, one per
-// XCD, each in vertex order.  Bucket 17 holds the tails above the workgroup
-// bin whose table still fits a workgroup's whole LDS (k_tc_big), bucket 16
-// those beyond (binary search, k_tc_huge).
-// Buckets 18 and 19 hold parts of tails whose walk is too long for one team
-// (see split_rule): entries (part << 32 | tail) in a list of their own, taken
-// by workgroup teams (18) and by waves (19) before everything else.
-constexpr int NBUCKET = 20;
-constexpr int BUCKET_HUGE = 16;
-constexpr int BUCKET_BIG = 17;
-constexpr int BUCKET_TEAM_PARTS = 18;
-constexpr int BUCKET_WAVE_PARTS = 19;
-constexpr int NLIST = 18;  // buckets whose tails share the u32 list
+// Work-queue buckets: three classes of eight.  Class PACK holds the tails that
+// a wave takes several at a time, SOLO the other wave tails, TEAM the
+// workgroup tails; the eight are size steps (by degree) or the contiguous
+// eighths of the tail range, one per XCD, each in vertex order (by vertex).
+// Then the tails beyond any LDS table (binary search, k_tc_huge) and those
+// above the workgroup bin whose table still fits a workgroup's whole LDS
+// (k_tc_big), and, in a list of their own, the parts of tails whose walk is
+// too long for one team (split_rule): entries (part << 32 | tail), taken by
+// workgroup teams and by waves before everything else.
+constexpr int CLASS_PACK = 0, CLASS_SOLO = 8, CLASS_TEAM = 16;
+constexpr int BUCKET_HUGE = 24;
+constexpr int BUCKET_BIG = 25;
+constexpr int NLIST = 26;  // buckets whose tails share the u32 list
+constexpr int BUCKET_TEAM_PARTS = 26;
+constexpr int BUCKET_WAVE_PARTS = 27;
+constexpr int NBUCKET = 28;
+// Tails of class PACK: at most 64 ids in S(x) and 64 walk entries.
+constexpr uint32_t PACK_MAX = KT_WAVE;
 // k_tc_big: one 1024-thread workgroup per CU with a 16384-slot table (128 KB
 // of LDS for keys and counters), for |S| <= 8192
 constexpr int BIG_THREADS = 1024;
@@ -65,7 +68,7 @@ constexpr int NXCD = 8;  // MI355X: workgroup i runs on XCD i % 8
 // work-queue header (u32 words at the start of the workspace); every counter
 // that waves update concurrently sits on its own 128-byte line so that the
 // queues of different buckets land on different L2 channels:
-//   [0, 20)               tails (parts) per bucket (written by binning, then read-only)
+//   [0, 28)               tails (parts) per bucket (written by binning, then read-only)
 //   Q_PULL + 32 * b       pull cursor of bucket b
 //   Q_FILL + 32 * b       fill cursor of bucket b (binning pass 2)
 enum : int { Q_CNT = 0, Q_PULL = 32, Q_FILL = 32 * (NBUCKET + 1), Q_STRIDE = 32, Q_WORDS = 32 * (2 * NBUCKET + 2) };
@@ -189,7 +192,7 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
     if (s == 0 || r == 0 || ((PLAIN || prm.pseudo2core) && s < 2)) return -1;
     if (s > prm.bsearch_min_deg) return BUCKET_HUGE;
     if (s > prm.group_max_deg) return BUCKET_BIG;
-    int b = (int)ceil_log2(s);  // 0..11
+    int b = (int)ceil_log2(s);  // size step, 0..11
     // a min-side walk covers the whole input row: a long row goes to a
     // bigger bucket (a workgroup team beyond 512 entries), whatever |S(x)|
     if (V.min_side()) b = max(b, min((int)ceil_log2(r) - 2, (int)ceil_log2(prm.group_max_deg)));
@@ -199,11 +202,9 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
         parts = (uint32_t)((r + split - 1) / split);
         return wave ? BUCKET_WAVE_PARTS : BUCKET_TEAM_PARTS;
     }
-    if (prm.order == TC_BY_VERTEX) {  // two classes per XCD, each in vertex order
-        const int xcd = (int)(((uint64_t)x * NXCD) / V.v.X);
-        return wave ? NXCD + xcd : xcd;
-    }
-    return b;
+    const int cls = !wave ? CLASS_TEAM : s <= PACK_MAX && r <= PACK_MAX ? CLASS_PACK : CLASS_SOLO;
+    if (prm.order == TC_BY_VERTEX) return cls + (int)(((uint64_t)x * NXCD) / V.v.X);
+    return cls + (cls == CLASS_TEAM ? max(b - 4, 0) : cls == CLASS_SOLO ? min(b, 8) - 1 : b);
 }
 
 // Grid-stride over tails; per-block bucket counts in LDS, one global atomic
@@ -846,13 +847,10 @@ __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, c
     team_sync<NW>();  // table reuse by the next tail
 }
 
-// Tails that a wave takes several at a time: at most 64 ids in S(x) and 64
-// walk entries, so that the entries and set members of a few such tails fill
-// one wave.  (One by one, each tail of R-MAT or G(n, m) -- 16 to 36 entries on
-// average -- cost the wave a chain of six dependent round trips with most of
-// its lanes idle: 12-19 us.)
-constexpr uint32_t PACK_MAX = KT_WAVE;
-
+// Tails that a wave takes several at a time, so that the entries and set
+// members of a few such tails fill one wave.  (One by one, each tail of R-MAT
+// or G(n, m) -- 16 to 36 entries on average -- cost the wave a chain of six
+// dependent round trips with most of its lanes idle: 12-19 us.)
 __device__ __forceinline__ uint32_t pack_slots(uint32_t ns) {  // load 1/8 to 1/4
     return 1u << max(ceil_log2(4ull * ns), 4u);
 }
@@ -934,6 +932,15 @@ struct Segment {
     uint32_t base, cnt;
 };
 
+// The segment of a class (a bucket of parts: that bucket): by vertex the
+// bucket of XCD sx, by degree all eight, largest first.
+template <class LdsT>
+__device__ __forceinline__ Segment class_segment(const LdsT& L, int cls, bool parts, bool by_vertex, uint32_t sx) {
+    if (parts) return {L.qbase[cls], L.qcnt[cls]};
+    if (by_vertex) return {L.qbase[cls + sx], L.qcnt[cls + sx]};
+    return {L.qbase[cls + NXCD - 1], L.qbase[cls] + L.qcnt[cls] - L.qbase[cls + NXCD - 1]};
+}
+
 // How a segment is shared out without a queue access: an atomic on one word
 // that many XCDs update costs 50-100 ns, one after the other (with every tail
 // taken from a queue, R-MAT n = 300,007 with 4 M pairs spent 1.2 of its
@@ -971,7 +978,6 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
     uint32_t* uid = uids + (LIST ? wave * KT_WAVE : 0);
     uint64_t my_total = 0;
     WorkStats wk;
-    const int wave_bucket_max = (int)ceil_log2(prm.wave_max_deg);
 
     // Every bucket's count and place in the list, read once.
     if (wave == 0) {
@@ -1007,13 +1013,10 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
     for (uint32_t k = 0; k <= (by_vertex ? NXCD : 1u); ++k) {
         const bool parts = k == 0;
         const uint32_t sx = (xcd + k - 1) % NXCD;  // by vertex: the segment's XCD
-        const Segment sg = parts       ? Segment{L.qbase[BUCKET_TEAM_PARTS], L.qcnt[BUCKET_TEAM_PARTS]}
-                           : by_vertex ? Segment{L.qbase[sx], L.qcnt[sx]}
-                                       : Segment{L.qbase[BUCKET_HUGE - 1],
-                                                 L.qbase[wave_bucket_max] - L.qbase[BUCKET_HUGE - 1]};
+        const Segment sg = class_segment(L, parts ? BUCKET_TEAM_PARTS : CLASS_TEAM, parts, by_vertex, sx);
         if (sg.cnt == 0) continue;
         const Shares sh(sg.cnt, parts || !by_vertex, sx, parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : team_parts);
-        uint32_t* pull = &q[Q_PULL + Q_STRIDE * (parts ? BUCKET_TEAM_PARTS : by_vertex ? (int)sx : 0)];
+        uint32_t* pull = &q[Q_PULL + Q_STRIDE * (parts ? BUCKET_TEAM_PARTS : CLASS_TEAM + (by_vertex ? (int)sx : 0))];
         const uint32_t fixed = sg.cnt <= 4 * sh.blocks ? sg.cnt : sh.blocks;
         uint32_t i = sh.mine ? sh.first : fixed;
         while (true) {
@@ -1037,35 +1040,35 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
             i = i < fixed ? i + sh.blocks : fixed;
         }
     }
-    // wave phase: independent waves with private tables, the same segments.
-    // A wave takes `grab` tails at a time: first the blocks of its
-    // workgroup's share (handed out by an LDS counter), then, where a wave
-    // gets many, the second half of the segment from its queue.
+    // wave phase: independent waves with private tables: the parts, the SOLO
+    // tails (a few per grab: they are the long ones, and a grab that holds
+    // several ends late), then the PACK tails.  Grabs come from the
+    // workgroup's share, handed out by an LDS counter, and, where a wave gets
+    // many, the last quarter of a segment from its queue.
     {
         uint32_t* keys = L.keys + wave * WAVE_SLOTS;
         uint32_t* tcnt = L.cnt + wave * WAVE_SLOTS;
         uint32_t* wovf = L.ovf + wave * (WAVE_SLOTS / 128);
-        for (uint32_t k = 0; k <= (by_vertex ? NXCD : 1u); ++k) {
-            const bool parts = k == 0;
+        const uint32_t segs = by_vertex ? NXCD : 1u;
+        for (uint32_t k = 0; k <= 2 * segs; ++k) {
+            const bool parts = k == 0, pack = k > segs;
             const uint32_t sx = (xcd + k - 1) % NXCD;
-            const Segment sg = parts       ? Segment{L.qbase[BUCKET_WAVE_PARTS], L.qcnt[BUCKET_WAVE_PARTS]}
-                               : by_vertex ? Segment{L.qbase[NXCD + sx], L.qcnt[NXCD + sx]}
-                                           : Segment{L.qbase[wave_bucket_max],
-                                                     L.qbase[0] + L.qcnt[0] - L.qbase[wave_bucket_max]};
+            const int cls = parts ? BUCKET_WAVE_PARTS : pack ? CLASS_PACK : CLASS_SOLO;
+            const Segment sg = class_segment(L, cls, parts, by_vertex, sx);
             if (sg.cnt == 0) continue;
             const Shares sh(sg.cnt, parts || !by_vertex, sx,
                             parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : wave_parts);
-            const uint32_t most = parts ? 4u : min(max(prm.wave_grab, 1u), (uint32_t)KT_WAVE);
-            const uint32_t grab = max(1u, min(most, sg.cnt / (2 * TC_WAVES * sh.blocks)));
+            const uint32_t most = pack ? min(max(prm.wave_grab, 1u), (uint32_t)KT_WAVE) : 2u;
+            const uint32_t grab = max(1u, min(most, sg.cnt / (4 * TC_WAVES * sh.blocks)));
             const uint32_t grabs = (sg.cnt + grab - 1) / grab;
-            const uint32_t fixed = grabs <= 8 * TC_WAVES * sh.blocks ? grabs : grabs / 2;
-            uint32_t* pull = &q[Q_PULL + Q_STRIDE * (parts ? BUCKET_WAVE_PARTS : by_vertex ? (int)(NXCD + sx) : 1)];
-            uint32_t* ctr = &L.qctr[parts ? BUCKET_WAVE_PARTS : by_vertex ? NXCD + sx : 1];
+            const uint32_t fixed = grabs <= 8 * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
+            const int qi = parts ? cls : cls + (by_vertex ? (int)sx : 0);
+            uint32_t* pull = &q[Q_PULL + Q_STRIDE * qi];
             bool own = sh.mine;
             while (true) {
                 uint32_t g = 0;
                 if (own) {
-                    if (lane == 0) g = sh.first + atomicAdd(ctr, 1u) * sh.blocks;
+                    if (lane == 0) g = sh.first + atomicAdd(&L.qctr[qi], 1u) * sh.blocks;
                     g = uniform(g);
                     own = g < fixed;
                 }
@@ -1097,7 +1100,7 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
                 }
                 // Consecutive small tails are taken together while their
                 // entries, set members and tables fit the wave.
-                const bool small = !LIST && !out.tail_count && lane < ng && bl.nr <= PACK_MAX && bl.ns <= PACK_MAX;
+                const bool small = !LIST && !out.tail_count && pack && lane < ng;
                 const uint32_t sr = wave_scan_dpp(small ? bl.nr : 0u), ss = wave_scan_dpp(small ? bl.ns : 0u),
                                st = wave_scan_dpp(small ? pack_slots(bl.ns) : 0u);
                 for (uint32_t j = 0; j < ng;) {
