@@ -303,11 +303,12 @@ struct PlainBufs {
     uint64_t* ws_radix;
     uint64_t* pv;
     uint64_t* small;  // [0] = err flags (u32), [1] = total, [2..] = tc stats
-    uint64_t entries;  // walk entries ws_tc's part list is sized for (0: none)
+    TcRoom room;      // what ws_tc has room for
 };
 
-// Lays out every buffer of the plain path; with base == nullptr only sizes.
-uint64_t plain_layout(void* base, uint32_t n, uint64_t nnz, uint64_t entries, int num_cus, bool host_in,
+// Lays out every buffer of the plain path; with base == nullptr only sizes
+// (rich: ws_tc has all the room that pays).
+uint64_t plain_layout(void* base, uint32_t n, uint64_t nnz, bool rich, int num_cus, bool host_in, bool want_pv,
                       bool want_pv_dev, bool unsorted, PlainBufs& B) {
     Carver cv{base, 0};
     const uint64_t m = nnz / 2;
@@ -323,7 +324,8 @@ uint64_t plain_layout(void* base, uint32_t n, uint64_t nnz, uint64_t entries, in
     B.oheads = static_cast<uint32_t*>(cv.take((m + 4) * 4));  // +4: 16-byte block reads past the end
     B.ws_orient = static_cast<uint64_t*>(cv.take(orient_ws_words(n, nnz) * 8));
     // also the scratch of the longest-list reduction of unsorted input
-    B.ws_tc = static_cast<uint64_t*>(cv.take(std::max(tc_ws_words(n, entries, num_cus), segsort_tmp_words()) * 8));
+    B.room = rich ? tc_room(nnz, m, want_pv ? n : 0) : TcRoom{};
+    B.ws_tc = static_cast<uint64_t*>(cv.take(std::max(tc_ws_words(n, B.room, num_cus), segsort_tmp_words()) * 8));
     B.pv = want_pv_dev ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(n, 1) * 8)) : nullptr;
     B.keys = B.alt = B.ws_radix = nullptr;
     if (unsorted) {
@@ -393,20 +395,28 @@ struct Workspace {
 };
 
 int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_off, const uint32_t* user_heads,
-                    bool host_in, bool pv_dev_needed, PlainBufs& B, bool& unsorted, const Workspace& ws = {}) {
+                    bool host_in, bool want_pv, bool pv_dev_needed, PlainBufs& B, bool& unsorted,
+                    const Workspace& ws = {}) {
     hipStream_t st = c->stream;
     unsorted = false;
-    // part list of the intersection: left out where only it does not fit a
-    // fixed workspace
-    uint64_t entries = nnz;
-    if (ws.fixed_base && plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, false, B) > ws.fixed_cap)
-        entries = 0;
-    uint64_t need = plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, false, B);
+    // the intersection's optional room is left out where only it does not fit
+    bool rich = true, sorting = false;
+    auto layout = [&](void* base) {
+        return plain_layout(base, n, nnz, rich, c->num_cus, host_in, want_pv, pv_dev_needed, sorting, B);
+    };
+    auto ensure = [&]() {
+        int r = ws.ensure(c, layout(nullptr));
+        if (r == KT_ENOMEM && rich) {
+            rich = false;
+            r = ws.ensure(c, layout(nullptr));
+        }
+        return r;
+    };
+    uint64_t need = layout(nullptr);
     trace("orientation: n=%u nnz=%llu workspace=%llu", n, (unsigned long long)nnz, (unsigned long long)need);
-    int rc = ws.ensure(c, need);
+    int rc = ensure();
     if (rc) return rc;
-    plain_layout(ws.base(c), n, nnz, entries, c->num_cus, host_in, pv_dev_needed, false, B);
-    B.entries = entries;
+    layout(ws.base(c));
     trace("workspace=%p bytes=%llu", ws.base(c), (unsigned long long)ws.cap(c));
     (void)hipEventRecord(c->ev[EV_START], st);
     rc = upload_and_count(c, n, nnz, user_off, user_heads, host_in, B);
@@ -452,20 +462,17 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
         if (flags & KT_ERR_MASK) return c->fail(KT_EINVAL, "malformed CSR: duplicate edge");
     } else if (flags & KT_FLAG_UNSORTED) {
         unsorted = true;
-        if (ws.fixed_base &&
-            plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B) > ws.fixed_cap)
-            entries = 0;
-        need = plain_layout(nullptr, n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B);
-        B.entries = entries;
+        sorting = true;
+        need = layout(nullptr);
         if (need > ws.cap(c)) {
             // growing the arena drops its contents: upload and count again
-            rc = ws.ensure(c, need);
+            rc = ensure();
             if (rc) return rc;
-            plain_layout(ws.base(c), n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B);
+            layout(ws.base(c));
             rc = upload_and_count(c, n, nnz, user_off, user_heads, host_in, B);
             if (rc) return rc;
         } else {
-            plain_layout(ws.base(c), n, nnz, entries, c->num_cus, host_in, pv_dev_needed, true, B);
+            layout(ws.base(c));
             if (!host_in) {
                 B.off = user_off;
                 B.heads = user_heads;
@@ -530,7 +537,7 @@ int kt::count_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, const uint3
     const bool pv_dev = want_pv && (flags & KT_DEVICE_OUTPUT);
     PlainBufs B;
     bool unsorted;
-    rc = run_orientation(c, n, nnz, offsets, heads, host_in, want_pv && !pv_dev, B, unsorted, ws);
+    rc = run_orientation(c, n, nnz, offsets, heads, host_in, want_pv, want_pv && !pv_dev, B, unsorted, ws);
     if (rc) return rc;
     hipStream_t st = c->stream;
     (void)hipEventRecord(c->ev[EV_PREP], st);
@@ -546,7 +553,9 @@ int kt::count_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, const uint3
         view.in_heads = B.heads;
         view.in_keep = orient_keep_bits(n, nnz, B.ws_orient);
     }
-    view.entries = B.entries;
+    view.sym_slots = nnz;
+    view.room = B.room;
+    view.deg = B.deg;
     TcOut out{pv, totals};
     trace("intersection: X=%u pv=%p", n, (void*)pv);
     // wave-bin tails per queue access for one graph: each grab costs a queue
@@ -617,7 +626,7 @@ extern "C" int kt_list_triangles(kt_ctx* c, uint32_t n, const uint64_t* offsets,
     const bool dev_out = (flags & KT_DEVICE_OUTPUT) != 0;
     PlainBufs B;
     bool unsorted;
-    rc = run_orientation(c, n, nnz, offsets, heads, host_in, false, B, unsorted);
+    rc = run_orientation(c, n, nnz, offsets, heads, host_in, false, false, B, unsorted);
     if (rc) return rc;
     // per-tail triangle counts, scanned in place into output offsets
     Carver cv{nullptr, 0};
@@ -709,7 +718,7 @@ extern "C" int kt_orient(kt_ctx* c, uint32_t n, const uint64_t* offsets, const u
     if (rc) return rc;
     PlainBufs B;
     bool unsorted;
-    rc = run_orientation(c, n, nnz, offsets, heads, !(flags & KT_DEVICE_INPUT), false, B, unsorted);
+    rc = run_orientation(c, n, nnz, offsets, heads, !(flags & KT_DEVICE_INPUT), false, false, B, unsorted);
     if (rc) return rc;
     hipStream_t st = c->stream;
     hipMemcpyKind kind = (flags & KT_DEVICE_OUTPUT) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;

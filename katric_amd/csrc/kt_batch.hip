@@ -83,7 +83,7 @@ __global__ void k_seg_final(uint32_t G, uint64_t* __restrict__ totals, uint32_t*
 }
 
 uint64_t batch_layout(void* base, uint32_t G, uint64_t N, uint64_t nnz, int num_cus, bool host_in, bool own_pv,
-                      bool unsorted, BatchBufs& B) {
+                      bool unsorted, bool rich, BatchBufs& B) {
     Carver cv{base, 0};
     B.small = static_cast<uint64_t*>(cv.take(64 * 8));
     B.off = nullptr;
@@ -97,7 +97,8 @@ uint64_t batch_layout(void* base, uint32_t G, uint64_t N, uint64_t nnz, int num_
     B.ooff = static_cast<uint64_t*>(cv.take((N + 1) * 8));
     B.oheads = static_cast<uint32_t*>(cv.take((nnz + 4) * 4));  // capacity nnz: no overflow without a host check
     B.ws_orient = static_cast<uint64_t*>(cv.take(orient_ws_words((uint32_t)N, nnz) * 8));
-    B.ws_tc = static_cast<uint64_t*>(cv.take(tc_ws_words((uint32_t)N, nnz, num_cus) * 8));
+    B.room = rich ? tc_room(nnz, nnz, N) : TcRoom{};
+    B.ws_tc = static_cast<uint64_t*>(cv.take(tc_ws_words((uint32_t)N, B.room, num_cus) * 8));
     B.pv = own_pv ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(N, 1) * 8)) : nullptr;
     B.totals = static_cast<uint64_t*>(cv.take(std::max<uint64_t>(G, 1) * 8));
     B.keys = B.alt = B.ws_radix = nullptr;
@@ -156,7 +157,9 @@ hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, cons
         v.in_heads = B.heads;
         v.in_keep = orient_keep_bits((uint32_t)N, nnz, B.ws_orient);
     }
-    v.entries = nnz;
+    v.sym_slots = nnz;
+    v.room = B.room;
+    v.deg = B.deg;
     // malformed input is never walked; unsorted input only once it is sorted
     // (the caller runs the pipeline again)
     v.gate = err;
@@ -232,10 +235,15 @@ extern "C" int kt_batch_count(kt_ctx* c, uint32_t G, const uint64_t* vertex_base
         const bool sort = attempt == 1;
         const bool radix = sort_mode == SORT_RADIX;
         BatchBufs B;
-        const uint64_t need = batch_layout(nullptr, G, N, nnz, c->num_cus, host_in, !pv_dev, radix, B);
-        rc = c->reserve(need);
+        // the intersection's optional room is left out where only it does not fit
+        bool rich = true;
+        rc = c->reserve(batch_layout(nullptr, G, N, nnz, c->num_cus, host_in, !pv_dev, radix, rich, B));
+        if (rc == KT_ENOMEM) {
+            rich = false;
+            rc = c->reserve(batch_layout(nullptr, G, N, nnz, c->num_cus, host_in, !pv_dev, radix, rich, B));
+        }
         if (rc) return rc;
-        batch_layout(c->arena, G, N, nnz, c->num_cus, host_in, !pv_dev, radix, B);
+        batch_layout(c->arena, G, N, nnz, c->num_cus, host_in, !pv_dev, radix, rich, B);
         if (!host_in) {
             B.off = offsets;
             B.heads = heads;

@@ -81,6 +81,7 @@ struct TcParams {
                               // tables to clear and flush per tail; 16 gave the same RMAT-22 time, batches 1 % slower)
     uint32_t wave_split = 0xffffffffu;  // walk entries per part of a wave / workgroup tail (set by the launch)
     uint32_t team_split = 0xffffffffu;
+    uint32_t hub_split = 0xffffffffu;
     uint32_t wave_grab = 32;  // wave-bin tails a wave takes per queue access (1..64), vertex order
     uint32_t bsearch_min_deg = 8192;  // |S(x)| above this: binary-search probes in global memory (<= 8192)
     uint32_t pseudo2core = 0; // skip tails with |S(x)| < 2 and count them (Config::pseudo2core)
@@ -102,6 +103,15 @@ enum : uint32_t {
 // then wave tails (TC_BY_VERTEX: tails of one graph of a batch, and their
 // data, stay together in time and cache).
 enum : uint32_t { TC_BY_DEGREE = 0, TC_BY_VERTEX = 1 };
+
+// Optional parts of the launch workspace; without them (all zero) every tail
+// is walked by one team with a hash table and every count goes straight to
+// per_vertex.  Callers leave them out where only they exceed a budget.
+struct TcRoom {
+    uint64_t entries = 0;    // upper bound of all tails' walk entries: list of the parts of long walks
+    uint64_t hub_slots = 0;  // oriented slots with a hub list entry (needs entries)
+    uint64_t pv_n = 0;       // per-vertex counts, one copy per XCD
+};
 
 // Generic "tail list" view for the intersection kernel:
 //   tails x in [0, X): hash set S(x) = sheads[s_off[x] .. s_off[x+1]),
@@ -136,9 +146,13 @@ struct TcView {
     const uint32_t* in_heads = nullptr;
     const uint64_t* in_keep = nullptr;
     uint64_t in_hash_max = 0;
-    // upper bound of all tails' walk entries, as given to tc_ws_words (0: the
-    // workspace has no part list, every tail is walked by one team)
-    uint64_t entries = 0;
+    // slots of the symmetric CSR whose whole orientation this is (0: not so):
+    // |S(x)| <= sqrt(slots), since every id in S(x) has at least |S(x)| slots
+    uint64_t sym_slots = 0;
+    TcRoom room;  // what the workspace has room for, as given to tc_ws_words
+    // plain views with room for hub lists: the order's degrees (S(x) holds ids
+    // whose degree is at least x's)
+    const uint32_t* deg = nullptr;
     // device flag word (nullable): with any of these bits set no tail is
     // queued, so input that failed its checks is never walked
     const uint32_t* gate = nullptr;
@@ -147,7 +161,8 @@ struct TcView {
 
 struct TcOut {
     uint64_t* per_vertex;       // nullable
-    uint64_t* totals;           // per graph (>= 1 entry)
+    uint64_t* totals;           // one entry
+    uint64_t pv_stride = 0;     // set by the launch: per_vertex is the first of one copy per XCD
     // triangle listing (plain views only): a counting launch with tail_count
     // set records every tail's number of emitted triangles; a listing launch
     // (tri set) writes tail x's triangles as (x, u, w) id triples from
@@ -174,13 +189,15 @@ struct BatchBufs {
     uint64_t* keys;
     uint64_t* alt;
     uint64_t* ws_radix;
+    TcRoom room;
 };
 // How a batch pipeline sorts the oriented lists: not at all (sorted input),
 // in place per list (every list at most segsort_max_len() ids), or by the
 // global radix sort (its scratch is in the layout).
 enum BatchSort : uint32_t { SORT_NONE = 0, SORT_SEGMENTED = 1, SORT_RADIX = 2 };
+// (rich: the intersection's workspace has all the room that pays)
 uint64_t batch_layout(void* base, uint32_t G, uint64_t N, uint64_t nnz, int num_cus, bool host_in, bool own_pv,
-                      bool unsorted, BatchBufs& B);
+                      bool unsorted, bool rich, BatchBufs& B);
 hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, const BatchBufs& B, uint32_t G, uint64_t N,
                           uint64_t nnz, uint64_t* pv, uint64_t* h_totals, uint64_t* h_small, uint32_t sort,
                           const uint64_t sym_key[2]);
@@ -188,9 +205,11 @@ hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, cons
 // longest oriented list of that run (B as it ran; synchronises st).
 hipError_t batch_sort_mode(hipStream_t st, const BatchBufs& B, uint64_t N, uint64_t* h_small, uint32_t& mode);
 
-// Words of the launch workspace for X tails whose walks hold at most `entries`
-// entries in all (0: no part list).
-uint64_t tc_ws_words(uint32_t X, uint64_t entries, int num_cus);
+// Words of the launch workspace for X tails.
+uint64_t tc_ws_words(uint32_t X, const TcRoom& room, int num_cus);
+// The room that pays for walks of at most `entries` entries, `slots` oriented
+// slots (0: the view has no hubs) and pv_n per-vertex counts (0: none).
+TcRoom tc_room(uint64_t entries, uint64_t slots, uint64_t pv_n);
 // Enqueues binning and the intersection kernels; returns the launch status.
 hipError_t tc_launch(const TcView& view, const TcOut& out, const TcParams& prm, uint64_t* ws, int num_cus,
                      hipStream_t st, hipEvent_t ev_begin, hipEvent_t ev_end);

@@ -114,6 +114,7 @@ struct ServeSlot {
     bool busy = false;
     bool sorted = false;
     bool large = false;  // the batch is one large request
+    bool rich = false;   // its layout has the intersection's optional room
     uint64_t batch_id = 0;
     uint64_t N = 0, nnz = 0;
 };
@@ -142,9 +143,9 @@ struct ServeState {
 // Device bytes of a slot's batch: the batch pipeline's buffers (with the
 // radix-sort scratch for a relaunch of unsorted lists that needs it) and the
 // gather descriptors after them.
-static uint64_t slot_bytes(const ServeState* S, uint32_t G, uint64_t N, uint64_t nnz, bool radix) {
+static uint64_t slot_bytes(const ServeState* S, uint32_t G, uint64_t N, uint64_t nnz, bool radix, bool rich = false) {
     BatchBufs B;
-    return ((batch_layout(nullptr, G, N, nnz, S->num_cus, true, true, radix, B) + 255) & ~255ull) + (uint64_t)G * sizeof(GatherDesc);
+    return ((batch_layout(nullptr, G, N, nnz, S->num_cus, true, true, radix, rich, B) + 255) & ~255ull) + (uint64_t)G * sizeof(GatherDesc);
 }
 
 static uint64_t req_bytes(const ServeState* S, const ServeReq* r) { return slot_bytes(S, 1, r->n, r->nnz, false); }
@@ -188,13 +189,20 @@ static int launch(ServeState* S, ServeSlot& sl, uint32_t sort) {
     }
     BatchBufs B;
     const bool radix = sort == SORT_RADIX;
-    const uint64_t used = (batch_layout(nullptr, G, N, nnz, S->num_cus, true, true, radix, B) + 255) & ~255ull;
     // a slot never holds more than its share of the budget (a relaunch with
-    // the radix-sort scratch can need more than admission counted)
+    // the radix-sort scratch can need more than admission counted); the
+    // intersection's optional room, which admission leaves out, is taken
+    // where it fits
     if (slot_bytes(S, G, N, nnz, radix) > S->slot_cap) return KT_ENOMEM;
-    int rc = slot_grow(sl, used + (uint64_t)G * sizeof(GatherDesc), G);
+    sl.rich = slot_bytes(S, G, N, nnz, radix, true) <= S->slot_cap;
+    int rc = slot_grow(sl, slot_bytes(S, G, N, nnz, radix, sl.rich), G);
+    if (rc == KT_ENOMEM && sl.rich) {
+        sl.rich = false;
+        rc = slot_grow(sl, slot_bytes(S, G, N, nnz, radix, false), G);
+    }
     if (rc) return rc;
-    batch_layout(sl.arena, G, N, nnz, S->num_cus, true, true, radix, B);
+    const uint64_t used =
+        (batch_layout(sl.arena, G, N, nnz, S->num_cus, true, true, radix, sl.rich, B) + 255) & ~255ull;
     GatherDesc* d_desc = reinterpret_cast<GatherDesc*>(static_cast<char*>(sl.arena) + used);
     uint64_t* vb = sl.h_meta;
     GatherDesc* desc = reinterpret_cast<GatherDesc*>(sl.h_meta + (sl.meta_cap + 1));
@@ -321,7 +329,7 @@ static void worker_main(ServeState* S) {
                 // same requests, with the oriented lists sorted (the sort
                 // chosen from the longest list of the run that found them)
                 BatchBufs B0;
-                batch_layout(sl.arena, (uint32_t)sl.reqs.size(), sl.N, sl.nnz, S->num_cus, true, true, false, B0);
+                batch_layout(sl.arena, (uint32_t)sl.reqs.size(), sl.N, sl.nnz, S->num_cus, true, true, false, sl.rich, B0);
                 uint32_t mode = SORT_RADIX;
                 int rc = batch_sort_mode(sl.stream, B0, sl.N, sl.h_small, mode) == hipSuccess ? KT_OK : KT_EHIP;
                 if (rc == KT_OK) rc = launch(S, sl, mode);

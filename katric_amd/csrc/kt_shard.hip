@@ -383,11 +383,12 @@ struct ShardBufs {
     uint2* rs;
     uint64_t* rs_cnt;
     uint32_t* tbnd;
+    TcRoom room;
 };
 
 
 uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t mtot, int num_cus, bool host_in,
-                      bool pv_dev, ShardBufs& B) {
+                      bool want_pv, bool pv_dev, bool rich, ShardBufs& B) {
     Carver cv{base, 0};
     const uint64_t nloc = in->range_bounds[in->rank + 1] - in->range_bounds[in->rank];
     const uint64_t X = nloc + in->n_ghost;
@@ -420,8 +421,9 @@ uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t 
     B.scan_tmp = static_cast<uint64_t*>(
         cv.take(scan_tmp_words(std::max(std::max<uint64_t>(X, in->n_msg), rs_words) + 1) * 8));
     // both phases use it: the list of the larger set of tails, the parts of the longer walk
-    B.tc_ws = static_cast<uint64_t*>(cv.take(
-        tc_ws_words((uint32_t)std::max<uint64_t>(X, in->n_msg), std::max(nnz, mtot), num_cus) * 8));
+    B.room = rich ? tc_room(std::max(nnz, mtot), 0, want_pv ? X : 0) : TcRoom{};
+    B.tc_ws = static_cast<uint64_t*>(
+        cv.take(tc_ws_words((uint32_t)std::max<uint64_t>(X, in->n_msg), B.room, num_cus) * 8));
     B.pv = pv_dev ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(X, 1) * 8)) : nullptr;
     B.rs = static_cast<uint2*>(cv.take((rs_words + 1) * 8));
     B.rs_cnt = static_cast<uint64_t*>(cv.take((rs_words + 1) * 8));
@@ -474,10 +476,15 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
         (in->n_msg && (!in->msg_src || !in->msg_offsets || (mtot && !in->msg_heads))))
         return c->fail(KT_EINVAL, "null shard array");
     ShardBufs B;
-    const uint64_t need = shard_layout(nullptr, in, nnz, mtot, c->num_cus, host_in, want_pv && !pv_dev, B);
-    rc = c->reserve(need);
+    // the intersection's optional room is left out where only it does not fit
+    bool rich = true;
+    rc = c->reserve(shard_layout(nullptr, in, nnz, mtot, c->num_cus, host_in, want_pv, want_pv && !pv_dev, rich, B));
+    if (rc == KT_ENOMEM) {
+        rich = false;
+        rc = c->reserve(shard_layout(nullptr, in, nnz, mtot, c->num_cus, host_in, want_pv, want_pv && !pv_dev, rich, B));
+    }
     if (rc) return rc;
-    shard_layout(c->arena, in, nnz, mtot, c->num_cus, host_in, want_pv && !pv_dev, B);
+    shard_layout(c->arena, in, nnz, mtot, c->num_cus, host_in, want_pv, want_pv && !pv_dev, rich, B);
     hipStream_t st = c->stream;
     (void)hipEventRecord(c->ev[EV_START], st);
     if (host_in) {
@@ -588,7 +595,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
             v.t_end = B.coff + 1;
             v.theads = B.cheads;
         }
-        v.entries = std::max(nnz, mtot);
+        v.room = B.room;
         TcOut o{pv, totals};
         rc = c->hip_check(tc_launch(v, o, c->prm, B.tc_ws, c->num_cus, st, c->ev[EV_TC0], c->ev[EV_TC1]),
                           "intersection launch");
@@ -620,7 +627,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
         // intersected ids; a CeTriC receiver without cut edges was compacted away
         v.stat_off = B.msg_off;
         v.stat_skip_empty = cetric ? 1u : 0u;
-        v.entries = std::max(nnz, mtot);
+        v.room = B.room;
         TcOut o{pv, totals + 1};
         // message tails have short owned parts: a whole workgroup on one of
         // them idles, so tails up to the largest wave table stay with one

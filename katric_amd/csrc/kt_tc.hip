@@ -55,7 +55,10 @@ constexpr int BUCKET_BIG = 25;
 constexpr int NLIST = 26;  // buckets whose tails share the u32 list
 constexpr int BUCKET_TEAM_PARTS = 26;
 constexpr int BUCKET_WAVE_PARTS = 27;
-constexpr int NBUCKET = 28;
+// Parts of the workgroup tails that k_tc_hub takes (every such tail, whole or
+// split).
+constexpr int BUCKET_HUB_PARTS = 28;
+constexpr int NBUCKET = 29;
 // Tails of class PACK: at most 64 ids in S(x) and 64 walk entries.
 constexpr uint32_t PACK_MAX = KT_WAVE;
 // k_tc_big: one 1024-thread workgroup per CU with a 16384-slot table (128 KB
@@ -68,13 +71,22 @@ constexpr int NXCD = 8;  // MI355X: workgroup i runs on XCD i % 8
 // work-queue header (u32 words at the start of the workspace); every counter
 // that waves update concurrently sits on its own 128-byte line so that the
 // queues of different buckets land on different L2 channels:
-//   [0, 28)               tails (parts) per bucket (written by binning, then read-only)
+//   [0, 29)               tails (parts) per bucket (written by binning, then read-only)
 //   Q_PULL + 32 * b       pull cursor of bucket b
 //   Q_FILL + 32 * b       fill cursor of bucket b (binning pass 2)
 enum : int { Q_CNT = 0, Q_PULL = 32, Q_FILL = 32 * (NBUCKET + 1), Q_STRIDE = 32, Q_WORDS = 32 * (2 * NBUCKET + 2) };
 // stats words after the queue header (the reference's work counters, and
 // the T-list ids the probes stream)
 enum : int { ST_WEDGE = 0, ST_ISZ = 1, ST_SKIP = 2, ST_STREAM = 3, ST_WORDS = 4 };
+// After the stats, every workgroup's sums (ST_* and the triangles), added up by
+// k_tc_finish: an atomic add per wave on the same few words held the last
+// workgroups of a launch up by 250 us.  Rows: binning, k_tc_huge, k_tc_big,
+// k_tc_hub, k_tc_main, of 1, 1, 1, 2 and 3 workgroups per CU.
+enum : int { SUM_TOTAL = ST_WORDS, SUM_WORDS = 5 };
+enum : int { ROW_BIN = 0, ROW_HUGE = 1, ROW_BIG = 2, ROW_HUB = 3, ROW_MAIN = 5, ROWS = 8 };
+static uint64_t head_words(int num_cus) {
+    return Q_WORDS / 2 + ST_WORDS + (uint64_t)ROWS * num_cus * SUM_WORDS;
+}
 
 template <bool PLAIN>
 struct View {
@@ -178,11 +190,195 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 }
 
 // ---------------------------------------------------------------------------
+// hubs: the (at most HUB_MAX) vertices of the highest degrees, numbered 0.. in
+// no particular order.  A hub's out-neighbours have at least its degree, so
+// they are hubs too: S(x) of a hub fits a table indexed by hub number, in
+// which a lookup is one 2-byte LDS read (k_tc_hub).
+// ---------------------------------------------------------------------------
+constexpr uint32_t HUB_MAX = 32000;            // 2-byte entries: 58 KB of LDS, two workgroups per CU
+constexpr uint32_t HUB_NONE = 2 * HUB_MAX;     // hub-list entry of any other id: its table entry stays empty
+constexpr uint32_t DEG_BINS = 1024;
+constexpr int HUB_BLOCKS = 256, HUB_HIST_THREADS = 256, HUB_NUMBER_THREADS = 256;
+
+// Monotone degree bin: exact below 64, then 32 steps per power of two.
+__device__ __forceinline__ uint32_t deg_bin(uint32_t d) {
+    if (d < 64) return d;
+    const uint32_t e = 31u - (uint32_t)__clz(d);
+    return 32 * (e - 4) + ((d >> (e - 5)) & 31);  // at most 32 * 27 + 31
+}
+
+// Hub workspace: degree histogram (vertices, then their degrees' sum, per
+// bin), then the lowest hub bin, the histogram's
+// finished blocks, the hubs numbered so far; the bits and number bases of 32
+// vertices each; the hub lists (2-byte entries, one per oriented slot).
+struct HubWs {
+    uint32_t* hist;
+    uint64_t* sum;
+    uint32_t* min_bin;
+    uint32_t* done;
+    uint32_t* count;
+    uint2* rs;
+    uint16_t* lists;
+};
+enum : uint64_t { HUB_HEAD_WORDS = DEG_BINS / 2 + DEG_BINS + 2 };
+
+static uint64_t hub_ws_words(uint32_t X, uint64_t slots) {
+    // lists are read 16 bytes at a time from any entry on
+    return slots ? HUB_HEAD_WORDS + ((uint64_t)X + 31) / 32 + (slots + 8 + 3) / 4 : 0;
+}
+
+static HubWs hub_ws(uint64_t* ws, uint32_t X) {
+    HubWs h;
+    h.hist = reinterpret_cast<uint32_t*>(ws);
+    h.sum = ws + DEG_BINS / 2;
+    h.min_bin = reinterpret_cast<uint32_t*>(h.sum + DEG_BINS);
+    h.done = h.min_bin + 1;
+    h.count = h.min_bin + 2;
+    h.rs = reinterpret_cast<uint2*>(ws + HUB_HEAD_WORDS);
+    h.lists = reinterpret_cast<uint16_t*>(h.rs + ((uint64_t)X + 31) / 32);
+    return h;
+}
+
+// Degree histogram; the last block picks the lowest bin such that no more
+// than HUB_MAX vertices are in it or above -- or none, where the hubs' rows
+// hold less than a quarter of the `entries`: numbering them and writing the
+// lists (0.5 ms for 106 M oriented slots of 768 mixed graphs, where hubs hold a
+// sixth) then costs more than k_tc_hub gains.
+__global__ void __launch_bounds__(HUB_HIST_THREADS) k_hub_hist(uint32_t X, const uint32_t* __restrict__ deg,
+                                                               uint64_t entries, HubWs h) {
+    __shared__ uint32_t bins[DEG_BINS];
+    __shared__ unsigned long long sums[DEG_BINS];
+    __shared__ uint32_t wcnt[HUB_HIST_THREADS / KT_WAVE];
+    __shared__ unsigned long long wsum[HUB_HIST_THREADS / KT_WAVE];
+    __shared__ uint32_t last, pick;
+    for (uint32_t i = threadIdx.x; i < DEG_BINS; i += HUB_HIST_THREADS) bins[i] = 0, sums[i] = 0;
+    __syncthreads();
+    // degrees below 8 are left out: a hub has more neighbours than that where hubs matter
+    for (uint64_t x = (uint64_t)blockIdx.x * HUB_HIST_THREADS + threadIdx.x; x < X;
+         x += (uint64_t)gridDim.x * HUB_HIST_THREADS) {
+        const uint32_t d = deg[x];
+        if (d >= 8) {
+            atomicAdd(&bins[deg_bin(d)], 1u);
+            atomicAdd(&sums[deg_bin(d)], (unsigned long long)d);
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < DEG_BINS; i += HUB_HIST_THREADS)
+        if (bins[i]) {
+            atomicAdd(&h.hist[i], bins[i]);
+            atomic_add_u64(&h.sum[i], sums[i]);
+        }
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        last = atomicAdd(h.done, 1u) == gridDim.x - 1;
+        pick = 8;
+    }
+    __syncthreads();
+    if (!last) return;
+    // thread t takes the bins 4t .. 4t + 3 counted from the top
+    constexpr uint32_t PER = DEG_BINS / HUB_HIST_THREADS;
+    uint32_t c[PER], cnt = 0;
+    for (uint32_t i = 0; i < PER; ++i) {
+        c[i] = __hip_atomic_load(&h.hist[DEG_BINS - 1 - (threadIdx.x * PER + i)], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+        cnt += c[i];
+    }
+    uint32_t run = wave_incl_sum(cnt);
+    if (lane_id() == KT_WAVE - 1) wcnt[threadIdx.x / KT_WAVE] = run;
+    __syncthreads();
+    for (uint32_t w = 0; w < threadIdx.x / KT_WAVE; ++w) run += wcnt[w];
+    run -= cnt;
+    for (uint32_t i = 0; i < PER; ++i) {
+        // the first bin from the top that no longer fits: hubs start above it
+        if (run <= HUB_MAX && run + c[i] > HUB_MAX) pick = DEG_BINS - (threadIdx.x * PER + i);
+        run += c[i];
+    }
+    __syncthreads();
+    uint64_t sum = 0;
+    for (uint32_t i = threadIdx.x; i < DEG_BINS; i += HUB_HIST_THREADS)
+        if (i >= pick) sum += __hip_atomic_load(&h.sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sum = wave_sum(sum);
+    if (lane_id() == 0) wsum[threadIdx.x / KT_WAVE] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sum = 0;
+        for (int w = 0; w < HUB_HIST_THREADS / KT_WAVE; ++w) sum += wsum[w];
+        *h.min_bin = 4 * sum >= entries ? pick : DEG_BINS;
+    }
+}
+
+// Numbers the hubs: block b takes a contiguous run of 64-vertex words, counts
+// its hubs, reserves their numbers with one atomic and writes the words.
+__global__ void __launch_bounds__(HUB_NUMBER_THREADS) k_hub_number(uint32_t X, const uint32_t* __restrict__ deg, HubWs h,
+                                                                 const uint32_t* __restrict__ q) {
+    if (q[BUCKET_HUB_PARTS] == 0) return;
+    constexpr uint32_t NW = HUB_NUMBER_THREADS / KT_WAVE;
+    __shared__ uint32_t wcnt[NW];
+    __shared__ uint32_t base;
+    const uint32_t wave = threadIdx.x / KT_WAVE, lane = lane_id();
+    const uint32_t min_bin = *h.min_bin;
+    // every wave takes a contiguous run of words
+    const uint64_t words = ((uint64_t)X + 63) / 64, waves = (uint64_t)gridDim.x * NW;
+    const uint64_t per = (words + waves - 1) / waves, w0 = min(words, ((uint64_t)blockIdx.x * NW + wave) * per),
+                   w1 = min(words, w0 + per);
+    auto hub_bits = [&](uint64_t w) {
+        const uint64_t x = 64 * w + lane;
+        return __ballot(x < X && deg_bin(deg[x]) >= min_bin);
+    };
+    uint32_t c = 0;
+    for (uint64_t w = w0; w < w1; ++w) c += (uint32_t)__popcll(hub_bits(w));
+    if (lane == 0) wcnt[wave] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (uint32_t i = 0; i < NW; ++i) t += wcnt[i];
+        base = t ? atomicAdd(h.count, t) : 0;
+    }
+    __syncthreads();
+    uint32_t at = base;
+    for (uint32_t i = 0; i < wave; ++i) at += wcnt[i];
+    for (uint64_t w = w0; w < w1; ++w) {
+        const uint64_t m = hub_bits(w);
+        const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+        if (lane == 0) h.rs[2 * w] = uint2{lo, at};
+        if (lane == 1 && 64 * w + 32 < X) h.rs[2 * w + 1] = uint2{hi, at + (uint32_t)__popc(lo)};
+        at += (uint32_t)__popcll(m);
+    }
+}
+
+// The hub list entry of every oriented slot: twice the hub's number (its
+// table entry's byte offset), HUB_NONE for other ids.  Bound by the 8-byte
+// gathers from the X / 4 byte table (L2) and HBM (4 bytes read, 2 written).
+__global__ void __launch_bounds__(256) k_hub_lists(uint32_t X, const uint64_t* __restrict__ off,
+                                                   const uint32_t* __restrict__ heads, HubWs h,
+                                                   const uint32_t* __restrict__ q) {
+    if (q[BUCKET_HUB_PARTS] == 0) return;
+    const uint64_t m = off[X], stride = (uint64_t)gridDim.x * 256;
+    constexpr int U = 4;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < m; i += U * stride) {
+        uint32_t id[U];
+        uint2 e[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) id[k] = heads[min(i + k * stride, m - 1)];
+#pragma unroll
+        for (int k = 0; k < U; ++k) e[k] = h.rs[id[k] >> 5];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const uint32_t bit = 1u << (id[k] & 31);
+            const uint32_t v = (e[k].x & bit) ? 2 * (e[k].y + (uint32_t)__popc(e[k].x & (bit - 1))) : HUB_NONE;
+            if (i + k * stride < m) h.lists[i + k * stride] = (uint16_t)v;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // binning: bucket tails by ceil(log2 |S(x)|), two passes (count, fill)
 // ---------------------------------------------------------------------------
 template <bool PLAIN>
-__device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams& prm, uint32_t x, uint64_t& s,
-                                           uint64_t& r, uint32_t& parts) {
+__device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams& prm,
+                                           const uint32_t* __restrict__ hub_min, uint32_t x, uint64_t& s, uint64_t& r,
+                                           uint32_t& parts) {
     uint64_t sb, se, rb, re;
     parts = 1;
     V.s_range(x, sb, se);
@@ -197,6 +393,10 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
     // bigger bucket (a workgroup team beyond 512 entries), whatever |S(x)|
     if (V.min_side()) b = max(b, min((int)ceil_log2(r) - 2, (int)ceil_log2(prm.group_max_deg)));
     const bool wave = b <= (int)ceil_log2(prm.wave_max_deg);
+    if (!wave && hub_min && deg_bin(V.v.deg[x]) >= *hub_min) {
+        parts = (uint32_t)((r + prm.hub_split - 1) / prm.hub_split);
+        return BUCKET_HUB_PARTS;
+    }
     const uint32_t split = wave ? prm.wave_split : prm.team_split;
     if (r > split) {
         parts = (uint32_t)((r + split - 1) / split);
@@ -208,12 +408,15 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
 }
 
 // Grid-stride over tails; per-block bucket counts in LDS, one global atomic
-// per bucket (and per stat) per block.
+// per bucket per block.
+constexpr int BIN_THREADS = 1024;
 template <bool PLAIN>
-__global__ void __launch_bounds__(256) k_tc_bin_count(View<PLAIN> V, TcParams prm, uint32_t* __restrict__ q,
-                                                      uint64_t* __restrict__ stats) {
+__global__ void __launch_bounds__(BIN_THREADS) k_tc_bin_count(View<PLAIN> V, TcParams prm, uint32_t* __restrict__ q,
+                                                      const uint32_t* __restrict__ hub_min,
+                                                      uint64_t* __restrict__ sums) {
     __shared__ uint32_t cnt[NBUCKET];
-    __shared__ uint64_t red[3][4];
+    constexpr int NW = BIN_THREADS / KT_WAVE;
+    __shared__ uint64_t red[3][NW];
     if (V.gated()) return;
     if (threadIdx.x < NBUCKET) cnt[threadIdx.x] = 0;
     __syncthreads();
@@ -221,7 +424,7 @@ __global__ void __launch_bounds__(256) k_tc_bin_count(View<PLAIN> V, TcParams pr
     for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < V.v.X; x += gridDim.x * blockDim.x) {
         uint64_t s, r;
         uint32_t parts;
-        int b = tail_bucket(V, prm, x, s, r, parts);
+        int b = tail_bucket(V, prm, hub_min, x, s, r, parts);
         if (b >= 0) atomicAdd(&cnt[b], parts);
         // pseudo2core: tails with fewer than two out-neighbours are skipped
         // and counted (cetric_edge_iterator.h:239-242)
@@ -262,12 +465,16 @@ __global__ void __launch_bounds__(256) k_tc_bin_count(View<PLAIN> V, TcParams pr
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint64_t a = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-        uint64_t c = red[1][0] + red[1][1] + red[1][2] + red[1][3];
-        uint64_t d = red[2][0] + red[2][1] + red[2][2] + red[2][3];
-        if (a) atomic_add_u64(&stats[ST_WEDGE], a);
-        if (c) atomic_add_u64(&stats[ST_ISZ], c);
-        if (d) atomic_add_u64(&stats[ST_SKIP], d);
+        uint64_t a = 0, c = 0, d = 0;
+        for (int w = 0; w < NW; ++w) {
+            a += red[0][w];
+            c += red[1][w];
+            d += red[2][w];
+        }
+        uint64_t* row = sums + (uint64_t)blockIdx.x * SUM_WORDS;
+        row[ST_WEDGE] = a;
+        row[ST_ISZ] = c;
+        row[ST_SKIP] = d;
     }
     if (threadIdx.x < NBUCKET && cnt[threadIdx.x]) atomicAdd(&q[Q_CNT + threadIdx.x], cnt[threadIdx.x]);
 }
@@ -288,7 +495,8 @@ __device__ __forceinline__ uint32_t bucket_base(const uint32_t* q, int b) {
 // bucket, reserves one range per bucket with a single global atomic, then
 // writes its tails into the reserved ranges.
 template <bool PLAIN>
-__global__ void __launch_bounds__(256) k_tc_bin_fill(View<PLAIN> V, TcParams prm, uint32_t* __restrict__ q,
+__global__ void __launch_bounds__(BIN_THREADS) k_tc_bin_fill(View<PLAIN> V, TcParams prm, uint32_t* __restrict__ q,
+                                                     const uint32_t* __restrict__ hub_min,
                                                      uint32_t* __restrict__ list, uint64_t* __restrict__ plist) {
     __shared__ uint32_t cnt[NBUCKET];
     __shared__ uint32_t pos[NBUCKET];
@@ -301,7 +509,7 @@ __global__ void __launch_bounds__(256) k_tc_bin_fill(View<PLAIN> V, TcParams prm
     for (uint32_t x = x0 + threadIdx.x; x < x1; x += blockDim.x) {
         uint64_t s, r;
         uint32_t parts;
-        int b = tail_bucket(V, prm, x, s, r, parts);
+        int b = tail_bucket(V, prm, hub_min, x, s, r, parts);
         if (b >= 0) atomicAdd(&cnt[b], parts);
     }
     __syncthreads();
@@ -313,7 +521,7 @@ __global__ void __launch_bounds__(256) k_tc_bin_fill(View<PLAIN> V, TcParams prm
     for (uint32_t x = x0 + threadIdx.x; x < x1; x += blockDim.x) {
         uint64_t s, r;
         uint32_t parts;
-        int b = tail_bucket(V, prm, x, s, r, parts);
+        int b = tail_bucket(V, prm, hub_min, x, s, r, parts);
         if (b < 0) continue;
         const uint32_t at = atomicAdd(&pos[b], parts);
         if (b < NLIST) {
@@ -548,6 +756,35 @@ struct WorkStats {
     __device__ __forceinline__ uint64_t recv() const { return uniform64(wave_sum(recv_lane)); }
     __device__ __forceinline__ uint64_t streamed() const { return uniform64(wave_sum(stream_lane)); }
 };
+
+// The workgroup's sums to its row (every wave calls it; `red` holds 4 words
+// per wave).
+template <int NW>
+__device__ __forceinline__ void flush_sums(uint64_t total, const WorkStats& wk, uint64_t* red, uint64_t* sums) {
+    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), recv = wk.recv();
+    const unsigned wave = threadIdx.x / KT_WAVE;
+    __syncthreads();
+    if (lane_id() == 0) {
+        red[4 * wave] = total;
+        red[4 * wave + 1] = wedge;
+        red[4 * wave + 2] = wedge + recv;
+        red[4 * wave + 3] = streamed;
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        uint64_t t = 0;
+        for (int i = 0; i < NW; ++i) t += red[4 * i + threadIdx.x];
+        const int at[4] = {SUM_TOTAL, ST_WEDGE, ST_ISZ, ST_STREAM};
+        sums[(uint64_t)blockIdx.x * SUM_WORDS + at[threadIdx.x]] = t;
+    }
+}
+
+// Per-vertex counts: adds on one word from all XCDs take 50-100 ns each, one
+// after the other, and every tail next to a hub adds to the hub's count: R-MAT
+// n = 300,007 (4 M pairs) spent 200 of 870 us waiting for them.  So the
+// workgroups of each XCD add to a copy of their own, and the copies are summed
+// at the end (128 bytes per vertex of traffic).
+__device__ __forceinline__ void own_copy(TcOut& out) { out.per_vertex += (blockIdx.x % NXCD) * out.pv_stride; }
 
 // What the walk probes: a hash table in LDS, or (huge tails) the sorted S(x).
 struct ProbeCtx {
@@ -970,7 +1207,8 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
                                                          uint32_t* __restrict__ q,
                                                          const uint32_t* __restrict__ list,
                                                          const uint64_t* __restrict__ plist,
-                                                         uint64_t* __restrict__ stats) {
+                                                         uint64_t* __restrict__ sums) {
+    own_copy(out);
     __shared__ Lds L;
     __shared__ uint32_t uids[LIST ? TC_THREADS : 1];  // a listing's neighbours, per wave
     const unsigned wave = threadIdx.x / KT_WAVE;
@@ -1126,32 +1364,7 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
             }
         }
     }
-    // flush the wave-uniform accumulators: one atomic per workgroup and counter
-    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), isz = wedge + wk.recv();
-    __syncthreads();
-    if (lane == 0) {
-        L.red[wave] = my_total;
-        L.keys[wave] = (uint32_t)wedge;
-        L.keys[TC_WAVES + wave] = (uint32_t)(wedge >> 32);
-        L.cnt[wave] = (uint32_t)isz;
-        L.cnt[TC_WAVES + wave] = (uint32_t)(isz >> 32);
-        L.keys[2 * TC_WAVES + wave] = (uint32_t)streamed;
-        L.keys[3 * TC_WAVES + wave] = (uint32_t)(streamed >> 32);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t t = 0, w = 0, z = 0, y = 0;
-        for (int i = 0; i < TC_WAVES; ++i) {
-            t += L.red[i];
-            w += ((uint64_t)L.keys[TC_WAVES + i] << 32) | L.keys[i];
-            z += ((uint64_t)L.cnt[TC_WAVES + i] << 32) | L.cnt[i];
-            y += ((uint64_t)L.keys[3 * TC_WAVES + i] << 32) | L.keys[2 * TC_WAVES + i];
-        }
-        if (t) atomic_add_u64(&out.totals[0], t);
-        if (w) atomic_add_u64(&stats[ST_WEDGE], w);
-        if (z) atomic_add_u64(&stats[ST_ISZ], z);
-        if (y) atomic_add_u64(&stats[ST_STREAM], y);
-    }
+    flush_sums<TC_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(L.keys), sums);
 }
 
 // Tails whose S(x) exceeds the LDS table: 8-wave teams, binary-search probes
@@ -1160,13 +1373,15 @@ template <bool PLAIN, bool LIST>
 __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out, TcParams prm,
                                                          uint32_t* __restrict__ q,
                                                          const uint32_t* __restrict__ list,
-                                                         uint64_t* __restrict__ stats) {
+                                                         uint64_t* __restrict__ sums) {
+    own_copy(out);
     __shared__ Lds L;
     __shared__ uint32_t uids[LIST ? TC_THREADS : 1];
     uint32_t* uid = uids + (LIST ? threadIdx.x / KT_WAVE * KT_WAVE : 0);
     uint64_t my_total = 0;
     WorkStats wk;
     const uint32_t cnt = q[Q_CNT + BUCKET_HUGE];
+    if (cnt == 0) return;
     const uint32_t base = bucket_base(q, BUCKET_HUGE);
     uint32_t* pull = &q[Q_PULL + Q_STRIDE * BUCKET_HUGE];
     while (true) {
@@ -1182,13 +1397,7 @@ __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out
         team_process<TC_WAVES, 1, false, PLAIN, LIST>(V, x, tail_bounds(V, x), L, nullptr, nullptr, nullptr, 0, 0,
                                                             prm.team_chunk, out, my_total, wk, uid);
     }
-    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), isz = wedge + wk.recv();
-    if (lane_id() == 0) {
-        if (my_total) atomic_add_u64(&out.totals[0], my_total);
-        if (wedge) atomic_add_u64(&stats[ST_WEDGE], wedge);
-        if (isz) atomic_add_u64(&stats[ST_ISZ], isz);
-        if (streamed) atomic_add_u64(&stats[ST_STREAM], streamed);
-    }
+    flush_sums<TC_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(L.keys), sums);
 }
 
 // Tails above the workgroup bin whose hash table fits one workgroup's LDS
@@ -1197,7 +1406,8 @@ __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out
 template <bool PLAIN, bool LIST>
 __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out, TcParams prm,
                                                         uint32_t* __restrict__ q, const uint32_t* __restrict__ list,
-                                                        uint64_t* __restrict__ stats) {
+                                                        uint64_t* __restrict__ sums) {
+    own_copy(out);
     __shared__ LdsBig L;
     __shared__ uint32_t uids[LIST ? BIG_THREADS : 1];
     uint32_t* uid = uids + (LIST ? threadIdx.x / KT_WAVE * KT_WAVE : 0);
@@ -1228,12 +1438,259 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
                                                             big_table + BIG_SLOTS, L.ovf, BIG_SLOTS, prm.table_shift,
                                                             prm.team_chunk, out, my_total, wk, uid);
     }
-    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), isz = wedge + wk.recv();
-    if (lane_id() == 0) {
-        if (my_total) atomic_add_u64(&out.totals[0], my_total);
-        if (wedge) atomic_add_u64(&stats[ST_WEDGE], wedge);
-        if (isz) atomic_add_u64(&stats[ST_ISZ], isz);
-        if (streamed) atomic_add_u64(&stats[ST_STREAM], streamed);
+    flush_sums<BIG_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(big_table), sums);
+}
+
+// ---------------------------------------------------------------------------
+// hub tails
+// ---------------------------------------------------------------------------
+constexpr int HUB_THREADS = 768;
+constexpr int HUB_WAVES = HUB_THREADS / KT_WAVE;
+struct HubPack {
+    uint2 rec[KT_WAVE];
+    union {
+        uint32_t bits[KT_WAVE];  // while a window is set up
+        uint32_t ucnt[KT_WAVE];  // while it is walked
+    };
+};
+constexpr uint64_t REC_BIAS = 1ull << 25;     // keeps a list's start less its blocks' ids above zero
+constexpr uint32_t REC_END = (1u << 25) - 1;  // low bits of rec.y: the list's end; above them the start's high bits
+
+constexpr uint32_t HUB_CNT = GROUP_SLOTS / 2 + 4;  // counters: 1 .. |S(x)|, |S(x)| <= 2048
+constexpr uint32_t HUB_LDS = (2 * HUB_MAX + 16) + 4 * HUB_CNT + HUB_WAVES * sizeof(HubPack);
+static_assert(2 * (HUB_LDS + 256) <= 160 * 1024, "two workgroups per CU");
+
+// Eight hub-list entries at 2-byte alignment; one global_load_dwordx4.
+struct __attribute__((packed, aligned(2))) Hubs8 {
+    uint32_t x, y, z, w;
+};
+
+// walk_lists over hub lists, eight entries (16 bytes) per block and lane:
+// tab (byte offsets from the list entries) holds the byte offset of a set
+// member's counter, zero for all others, so a lookup is one 2-byte LDS read
+// and one compare, against five compares and an address of two instructions
+// in a hash bucket.
+__device__ __forceinline__ uint32_t walk_hub_lists(const uint16_t* __restrict__ lists, uint64_t tb, uint64_t rem,
+                                                   const char* tab, char* cnt, HubPack& pk, uint64_t& total) {
+    const uint32_t lane = lane_id();
+    const uint16_t* __restrict__ T = lists - REC_BIAS;
+    uint32_t mine = 0;
+    total = 0;
+    while (true) {
+        const uint32_t len = (uint32_t)min<uint64_t>(rem, ROUND_IDS);
+        const uint64_t nem = __builtin_amdgcn_ballot_w64(len != 0);
+        if (nem == 0) break;
+        const uint32_t nb = (len + 7) >> 3;
+        const uint32_t incl = wave_scan_dpp(nb);
+        const uint32_t first = incl - nb;
+        const uint32_t blocks = readlane32(incl, KT_WAVE - 1);
+        const uint32_t rank = rank_below(nem, 0);
+        const bool bounded = len != 0 && rank != 0;
+        if (len) {
+            const uint64_t t0 = tb + REC_BIAS - 8ull * first;
+            pk.rec[rank] = uint2{(uint32_t)t0, (len + 8 * first) | ((uint32_t)(t0 >> 32) << 25)};
+        }
+        for (uint32_t w0 = 0; w0 < blocks; w0 += WINDOW) {
+            pk.bits[lane] = 0;
+            wave_sync();
+            const uint32_t at = first - 1 - w0;
+            if (bounded && at < WINDOW) atomicOr(&pk.bits[at >> 5], 1u << (at & 31));
+            wave_sync();
+            const uint32_t bits = pk.bits[lane];
+            uint32_t base = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(bounded && first <= w0));
+            wave_sync();
+            pk.ucnt[lane] = 0;
+            wave_sync();
+            const uint32_t steps = min((blocks - w0 + KT_WAVE - 1) / KT_WAVE, WINDOW / KT_WAVE);
+            uint64_t ends = 0;
+            uint32_t rk = 0;
+            int lim = 0;
+            Hubs8 q;
+            // (s == steps, loaded but not probed: every lane takes the step's
+            // first block, which is in list `base`, or the last block there is)
+            auto load = [&](uint32_t s) {
+                const bool over = s == steps;
+                const int l0 = over ? 0 : (int)(2 * s);
+                ends = over ? 0 : (uint64_t)readlane32(bits, l0) | ((uint64_t)readlane32(bits, l0 + 1) << 32);
+                rk = rank_below(ends, base);
+                base += (uint32_t)__popcll(ends);
+                const uint2 r = pk.rec[rk];
+                const uint32_t p = w0 + s * KT_WAVE + (over ? 0 : lane);
+                lim = p < blocks ? (int)(r.y & REC_END) - (int)(8 * p) : 0;
+                q = *reinterpret_cast<const Hubs8*>(
+                    T + ((((uint64_t)(r.y >> 25) << 32) | r.x) + 8ull * min(p, blocks - 1)));
+            };
+            load(0);
+            for (uint32_t s = 0; s < steps; ++s) {
+                const uint32_t d[4] = {q.x, q.y, q.z, q.w};
+                const uint64_t c_ends = ends;
+                const uint32_t c_rk = rk;
+                const int c_lim = lim;
+                load(s + 1);
+                uint32_t t[8];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    t[2 * k] = *reinterpret_cast<const uint16_t*>(tab + (d[k] & 0xffffu));
+                    t[2 * k + 1] = *reinterpret_cast<const uint16_t*>(tab + (d[k] >> 16));
+                }
+                uint32_t nh = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const bool hit = k < c_lim && t[k] != 0;
+                    nh += hit ? 1u : 0u;
+                    if (hit) atomicAdd(reinterpret_cast<uint32_t*>(cnt + t[k]), 1u);
+                }
+                if (__builtin_amdgcn_ballot_w64(nh != 0)) {
+                    const uint32_t sum = wave_scan_dpp(nh);
+                    total += readlane32(sum, KT_WAVE - 1);
+                    const bool end = (c_ends >> lane) & 1;
+                    if (end || lane == KT_WAVE - 1) atomicAdd(&pk.ucnt[c_rk], sum);
+                    if (end && lane != KT_WAVE - 1) atomicSub(&pk.ucnt[c_rk + 1], sum);
+                }
+            }
+            wave_sync();
+            if (len) mine += pk.ucnt[rank];
+            wave_sync();
+        }
+        tb += len;
+        rem -= len;
+    }
+    return mine;
+}
+
+// Workgroup tails that are hubs, part by part: 16-wave teams, two workgroups
+// per CU, each with a table of one entry per hub in dynamic LDS.  The table is
+// empty between parts (the thread that set an entry clears it).
+__global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6)))
+    k_tc_hub(View<true> V, TcOut out, TcParams prm, uint32_t* __restrict__ q, const uint64_t* __restrict__ plist,
+             const uint16_t* __restrict__ lists, uint64_t* __restrict__ sums) {
+    own_copy(out);
+    extern __shared__ uint32_t hub_lds[];
+    __shared__ uint64_t red[HUB_WAVES];
+    __shared__ uint32_t next_u, bcast;
+    const uint32_t parts = q[Q_CNT + BUCKET_HUB_PARTS];
+    if (parts == 0) return;
+    const uint32_t base = bucket_base(q, BUCKET_HUB_PARTS);
+    uint32_t* pull = &q[Q_PULL + Q_STRIDE * BUCKET_HUB_PARTS];
+    // counters first: their byte offsets from the start fit two bytes, and a
+    // table entry is one
+    char* cnt = reinterpret_cast<char*>(hub_lds);
+    char* tab = cnt + 4 * HUB_CNT;
+    const uint32_t tid = threadIdx.x, wave = tid / KT_WAVE, lane = lane_id();
+    HubPack& pk = reinterpret_cast<HubPack*>(tab + 2 * HUB_MAX + 16)[wave];
+    for (uint32_t i = tid; i < (2 * HUB_MAX + 16) / 4 + HUB_CNT; i += HUB_THREADS) hub_lds[i] = 0;
+    __syncthreads();
+    uint64_t my_total = 0;
+    WorkStats wk;
+    const uint32_t fixed = parts <= 4 * gridDim.x ? parts : parts - parts / 4;
+    uint32_t i = blockIdx.x;
+    // the tail and bounds of the fixed share's next part, loaded a part ahead
+    uint64_t xp_nx = i < parts ? plist[base + i] : 0;
+    TailBounds tb_nx = part_bounds(V, (uint32_t)xp_nx, (uint32_t)(xp_nx >> 32), prm.hub_split);
+    while (true) {
+        if (i >= fixed) {
+            if (fixed == parts) break;
+            if (tid == 0)
+                bcast = (__hip_atomic_load(pull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= parts - fixed)
+                            ? parts
+                            : fixed + atomicAdd(pull, 1u);
+            __syncthreads();
+            i = bcast;
+            __syncthreads();
+            if (i >= parts) break;
+            xp_nx = plist[base + i];
+            tb_nx = part_bounds(V, (uint32_t)xp_nx, (uint32_t)(xp_nx >> 32), prm.hub_split);
+        }
+        const uint32_t x = uniform((uint32_t)xp_nx);
+        const TailBounds tb = tb_nx;
+        const uint64_t sb = uniform64(tb.sb), rb = uniform64(tb.rb);
+        const uint32_t ns = uniform(tb.ns), nr = uniform(tb.nr);
+        const uint32_t chunk = min((uint32_t)KT_WAVE, max(1u, (nr + 2 * HUB_WAVES - 1) / (2 * HUB_WAVES)));
+        uint32_t k = wave * chunk;
+        uint32_t u_nx = 0, kw_nx = 0;
+        if (k < nr && lane < min(chunk, nr - k)) V.entry_head(rb + k + lane, u_nx, kw_nx);
+        for (uint32_t j = tid; j < ns; j += HUB_THREADS)
+            *reinterpret_cast<uint16_t*>(tab + lists[sb + j]) = (uint16_t)(4 * (j + 1));
+        if (tid == 0) next_u = HUB_WAVES * chunk;
+        const uint32_t i_nx = i + gridDim.x;
+        if (i_nx < fixed) xp_nx = plist[base + i_nx];
+        __syncthreads();
+        uint64_t hsum = 0;
+        while (k < nr) {
+            const uint32_t c = min(chunk, nr - k), u = u_nx, kw = kw_nx;
+            uint32_t nk = 0;
+            if (lane == 0) nk = atomicAdd(&next_u, chunk);
+            nk = uniform(nk);
+            if (nk < nr && lane < min(chunk, nr - nk)) V.entry_head(rb + nk + lane, u_nx, kw_nx);
+            uint64_t b = 0, e = 0, stl = 0;
+            bool stc = false;
+            if (lane < c) V.entry_bounds(rb + k + lane, u, kw, ns, b, e, stl, stc);
+            const uint64_t len = e > b ? e - b : 0;
+            wk.wedge_lane += stl;
+            wk.recv_lane += stc ? ns : 0u;
+            wk.stream_lane += len;
+            uint64_t hits;
+            const uint32_t h = walk_hub_lists(lists, b, len, tab, cnt, pk, hits);
+            if (h && out.per_vertex) atomic_add_u64(&out.per_vertex[u], h);
+            hsum += hits;
+            k = nk;
+        }
+        if (lane == 0) red[wave] = hsum;
+        if (i_nx < fixed) tb_nx = part_bounds(V, (uint32_t)xp_nx, (uint32_t)(xp_nx >> 32), prm.hub_split);
+        __syncthreads();
+        for (uint32_t j = tid; j < ns; j += HUB_THREADS) {
+            uint32_t* p = reinterpret_cast<uint32_t*>(cnt + 4 * (j + 1));
+            const uint32_t c = *p;
+            if (c) {
+                if (out.per_vertex) atomic_add_u64(&out.per_vertex[V.v.sheads[sb + j]], c);
+                *p = 0;
+            }
+            *reinterpret_cast<uint16_t*>(tab + lists[sb + j]) = 0;
+        }
+        if (tid == 0) {
+            hsum = 0;
+            for (int w = 0; w < HUB_WAVES; ++w) hsum += red[w];
+            if (hsum) {
+                if (out.per_vertex) atomic_add_u64(&out.per_vertex[x], hsum);
+                my_total += hsum;
+            }
+        }
+        __syncthreads();
+        i = i < fixed ? i_nx : fixed;
+    }
+    flush_sums<HUB_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(hub_lds), sums);
+}
+
+// Adds up the per-XCD copies of the n per-vertex counts (n == 0: none) and,
+// in the first block, the workgroups' sums.
+__global__ void __launch_bounds__(256) k_tc_finish(uint64_t n, const uint64_t* __restrict__ copies,
+                                                   uint64_t* __restrict__ pv, uint32_t rows,
+                                                   const uint64_t* __restrict__ sums, uint64_t* __restrict__ stats,
+                                                   uint64_t* __restrict__ total) {
+    for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) {
+        uint64_t s = 0;
+#pragma unroll
+        for (int c = 0; c < NXCD; ++c) s += copies[c * n + v];
+        if (s) pv[v] += s;
+    }
+    if (blockIdx.x != 0) return;
+    __shared__ uint64_t red[256 / KT_WAVE][SUM_WORDS];
+    uint64_t t[SUM_WORDS] = {};
+    for (uint32_t r = threadIdx.x; r < rows; r += 256)
+#pragma unroll
+        for (int k = 0; k < SUM_WORDS; ++k) t[k] += sums[(uint64_t)r * SUM_WORDS + k];
+#pragma unroll
+    for (int k = 0; k < SUM_WORDS; ++k) {
+        const uint64_t w = wave_sum(t[k]);
+        if (lane_id() == 0) red[threadIdx.x / KT_WAVE][k] = w;
+    }
+    __syncthreads();
+    if (threadIdx.x < SUM_WORDS) {
+        const uint64_t x = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+        if (threadIdx.x == SUM_TOTAL)
+            *total += x;
+        else
+            stats[threadIdx.x] = x;
     }
 }
 
@@ -1244,7 +1701,7 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
 // long rows (an R-MAT hub's row has a large share of all entries) do not
 // leave the rest of the chip waiting for the team that drew them.
 struct Split {
-    uint32_t wave, team;
+    uint32_t wave, team, hub;
 };
 
 static Split split_rule(uint64_t entries, int num_cus) {
@@ -1254,36 +1711,58 @@ static Split split_rule(uint64_t entries, int num_cus) {
         while (p < want && p < hi) p <<= 1;
         return (uint32_t)p;
     };
-    return {size(entries / (2 * waves), 16, 1024), size(entries / (4 * teams), 128, 4096)};
+    return {size(entries / (2 * waves), 16, 1024), size(entries / (4 * teams), 128, 4096),
+            size(entries / (16 * (uint64_t)num_cus), 256, 4096)};
 }
 
 // A walk of r > split entries becomes ceil(r / split) <= 2 r / split parts.
-static uint64_t max_parts(uint64_t entries, const Split& s) {
-    return 2 * entries / s.team + (s.wave < 1024 ? 2 * entries / s.wave : 0);
+// A hub tail is at least one part.
+static uint64_t max_parts(uint64_t entries, const Split& s, bool hubs) {
+    if (!entries) return 0;
+    return 2 * entries / s.team + (s.wave < 1024 ? 2 * entries / s.wave : 0) +
+           (hubs ? HUB_MAX + 2 * entries / s.hub : 0);
 }
 
-uint64_t tc_ws_words(uint32_t X, uint64_t entries, int num_cus) {
-    // queue header (u32) + stats (u64) + one u32 list of X + the part list
-    return Q_WORDS / 2 + ST_WORDS + (uint64_t(X) + 1) / 2 + 1 +
-           (entries ? max_parts(entries, split_rule(entries, num_cus)) : 0);
+static uint64_t parts_of(const TcRoom& r, int num_cus) {
+    return max_parts(r.entries, split_rule(r.entries, num_cus), r.hub_slots != 0);
+}
+
+// queue header, stats and sums; one u32 list of X; the part list, the
+// hubs, the copies of the per-vertex counts
+uint64_t tc_ws_words(uint32_t X, const TcRoom& room, int num_cus) {
+    return head_words(num_cus) + (uint64_t(X) + 1) / 2 + 1 + parts_of(room, num_cus) +
+           hub_ws_words(X, room.hub_slots) + NXCD * room.pv_n;
+}
+
+TcRoom tc_room(uint64_t entries, uint64_t slots, uint64_t pv_n) {
+    TcRoom r;
+    r.entries = entries;
+    // below, the launches for the hubs cost what they gain (R-MAT n = 65,521 with
+    // 1.8 M entries: 206 us without, 213 us with)
+    if (entries >= (1ull << 22)) r.hub_slots = slots;
+    if (pv_n <= (1ull << 22)) r.pv_n = pv_n;
+    return r;
 }
 
 uint64_t* tc_stats_ptr(uint64_t* ws) { return ws + Q_WORDS / 2; }
 
 template <bool PLAIN>
-static hipError_t launch_impl(const TcView& view, const TcOut& out, const TcParams& prm, uint64_t* ws, int num_cus,
+static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const TcParams& prm, uint64_t* ws, int num_cus,
                               hipStream_t st, hipEvent_t ev_begin, hipEvent_t ev_end) {
     (void)hipGetLastError();  // a status left by an earlier call is not this launch's
     View<PLAIN> V;
     V.v = view;
+    TcOut out = user_out;
     // min-side walks move triangles between tails: listing launches (and
     // their per-tail counting pass) keep every triangle at its first vertex
     if (out.tri || out.tail_count) V.v.in_off = nullptr;
     uint32_t* q = reinterpret_cast<uint32_t*>(ws);
     uint64_t* stats = ws + Q_WORDS / 2;
-    uint32_t* list = reinterpret_cast<uint32_t*>(stats + ST_WORDS);
-    uint64_t* plist = stats + ST_WORDS + (uint64_t(view.X) + 1) / 2 + 1;
-    fill_u64(ws, Q_WORDS / 2 + ST_WORDS, 0, st);
+    uint64_t* sums = stats + ST_WORDS;
+    auto row = [&](int r) { return sums + (uint64_t)r * num_cus * SUM_WORDS; };
+    uint32_t* list = reinterpret_cast<uint32_t*>(ws + head_words(num_cus));
+    uint64_t* plist = ws + head_words(num_cus) + (uint64_t(view.X) + 1) / 2 + 1;
+    fill_u64(ws, head_words(num_cus), 0, st);
     TcParams p = prm;
     if (p.wave_max_deg > WAVE_SLOTS / 2) p.wave_max_deg = WAVE_SLOTS / 2;
     if (p.group_max_deg > GROUP_SLOTS / 2) p.group_max_deg = GROUP_SLOTS / 2;
@@ -1296,48 +1775,87 @@ static hipError_t launch_impl(const TcView& view, const TcOut& out, const TcPara
     V.v.in_hash_max = p.bsearch_min_deg;
     // parts: the workspace holds the part list of view.entries entries; a
     // listing writes whole tails
-    p.wave_split = p.team_split = 0xffffffffu;
-    if (view.entries && !out.tri && !out.tail_count) {
-        const Split sp = split_rule(view.entries, num_cus);
+    p.wave_split = p.team_split = p.hub_split = 0xffffffffu;
+    HubWs hub{};
+    uint64_t* room = plist + parts_of(view.room, num_cus);
+    if (view.room.entries && !out.tri && !out.tail_count) {
+        const Split sp = split_rule(view.room.entries, num_cus);
         p.team_split = sp.team;
         if (sp.wave < 1024) p.wave_split = sp.wave;
+        if (PLAIN && view.room.hub_slots && view.deg && view.X) {
+            p.hub_split = sp.hub;
+            hub = hub_ws(room, view.X);
+            fill_u64(room, HUB_HEAD_WORDS, 0, st);
+            // few blocks: each adds up to a thousand bins to the global ones
+            k_hub_hist<<<std::clamp<unsigned>(view.X / (32 * HUB_HIST_THREADS), 1, HUB_BLOCKS), HUB_HIST_THREADS, 0,
+                         st>>>(view.X, view.deg, view.room.entries, hub);
+        }
+    }
+    room += hub_ws_words(view.X, view.room.hub_slots);
+    uint64_t* const pv = user_out.per_vertex;
+    if (pv && view.room.pv_n) {
+        out.per_vertex = room;
+        out.pv_stride = view.room.pv_n;
+        fill_u64(room, NXCD * view.room.pv_n, 0, st);
     }
     // a min-side walk covers in- and out-neighbours and streams from only
     // some of them: four times the entries per team grab
     if (V.v.in_off) p.team_chunk = std::min<uint32_t>(4 * std::max<uint32_t>(p.team_chunk, 1), KT_WAVE);
     if (view.X > 0) {
-        const unsigned g = std::min<unsigned>((view.X + 255) / 256, (unsigned)num_cus * 8);
-        k_tc_bin_count<PLAIN><<<g, 256, 0, st>>>(V, p, q, stats);
-        k_tc_bin_fill<PLAIN><<<g, 256, 0, st>>>(V, p, q, list, plist);
+        const unsigned g = std::min<unsigned>((view.X + BIN_THREADS - 1) / BIN_THREADS, (unsigned)num_cus);
+        k_tc_bin_count<PLAIN><<<g, BIN_THREADS, 0, st>>>(V, p, q, hub.min_bin, row(ROW_BIN));
+        k_tc_bin_fill<PLAIN><<<g, BIN_THREADS, 0, st>>>(V, p, q, hub.min_bin, list, plist);
     }
     // no more workgroups than fit at once (three per CU): shares are fixed per
     // workgroup, and one that starts late would hold its share back
     const unsigned grid = (unsigned)num_cus * std::clamp<unsigned>(p.grid_per_cu, 1, 3);
+    auto finish = [&]() {
+        const uint64_t n = out.pv_stride;
+        k_tc_finish<<<(unsigned)std::clamp<uint64_t>((n + 255) / 256, 1, 4096), 256, 0, st>>>(
+            n, out.per_vertex, pv, (uint32_t)(ROWS * num_cus), sums, stats, out.totals);
+    };
     constexpr uint32_t big_lds = 2 * BIG_SLOTS * sizeof(uint32_t);
     if constexpr (PLAIN) {
         if (out.tri) {  // listing: streamed walks only
-            k_tc_huge<PLAIN, true><<<(unsigned)num_cus, TC_THREADS, 0, st>>>(V, out, p, q, list, stats);
+            k_tc_huge<PLAIN, true><<<(unsigned)num_cus, TC_THREADS, 0, st>>>(V, out, p, q, list, row(ROW_HUGE));
             static const hipError_t big_list_ok =
                 hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tc_big<PLAIN, true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)big_lds);
             if (big_list_ok != hipSuccess) return big_list_ok;
-            k_tc_big<PLAIN, true><<<(unsigned)num_cus, BIG_THREADS, big_lds, st>>>(V, out, p, q, list, stats);
+            k_tc_big<PLAIN, true><<<(unsigned)num_cus, BIG_THREADS, big_lds, st>>>(V, out, p, q, list, row(ROW_BIG));
             if (ev_begin) (void)hipEventRecord(ev_begin, st);
-            k_tc_main<PLAIN, true><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, plist, stats);
+            k_tc_main<PLAIN, true><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, plist, row(ROW_MAIN));
+            finish();
             if (ev_end) (void)hipEventRecord(ev_end, st);
             return hipGetLastError();
         }
     }
     // huge and big tails are rare: one workgroup per CU; they exit at once
-    // when there are none
-    k_tc_huge<PLAIN, false><<<(unsigned)num_cus, TC_THREADS, 0, st>>>(V, out, p, q, list, stats);
-    static const hipError_t big_ok =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tc_big<PLAIN, false>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)big_lds);
-    if (big_ok != hipSuccess) return big_ok;
-    k_tc_big<PLAIN, false><<<(unsigned)num_cus, BIG_THREADS, big_lds, st>>>(V, out, p, q, list, stats);
+    // when there are none, and are not launched where none can be
+    auto longer = [&](uint64_t s) { return view.sym_slots == 0 || view.sym_slots > s * s; };
+    if (longer(p.bsearch_min_deg))
+        k_tc_huge<PLAIN, false><<<(unsigned)num_cus, TC_THREADS, 0, st>>>(V, out, p, q, list, row(ROW_HUGE));
+    if (longer(p.group_max_deg)) {
+        static const hipError_t big_ok =
+            hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tc_big<PLAIN, false>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)big_lds);
+        if (big_ok != hipSuccess) return big_ok;
+        k_tc_big<PLAIN, false><<<(unsigned)num_cus, BIG_THREADS, big_lds, st>>>(V, out, p, q, list, row(ROW_BIG));
+    }
     if (ev_begin) (void)hipEventRecord(ev_begin, st);
-    k_tc_main<PLAIN, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, plist, stats);
+    if constexpr (PLAIN) {
+        if (hub.lists) {
+            static const hipError_t hub_ok = hipFuncSetAttribute(
+                reinterpret_cast<const void*>(&k_tc_hub), hipFuncAttributeMaxDynamicSharedMemorySize, (int)HUB_LDS);
+            if (hub_ok != hipSuccess) return hub_ok;
+            k_hub_number<<<HUB_BLOCKS, HUB_NUMBER_THREADS, 0, st>>>(view.X, view.deg, hub, q);
+            k_hub_lists<<<(unsigned)std::min<uint64_t>((view.room.hub_slots + 1023) / 1024, (uint64_t)num_cus * 16), 256, 0,
+                          st>>>(view.X, view.s_off, view.sheads, hub, q);
+            k_tc_hub<<<2 * (unsigned)num_cus, HUB_THREADS, HUB_LDS, st>>>(V, out, p, q, plist, hub.lists, row(ROW_HUB));
+        }
+    }
+    k_tc_main<PLAIN, false><<<grid, TC_THREADS, 0, st>>>(V, out, p, q, list, plist, row(ROW_MAIN));
+    finish();
     if (ev_end) (void)hipEventRecord(ev_end, st);
     return hipGetLastError();  // a launch that did not start (e.g. LDS beyond the device's limit)
 }

@@ -1,0 +1,124 @@
+"""How the intersection shares out tails, at the sizes where that can go wrong.
+
+Closed forms (cliques, wheels) for the edges of packs, parts, list blocks and
+windows; the oracle for a skewed graph whose workgroup tails are partly hubs.
+"""
+import numpy as np
+import pytest
+
+import katric_amd as K
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _cliques(sizes):
+    """Disjoint cliques: (graph, per-vertex counts)."""
+    edges, pv, at = [], [], 0
+    for k in sizes:
+        iu = np.triu_indices(k, 1)
+        edges.append(np.stack(iu, 1) + at)
+        pv.append(np.full(k, (k - 1) * (k - 2) // 2, np.uint64))
+        at += k
+    return K.Graph.from_edges(at, np.concatenate(edges)), np.concatenate(pv)
+
+
+def _wheel(n):
+    """Vertex 0 joined to a cycle of n - 1 > 3 vertices."""
+    rim = np.arange(1, n)
+    e = np.concatenate([np.stack([np.zeros(n - 1, np.int64), rim], 1),
+                        np.stack([rim, np.roll(rim, -1)], 1)])
+    pv = np.full(n, 2, np.uint64)
+    pv[0] = n - 1
+    return K.Graph.from_edges(n, e), pv
+
+
+@pytest.fixture
+def knobs(ctx):
+    saved = ctx.params()
+    yield ctx.set_params
+    ctx.set_params(**saved)
+
+
+def _check(ctx, g, pv):
+    total, got = ctx.count(g)
+    np.testing.assert_array_equal(got, pv)
+    assert total == int(pv.sum()) // 3
+
+
+@pytest.mark.parametrize("order", [K.ORDER_DEGREE, K.ORDER_VERTEX])
+@pytest.mark.parametrize("min_side", [0, 1])
+# one wave's pack: 64 set members and 64 entries; its tables: 512 slots
+@pytest.mark.parametrize("sizes", [[2, 3, 4, 5] * 40, [63, 64, 65, 66, 67], [3] * 500 + [33, 64, 65] * 8,
+                                   list(range(2, 140))])
+def test_packs(ctx, knobs, sizes, min_side, order):
+    knobs(min_side=min_side, order=order)
+    g, pv = _cliques(sizes)
+    _check(ctx, g, pv)
+
+
+@pytest.mark.parametrize("order", [K.ORDER_DEGREE, K.ORDER_VERTEX])
+# a row of one part, two parts, and of many parts (the least and the largest part size)
+@pytest.mark.parametrize("n", [5, 17, 65, 513, 514, 1025, 4097, 5000, 300_001])
+def test_long_rows(ctx, knobs, n, order):
+    knobs(order=order)
+    g, pv = _wheel(n)
+    _check(ctx, g, pv)
+
+
+@pytest.mark.parametrize("wave_max_deg", [2, 128, 256])
+# cliques beyond 2^22 slots have hub tails (every vertex is one) with list lengths over the blocks of
+# eight and the windows of 2048 blocks; 2100 also has tails above the workgroup bin
+@pytest.mark.parametrize("k", [1025, 2049, 2052, 2100])
+def test_hub_cliques(ctx, knobs, k, wave_max_deg):
+    knobs(wave_max_deg=wave_max_deg)
+    g, pv = _cliques([k, 5, 64])
+    _check(ctx, g, pv)
+
+
+@pytest.mark.parametrize("per_vertex", [True, False])
+@pytest.mark.parametrize("unsorted", [False, True])
+def test_hubs_and_others(ctx, knobs, unsorted, per_vertex):
+    knobs(wave_max_deg=32)
+    g = K.gen_rmat(18, 16, seed=5)  # 262144 vertices: more than there are hubs
+    ot, opv, ost = O.run_shmem(g, threads=4)
+    if unsorted:
+        heads = g.heads.copy()
+        for v in range(g.n):
+            a, b = int(g.offsets[v]), int(g.offsets[v + 1])
+            heads[a:b] = heads[a:b][::-1]
+        g = K.Graph(g.n, g.offsets, heads)
+    total, pv = ctx.count(g, per_vertex=per_vertex)
+    assert total == ot
+    if per_vertex:
+        np.testing.assert_array_equal(pv, opv)
+    st = ctx.stats()
+    assert st["wedge_checks"] == ost["wedge_checks"]
+    assert st["intersection_size_local"] == ost["intersection_size_local"]
+
+
+def test_no_hubs_in_a_regular_graph(ctx):
+    # a circulant graph of 40000 vertices and degree 32: one degree bin, more
+    # vertices than hubs can be.  i ~ i + 1 .. i + 16: triangles at i are pairs
+    # (a, b) of distinct offsets in +-1 .. +-16 whose difference is one too
+    n, k = 40_000, 16
+    i = np.arange(n)
+    e = np.concatenate([np.stack([i, (i + d) % n], 1) for d in range(1, k + 1)])
+    offs = [d for d in range(-k, k + 1) if d]
+    per = sum(1 for a in offs for b in offs if a < b and 0 < b - a <= k)
+    _check(ctx, K.Graph.from_edges(n, e), np.full(n, per, np.uint64))
+
+
+def test_tight_budget_counts_without_the_optional_room():
+    # a budget that holds the buffers every count needs, but not part list,
+    # hub lists and per-vertex copies beside them
+    g = K.gen_rmat(16, 16, seed=3)
+    want = O.run_shmem(g, threads=4)
+    with K.Context(0) as free:
+        free.count(g)
+        rich = free.device_bytes()
+    with K.Context(0, hbm_budget_bytes=rich - 64 * g.n) as tight:
+        total, pv = tight.count(g)
+        assert tight.device_bytes() < rich - 64 * g.n + 1
+    assert total == want[0]
+    np.testing.assert_array_equal(pv, want[1])
