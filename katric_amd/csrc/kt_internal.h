@@ -48,6 +48,11 @@ void sym_check_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint3
 void random_keys(uint64_t key[2]);
 void orient_write_launch(uint32_t n, uint64_t nnz, const uint32_t* heads, uint32_t* oheads, uint64_t* ws,
                          hipStream_t st);
+// Writes the entries of heads[0, nnz) whose bit is set to out, in order; bits
+// hold 64 entries a word, tile_off the number of set bits before every tile of
+// 2048 entries.
+void emit_bits_launch(uint64_t nnz, const uint32_t* heads, const uint64_t* bits, const uint64_t* tile_off,
+                      uint32_t* out, hipStream_t st);
 // The keep bitmask of the input slots (bit i: slot i is an out-edge) inside
 // the orientation workspace; valid after orient_count_launch.
 const uint64_t* orient_keep_bits(uint32_t n, uint64_t nnz, const uint64_t* ws);

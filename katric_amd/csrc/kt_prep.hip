@@ -986,8 +986,14 @@ void random_keys(uint64_t key[2]) {
 // input showed a symmetric, well-formed CSR (kept == nnz / 2).
 void orient_write_launch(uint32_t n, uint64_t nnz, const uint32_t* heads, uint32_t* oheads, uint64_t* ws,
                          hipStream_t st) {
-    OrientWs w = orient_ws(n, nnz, ws);
-    if (w.tiles > 0) k_orient_emit<<<(unsigned)w.tiles, OR_THREADS, 0, st>>>(nnz, heads, w.bits, w.tile_off, oheads);
+    const OrientWs w = orient_ws(n, nnz, ws);
+    emit_bits_launch(nnz, heads, w.bits, w.tile_off, oheads, st);
+}
+
+void emit_bits_launch(uint64_t nnz, const uint32_t* heads, const uint64_t* bits, const uint64_t* tile_off,
+                      uint32_t* out, hipStream_t st) {
+    const uint64_t tiles = (nnz + OR_TILE - 1) / OR_TILE;
+    if (tiles > 0) k_orient_emit<<<(unsigned)tiles, OR_THREADS, 0, st>>>(nnz, heads, bits, tile_off, out);
 }
 
 void make_keys(uint32_t n, uint64_t m, const uint64_t* ooff, const uint32_t* oheads, uint64_t* keys,

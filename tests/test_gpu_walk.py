@@ -122,3 +122,31 @@ def test_tight_budget_counts_without_the_optional_room():
         assert tight.device_bytes() < rich - 64 * g.n + 1
     assert total == want[0]
     np.testing.assert_array_equal(pv, want[1])
+
+
+@pytest.mark.parametrize("lens", [
+    [(0, 5), (5, 0), (0, 0), (1, 1)],                      # empty lists
+    [(2047, 10), (1, 2048), (2048, 3000), (2049, 1)],      # a tile's edges
+    [(6000, 7), (7, 6000), (64, 64), (63, 65)] * 3,        # lists over several tiles
+    [(1, 1)] * 3000 + [(0, 1)] * 5000 + [(3, 2)] * 100,    # more pairs than a tile has ids
+])
+def test_intersect_tiles(ctx, lens):
+    rng = np.random.default_rng(7)
+    pairs = [tuple(np.sort(rng.choice(2 * (la + lb) + 1, n, replace=False)).astype(np.uint32) for n in (la, lb))
+             for la, lb in lens]
+    counts, matches = ctx.intersect(pairs)
+    for (a, b), c, m in zip(pairs, counts, matches):
+        want = np.intersect1d(a, b)
+        assert c == len(want)
+        np.testing.assert_array_equal(m, want)
+
+
+@pytest.mark.parametrize("at", [0, 63, 64, 2047, 2048, 4999])
+def test_intersect_order_check_at_tile_edges(ctx, at):
+    ids = np.arange(1, 5002, dtype=np.uint32)
+    bad = ids.copy()
+    bad[at + 1] = bad[at]
+    for pair in ((bad, ids), (ids, bad)):
+        with pytest.raises(K.KatricError):
+            ctx.intersect([pair])
+    assert ctx.intersect([(ids, ids[::2])])[0].tolist() == [2501]
