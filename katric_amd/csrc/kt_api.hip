@@ -1,5 +1,6 @@
 // C ABI of katric_amd: context, device workspace, plain count / orient.
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -128,6 +129,26 @@ void kt_ctx::release_aux() {
         aux[i] = nullptr;
         aux_bytes[i] = 0;
     }
+}
+
+namespace kt {
+__global__ void k_peek(const uint64_t* a, const uint64_t* b, uint64_t* host) {
+    host[0] = *a;
+    host[1] = *b;
+}
+}  // namespace kt
+
+int kt_ctx::read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what) {
+    // a kernel that writes to page-locked memory: one round trip of a few
+    // microseconds instead of two copies and two waits
+    k_peek<<<1, 1, 0, stream>>>(a, b, host_small + 62);
+    int rc = hip_check(hipGetLastError(), what);
+    if (!rc) rc = hip_check(hipStreamSynchronize(stream), what);
+    if (!rc) {
+        out[0] = host_small[62];
+        out[1] = host_small[63];
+    }
+    return rc;
 }
 
 int kt_ctx::read_u64(const uint64_t* dev, uint64_t* out, const char* what) {
@@ -342,9 +363,10 @@ int bits_for(uint64_t x) {
     return b;
 }
 
-// Uploads host input (if any) and runs the count pass of the orientation.
+// Uploads host input (if any) and runs the count pass of the orientation; with
+// `wait`, its flags and kept slots are then in c->host_small[0] and [1].
 int upload_and_count(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_off, const uint32_t* user_heads,
-                     bool host_in, PlainBufs& B) {
+                     bool host_in, PlainBufs& B, bool wait = true) {
     hipStream_t st = c->stream;
     int rc;
     if (host_in) {
@@ -362,12 +384,16 @@ int upload_and_count(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_o
         B.off = user_off;
         B.heads = user_heads;
     }
-    (void)hipEventRecord(c->ev[EV_H2D], st);
+    if (host_in) (void)hipEventRecord(c->ev[EV_H2D], st);
     trace("upload done, launching count pass");
-    fill_u64(B.small, 64, 0, st);
+    ClearList cl;
+    cl.add(B.small, 64);
+    tc_clear(B.ws_tc, n, B.room, c->num_cus, cl);
+    clear(cl, st);
     OrientCheck chk{{c->sym_key[0], c->sym_key[1]}};
     orient_count_launch(n, nnz, B.off, B.heads, B.deg, B.ooff, B.ws_orient, reinterpret_cast<uint32_t*>(B.small), chk,
                         st);
+    if (!wait) return KT_OK;
     rc = c->hip_check(hipMemcpyAsync(c->host_small, B.small, 8, hipMemcpyDeviceToHost, st), "D2H flags");
     if (rc) return rc;
     rc = c->hip_check(hipMemcpyAsync(c->host_small + 1, B.ooff + n, 8, hipMemcpyDeviceToHost, st), "D2H kept");
@@ -394,9 +420,35 @@ struct Workspace {
     }
 };
 
+int check_flags(kt_ctx* c, uint32_t flags, uint64_t kept, uint64_t nnz) {
+    if (flags & (KT_ERR_MASK & ~KT_ERR_ASYMMETRIC)) {
+        return c->fail(KT_EINVAL, "malformed CSR:%s%s%s%s", (flags & KT_ERR_OFFSETS) ? " bad offsets" : "",
+                       (flags & KT_ERR_HEAD_RANGE) ? " head id >= n" : "",
+                       (flags & KT_ERR_SELF_LOOP) ? " self-loop" : "",
+                       (flags & KT_ERR_DUPLICATE) ? " duplicate edge" : "");
+    }
+    if (flags & KT_ERR_ASYMMETRIC)
+        return c->fail(KT_EINVAL, "CSR is not symmetric (some slot v -> u has no slot u -> v)");
+    if (2 * kept != nnz) {
+        return c->fail(KT_EINVAL, "CSR is not symmetric (%llu oriented edges for %llu slots)",
+                       (unsigned long long)kept, (unsigned long long)nnz);
+    }
+    return KT_OK;
+}
+
+// No list of such a CSR is longer than the in-place sort takes (|N+(v)| <=
+// sqrt(nnz)), so whether its lists need sorting is the device's affair and the
+// whole call can be queued at once: the flags of the checks keep every later
+// kernel from writing or walking anything when the input is malformed.
+bool one_round(uint64_t nnz, const PlainBufs& B, bool want_pv) {
+    return nnz <= (uint64_t)segsort_max_len() * segsort_max_len() && B.room.entries && (!want_pv || B.room.pv_n);
+}
+
+// With *queued, a call that is `one_round` returns with everything queued and
+// *queued set; its flags are still to be read.
 int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_off, const uint32_t* user_heads,
                     bool host_in, bool want_pv, bool pv_dev_needed, PlainBufs& B, bool& unsorted,
-                    const Workspace& ws = {}) {
+                    const Workspace& ws = {}, bool* queued = nullptr) {
     hipStream_t st = c->stream;
     unsorted = false;
     // the intersection's optional room is left out where only it does not fit
@@ -419,23 +471,23 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
     layout(ws.base(c));
     trace("workspace=%p bytes=%llu", ws.base(c), (unsigned long long)ws.cap(c));
     (void)hipEventRecord(c->ev[EV_START], st);
+    if (queued && one_round(nnz, B, want_pv)) {
+        *queued = true;
+        uint32_t* err = reinterpret_cast<uint32_t*>(B.small);
+        rc = upload_and_count(c, n, nnz, user_off, user_heads, host_in, B, false);
+        if (rc) return rc;
+        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, err, st);
+        const uint64_t len = std::min<uint64_t>((uint64_t)std::sqrt((double)nnz) + 1, segsort_max_len());
+        segsort_launch(n, B.ooff, B.oheads, err, len, c->num_cus, st);
+        return KT_OK;
+    }
     rc = upload_and_count(c, n, nnz, user_off, user_heads, host_in, B);
     if (rc) return rc;
     uint32_t flags = static_cast<uint32_t>(c->host_small[0]);
     uint64_t kept = c->host_small[1];
     trace("count pass: flags=0x%x kept=%llu", flags, (unsigned long long)kept);
-    if (flags & (KT_ERR_MASK & ~KT_ERR_ASYMMETRIC)) {
-        return c->fail(KT_EINVAL, "malformed CSR:%s%s%s%s", (flags & KT_ERR_OFFSETS) ? " bad offsets" : "",
-                       (flags & KT_ERR_HEAD_RANGE) ? " head id >= n" : "",
-                       (flags & KT_ERR_SELF_LOOP) ? " self-loop" : "",
-                       (flags & KT_ERR_DUPLICATE) ? " duplicate edge" : "");
-    }
-    if (flags & KT_ERR_ASYMMETRIC)
-        return c->fail(KT_EINVAL, "CSR is not symmetric (some slot v -> u has no slot u -> v)");
-    if (2 * kept != nnz) {
-        return c->fail(KT_EINVAL, "CSR is not symmetric (%llu oriented edges for %llu slots)",
-                       (unsigned long long)kept, (unsigned long long)nnz);
-    }
+    rc = check_flags(c, flags, kept, nnz);
+    if (rc) return rc;
     const uint64_t m = nnz / 2;
     uint64_t max_len = 0;
     if (flags & KT_FLAG_UNSORTED) {
@@ -452,7 +504,7 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
     }
     if ((flags & KT_FLAG_UNSORTED) && max_len <= segsort_max_len()) {
         unsorted = true;
-        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, st);
+        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, reinterpret_cast<uint32_t*>(B.small), st);
         segsort_launch(n, B.ooff, B.oheads, reinterpret_cast<uint32_t*>(B.small), max_len, c->num_cus, st);
         rc = c->hip_check(hipMemcpyAsync(c->host_small, B.small, 8, hipMemcpyDeviceToHost, st), "D2H flags");
         if (rc) return rc;
@@ -478,7 +530,7 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
                 B.heads = user_heads;
             }
         }
-        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, st);
+        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, reinterpret_cast<uint32_t*>(B.small), st);
         make_keys(n, m, B.ooff, B.oheads, B.keys, st);
         radix_sort_u64(B.keys, B.alt, m, 32 + bits_for(n), B.ws_radix, st);
         keys_to_heads(m, B.keys, B.oheads, reinterpret_cast<uint32_t*>(B.small), st);
@@ -489,7 +541,7 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
         flags = static_cast<uint32_t>(c->host_small[0]);
         if (flags & KT_ERR_MASK) return c->fail(KT_EINVAL, "malformed CSR: duplicate edge");
     } else {
-        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, st);
+        orient_write_launch(n, nnz, B.heads, B.oheads, B.ws_orient, reinterpret_cast<uint32_t*>(B.small), st);
     }
     c->stats.oriented_edges = kept;
     c->stats.vertices = n;
@@ -500,9 +552,7 @@ int run_orientation(kt_ctx* c, uint32_t n, uint64_t nnz, const uint64_t* user_of
 int read_nnz(kt_ctx* c, uint32_t n, const uint64_t* offsets, uint32_t flags, uint64_t& nnz) {
     if (flags & KT_DEVICE_INPUT) {
         uint64_t v[2] = {0, 0};
-        int rc = c->read_u64(offsets, v, "D2H offsets[0]");
-        if (rc) return rc;
-        rc = c->read_u64(offsets + n, v + 1, "D2H offsets[n]");
+        int rc = c->read_2u64(offsets, offsets + n, v, "D2H offsets");
         if (rc) return rc;
         if (v[0] != 0) return c->fail(KT_EINVAL, "offsets[0] != 0");
         nnz = v[1];
@@ -536,15 +586,20 @@ int kt::count_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, const uint3
     const bool want_pv = per_vertex_out != nullptr;
     const bool pv_dev = want_pv && (flags & KT_DEVICE_OUTPUT);
     PlainBufs B;
-    bool unsorted;
-    rc = run_orientation(c, n, nnz, offsets, heads, host_in, want_pv, want_pv && !pv_dev, B, unsorted, ws);
+    bool unsorted, queued = false;
+    rc = run_orientation(c, n, nnz, offsets, heads, host_in, want_pv, want_pv && !pv_dev, B, unsorted, ws, &queued);
     if (rc) return rc;
     hipStream_t st = c->stream;
     (void)hipEventRecord(c->ev[EV_PREP], st);
     uint64_t* pv = want_pv ? (pv_dev ? per_vertex_out : B.pv) : nullptr;
-    if (pv) fill_u64(pv, n, 0, st);
+    if (pv && !B.room.pv_n) fill_u64(pv, n, 0, st);
     uint64_t* totals = B.small + 1;
     TcView view{};
+    view.cleared = queued || !unsorted;  // by the count pass (the longest list's search writes there too)
+    view.gate = reinterpret_cast<uint32_t*>(B.small);
+    view.gate_bits = KT_ERR_MASK;
+    view.host_out = c->host_small;
+    view.kept = B.ooff + n;
     view.X = n;
     view.s_off = B.ooff;
     view.sheads = B.oheads;
@@ -571,32 +626,43 @@ int kt::count_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, const uint3
                       "intersection launch");
     if (rc) return rc;
     (void)hipEventRecord(c->ev[EV_COUNT], st);
-    uint64_t* tstats = tc_stats_ptr(B.ws_tc);
-    rc = c->hip_check(hipMemcpyAsync(c->host_small + 1, totals, 8, hipMemcpyDeviceToHost, st), "D2H total");
-    if (rc) return rc;
-    rc = c->hip_check(hipMemcpyAsync(c->host_small + 2, tstats, 32, hipMemcpyDeviceToHost, st), "D2H stats");
-    if (rc) return rc;
-    if (want_pv && !pv_dev) {
+    const bool copy_pv = want_pv && !pv_dev;
+    if (queued || !copy_pv) {
+        rc = c->hip_check(hipStreamSynchronize(st), "count");
+        if (rc) return rc;
+    }
+    if (queued) {
+        const uint32_t fl = (uint32_t)c->host_small[0];
+        unsorted = (fl & KT_FLAG_UNSORTED) != 0;
+        rc = check_flags(c, fl, c->host_small[1], nnz);
+        if (rc) return rc;
+        c->stats.oriented_edges = c->host_small[1];
+        c->stats.vertices = n;
+        c->stats.input_slots = nnz;
+    }
+    if (copy_pv) {
         rc = c->hip_check(hipMemcpyAsync(per_vertex_out, pv, uint64_t(n) * 8, hipMemcpyDeviceToHost, st),
                           "D2H per-vertex");
         if (rc) return rc;
+        (void)hipEventRecord(c->ev[EV_END], st);
+        rc = c->hip_check(hipStreamSynchronize(st), "count");
+        if (rc) return rc;
     }
-    (void)hipEventRecord(c->ev[EV_END], st);
-    rc = c->hip_check(hipStreamSynchronize(st), "count");
-    if (rc) return rc;
-    trace("count done: total=%llu", (unsigned long long)c->host_small[1]);
-    *total_out = c->host_small[1];
-    c->stats.local_triangles = c->host_small[1];
-    c->stats.wedge_checks = c->host_small[2];
-    c->stats.intersection_size_local = c->host_small[3];
-    c->stats.skipped_nodes = c->host_small[4];
-    c->stats.streamed_ids = c->host_small[5];
-    c->timing.h2d_ms = c->elapsed(EV_START, EV_H2D);
-    c->timing.prep_ms = c->elapsed(EV_H2D, EV_PREP);
+    trace("count done: total=%llu", (unsigned long long)c->host_small[2]);
+    *total_out = c->host_small[2];
+    c->stats.local_triangles = c->host_small[2];
+    c->stats.wedge_checks = c->host_small[3];
+    c->stats.intersection_size_local = c->host_small[4];
+    c->stats.skipped_nodes = c->host_small[5];
+    c->stats.streamed_ids = c->host_small[6];
+    // (events that would fall together are recorded once)
+    const int h2d = host_in ? EV_H2D : EV_START, end = copy_pv ? EV_END : EV_COUNT;
+    c->timing.h2d_ms = host_in ? c->elapsed(EV_START, EV_H2D) : 0.f;
+    c->timing.prep_ms = c->elapsed(h2d, EV_PREP);
     c->timing.count_ms = c->elapsed(EV_PREP, EV_COUNT);
     c->timing.intersect_ms = c->elapsed(EV_TC0, EV_TC1);
-    c->timing.d2h_ms = c->elapsed(EV_COUNT, EV_END);
-    c->timing.total_ms = c->elapsed(EV_START, EV_END);
+    c->timing.d2h_ms = copy_pv ? c->elapsed(EV_COUNT, EV_END) : 0.f;
+    c->timing.total_ms = c->elapsed(EV_START, end);
     return KT_OK;
 }
 
@@ -691,8 +757,8 @@ extern "C" int kt_list_triangles(kt_ctx* c, uint32_t n, const uint64_t* offsets,
     (void)hipEventRecord(c->ev[EV_END], st);
     rc = c->hip_check(hipStreamSynchronize(st), "listing");
     if (rc) return rc;
-    c->timing.h2d_ms = c->elapsed(EV_START, EV_H2D);
-    c->timing.prep_ms = c->elapsed(EV_H2D, EV_PREP);
+    c->timing.h2d_ms = host_in ? c->elapsed(EV_START, EV_H2D) : 0.f;
+    c->timing.prep_ms = c->elapsed(host_in ? EV_H2D : EV_START, EV_PREP);
     c->timing.count_ms = c->elapsed(EV_PREP, EV_COUNT);
     c->timing.intersect_ms = c->elapsed(EV_TC0, EV_TC1);
     c->timing.d2h_ms = c->elapsed(EV_COUNT, EV_END);

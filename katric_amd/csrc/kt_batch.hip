@@ -133,12 +133,17 @@ hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, cons
                           uint64_t nnz, uint64_t* pv, uint64_t* h_totals, uint64_t* h_small, uint32_t sort,
                           const uint64_t sym_key[2]) {
     uint32_t* err = reinterpret_cast<uint32_t*>(B.small);
-    fill_u64(B.small, 64, 0, st);
+    ClearList cl;
+    cl.add(B.small, 64);
+    cl.add(pv, N);
+    cl.add(B.totals, G);
+    tc_clear(B.ws_tc, (uint32_t)N, B.room, num_cus, cl);
+    clear(cl, st);
     // heads must stay inside their row's graph: a union with edges between
     // graphs is not a batch of independent graphs
     OrientCheck chk{{sym_key[0], sym_key[1]}, B.vbase, G};
     orient_count_launch((uint32_t)N, nnz, B.off, B.heads, B.deg, B.ooff, B.ws_orient, err, chk, st);
-    orient_write_launch((uint32_t)N, nnz, B.heads, B.oheads, B.ws_orient, st);
+    orient_write_launch((uint32_t)N, nnz, B.heads, B.oheads, B.ws_orient, err, st);
     if (sort == SORT_SEGMENTED) {
         segsort_launch((uint32_t)N, B.ooff, B.oheads, err, segsort_max_len(), num_cus, st);
     } else if (sort == SORT_RADIX) {
@@ -147,8 +152,8 @@ hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, cons
         radix_sort_u64(B.keys, B.alt, m, 32 + bits_for(N), B.ws_radix, st);
         keys_to_heads(m, B.keys, B.oheads, err, st);
     }
-    fill_u64(pv, N, 0, st);
     TcView v{};
+    v.cleared = true;
     v.X = (uint32_t)N;
     v.s_off = B.ooff;
     v.sheads = B.oheads;
@@ -167,7 +172,6 @@ hipError_t batch_pipeline(hipStream_t st, int num_cus, const TcParams& prm, cons
     TcOut o{pv, B.small + 2};
     const hipError_t le = tc_launch(v, o, prm, B.ws_tc, num_cus, st, nullptr, nullptr);
     if (le != hipSuccess) return le;
-    fill_u64(B.totals, G, 0, st);
     k_seg_partial<<<(unsigned)std::clamp<uint64_t>((N + SEG_CHUNK * 4 - 1) / (SEG_CHUNK * 4), 1, 16384), 256, 0, st>>>(
         G, N, B.vbase, pv, B.totals);
     k_seg_final<<<std::min<uint32_t>((G + 255) / 256, 1024), 256, 0, st>>>(G, B.totals, err);

@@ -69,6 +69,7 @@ struct kt_ctx {
     int reserve_aux(int i, uint64_t bytes);
     void release_aux();
     // One device word, read in order after the work queued on `stream`.
+    int read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what);
     int read_u64(const uint64_t* dev, uint64_t* out, const char* what);
     void destroy_extensions();
 };

@@ -46,20 +46,22 @@ void sym_check_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint3
                       uint32_t* err, const OrientCheck& chk, hipStream_t st);
 // A random key pair for OrientCheck.
 void random_keys(uint64_t key[2]);
+// (err: device flags; with an error among them nothing is written)
 void orient_write_launch(uint32_t n, uint64_t nnz, const uint32_t* heads, uint32_t* oheads, uint64_t* ws,
-                         hipStream_t st);
+                         const uint32_t* err, hipStream_t st);
 // Writes the entries of heads[0, nnz) whose bit is set to out, in order; bits
 // hold 64 entries a word, tile_off the number of set bits before every tile of
 // 2048 entries.
 void emit_bits_launch(uint64_t nnz, const uint32_t* heads, const uint64_t* bits, const uint64_t* tile_off,
-                      uint32_t* out, hipStream_t st);
+                      uint32_t* out, const uint32_t* err, hipStream_t st);
 // The keep bitmask of the input slots (bit i: slot i is an out-edge) inside
 // the orientation workspace; valid after orient_count_launch.
 const uint64_t* orient_keep_bits(uint32_t n, uint64_t nnz, const uint64_t* ws);
 void make_keys(uint32_t n, uint64_t m, const uint64_t* ooff, const uint32_t* oheads, uint64_t* keys,
                hipStream_t st);
 void keys_to_heads(uint64_t m, const uint64_t* keys, uint32_t* oheads, uint32_t* err, hipStream_t st);
-// Segmented in-place sort of the oriented lists oheads[ooff[v] .. ooff[v+1])
+// Segmented in-place sort, where the device flags err say that lists are
+// unsorted (and nothing worse), of the oriented lists oheads[ooff[v] .. ooff[v+1])
 // of up to segsort_max_len() ids each, max_len being the longest (duplicates
 // set KT_ERR_DUPLICATE); max_len_launch writes the longest list's length to
 // *out, using tmp (segsort_tmp_words() words).
@@ -73,6 +75,18 @@ void segsort_launch(uint32_t n, const uint64_t* ooff, uint32_t* oheads, uint32_t
 // pipeline stays capturable in a HIP graph.
 void fill_u64(uint64_t* p, uint64_t count, uint64_t value, hipStream_t st);
 void fill_u32(uint32_t* p, uint64_t count, uint32_t value, hipStream_t st);
+// Several ranges of words zeroed by one launch.
+struct ClearList {
+    uint64_t* p[6];
+    uint64_t n[6];
+    uint32_t count = 0;
+    void add(uint64_t* q, uint64_t words) {
+        if (!words) return;
+        p[count] = q;
+        n[count++] = words;
+    }
+};
+void clear(const ClearList& c, hipStream_t st);
 
 // Intersection tuning knobs (bin thresholds, table sizes); see kt_tc.hip.
 struct TcParams {
@@ -162,6 +176,12 @@ struct TcView {
     // queued, so input that failed its checks is never walked
     const uint32_t* gate = nullptr;
     uint32_t gate_bits = 0;
+    bool cleared = false;  // the caller cleared tc_clear's ranges
+    // host words (page-locked; nullable) that receive the gate word, *kept, the
+    // total and the four work counters at the end; with them, per_vertex is
+    // assigned (room.pv_n set) and left alone when the gate is closed
+    uint64_t* host_out = nullptr;
+    const uint64_t* kept = nullptr;
 };
 
 struct TcOut {
@@ -215,6 +235,8 @@ uint64_t tc_ws_words(uint32_t X, const TcRoom& room, int num_cus);
 // The room that pays for walks of at most `entries` entries, `slots` oriented
 // slots (0: the view has no hubs) and pv_n per-vertex counts (0: none).
 TcRoom tc_room(uint64_t entries, uint64_t slots, uint64_t pv_n);
+// Adds the ranges of the launch workspace that have to be zero.
+void tc_clear(uint64_t* ws, uint32_t X, const TcRoom& room, int num_cus, ClearList& c);
 // Enqueues binning and the intersection kernels; returns the launch status.
 hipError_t tc_launch(const TcView& view, const TcOut& out, const TcParams& prm, uint64_t* ws, int num_cus,
                      hipStream_t st, hipEvent_t ev_begin, hipEvent_t ev_end);

@@ -329,7 +329,7 @@ extern "C" int kt_intersect(kt_ctx* c, uint64_t num_pairs, const uint64_t* a_off
             dm = static_cast<uint32_t*>(c->aux[1]);
         }
         if (tiles)
-            emit_bits_launch(na, a, bits, toff, dm, st);
+            emit_bits_launch(na, a, bits, toff, dm, nullptr, st);
         else
             k_isect<true><<<grid, IS_THREADS, 0, st>>>(P, aoff, a, na, boff, b, nb, nullptr, toff, dm, err);
         if (!dev_out) {

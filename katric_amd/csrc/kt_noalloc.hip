@@ -18,7 +18,9 @@
 
 namespace kt {
 
-constexpr uint64_t NOALLOC_BYTES = KT_NOALLOC_SCRATCH_BYTES;
+// a little more than promised: the intersection's queue and sums (150 KB) come
+// on top of what the limit in the header counts
+constexpr uint64_t NOALLOC_BYTES = KT_NOALLOC_SCRATCH_BYTES + (256ull << 10);
 constexpr int MAX_DEVICES = 64;
 
 // the workspace (per GPU); every kernel of a call is handed scratch_ptr[d]

@@ -112,14 +112,20 @@ void scan_u64(const uint64_t* in, uint64_t* out, uint64_t len, uint64_t* tmp, hi
 // ---------------------------------------------------------------------------
 // degrees + offset validation
 // ---------------------------------------------------------------------------
+// Also clears the out-degrees (n + 1) and notes the rows that hold the first
+// and last slot of every `tile`-slot tile (bnd: two entries per tile; with
+// offsets that fail the check some keep what the workspace held).
 __global__ void k_degree(uint32_t n, uint64_t nnz, const uint64_t* __restrict__ off, uint32_t* __restrict__ deg,
-                         uint8_t* __restrict__ ncls, uint32_t* __restrict__ err) {
+                         uint8_t* __restrict__ ncls, uint64_t* __restrict__ dplus, uint64_t tile,
+                         uint32_t* __restrict__ bnd, uint32_t* __restrict__ err) {
     // blockDim is a multiple of 64: vertices 2i and 2i+1 sit in one wave
     const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v == 0 && (off[0] != 0 || off[n] != nnz)) atomicOr(err, KT_ERR_OFFSETS);
     uint32_t c = 0;
+    uint64_t a = 0, b = 0;
     if (v < n) {
-        const uint64_t a = off[v], b = off[v + 1];
+        a = off[v];
+        b = off[v + 1];
         uint32_t d = 0;
         if (b < a || b - a > 0xffffffffull)
             atomicOr(err, KT_ERR_OFFSETS);
@@ -128,8 +134,16 @@ __global__ void k_degree(uint32_t n, uint64_t nnz, const uint64_t* __restrict__ 
         deg[v] = d;
         c = deg_class4(d);
     }
+    if (v <= n) dplus[v] = 0;
     const uint32_t c1 = (uint32_t)__shfl_down((int)c, 1, KT_WAVE);
     if (v < n && (v & 1) == 0) ncls[v >> 1] = (uint8_t)(c | (v + 1 < n ? c1 << 4 : 0u));
+    b = min(b, nnz);
+    if (b > a)
+        for (uint64_t t = a / tile; t * tile < b; ++t) {
+            if (t * tile >= a) bnd[2 * t] = (uint32_t)v;
+            const uint64_t last = min((t + 1) * tile, nnz) - 1;
+            if (last >= a && last < b) bnd[2 * t + 1] = (uint32_t)v;
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -238,7 +252,7 @@ __global__ void __launch_bounds__(OR_THREADS)
     for (int i = tid; i < OR_TILE; i += OR_THREADS) rowcnt[i] = 0;
     if (tid == 0) bflags = 0;
     uint32_t lo, hi;
-    tile_rows<OR_THREADS, OR_ITEMS>(off, n, tile0, tend, marks, bnd, wmax, lo, hi, tbnd);
+    tile_rows<OR_THREADS, OR_ITEMS>(off, n, tile0, tend, marks, bnd, wmax, lo, hi, tbnd, err);
     const uint64_t nrows = (uint64_t)hi - lo + 1;
     const bool lds_rows = nrows <= OR_TILE;
     TileGraphs tg{};
@@ -361,34 +375,145 @@ __global__ void __launch_bounds__(OR_THREADS)
     }
 }
 
-// Folds the per-tile pair checksums (tiles entries) and the kept count into
-// the error flags: a symmetric CSR keeps exactly half of its slots and its
-// checksum is zero.  One 1024-thread block, eight independent loads in flight
-// per thread (a batch of 2^31 slots has half a million tiles).
-constexpr int SYM_FINAL_THREADS = 1024;
-__global__ void __launch_bounds__(SYM_FINAL_THREADS) k_sym_final(const uint64_t* __restrict__ sym_part,
-                                                                 uint64_t tiles, const uint64_t* __restrict__ kept,
-                                                                 uint64_t nnz, uint32_t* __restrict__ err) {
+// The sum of the per-tile pair checksums, by a 1024-thread block: eight
+// independent loads in flight per thread (a batch of 2^31 slots has half a
+// million tiles).  The total is thread 0's.
+constexpr int ONE_THREADS = 1024;
+__device__ __forceinline__ uint64_t sym_sum(const uint64_t* __restrict__ sym_part, uint64_t tiles, uint64_t* lw) {
     constexpr int U = 8;
-    __shared__ uint64_t lw[SYM_FINAL_THREADS / KT_WAVE];
     uint64_t s[U] = {};
     uint64_t i = threadIdx.x;
-    for (; i + (U - 1) * SYM_FINAL_THREADS < tiles; i += U * SYM_FINAL_THREADS)
+    for (; i + (U - 1) * ONE_THREADS < tiles; i += U * ONE_THREADS)
 #pragma unroll
-        for (int k = 0; k < U; ++k) s[k] += sym_part[i + (uint64_t)k * SYM_FINAL_THREADS];
-    for (; i < tiles; i += SYM_FINAL_THREADS) s[0] += sym_part[i];
+        for (int k = 0; k < U; ++k) s[k] += sym_part[i + (uint64_t)k * ONE_THREADS];
+    for (; i < tiles; i += ONE_THREADS) s[0] += sym_part[i];
 #pragma unroll
     for (int k = 1; k < U; ++k) s[0] += s[k];
-    const uint64_t w = wave_incl_sum(s[0]);
-    if (lane_id() == KT_WAVE - 1) lw[threadIdx.x / KT_WAVE] = w;
+    const uint64_t w = wave_sum(s[0]);
+    if (lane_id() == 0) lw[threadIdx.x / KT_WAVE] = w;
     __syncthreads();
-    if (threadIdx.x != 0) return;
     uint64_t tot = 0;
+    if (threadIdx.x == 0)
+        for (int k = 0; k < ONE_THREADS / KT_WAVE; ++k) tot += lw[k];
+    return tot;
+}
+
+// Folds the per-tile pair checksums (tiles entries) into the error flags: the
+// checksum of a symmetric CSR is zero.
+__global__ void __launch_bounds__(ONE_THREADS) k_sym_final(const uint64_t* __restrict__ sym_part, uint64_t tiles,
+                                                           uint32_t* __restrict__ err) {
+    __shared__ uint64_t lw[ONE_THREADS / KT_WAVE];
+    if (sym_sum(sym_part, tiles, lw) != 0) atomicOr(err, KT_ERR_ASYMMETRIC);
+}
+
+// The two scans behind the orientation count pass, together: kept slots per
+// tile and out-degrees (each three launches of its own before, of 4 to 6 us).
+// Short arrays take one block (k_scan_one); longer ones per-tile sums, their
+// scan by k_scan_one, and a pass that adds the tiles' bases.
+struct ScanJob {
+    const uint64_t* in;
+    uint64_t* out;  // len + 1 entries; may alias in
+    uint64_t len;
+    uint64_t* sums;  // tiles + 1 entries
+    uint64_t tiles;
+};
+
+// Exclusive scan of len entries by one block, four per thread and step;
+// returns the total.
+__device__ __forceinline__ uint64_t scan_block(const uint64_t* in, uint64_t* out, uint64_t len, uint64_t* lw) {
+    constexpr int I = 4;
+    uint64_t carry = 0;
+    for (uint64_t i0 = 0; i0 < len; i0 += ONE_THREADS * I) {
+        const uint64_t i = i0 + threadIdx.x * I;
+        uint64_t v[I], s = 0;
 #pragma unroll
-    for (int k = 0; k < SYM_FINAL_THREADS / KT_WAVE; ++k) tot += lw[k];
-    bool bad = tot != 0;
-    if (kept) bad |= 2 * kept[0] != nnz;
-    if (bad) atomicOr(err, KT_ERR_ASYMMETRIC);
+        for (int k = 0; k < I; ++k) {
+            v[k] = i + k < len ? in[i + k] : 0;
+            s += v[k];
+        }
+        const uint64_t incl = wave_incl_sum(s);
+        if (lane_id() == KT_WAVE - 1) lw[threadIdx.x / KT_WAVE] = incl;
+        __syncthreads();
+        uint64_t run = carry + incl - s;
+#pragma unroll
+        for (unsigned w = 0; w < ONE_THREADS / KT_WAVE; ++w) {
+            const uint64_t t = lw[w];
+            if (w < threadIdx.x / KT_WAVE) run += t;
+            carry += t;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < I; ++k) {
+            if (i + k < len) out[i + k] = run;
+            run += v[k];
+        }
+    }
+    if (threadIdx.x == 0) out[len] = carry;
+    return carry;
+}
+
+// Scans both arrays (or their tiles' sums); then the checks of the whole CSR: a
+// symmetric one keeps exactly half of its slots -- the second array's total --
+// and its checksum is zero.
+__global__ void __launch_bounds__(ONE_THREADS)
+    k_scan_one(const uint64_t* in0, uint64_t* out0, uint64_t len0, const uint64_t* in1, uint64_t* out1, uint64_t len1,
+               const uint64_t* __restrict__ sym_part, uint64_t tiles, uint64_t nnz, uint32_t* __restrict__ err) {
+    __shared__ uint64_t lw[ONE_THREADS / KT_WAVE];
+    scan_block(in0, out0, len0, lw);
+    const uint64_t kept = scan_block(in1, out1, len1, lw);
+    const uint64_t sym = sym_sum(sym_part, tiles, lw);
+    if (threadIdx.x == 0 && (sym != 0 || 2 * kept != nnz)) atomicOr(err, KT_ERR_ASYMMETRIC);
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(ScanJob a, ScanJob b) {
+    __shared__ uint64_t lw[SCAN_THREADS / KT_WAVE];
+    const bool second = blockIdx.x >= a.tiles;
+    const uint64_t* in = second ? b.in : a.in;
+    const uint64_t len = second ? b.len : a.len, tile = second ? blockIdx.x - a.tiles : blockIdx.x;
+    const uint64_t base = tile * SCAN_TILE + threadIdx.x;
+    uint64_t s = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i)
+        if (base + i * SCAN_THREADS < len) s += in[base + i * SCAN_THREADS];
+    uint64_t tot;
+    block_excl_sum(s, lw, &tot);
+    if (threadIdx.x == 0) (second ? b.sums : a.sums)[tile] = tot;
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob a, ScanJob b) {
+    __shared__ uint64_t lw[SCAN_THREADS / KT_WAVE];
+    const bool second = blockIdx.x >= a.tiles;
+    const ScanJob j{second ? b.in : a.in, second ? b.out : a.out, second ? b.len : a.len, second ? b.sums : a.sums,
+                    second ? b.tiles : a.tiles};
+    const uint64_t tile = second ? blockIdx.x - a.tiles : blockIdx.x;
+    const uint64_t base = tile * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
+    uint64_t v[SCAN_ITEMS], s = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i) {
+        v[i] = (base + i < j.len) ? j.in[base + i] : 0;
+        s += v[i];
+    }
+    uint64_t tot;
+    uint64_t run = block_excl_sum(s, lw, &tot) + j.sums[tile];
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i) {
+        if (base + i < j.len) j.out[base + i] = run;
+        run += v[i];
+    }
+    if (tile == j.tiles - 1 && threadIdx.x == 0) j.out[j.len] = j.sums[j.tiles];
+}
+
+// (one block up to 16384 entries: four steps)
+static void orient_scans(ScanJob a, ScanJob b, const uint64_t* sym, uint64_t tiles, uint64_t nnz, uint32_t* err,
+                         hipStream_t st) {
+    if (a.len <= 4 * SCAN_TILE && b.len <= 4 * SCAN_TILE) {
+        k_scan_one<<<1, ONE_THREADS, 0, st>>>(a.in, a.out, a.len, b.in, b.out, b.len, sym, tiles, nnz, err);
+        return;
+    }
+    const unsigned g = (unsigned)(a.tiles + b.tiles);
+    k_scan_sums<<<g, SCAN_THREADS, 0, st>>>(a, b);
+    k_scan_one<<<1, ONE_THREADS, 0, st>>>(a.sums, a.sums, a.tiles, b.sums, b.sums, b.tiles, sym, tiles, nnz, err);
+    k_scan_apply<<<g, SCAN_THREADS, 0, st>>>(a, b);
 }
 
 // Validation of a whole CSR without orienting it (rows resolved per tile as
@@ -455,7 +580,8 @@ __global__ void __launch_bounds__(OR_THREADS)
 // which each wave derives all its output positions.
 __global__ void __launch_bounds__(OR_THREADS)
     k_orient_emit(uint64_t nnz, const uint32_t* __restrict__ heads, const uint64_t* __restrict__ keep_bits,
-                  const uint64_t* __restrict__ tile_off, uint32_t* __restrict__ oheads) {
+                  const uint64_t* __restrict__ tile_off, uint32_t* __restrict__ oheads,
+                  const uint32_t* __restrict__ err) {
     constexpr int NW = OR_THREADS / KT_WAVE;
     __shared__ uint32_t wcnt[OR_ITEMS][NW];
     const uint64_t tile0 = (uint64_t)blockIdx.x * OR_TILE;
@@ -469,6 +595,8 @@ __global__ void __launch_bounds__(OR_THREADS)
         hv[k] = (w0 + lane < nnz) ? heads[w0 + lane] : 0u;
     }
     uint64_t base = tile_off[blockIdx.x];
+    // input that failed its checks may keep more slots than oheads has room for
+    if (err && (*err & KT_ERR_MASK)) return;
 #pragma unroll
     for (int k = 0; k < OR_ITEMS; ++k)
         if (lane == 0) wcnt[k][wave] = (uint32_t)__popcll(bits[k]);
@@ -523,6 +651,10 @@ constexpr uint32_t SEG_THREAD_MAX = 16;
 constexpr uint32_t SEG_WAVE_MAX = 1024;
 constexpr uint32_t SEG_MAX = 4096;
 constexpr int SEG_BLOCK = 256;
+
+__device__ __forceinline__ bool unsorted_only(uint32_t flags) {
+    return (flags & (KT_FLAG_UNSORTED | KT_ERR_MASK)) == KT_FLAG_UNSORTED;
+}
 
 __device__ __forceinline__ void cas(uint32_t& a, uint32_t& b) {
     const uint32_t lo = min(a, b), hi = max(a, b);
@@ -587,9 +719,12 @@ __device__ __forceinline__ uint32_t wave_sort_list(uint32_t* __restrict__ p, uin
 // Rows of 64-row chunks, one chunk per wave: lists of <= 16 ids sorted by
 // their own lane, then the chunk's lists of 17..1024 ids one after another by
 // the whole wave.
+// A list above max_len, which no list of a simple graph exceeds, holds an edge
+// twice.
 __global__ void __launch_bounds__(SEG_BLOCK) k_segsort_small(uint32_t n, const uint64_t* __restrict__ ooff,
-                                                             uint32_t* __restrict__ oheads,
+                                                             uint32_t* __restrict__ oheads, uint64_t max_len,
                                                              uint32_t* __restrict__ err) {
+    if (!unsorted_only(*err)) return;
     const uint32_t lane = lane_id();
     const uint64_t nw = (uint64_t)gridDim.x * (SEG_BLOCK / KT_WAVE);
     uint32_t flags = 0;
@@ -601,6 +736,7 @@ __global__ void __launch_bounds__(SEG_BLOCK) k_segsort_small(uint32_t n, const u
             e = ooff[v + 1];
         }
         const uint32_t len = (uint32_t)(e - b);
+        if (e - b > max_len) flags |= KT_ERR_DUPLICATE;
         if (len >= 2 && len <= SEG_THREAD_MAX) {
             uint32_t a[SEG_THREAD_MAX];
 #pragma unroll
@@ -659,8 +795,14 @@ __global__ void __launch_bounds__(SEG_BLOCK) k_segsort_large(uint32_t n, const u
     __shared__ uint32_t rows[SEG_BLOCK];
     __shared__ uint32_t nrows;
     __shared__ uint32_t bflags;
+    __shared__ bool run;
     const uint32_t tid = threadIdx.x;
-    if (tid == 0) bflags = 0;
+    if (tid == 0) {
+        bflags = 0;
+        run = unsorted_only(*err);
+    }
+    __syncthreads();
+    if (!run) return;
     for (uint64_t c0 = (uint64_t)blockIdx.x * SEG_BLOCK; c0 < n; c0 += (uint64_t)gridDim.x * SEG_BLOCK) {
         if (tid == 0) nrows = 0;
         __syncthreads();
@@ -752,7 +894,7 @@ void segsort_launch(uint32_t n, const uint64_t* ooff, uint32_t* oheads, uint32_t
     if (n == 0 || max_len < 2) return;
     const uint64_t chunks = ((uint64_t)n + KT_WAVE - 1) / KT_WAVE;
     const uint32_t g1 = (uint32_t)std::min<uint64_t>((chunks + 3) / 4, (uint64_t)num_cus * 32);
-    k_segsort_small<<<g1, SEG_BLOCK, 0, st>>>(n, ooff, oheads, err);
+    k_segsort_small<<<g1, SEG_BLOCK, 0, st>>>(n, ooff, oheads, max_len, err);
     if (max_len <= SEG_WAVE_MAX) return;
     const uint32_t g2 = (uint32_t)std::min<uint64_t>(((uint64_t)n + SEG_BLOCK - 1) / SEG_BLOCK, (uint64_t)num_cus * 8);
     k_segsort_large<<<g2, SEG_BLOCK, 0, st>>>(n, ooff, oheads, err);
@@ -890,6 +1032,12 @@ struct OrientWs {
     uint32_t* tgraph;    // 2 * tiles: batch, graphs of each tile's first and last row
 };
 
+// The sums of both scans (no more than the scans took one after the other).
+static uint64_t orient_scan_words(uint32_t n, uint64_t tiles) {
+    return std::max(std::max(scan_tmp_words(tiles + 1), scan_tmp_words((uint64_t)n + 1)),
+                    (tiles + SCAN_TILE - 1) / SCAN_TILE + ((uint64_t)n + SCAN_TILE - 1) / SCAN_TILE + 2);
+}
+
 static OrientWs orient_ws(uint32_t n, uint64_t nnz, uint64_t* ws) {
     OrientWs w;
     w.tiles = (nnz + OR_TILE - 1) / OR_TILE;
@@ -900,7 +1048,7 @@ static OrientWs orient_ws(uint32_t n, uint64_t nnz, uint64_t* ws) {
     w.dplus = w.bits + (nnz + 63) / 64 + 1;
     w.tbnd = reinterpret_cast<uint32_t*>(w.dplus + (uint64_t)n + 1);
     w.stmp = w.dplus + (uint64_t)n + 1 + w.tiles;
-    uint64_t* after = w.stmp + std::max(scan_tmp_words(w.tiles + 1), scan_tmp_words((uint64_t)n + 1));
+    uint64_t* after = w.stmp + orient_scan_words(n, w.tiles);
     w.ncls = reinterpret_cast<uint8_t*>(after);
     w.tgraph = reinterpret_cast<uint32_t*>(after + ((uint64_t)n + 15) / 16);
     return w;
@@ -913,7 +1061,7 @@ const uint64_t* orient_keep_bits(uint32_t n, uint64_t nnz, const uint64_t* ws) {
 uint64_t orient_ws_words(uint32_t n, uint64_t nnz) {
     uint64_t tiles = (nnz + OR_TILE - 1) / OR_TILE;
     return (tiles + 1) + 2 * (tiles + 1) + (nnz + 63) / 64 + 1 + (uint64_t)n + 1 + tiles +
-           std::max(scan_tmp_words(tiles + 1), scan_tmp_words((uint64_t)n + 1)) + ((uint64_t)n + 15) / 16 + tiles;
+           orient_scan_words(n, tiles) + ((uint64_t)n + 15) / 16 + tiles;
 }
 
 // Rows of the first and last slot of every `tile`-slot tile of a CSR whose
@@ -930,12 +1078,10 @@ void tile_bounds_launch(uint32_t n, uint64_t nnz, uint64_t tile, const uint64_t*
 void orient_count_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint32_t* heads, uint32_t* deg,
                          uint64_t* ooff, uint64_t* ws, uint32_t* err, const OrientCheck& chk, hipStream_t st) {
     OrientWs w = orient_ws(n, nnz, ws);
-    k_degree<<<(n + 255) / 256, 256, 0, st>>>(n, nnz, off, deg, w.ncls, err);
-    fill_u64(w.dplus, (uint64_t)n + 1, 0, st);
+    k_degree<<<(unsigned)(((uint64_t)n + 256) / 256), 256, 0, st>>>(n, nnz, off, deg, w.ncls, w.dplus, OR_TILE, w.tbnd,
+                                                                   err);
     if (w.tiles > 0) {
         const CheckArgs ck{chk.key[0], chk.key[1], chk.G ? chk.vbase : nullptr, chk.G, w.tgraph};
-        fill_u32(w.tbnd, 2 * w.tiles, 0, st);
-        k_tile_bounds<<<(n + 255) / 256, 256, 0, st>>>(n, nnz, OR_TILE, off, w.tbnd);
         if (ck.vbase) {
             k_tile_graphs<<<(unsigned)((w.tiles + 255) / 256), 256, 0, st>>>(n, w.tiles, w.tbnd, ck.vbase, ck.G,
                                                                             w.tgraph);
@@ -945,12 +1091,10 @@ void orient_count_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const ui
             k_orient_keep<false><<<(unsigned)w.tiles, OR_THREADS, 0, st>>>(n, nnz, off, heads, deg, w.ncls, w.tbnd,
                                                                           w.bits, w.dplus, w.tile_cnt, err, ck, w.sym);
         }
-        scan_u64(w.tile_cnt, w.tile_off, w.tiles, w.stmp, st);
-    } else {
-        fill_u64(w.tile_off, 1, 0, st);
     }
-    scan_u64(w.dplus, ooff, n, w.stmp, st);
-    k_sym_final<<<1, SYM_FINAL_THREADS, 0, st>>>(w.sym, w.tiles, ooff + n, nnz, err);
+    ScanJob a{w.tile_cnt, w.tile_off, w.tiles, w.stmp, (w.tiles + SCAN_TILE - 1) / SCAN_TILE};
+    ScanJob b{w.dplus, ooff, n, w.stmp + a.tiles + 1, ((uint64_t)n + SCAN_TILE - 1) / SCAN_TILE};
+    orient_scans(a, b, w.sym, w.tiles, nnz, err, st);
 }
 
 uint64_t sym_ws_words(uint32_t n, uint64_t nnz) {
@@ -970,7 +1114,7 @@ void sym_check_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint3
         k_tile_bounds<<<(n + 255) / 256, 256, 0, st>>>(n, nnz, OR_TILE, off, tbnd);
         k_sym_tiles<<<(unsigned)tiles, OR_THREADS, 0, st>>>(n, nnz, off, heads, tbnd, err, ck, sym);
     }
-    k_sym_final<<<1, SYM_FINAL_THREADS, 0, st>>>(sym, (tiles > 0 && n > 0) ? tiles : 0, nullptr, nnz, err);
+    k_sym_final<<<1, ONE_THREADS, 0, st>>>(sym, (tiles > 0 && n > 0) ? tiles : 0, err);
 }
 
 void random_keys(uint64_t key[2]) {
@@ -982,18 +1126,17 @@ void random_keys(uint64_t key[2]) {
     }
 }
 
-// Writes the oriented heads; only valid after orient_count_launch on the same
-// input showed a symmetric, well-formed CSR (kept == nnz / 2).
+// Writes the oriented heads, after orient_count_launch on the same input.
 void orient_write_launch(uint32_t n, uint64_t nnz, const uint32_t* heads, uint32_t* oheads, uint64_t* ws,
-                         hipStream_t st) {
+                         const uint32_t* err, hipStream_t st) {
     const OrientWs w = orient_ws(n, nnz, ws);
-    emit_bits_launch(nnz, heads, w.bits, w.tile_off, oheads, st);
+    emit_bits_launch(nnz, heads, w.bits, w.tile_off, oheads, err, st);
 }
 
 void emit_bits_launch(uint64_t nnz, const uint32_t* heads, const uint64_t* bits, const uint64_t* tile_off,
-                      uint32_t* out, hipStream_t st) {
+                      uint32_t* out, const uint32_t* err, hipStream_t st) {
     const uint64_t tiles = (nnz + OR_TILE - 1) / OR_TILE;
-    if (tiles > 0) k_orient_emit<<<(unsigned)tiles, OR_THREADS, 0, st>>>(nnz, heads, bits, tile_off, out);
+    if (tiles > 0) k_orient_emit<<<(unsigned)tiles, OR_THREADS, 0, st>>>(nnz, heads, bits, tile_off, out, err);
 }
 
 void make_keys(uint32_t n, uint64_t m, const uint64_t* ooff, const uint32_t* oheads, uint64_t* keys,

@@ -1663,16 +1663,25 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
 
 // Adds up the per-XCD copies of the n per-vertex counts (n == 0: none) and,
 // in the first block, the workgroups' sums.
+// With `host` (page-locked words) the results go there too: gate word, kept
+// slots, total, work counters; then the per-vertex counts are assigned, and
+// left alone when the gate is closed.
 __global__ void __launch_bounds__(256) k_tc_finish(uint64_t n, const uint64_t* __restrict__ copies,
                                                    uint64_t* __restrict__ pv, uint32_t rows,
                                                    const uint64_t* __restrict__ sums, uint64_t* __restrict__ stats,
-                                                   uint64_t* __restrict__ total) {
-    for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) {
-        uint64_t s = 0;
+                                                   uint64_t* __restrict__ total, uint64_t* __restrict__ host,
+                                                   const uint32_t* __restrict__ gate, uint32_t gate_bits,
+                                                   const uint64_t* __restrict__ kept) {
+    if (!host || !(*gate & gate_bits))
+        for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) {
+            uint64_t s = 0;
 #pragma unroll
-        for (int c = 0; c < NXCD; ++c) s += copies[c * n + v];
-        if (s) pv[v] += s;
-    }
+            for (int c = 0; c < NXCD; ++c) s += copies[c * n + v];
+            if (host)
+                pv[v] = s;
+            else if (s)
+                pv[v] += s;
+        }
     if (blockIdx.x != 0) return;
     __shared__ uint64_t red[256 / KT_WAVE][SUM_WORDS];
     uint64_t t[SUM_WORDS] = {};
@@ -1691,6 +1700,13 @@ __global__ void __launch_bounds__(256) k_tc_finish(uint64_t n, const uint64_t* _
             *total += x;
         else
             stats[threadIdx.x] = x;
+        if (host) {
+            host[threadIdx.x == SUM_TOTAL ? 2 : 3 + threadIdx.x] = x;
+            if (threadIdx.x == 0) {
+                host[0] = *gate;
+                host[1] = *kept;
+            }
+        }
     }
 }
 
@@ -1734,6 +1750,13 @@ uint64_t tc_ws_words(uint32_t X, const TcRoom& room, int num_cus) {
            hub_ws_words(X, room.hub_slots) + NXCD * room.pv_n;
 }
 
+void tc_clear(uint64_t* ws, uint32_t X, const TcRoom& room, int num_cus, ClearList& c) {
+    c.add(ws, head_words(num_cus));
+    uint64_t* p = ws + head_words(num_cus) + (uint64_t(X) + 1) / 2 + 1 + parts_of(room, num_cus);
+    if (room.hub_slots) c.add(p, HUB_HEAD_WORDS);
+    c.add(p + hub_ws_words(X, room.hub_slots), NXCD * room.pv_n);
+}
+
 TcRoom tc_room(uint64_t entries, uint64_t slots, uint64_t pv_n) {
     TcRoom r;
     r.entries = entries;
@@ -1762,7 +1785,13 @@ static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const T
     auto row = [&](int r) { return sums + (uint64_t)r * num_cus * SUM_WORDS; };
     uint32_t* list = reinterpret_cast<uint32_t*>(ws + head_words(num_cus));
     uint64_t* plist = ws + head_words(num_cus) + (uint64_t(view.X) + 1) / 2 + 1;
-    fill_u64(ws, head_words(num_cus), 0, st);
+    if (!view.cleared) {
+        TcRoom r = view.room;
+        if (!user_out.per_vertex) r.pv_n = 0;
+        ClearList cl;
+        tc_clear(ws, view.X, r, num_cus, cl);
+        clear(cl, st);
+    }
     TcParams p = prm;
     if (p.wave_max_deg > WAVE_SLOTS / 2) p.wave_max_deg = WAVE_SLOTS / 2;
     if (p.group_max_deg > GROUP_SLOTS / 2) p.group_max_deg = GROUP_SLOTS / 2;
@@ -1785,7 +1814,6 @@ static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const T
         if (PLAIN && view.room.hub_slots && view.deg && view.X) {
             p.hub_split = sp.hub;
             hub = hub_ws(room, view.X);
-            fill_u64(room, HUB_HEAD_WORDS, 0, st);
             // few blocks: each adds up to a thousand bins to the global ones
             k_hub_hist<<<std::clamp<unsigned>(view.X / (32 * HUB_HIST_THREADS), 1, HUB_BLOCKS), HUB_HIST_THREADS, 0,
                          st>>>(view.X, view.deg, view.room.entries, hub);
@@ -1796,7 +1824,6 @@ static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const T
     if (pv && view.room.pv_n) {
         out.per_vertex = room;
         out.pv_stride = view.room.pv_n;
-        fill_u64(room, NXCD * view.room.pv_n, 0, st);
     }
     // a min-side walk covers in- and out-neighbours and streams from only
     // some of them: four times the entries per team grab
@@ -1812,7 +1839,8 @@ static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const T
     auto finish = [&]() {
         const uint64_t n = out.pv_stride;
         k_tc_finish<<<(unsigned)std::clamp<uint64_t>((n + 255) / 256, 1, 4096), 256, 0, st>>>(
-            n, out.per_vertex, pv, (uint32_t)(ROWS * num_cus), sums, stats, out.totals);
+            n, out.per_vertex, pv, (uint32_t)(ROWS * num_cus), sums, stats, out.totals, view.host_out, view.gate,
+            view.gate_bits, view.kept);
     };
     constexpr uint32_t big_lds = 2 * BIG_SLOTS * sizeof(uint32_t);
     if constexpr (PLAIN) {

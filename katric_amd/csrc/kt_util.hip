@@ -17,6 +17,20 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint64_t count, uint32_t va
         p[i] = value;
 }
 
+__global__ void __launch_bounds__(256) k_clear(ClearList c) {
+    const uint64_t n = c.n[blockIdx.y];
+    uint64_t* p = c.p[blockIdx.y];
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) p[i] = 0;
+}
+
+void clear(const ClearList& c, hipStream_t st) {
+    if (c.count == 0) return;
+    uint64_t most = 0;
+    for (uint32_t i = 0; i < c.count; ++i) most = c.n[i] > most ? c.n[i] : most;
+    const uint64_t g = (most + 1023) / 1024;
+    k_clear<<<dim3((unsigned)(g > 4096 ? 4096 : g), c.count), 256, 0, st>>>(c);
+}
+
 static unsigned fill_grid(uint64_t count) {
     uint64_t g = (count + 255) / 256;
     if (g > 8192) g = 8192;

@@ -150,3 +150,38 @@ def test_intersect_order_check_at_tile_edges(ctx, at):
         with pytest.raises(K.KatricError):
             ctx.intersect([pair])
     assert ctx.intersect([(ids, ids[::2])])[0].tolist() == [2501]
+
+
+@pytest.mark.parametrize("k", [2, 3, 40, 600, 3000])
+def test_repeated_edges_in_unsorted_rows(ctx, k):
+    # a triangle whose edges all come k times, never twice in a row: only the
+    # sort can see it, and with many copies the lists are longer than a simple
+    # graph's can be
+    rows = [[1, 2] * k, [2, 0] * k, [0, 1] * k]
+    off = np.array([0, 2 * k, 4 * k, 6 * k], np.uint64)
+    with pytest.raises(K.KatricError):
+        ctx.count(K.Graph(3, off, np.concatenate(rows).astype(np.uint32)))
+    g, pv = _cliques([5, 9])
+    _check(ctx, g, pv)  # the context is none the worse
+
+
+@pytest.mark.parametrize("n", [1, 2, 4095, 4096, 16383, 16384, 16385, 70_001])
+@pytest.mark.parametrize("unsorted", [False, True])
+def test_scan_sizes(ctx, n, unsorted):
+    # a path of n vertices with a triangle at its end where there is room
+    e = np.stack([np.arange(n - 1), np.arange(1, n)], 1)
+    tri = n >= 3
+    if tri:
+        e = np.concatenate([e, [[n - 3, n - 1]]])
+    g = K.Graph.from_edges(n, e)
+    if unsorted and tri:
+        heads = g.heads.copy()
+        a, b = int(g.offsets[n - 2]), int(g.offsets[n - 1])
+        heads[a:b] = heads[a:b][::-1]
+        g = K.Graph(n, g.offsets, heads)
+    pv = np.zeros(n, np.uint64)
+    if tri:
+        pv[n - 3:] = 1
+    _check(ctx, g, pv)
+    o = ctx.orient(g)
+    assert int(o.offsets[-1]) == len(e)
