@@ -1465,13 +1465,18 @@ struct __attribute__((packed, aligned(2))) Hubs8 {
     uint32_t x, y, z, w;
 };
 
+typedef __attribute__((address_space(3))) uint32_t LdsWord;
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+
 // walk_lists over hub lists, eight entries (16 bytes) per block and lane:
-// tab (byte offsets from the list entries) holds the byte offset of a set
+// tab (byte offsets from the list entries) holds the LDS address of a set
 // member's counter, zero for all others, so a lookup is one 2-byte LDS read
 // and one compare, against five compares and an address of two instructions
 // in a hash bucket.
 __device__ __forceinline__ uint32_t walk_hub_lists(const uint16_t* __restrict__ lists, uint64_t tb, uint64_t rem,
-                                                   const char* tab, char* cnt, HubPack& pk, uint64_t& total) {
+                                                   const char* tab, HubPack& pk, uint64_t& total) {
     const uint32_t lane = lane_id();
     const uint16_t* __restrict__ T = lists - REC_BIAS;
     uint32_t mine = 0;
@@ -1538,7 +1543,9 @@ __device__ __forceinline__ uint32_t walk_hub_lists(const uint16_t* __restrict__ 
                 for (int k = 0; k < 8; ++k) {
                     const bool hit = k < c_lim && t[k] != 0;
                     nh += hit ? 1u : 0u;
-                    if (hit) atomicAdd(reinterpret_cast<uint32_t*>(cnt + t[k]), 1u);
+                    if (hit)
+                        __hip_atomic_fetch_add(reinterpret_cast<LdsWord*>((uintptr_t)t[k]), 1u, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
                 if (__builtin_amdgcn_ballot_w64(nh != 0)) {
                     const uint32_t sum = wave_scan_dpp(nh);
@@ -1572,10 +1579,10 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
     if (parts == 0) return;
     const uint32_t base = bucket_base(q, BUCKET_HUB_PARTS);
     uint32_t* pull = &q[Q_PULL + Q_STRIDE * BUCKET_HUB_PARTS];
-    // counters first: their byte offsets from the start fit two bytes, and a
-    // table entry is one
+    // counters first: their LDS addresses fit two bytes, and a table entry is one
     char* cnt = reinterpret_cast<char*>(hub_lds);
     char* tab = cnt + 4 * HUB_CNT;
+    const uint32_t cnt0 = lds_address(cnt);
     const uint32_t tid = threadIdx.x, wave = tid / KT_WAVE, lane = lane_id();
     HubPack& pk = reinterpret_cast<HubPack*>(tab + 2 * HUB_MAX + 16)[wave];
     for (uint32_t i = tid; i < (2 * HUB_MAX + 16) / 4 + HUB_CNT; i += HUB_THREADS) hub_lds[i] = 0;
@@ -1610,7 +1617,7 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
         uint32_t u_nx = 0, kw_nx = 0;
         if (k < nr && lane < min(chunk, nr - k)) V.entry_head(rb + k + lane, u_nx, kw_nx);
         for (uint32_t j = tid; j < ns; j += HUB_THREADS)
-            *reinterpret_cast<uint16_t*>(tab + lists[sb + j]) = (uint16_t)(4 * (j + 1));
+            *reinterpret_cast<uint16_t*>(tab + lists[sb + j]) = (uint16_t)(cnt0 + 4 * (j + 1));
         if (tid == 0) next_u = HUB_WAVES * chunk;
         const uint32_t i_nx = i + gridDim.x;
         if (i_nx < fixed) xp_nx = plist[base + i_nx];
@@ -1630,7 +1637,7 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
             wk.recv_lane += stc ? ns : 0u;
             wk.stream_lane += len;
             uint64_t hits;
-            const uint32_t h = walk_hub_lists(lists, b, len, tab, cnt, pk, hits);
+            const uint32_t h = walk_hub_lists(lists, b, len, tab, pk, hits);
             if (h && out.per_vertex) atomic_add_u64(&out.per_vertex[u], h);
             hsum += hits;
             k = nk;
