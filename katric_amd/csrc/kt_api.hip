@@ -132,23 +132,29 @@ void kt_ctx::release_aux() {
 }
 
 namespace kt {
-__global__ void k_peek(const uint64_t* a, const uint64_t* b, uint64_t* host) {
-    host[0] = *a;
-    host[1] = *b;
+struct PeekList {
+    const uint64_t* p[4];
+};
+__global__ void k_peek(PeekList l, int count, uint64_t* host) {
+    if ((int)threadIdx.x < count) host[threadIdx.x] = *l.p[threadIdx.x];
 }
 }  // namespace kt
 
-int kt_ctx::read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what) {
+int kt_ctx::read_words(const uint64_t* const* dev, int count, uint64_t* out, const char* what) {
     // a kernel that writes to page-locked memory: one round trip of a few
-    // microseconds instead of two copies and two waits
-    k_peek<<<1, 1, 0, stream>>>(a, b, host_small + 62);
+    // microseconds instead of a copy each
+    kt::PeekList l{};
+    for (int i = 0; i < count; ++i) l.p[i] = dev[i];
+    k_peek<<<1, 4, 0, stream>>>(l, count, host_small + 60);
     int rc = hip_check(hipGetLastError(), what);
     if (!rc) rc = hip_check(hipStreamSynchronize(stream), what);
-    if (!rc) {
-        out[0] = host_small[62];
-        out[1] = host_small[63];
-    }
+    for (int i = 0; !rc && i < count; ++i) out[i] = host_small[60 + i];
     return rc;
+}
+
+int kt_ctx::read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what) {
+    const uint64_t* p[2] = {a, b};
+    return read_words(p, 2, out, what);
 }
 
 int kt_ctx::read_u64(const uint64_t* dev, uint64_t* out, const char* what) {

@@ -70,6 +70,8 @@ struct kt_ctx {
     void release_aux();
     // One device word, read in order after the work queued on `stream`.
     int read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what);
+    // Up to four of them with one launch and one wait.
+    int read_words(const uint64_t* const* dev, int count, uint64_t* out, const char* what);
     int read_u64(const uint64_t* dev, uint64_t* out, const char* what);
     void destroy_extensions();
 };
@@ -79,8 +81,12 @@ void kt_serve_release(kt_ctx* c);
 
 namespace kt {
 uint64_t* tc_stats_ptr(uint64_t* ws);
-// kt_count_shard without taking the context lock (kt_shard.hip)
-int count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out);
+// kt_count_shard without taking the context lock (kt_shard.hip); sizes: those of
+// device inputs, where the caller knows them
+struct ShardSizes {
+    uint64_t slots, entries;  // offsets[n_local], msg_offsets[n_msg]
+};
+int count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, const ShardSizes* sizes = nullptr);
 // kt_count without taking the context lock; with fixed_ws the device
 // workspace is that region (fixed_ws_bytes long) instead of the context's
 // arena, and nothing is allocated (kt_api.hip)

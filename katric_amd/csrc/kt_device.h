@@ -187,6 +187,20 @@ __device__ __forceinline__ void tile_rows(const uint64_t* __restrict__ off, uint
     __syncthreads();
 }
 
+// Notes the row v = [a, b) of a CSR with len entries as the row of the first and
+// last entry of every tile of `tile` entries whose first or last entry it holds
+// (bnd: two entries per tile).
+__device__ __forceinline__ void note_tiles(uint32_t v, uint64_t a, uint64_t b, uint64_t len, uint64_t tile,
+                                           uint32_t* __restrict__ bnd) {
+    b = min(b, len);
+    if (b <= a) return;
+    for (uint64_t t = a / tile; t * tile < b; ++t) {
+        if (t * tile >= a) bnd[2 * t] = v;
+        const uint64_t last = min((t + 1) * tile, len) - 1;
+        if (last >= a && last < b) bnd[2 * t + 1] = v;
+    }
+}
+
 // Sum over the wave with DPP row shifts and row broadcasts (no LDS traffic):
 // an inclusive scan within each 16-lane row by shifts of 1, 2, 4, 8 (lanes
 // shifted in from outside the row read 0), then lane 15 of rows 0 and 2 into

@@ -15,6 +15,9 @@
 #define KT_ERR_SEGMENT 0x40u     // batch: a graph's per-vertex sum is not a multiple of 3
 #define KT_ERR_ASYMMETRIC 0x80u  // some slot v -> u has no slot u -> v (pair checksum or kept count)
 #define KT_ERR_MASK 0xffu
+#define KT_FLAG_OVER_WAVE 0x200u    // shard: a list longer than segsort_wave_len()
+#define KT_FLAG_OVER_GROUP 0x400u   // shard: a list longer than segsort_max_len()
+#define KT_FLAG_LONG_MESSAGE 0x800u // shard: a message with more than segsort_wave_len() known entries
 
 namespace kt {
 
@@ -23,7 +26,6 @@ uint64_t scan_tmp_words(uint64_t len);
 void scan_u64(const uint64_t* in, uint64_t* out, uint64_t len, uint64_t* tmp, hipStream_t st);
 uint64_t radix_tmp_words(uint64_t len);
 void radix_sort_u64(uint64_t* keys, uint64_t* alt, uint64_t len, int bits, uint64_t* tmp, hipStream_t st);
-void tile_bounds_launch(uint32_t n, uint64_t nnz, uint64_t tile, const uint64_t* off, uint32_t* bnd, hipStream_t st);
 uint64_t orient_ws_words(uint32_t n, uint64_t nnz);
 // Validation of a symmetric CSR beside the orientation count pass.  Every
 // slot v -> u adds +h(min, max) (v < u) or -h(min, max) (v > u) of the
@@ -41,7 +43,11 @@ void orient_count_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const ui
                          uint64_t* ooff, uint64_t* ws, uint32_t* err, const OrientCheck& chk, hipStream_t st);
 // Pair checksum, self-loop, range and (sorted-row) duplicate checks of a whole
 // symmetric CSR without orienting it; ws holds sym_ws_words(n, nnz) words.
+// The caller fills sym_tile_bounds first: the rows of every tile's first and
+// last slot, tiles of SYM_TILE slots.
+constexpr uint64_t SYM_TILE = 2048;
 uint64_t sym_ws_words(uint32_t n, uint64_t nnz);
+uint32_t* sym_tile_bounds(uint64_t nnz, uint64_t* ws);
 void sym_check_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint32_t* heads, uint64_t* ws,
                       uint32_t* err, const OrientCheck& chk, hipStream_t st);
 // A random key pair for OrientCheck.
@@ -67,7 +73,9 @@ void keys_to_heads(uint64_t m, const uint64_t* keys, uint32_t* oheads, uint32_t*
 // *out, using tmp (segsort_tmp_words() words).
 uint64_t segsort_tmp_words();
 void max_len_launch(uint32_t n, const uint64_t* ooff, uint64_t* tmp, uint64_t* out, hipStream_t st);
-uint32_t segsort_max_len();
+// segsort_wave_len(): lists up to it are sorted by one wave.
+constexpr __host__ __device__ uint32_t segsort_max_len() { return 4096; }
+constexpr __host__ __device__ uint32_t segsort_wave_len() { return 1024; }
 void segsort_launch(uint32_t n, const uint64_t* ooff, uint32_t* oheads, uint32_t* err, uint64_t max_len, int num_cus,
                     hipStream_t st);
 
@@ -177,6 +185,7 @@ struct TcView {
     const uint32_t* gate = nullptr;
     uint32_t gate_bits = 0;
     bool cleared = false;  // the caller cleared tc_clear's ranges
+    uint64_t longest = 0;  // no list S is longer (0: not known)
     // host words (page-locked; nullable) that receive the gate word, *kept, the
     // total and the four work counters at the end; with them, per_vertex is
     // assigned (room.pv_n set) and left alone when the gate is closed

@@ -58,7 +58,10 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_tile_reduce(const uint64_t* __
     if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// out[i] = tile_base[tile] + exclusive prefix within the tile; out[len] = grand total.
+// out[i] = tile_base[tile] + exclusive prefix within the tile; out[len] = grand
+// total.  SUMS: tile_base holds the tiles' sums, and the block adds up those
+// before its own.
+template <bool SUMS>
 __global__ void __launch_bounds__(SCAN_THREADS) k_tile_scan(const uint64_t* __restrict__ in, uint64_t len,
                                                              const uint64_t* __restrict__ tile_base,
                                                              uint64_t* __restrict__ out) {
@@ -71,16 +74,25 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_tile_scan(const uint64_t* __re
         v[i] = (base + i < len) ? in[base + i] : 0;
         s += v[i];
     }
+    uint64_t before = tile_base && !SUMS ? tile_base[blockIdx.x] : 0;
+    if constexpr (SUMS) {
+        uint64_t part = 0;
+        for (uint32_t t = threadIdx.x; t < blockIdx.x; t += SCAN_THREADS) part += tile_base[t];
+        block_excl_sum(part, lw, &before);
+    }
     uint64_t tot;
-    uint64_t run = block_excl_sum(s, lw, &tot) + (tile_base ? tile_base[blockIdx.x] : 0);
+    uint64_t run = block_excl_sum(s, lw, &tot) + before;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) {
         if (base + i < len) out[base + i] = run;
         run += v[i];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
-        out[len] = (tile_base ? tile_base[blockIdx.x] : 0) + tot;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[len] = before + tot;
 }
+
+// Up to this many tiles every block adds up the sums before its own (4 loads a
+// thread) in place of a launch that scans them.
+constexpr uint64_t SCAN_SUMS_MAX = 4 * SCAN_THREADS;
 
 uint64_t scan_tmp_words(uint64_t len) {
     uint64_t words = 0;
@@ -99,14 +111,18 @@ void scan_u64(const uint64_t* in, uint64_t* out, uint64_t len, uint64_t* tmp, hi
     }
     uint64_t tiles = (len + SCAN_TILE - 1) / SCAN_TILE;
     if (tiles == 1) {
-        k_tile_scan<<<1, SCAN_THREADS, 0, st>>>(in, len, nullptr, out);
+        k_tile_scan<false><<<1, SCAN_THREADS, 0, st>>>(in, len, nullptr, out);
         return;
     }
     uint64_t* sums = tmp;
     uint64_t* sums_off = tmp + tiles + 1;
     k_tile_reduce<<<(unsigned)tiles, SCAN_THREADS, 0, st>>>(in, len, sums);
+    if (tiles <= SCAN_SUMS_MAX) {
+        k_tile_scan<true><<<(unsigned)tiles, SCAN_THREADS, 0, st>>>(in, len, sums, out);
+        return;
+    }
     scan_u64(sums, sums_off, tiles, tmp + 2 * (tiles + 1), st);
-    k_tile_scan<<<(unsigned)tiles, SCAN_THREADS, 0, st>>>(in, len, sums_off, out);
+    k_tile_scan<false><<<(unsigned)tiles, SCAN_THREADS, 0, st>>>(in, len, sums_off, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -137,13 +153,7 @@ __global__ void k_degree(uint32_t n, uint64_t nnz, const uint64_t* __restrict__ 
     if (v <= n) dplus[v] = 0;
     const uint32_t c1 = (uint32_t)__shfl_down((int)c, 1, KT_WAVE);
     if (v < n && (v & 1) == 0) ncls[v >> 1] = (uint8_t)(c | (v + 1 < n ? c1 << 4 : 0u));
-    b = min(b, nnz);
-    if (b > a)
-        for (uint64_t t = a / tile; t * tile < b; ++t) {
-            if (t * tile >= a) bnd[2 * t] = (uint32_t)v;
-            const uint64_t last = min((t + 1) * tile, nnz) - 1;
-            if (last >= a && last < b) bnd[2 * t + 1] = (uint32_t)v;
-        }
+    note_tiles((uint32_t)v, a, b, nnz, tile, bnd);
 }
 
 // ---------------------------------------------------------------------------
@@ -166,22 +176,6 @@ constexpr int OR_TILE = OR_THREADS * OR_ITEMS;
 // local (distributed_graph.h:147-163).
 __device__ __forceinline__ bool keep_edge(uint32_t v, uint32_t dv, uint32_t u, uint32_t du) {
     return dv < du || (dv == du && v < u);
-}
-
-// bnd[2t] / bnd[2t+1] = the rows holding the first / last slot of tile t
-// (tiles of `tile` slots), written by the row that holds them, so every tile
-// resolves its rows without a dependent search (bnd is pre-filled with 0).
-__global__ void k_tile_bounds(uint32_t n, uint64_t nnz, uint64_t tile, const uint64_t* __restrict__ off,
-                              uint32_t* __restrict__ bnd) {
-    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-        const uint64_t a = off[v], b = min(off[v + 1], nnz);
-        if (b <= a) continue;  // empty row (or offsets the validation will reject)
-        for (uint64_t t = a / tile; t * tile < b; ++t) {
-            if (t * tile >= a) bnd[2 * t] = v;
-            const uint64_t last = min((t + 1) * tile, nnz) - 1;
-            if (last >= a && last < b) bnd[2 * t + 1] = v;
-        }
-    }
 }
 
 // Graph bounds of a tile's rows for the batch range check: the graphs of its
@@ -533,7 +527,7 @@ __global__ void __launch_bounds__(OR_THREADS)
     const unsigned tid = threadIdx.x, lane = lane_id();
     if (tid == 0) bflags = 0;
     uint32_t lo, hi;
-    tile_rows<OR_THREADS, OR_ITEMS>(off, n, tile0, tend, marks, bnd, wmax, lo, hi, tbnd);
+    tile_rows<OR_THREADS, OR_ITEMS>(off, n, tile0, tend, marks, bnd, wmax, lo, hi, tbnd, err);
     uint32_t flags = 0;
     uint64_t s0 = 0;
 #pragma unroll 4
@@ -648,8 +642,8 @@ __global__ void k_keys_to_heads(uint64_t m, const uint64_t* __restrict__ keys, u
 // neighbours after the sort are duplicate edges.
 // ---------------------------------------------------------------------------
 constexpr uint32_t SEG_THREAD_MAX = 16;
-constexpr uint32_t SEG_WAVE_MAX = 1024;
-constexpr uint32_t SEG_MAX = 4096;
+constexpr uint32_t SEG_WAVE_MAX = segsort_wave_len();
+constexpr uint32_t SEG_MAX = segsort_max_len();
 constexpr int SEG_BLOCK = 256;
 
 __device__ __forceinline__ bool unsorted_only(uint32_t flags) {
@@ -716,22 +710,23 @@ __device__ __forceinline__ uint32_t wave_sort_list(uint32_t* __restrict__ p, uin
     return f;
 }
 
-// Rows of 64-row chunks, one chunk per wave: lists of <= 16 ids sorted by
+// Rows of `rows`-row chunks (a power of two up to 64), one chunk per wave: lists of <= 16 ids sorted by
 // their own lane, then the chunk's lists of 17..1024 ids one after another by
 // the whole wave.
 // A list above max_len, which no list of a simple graph exceeds, holds an edge
 // twice.
-__global__ void __launch_bounds__(SEG_BLOCK) k_segsort_small(uint32_t n, const uint64_t* __restrict__ ooff,
+__global__ void __launch_bounds__(SEG_BLOCK) k_segsort_small(uint32_t n, uint32_t rows,
+                                                             const uint64_t* __restrict__ ooff,
                                                              uint32_t* __restrict__ oheads, uint64_t max_len,
                                                              uint32_t* __restrict__ err) {
     if (!unsorted_only(*err)) return;
     const uint32_t lane = lane_id();
     const uint64_t nw = (uint64_t)gridDim.x * (SEG_BLOCK / KT_WAVE);
     uint32_t flags = 0;
-    for (uint64_t c = (uint64_t)blockIdx.x * (SEG_BLOCK / KT_WAVE) + threadIdx.x / KT_WAVE; c * KT_WAVE < n; c += nw) {
-        const uint64_t v = c * KT_WAVE + lane;
+    for (uint64_t c = (uint64_t)blockIdx.x * (SEG_BLOCK / KT_WAVE) + threadIdx.x / KT_WAVE; c * rows < n; c += nw) {
+        const uint64_t v = c * rows + lane;
         uint64_t b = 0, e = 0;
-        if (v < n) {
+        if (v < n && lane < rows) {
             b = ooff[v];
             e = ooff[v + 1];
         }
@@ -887,14 +882,16 @@ void max_len_launch(uint32_t n, const uint64_t* ooff, uint64_t* tmp, uint64_t* o
     k_max_final<<<1, 256, 0, st>>>(g, part, out);
 }
 
-uint32_t segsort_max_len() { return SEG_MAX; }
-
 void segsort_launch(uint32_t n, const uint64_t* ooff, uint32_t* oheads, uint32_t* err, uint64_t max_len, int num_cus,
                     hipStream_t st) {
     if (n == 0 || max_len < 2) return;
-    const uint64_t chunks = ((uint64_t)n + KT_WAVE - 1) / KT_WAVE;
+    // a chunk's longer lists wait for each other: fewer rows per chunk while
+    // the chip holds more waves
+    uint32_t rows = KT_WAVE;
+    while (rows > 8 && n / rows < (uint32_t)num_cus * 64) rows /= 2;
+    const uint64_t chunks = ((uint64_t)n + rows - 1) / rows;
     const uint32_t g1 = (uint32_t)std::min<uint64_t>((chunks + 3) / 4, (uint64_t)num_cus * 32);
-    k_segsort_small<<<g1, SEG_BLOCK, 0, st>>>(n, ooff, oheads, max_len, err);
+    k_segsort_small<<<g1, SEG_BLOCK, 0, st>>>(n, rows, ooff, oheads, max_len, err);
     if (max_len <= SEG_WAVE_MAX) return;
     const uint32_t g2 = (uint32_t)std::min<uint64_t>(((uint64_t)n + SEG_BLOCK - 1) / SEG_BLOCK, (uint64_t)num_cus * 8);
     k_segsort_large<<<g2, SEG_BLOCK, 0, st>>>(n, ooff, oheads, err);
@@ -1066,13 +1063,6 @@ uint64_t orient_ws_words(uint32_t n, uint64_t nnz) {
 
 // Rows of the first and last slot of every `tile`-slot tile of a CSR whose
 // offsets start at 0 (bnd: 2 entries per tile), for tile_rows.
-void tile_bounds_launch(uint32_t n, uint64_t nnz, uint64_t tile, const uint64_t* off, uint32_t* bnd, hipStream_t st) {
-    const uint64_t tiles = (nnz + tile - 1) / tile;
-    if (!tiles || !n) return;
-    fill_u32(bnd, 2 * tiles, 0, st);
-    k_tile_bounds<<<(unsigned)(((uint64_t)n + 255) / 256), 256, 0, st>>>(n, nnz, tile, off, bnd);
-}
-
 // Degrees, validation flags, keep bitmask, d+ per row and its scan into ooff
 // (ooff[n] = kept total), per-tile kept counts and their scan.
 void orient_count_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint32_t* heads, uint32_t* deg,
@@ -1103,15 +1093,18 @@ uint64_t sym_ws_words(uint32_t n, uint64_t nnz) {
     return 2 * (tiles + 1);  // per-tile checksums, then the tiles' row bounds
 }
 
+uint32_t* sym_tile_bounds(uint64_t nnz, uint64_t* ws) {
+    return reinterpret_cast<uint32_t*>(ws + (nnz + SYM_TILE - 1) / SYM_TILE + 1);
+}
+
 void sym_check_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint32_t* heads, uint64_t* ws,
                       uint32_t* err, const OrientCheck& chk, hipStream_t st) {
+    static_assert(OR_TILE == SYM_TILE, "the caller's tiles");
     const uint64_t tiles = (nnz + OR_TILE - 1) / OR_TILE;
     uint64_t* sym = ws;
-    uint32_t* tbnd = reinterpret_cast<uint32_t*>(ws + tiles + 1);
+    const uint32_t* tbnd = sym_tile_bounds(nnz, ws);
     if (tiles > 0 && n > 0) {
         const CheckArgs ck{chk.key[0], chk.key[1], nullptr, 0, nullptr};
-        fill_u32(tbnd, 2 * tiles, 0, st);
-        k_tile_bounds<<<(n + 255) / 256, 256, 0, st>>>(n, nnz, OR_TILE, off, tbnd);
         k_sym_tiles<<<(unsigned)tiles, OR_THREADS, 0, st>>>(n, nnz, off, heads, tbnd, err, ck, sym);
     }
     k_sym_final<<<1, ONE_THREADS, 0, st>>>(sym, (tiles > 0 && n > 0) ? tiles : 0, err);

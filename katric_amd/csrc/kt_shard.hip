@@ -6,13 +6,13 @@
 // reference's node_ordering::id_outward(rank) (owned first, then by id,
 // distributed_graph.h:102-112), and the ghost part of a list is its suffix.
 //
-// Preprocessing (one radix sort):
+// Preprocessing (lists placed by rank and sorted one by one):
 //   every owned slot (v, u) with c = map(u) contributes
 //     (v, c)  if (deg v, v) < (deg u, u)           -- N+(v), global degrees
 //     (c, v)  if not, c is a ghost and cetric-x     -- ghost_adj(c)
 //   (remove_in_edges_and_expand_ghosts, distributed_graph.h:1057-1169, with
-//   node_ordering::degree on exchanged ghost degrees, :113-146).  The sorted
-//   (tail << b | head) keys form a CSR L over the combined space.
+//   node_ordering::degree on exchanged ghost degrees, :113-146), and the sorted
+//   lists form a CSR L over the combined space.
 // Local phase (same intersection kernel as the plain path):
 //   cetric-x: every tail x (owned or ghost), S = R = L(x), T(u) = L(u)
 //             (run_local_sequential_with_ghosts, cetric_edge_iterator.h:300-388);
@@ -51,17 +51,30 @@ struct ShardMap {
         if (u >= n_all) return 0xffffffffu;
         const uint2 e = rs[u >> 5];
         const uint32_t bit = 1u << (u & 31);
-        return (e.x & bit) ? nl + e.y + (uint32_t)__popc(e.x & (bit - 1)) : 0xffffffffu;
+        // (the bound matters for a table that fails its check only)
+        return (e.x & bit) ? nl + min(e.y + (uint32_t)__popc(e.x & (bit - 1)), ng - 1) : 0xffffffffu;
     }
     __device__ __forceinline__ uint32_t gid(uint32_t c) const { return c < nl ? from + c : ghost_ids[c - nl]; }
 };
 
+// One pass over the combined index space and the messages: degrees, the ghosts'
+// rank-select table, the row bounds of the slot and message-entry tiles, and the
+// checks of both offset arrays and of the ghost table.
+//
+// Ghost ids ascend, so the first ghost of a table word owns it: it reads the up
+// to 31 ids after its own, and its index is the word's prefix.  Words without a
+// ghost stay zero.  (The bits were set by atomics and counted, scanned and
+// spread by four more launches: six in all, 85 us for 77,000 ghosts among 2^18
+// ids in the CeTriC shard of an R-MAT graph; this one takes 8.)  Only
+// strictly ascending ids are taken, so every index below is in range.
 __global__ void k_shard_prepare(ShardMap M, uint64_t nnz, const uint64_t* __restrict__ off,
                                 const uint64_t* __restrict__ ghost_degree, uint32_t* __restrict__ deg,
+                                uint32_t* __restrict__ tbnd, uint2* __restrict__ rs, uint32_t nmsg, uint64_t mtot,
+                                const uint64_t* __restrict__ moff, uint32_t* __restrict__ mbnd,
                                 uint32_t* __restrict__ err) {
-    const uint64_t X = (uint64_t)M.nl + M.ng;
-    for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < X; c += (uint64_t)gridDim.x * blockDim.x) {
-        if (c == 0 && (off[0] != 0 || off[M.nl] != nnz)) atomicOr(err, KT_ERR_OFFSETS);
+    const uint64_t X = (uint64_t)M.nl + M.ng, all = max(X, (uint64_t)nmsg);
+    for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < all; c += (uint64_t)gridDim.x * blockDim.x) {
+        if (c == 0) atomicOr(err, (off[0] != 0 || off[M.nl] != nnz) ? KT_ERR_OFFSETS | KT_FLAG_UNSORTED : KT_FLAG_UNSORTED);
         if (c < M.nl) {
             uint64_t a = off[c], b = off[c + 1];
             if (b < a || b - a > 0xffffffffull) {
@@ -69,38 +82,36 @@ __global__ void k_shard_prepare(ShardMap M, uint64_t nnz, const uint64_t* __rest
                 deg[c] = 0;
             } else {
                 deg[c] = (uint32_t)(b - a);
+                note_tiles((uint32_t)c, a, b, nnz, SH_TILE, tbnd);
             }
-        } else {
-            const uint64_t g = c - M.nl;
+        } else if (c < X) {
+            const uint32_t g = (uint32_t)(c - M.nl);
             const uint32_t id = M.ghost_ids[g];
-            if ((id >= M.from && id < M.to) || (g > 0 && M.ghost_ids[g - 1] >= id)) atomicOr(err, KT_ERR_GHOST);
+            const uint32_t prev = g > 0 ? M.ghost_ids[g - 1] : 0u;
+            if ((id >= M.from && id < M.to) || (g > 0 && prev >= id) || id >= M.n_all) atomicOr(err, KT_ERR_GHOST);
             uint64_t d = ghost_degree[g];
             deg[c] = d > 0xffffffffull ? 0xffffffffu : (uint32_t)d;
+            if (id < M.n_all && (g == 0 || (prev >> 5) != (id >> 5))) {
+                uint32_t bits = 1u << (id & 31), last = id;
+                bool in = true;
+#pragma unroll
+                for (uint32_t j = 1; j < 32; ++j) {
+                    const uint32_t x = M.ghost_ids[min((uint64_t)g + j, (uint64_t)M.ng - 1)];
+                    in = in && x > last && (x >> 5) == (id >> 5);
+                    bits |= in ? 1u << (x & 31) : 0u;
+                    last = x;
+                }
+                rs[id >> 5] = make_uint2(bits, g);
+            }
+        }
+        if (c < nmsg) {
+            const uint64_t a = moff[c], b = moff[c + 1];
+            if (b < a || b > mtot)
+                atomicOr(err, KT_ERR_MESSAGE);
+            else
+                note_tiles((uint32_t)c, c ? a : 0, b, mtot, SH_TILE, mbnd);  // (entries before the first message: row 0)
         }
     }
-}
-
-// Ghost bits of the rank-select table (zeroed before): word w of the table
-// is rs32[2w], its prefix count rs32[2w + 1].
-__global__ void k_ghost_bits(uint32_t ng, const uint32_t* __restrict__ ghost_ids, uint32_t n_all,
-                             uint32_t* __restrict__ rs32, uint32_t* __restrict__ err) {
-    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += gridDim.x * blockDim.x) {
-        const uint32_t id = ghost_ids[g];
-        if (id < n_all)
-            atomicOr(&rs32[2 * (id >> 5)], 1u << (id & 31));
-        else
-            atomicOr(err, KT_ERR_GHOST);
-    }
-}
-
-__global__ void k_rs_count(uint64_t words, const uint2* __restrict__ rs, uint64_t* __restrict__ cnt) {
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += (uint64_t)gridDim.x * blockDim.x)
-        cnt[w] = __popc(rs[w].x);
-}
-
-__global__ void k_rs_prefix(uint64_t words, const uint64_t* __restrict__ pre, uint2* __restrict__ rs) {
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += (uint64_t)gridDim.x * blockDim.x)
-        rs[w].y = (uint32_t)pre[w];
 }
 
 __device__ __forceinline__ bool c_less(const ShardMap& M, const uint32_t* deg, uint32_t a, uint32_t b) {
@@ -109,13 +120,18 @@ __device__ __forceinline__ bool c_less(const ShardMap& M, const uint32_t* deg, u
 }
 
 // Owned slots -> (tail, head) keys of N+ lists and (cetric-x) ghost lists,
-// appended in any order (they are sorted next): every wave counts its keys
-// over the tile's 16 slot rounds, and one atomic per workgroup reserves the
-// workgroup's output range.
+// appended in any order, each with its rank among its tail's entries; the
+// tails' counts are left in cnt (zeroed by the caller).  Every wave counts its
+// keys over the tile's 16 slot rounds, and one atomic per workgroup reserves
+// the workgroup's output range.  The ranks come from the counts' atomics: a
+// run of a wave's slots with one owned tail takes one, a ghost list's entry its
+// own (few per ghost: an entry's owned head follows the ghost in degree order).
+// All of a thread's atomics are in flight together.
 __global__ void __launch_bounds__(SH_THREADS)
     k_shard_entries(ShardMap M, uint64_t nnz, const uint64_t* __restrict__ off, const uint32_t* __restrict__ tbnd,
                     const uint32_t* __restrict__ heads, const uint32_t* __restrict__ deg, int bits, int ghost_lists,
-                    uint64_t* __restrict__ keys, uint64_t* __restrict__ nkeys, uint32_t* __restrict__ err) {
+                    uint64_t* __restrict__ keys, uint32_t* __restrict__ rank, uint64_t* __restrict__ cnt,
+                    uint64_t* __restrict__ nkeys, uint32_t* __restrict__ err) {
     constexpr int NW = SH_THREADS / KT_WAVE;
     __shared__ uint32_t marks[SH_TILE];
     __shared__ uint32_t wmax[NW];
@@ -125,7 +141,7 @@ __global__ void __launch_bounds__(SH_THREADS)
     const uint64_t tile0 = (uint64_t)blockIdx.x * SH_TILE;
     const uint64_t tend = min(tile0 + SH_TILE, nnz);
     uint32_t lo, hi;
-    tile_rows<SH_THREADS, SH_ITEMS>(off, M.nl, tile0, tend, marks, bnd, wmax, lo, hi, tbnd);
+    tile_rows<SH_THREADS, SH_ITEMS>(off, M.nl, tile0, tend, marks, bnd, wmax, lo, hi, tbnd, err);
     const unsigned tid = threadIdx.x, wave = tid / KT_WAVE;
     uint32_t cs[SH_ITEMS];
 #pragma unroll
@@ -134,7 +150,7 @@ __global__ void __launch_bounds__(SH_THREADS)
         cs[k] = sl < tend ? M.map(heads[sl]) : 0u;
     }
     uint32_t flags = 0, count = 0;
-    uint64_t key[SH_ITEMS], pm[SH_ITEMS];
+    uint64_t pm[SH_ITEMS], om[SH_ITEMS];
 #pragma unroll
     for (int k = 0; k < SH_ITEMS; ++k) {
         const unsigned i = k * SH_THREADS + tid;
@@ -150,9 +166,28 @@ __global__ void __launch_bounds__(SH_THREADS)
                 in_e = ghost_lists && !out_e && c >= M.nl;
             }
         }
-        key[k] = out_e ? (((uint64_t)v << bits) | c) : (((uint64_t)c << bits) | v);
-        pm[k] = __ballot(out_e || in_e);
+        om[k] = __ballot(out_e);
+        pm[k] = om[k] | __ballot(in_e);
         count += (uint32_t)__popcll(pm[k]);
+    }
+    // this lane's entries of round k: the owned ones before it in its row's run
+    const uint64_t lt = lanemask_lt(), me = 1ull << lane_id();
+    uint32_t base[SH_ITEMS];
+#pragma unroll
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const uint32_t m = marks[k * SH_THREADS + tid], mp = __shfl_up(m, 1, 64);
+        const uint64_t starts = __ballot(lane_id() == 0 || m != mp);
+        const int s = 63 - __clzll((long long)(starts & (lt | me)));
+        const uint64_t after = starts & ~(lt | me);
+        const uint64_t run = om[k] & (~0ull << s) & (after ? (after & -after) - 1 : ~0ull);
+        const bool own = (om[k] & me) != 0;
+        const int lead = run ? __ffsll((unsigned long long)run) - 1 : 0;
+        uint32_t got = 0;
+        if ((pm[k] & me) && (!own || lead == (int)lane_id()))
+            got = (uint32_t)atomic_add_u64(&cnt[own ? lo + m : cs[k]], own ? (uint64_t)__popcll(run) : 1ull);
+        base[k] = __shfl(got, own ? lead : (int)lane_id(), 64) + (own ? (uint32_t)__popcll(run & lt) : 0u);
+        if (pm[k] & me) flags |= (base[k] >= segsort_wave_len() ? KT_FLAG_OVER_WAVE : 0u) |
+                                 (base[k] >= segsort_max_len() ? KT_FLAG_OVER_GROUP : 0u);
     }
     or_flags(err, flags);
     if (lane_id() == 0) wtot[wave] = count;
@@ -163,41 +198,38 @@ __global__ void __launch_bounds__(SH_THREADS)
         bbase = t ? atomic_add_u64(nkeys, t) : 0;
     }
     __syncthreads();
-    uint64_t base = bbase;
-    for (unsigned w = 0; w < wave; ++w) base += wtot[w];
+    uint64_t at = bbase;
+    for (unsigned w = 0; w < wave; ++w) at += wtot[w];
 #pragma unroll
     for (int k = 0; k < SH_ITEMS; ++k) {
-        if ((pm[k] >> lane_id()) & 1) keys[base + __popcll(pm[k] & lanemask_lt())] = key[k];
-        base += __popcll(pm[k]);
+        if (pm[k] & me) {
+            const uint64_t v = lo + marks[k * SH_THREADS + tid], c = cs[k], p = at + __popcll(pm[k] & lt);
+            keys[p] = (om[k] & me) ? (v << bits) | c : (c << bits) | v;
+            rank[p] = base[k];
+        }
+        at += __popcll(pm[k]);
     }
 }
 
-// Sorted keys -> heads of the CSR over X tails, and the list length of every
-// tail in cnt[0, X) (zeroed by the caller; an exclusive scan makes it the
-// offsets).  Runs of equal tails inside a wave add their length with one
-// atomic from the run's last lane.
-__global__ void k_keys_csr(uint64_t M, int bits, const uint64_t* __restrict__ keys, uint64_t* __restrict__ cnt,
-                           uint32_t* __restrict__ cheads, uint32_t* __restrict__ err) {
+// Every entry to its rank's place in its tail's list.
+__global__ void k_shard_place(uint64_t M, int bits, const uint64_t* __restrict__ keys,
+                              const uint32_t* __restrict__ rank, const uint64_t* __restrict__ coff,
+                              uint32_t* __restrict__ cheads) {
     const uint64_t mask = (1ull << bits) - 1;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x; i0 < M; i0 += stride) {  // wave-uniform trip count
-        const uint64_t i = i0 + threadIdx.x;
-        const bool in = i < M;
-        const uint64_t k = in ? keys[i] : ~0ull;
-        const uint64_t t = k >> bits;
-        if (in) {
-            cheads[i] = (uint32_t)(k & mask);
-            if (i > 0 && keys[i - 1] == k) atomicOr(err, KT_ERR_DUPLICATE);
-        }
-        const uint64_t tn = __shfl_down(t, 1, 64);
-        const unsigned lane = lane_id();
-        const bool end = in && (lane == KT_WAVE - 1 || i + 1 == M || tn != t);
-        const uint64_t ends = __ballot(end);
-        if (end) {
-            const uint64_t below = ends & lanemask_lt();
-            const int prev = below ? 63 - __clzll((long long)below) : -1;
-            atomic_add_u64(&cnt[t], (uint64_t)((int)lane - prev));
-        }
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < M; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t k = keys[i];
+        cheads[coff[k >> bits] + rank[i]] = (uint32_t)(k & mask);
+    }
+}
+
+// Sorted keys -> heads of the CSR (lists above the segmented sort's longest).
+__global__ void k_keys_csr(uint64_t M, int bits, const uint64_t* __restrict__ keys, uint32_t* __restrict__ cheads,
+                           uint32_t* __restrict__ err) {
+    const uint64_t mask = (1ull << bits) - 1;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < M; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t k = keys[i];
+        cheads[i] = (uint32_t)(k & mask);
+        if (i > 0 && keys[i - 1] == k) atomicOr(err, KT_ERR_DUPLICATE);
     }
 }
 
@@ -217,128 +249,181 @@ __global__ void k_cut_begin(uint32_t nl, const uint64_t* __restrict__ coff, cons
     cut[u] = lo;
 }
 
-// Messages are walked by groups of MSG_G lanes (one message per group; most
-// messages are short), each lane taking MSG_E consecutive entries per step so
-// that a message of up to 64 ids takes one step, its loads and rank-select
-// gathers all in flight together.
-constexpr unsigned MSG_G = 8;
-constexpr unsigned MSG_E = 8;
-
-__device__ __forceinline__ uint32_t group_sum(uint32_t x) {
-#pragma unroll
-    for (unsigned d = MSG_G / 2; d >= 1; d >>= 1) x += __shfl_xor(x, d, MSG_G);
-    return x;
-}
-
-// One step of a group over entries [p0, p0 + MSG_G * MSG_E) of a message
-// ending at e: this lane's entries p0 + gl + MSG_G * k (round k covers
-// MSG_G consecutive entries, one per lane, so every load and store of a
-// round is one contiguous run) and their combined indices (0xffffffff past
-// the end or unknown to the rank).
-struct MsgStep {
-    uint32_t x[MSG_E], c[MSG_E];
-    __device__ __forceinline__ static uint64_t at(uint64_t p0, unsigned gl, unsigned k) {
-        return p0 + gl + MSG_G * k;
-    }
-    __device__ __forceinline__ void load(const ShardMap& M, const uint32_t* __restrict__ mheads, uint64_t p0,
-                                         unsigned gl, uint64_t e) {
-#pragma unroll
-        for (unsigned k = 0; k < MSG_E; ++k) x[k] = (at(p0, gl, k) < e) ? mheads[at(p0, gl, k)] : 0u;
-#pragma unroll
-        for (unsigned k = 0; k < MSG_E; ++k) c[k] = (at(p0, gl, k) < e) ? M.map(x[k]) : 0xffffffffu;
-    }
-    // the combined indices stored by a previous pass at the entries' positions
-    __device__ __forceinline__ void load_mapped(const uint32_t* __restrict__ mapped, uint64_t p0, unsigned gl,
-                                                uint64_t e) {
-#pragma unroll
-        for (unsigned k = 0; k < MSG_E; ++k) c[k] = (at(p0, gl, k) < e) ? mapped[at(p0, gl, k)] : 0xffffffffu;
-    }
+// Messages are taken as one flat run of entries, in tiles of SH_TILE: with O(p)
+// and G(p) the owned and the ghost entries before entry p, and b, e a message's
+// first entry and its end, an owned entry p goes to O(p) + G(b), a ghost entry
+// to O(e) + G(p) -- the message's owned entries, then its ghosts, each in
+// message order.  A count pass gives every 64 entries' bits and every tile's
+// totals; a thread per message then ranks its b and e, and a write pass places
+// the entries.  Short and long messages take the same time (8 lanes per message
+// took 126 + 44 us for the 241,000 messages of an R-MAT CeTriC shard, most of it
+// one long message's steps; the three passes take 60).
+struct MsgWord {
+    uint64_t own, ghost;      // entry classes of 64 entries
+    uint32_t pre_own, pre_ghost;  // those of the tile's words before
 };
 
-// This group's bits of a wave ballot (lane gl of the group = bit gl).
-__device__ __forceinline__ uint32_t group_bits(uint64_t ballot) {
-    return (uint32_t)(ballot >> (lane_id() & ~(MSG_G - 1))) & ((1u << MSG_G) - 1);
+// No pass of the messages runs on offsets that fail their check, and none needs
+// to where an entry was found bad.  Block-wide.
+__device__ __forceinline__ bool messages_bad(const uint32_t* err, uint32_t* word) {
+    if (threadIdx.x == 0) *word = *err;
+    __syncthreads();
+    return (*word & KT_ERR_MASK) != 0;
 }
 
-// Per message: owned / ghost entry counts; sender -> combined index.  The
-// combined index of every entry is stored at the entry's position in `mapped`
-// (one streaming write instead of a second round of rank-select gathers).
-__global__ void k_msg_count(ShardMap M, uint32_t nmsg, uint64_t mtot, const uint32_t* __restrict__ src,
-                            const uint64_t* __restrict__ moff, const uint32_t* __restrict__ mheads,
-                            uint64_t* __restrict__ kept, uint32_t* __restrict__ nown, uint32_t* __restrict__ tail_id,
-                            uint32_t* __restrict__ mapped, uint32_t* __restrict__ err) {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t groups = (uint64_t)gridDim.x * blockDim.x / MSG_G;
-    const unsigned gl = lane_id() & (MSG_G - 1);
-    uint32_t flags = 0;
-    for (uint64_t i = t / MSG_G; i < nmsg; i += groups) {
-        const uint64_t b = moff[i], e = moff[i + 1];
-        const bool bad = e < b || e > mtot;
-        uint32_t own = 0, gh = 0;  // this lane's share
-        if (!bad) {
-            for (uint64_t p0 = b; p0 < e; p0 += MSG_G * MSG_E) {  // uniform over the group
-                MsgStep s;
-                s.load(M, mheads, p0, gl, e);
-                // the entry after this step's last one (read by the group's last lane)
-                const uint64_t pn = p0 + MSG_G * MSG_E;
-                const uint32_t xn = (gl == MSG_G - 1 && pn < e) ? mheads[pn] : 0u;
+// Combined index of every entry (to mapped; entries of no message are unknown),
+// order of the messages, and the entry classes.
+__global__ void __launch_bounds__(SH_THREADS)
+    k_msg_map(ShardMap M, uint32_t nmsg, uint64_t mtot, const uint64_t* __restrict__ moff,
+              const uint32_t* __restrict__ mbnd, const uint32_t* __restrict__ mheads, uint32_t* __restrict__ mapped,
+              MsgWord* __restrict__ words, uint64_t* __restrict__ tcnt, uint32_t* __restrict__ err) {
+    constexpr int NW = SH_THREADS / KT_WAVE;
+    static_assert(SH_ITEMS * NW == KT_WAVE, "a lane per word of a tile");
+    __shared__ uint32_t marks[SH_TILE];
+    __shared__ uint32_t wmax[NW];
+    __shared__ uint32_t bnd[2];
+    __shared__ uint64_t wo[KT_WAVE], wg[KT_WAVE];
+    if (messages_bad(err, bnd)) return;
+    const uint64_t tile0 = (uint64_t)blockIdx.x * SH_TILE;
+    const uint64_t tend = min(tile0 + SH_TILE, mtot);
+    uint32_t lo, hi;
+    __syncthreads();  // bnd has been read
+    tile_rows<SH_THREADS, SH_ITEMS>(moff, nmsg, tile0, tend, marks, bnd, wmax, lo, hi, mbnd);
+    const uint64_t first = moff[0];
+    const unsigned tid = threadIdx.x, wave = tid / KT_WAVE;
+    uint32_t x[SH_ITEMS], nx[SH_ITEMS], c[SH_ITEMS];
 #pragma unroll
-                for (unsigned k = 0; k < MSG_E; ++k) {
-                    // successor of entry (k, gl): lane gl + 1 of round k, or lane 0
-                    // of round k + 1 (shuffles outside any branch: the group is whole)
-                    const uint32_t up = __shfl_down(s.x[k], 1, MSG_G);
-                    const uint32_t first = __shfl(s.x[k + 1 < MSG_E ? k + 1 : k], 0, MSG_G);
-                    const uint32_t nx = gl + 1 < MSG_G ? up : (k + 1 < MSG_E ? first : xn);
-                    const uint64_t q = MsgStep::at(p0, gl, k);
-                    if (q >= e) continue;
-                    mapped[q] = s.c[k];
-                    if (q + 1 < e && nx <= s.x[k]) flags |= KT_ERR_MESSAGE;
-                    own += s.c[k] < M.nl ? 1u : 0u;
-                    gh += (s.c[k] != 0xffffffffu && s.c[k] >= M.nl) ? 1u : 0u;
-                }
-            }
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const uint64_t p = tile0 + k * SH_THREADS + tid;
+        x[k] = p < tend ? mheads[p] : 0u;
+        nx[k] = p + 1 < mtot ? mheads[p + 1] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const uint64_t p = tile0 + k * SH_THREADS + tid;
+        c[k] = p < tend && p >= first ? M.map(x[k]) : 0xffffffffu;
+    }
+    uint32_t flags = 0;
+#pragma unroll
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const uint32_t i = k * SH_THREADS + tid;
+        const uint64_t p = tile0 + i;
+        if (p < tend) {
+            mapped[p] = c[k];
+            const bool same = i + 1 < SH_TILE ? p + 1 < tend && marks[i + 1 < SH_TILE ? i + 1 : i] == marks[i]
+                                              : p + 1 < moff[(uint64_t)lo + marks[i] + 1];
+            if (p >= first && same && nx[k] <= x[k]) flags |= KT_ERR_MESSAGE;
         }
-        own = group_sum(own);
-        gh = group_sum(gh);
-        if (gl == 0) {
-            const uint32_t a = M.map(src[i]);
-            if (bad || a == 0xffffffffu || a < M.nl) flags |= KT_ERR_MESSAGE;
-            tail_id[i] = (a == 0xffffffffu) ? 0u : a;
-            kept[i] = own + gh;
-            nown[i] = own;
+        const uint64_t ob = __ballot(c[k] < M.nl), gb = __ballot(c[k] != 0xffffffffu && c[k] >= M.nl);
+        if (lane_id() == 0) {
+            wo[k * NW + wave] = ob;
+            wg[k * NW + wave] = gb;
         }
+    }
+    or_flags(err, flags);
+    __syncthreads();
+    if (wave != 0) return;
+    MsgWord w{wo[tid], wg[tid], 0, 0};
+    const uint64_t n = (uint64_t)__popcll(w.own) << 32 | (uint32_t)__popcll(w.ghost);
+    const uint64_t incl = wave_incl_sum(n);
+    w.pre_own = (uint32_t)((incl - n) >> 32);
+    w.pre_ghost = (uint32_t)(incl - n);
+    if (tile0 + tid * 64 < tend) words[tile0 / 64 + tid] = w;
+    if (tid == KT_WAVE - 1) {
+        tcnt[blockIdx.x] = incl >> 32;
+        tcnt[gridDim.x + blockIdx.x] = (uint32_t)incl;
+    }
+}
+
+// Owned and ghost entries before entry p; toff: scan of the tiles' owned, then
+// ghost counts.
+__device__ __forceinline__ void msg_ranks(uint64_t p, uint64_t mtot, uint64_t tiles, const MsgWord* __restrict__ words,
+                                          const uint64_t* __restrict__ toff, uint64_t& own, uint64_t& ghost) {
+    const uint64_t t = min(p / SH_TILE, tiles);
+    own = toff[t];
+    ghost = toff[tiles + t] - toff[tiles];
+    if (p >= mtot) {
+        own = toff[tiles];
+        ghost = toff[2 * tiles] - toff[tiles];
+        return;
+    }
+    const MsgWord w = words[p / 64];
+    const uint64_t lt = (1ull << (p & 63)) - 1;
+    own += w.pre_own + (uint32_t)__popcll(w.own & lt);
+    ghost += w.pre_ghost + (uint32_t)__popcll(w.ghost & lt);
+}
+
+// Per message: its list in the output, the list's first ghost, the ghosts
+// before it, and its sender's combined index.
+__global__ void k_msg_place(ShardMap M, uint32_t nmsg, uint64_t mtot, uint64_t tiles, const uint32_t* __restrict__ src,
+                            const uint64_t* __restrict__ moff, const MsgWord* __restrict__ words,
+                            const uint64_t* __restrict__ toff, uint64_t* __restrict__ out_off,
+                            uint64_t* __restrict__ split, uint64_t* __restrict__ gbeg, uint32_t* __restrict__ tail_id,
+                            uint32_t* __restrict__ err) {
+    if (*err & KT_ERR_MASK) return;
+    uint32_t flags = 0;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nmsg; i += gridDim.x * blockDim.x) {
+        uint64_t o0, g0, o1, g1;
+        msg_ranks(moff[i], mtot, tiles, words, toff, o0, g0);
+        msg_ranks(moff[i + 1], mtot, tiles, words, toff, o1, g1);
+        const uint32_t a = M.map(src[i]);
+        if (a == 0xffffffffu || a < M.nl) flags |= KT_ERR_MESSAGE;
+        if (o1 + g1 - o0 - g0 > segsort_wave_len()) flags |= KT_FLAG_LONG_MESSAGE;
+        tail_id[i] = (a == 0xffffffffu) ? 0u : a;
+        out_off[i] = o0 + g0;
+        split[i] = o1 + g0;
+        gbeg[i] = g0;
+        if (i + 1 == nmsg) out_off[nmsg] = o1 + g1;
     }
     or_flags(err, flags);
 }
 
-// Per message: owned entries then ghost entries, each in message order.
-__global__ void k_msg_write(uint32_t nl, uint32_t nmsg, uint64_t mtot, const uint64_t* __restrict__ moff,
-                            const uint32_t* __restrict__ mapped, const uint64_t* __restrict__ coff_msg,
-                            const uint32_t* __restrict__ nown, uint32_t* __restrict__ out,
-                            uint64_t* __restrict__ split) {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t groups = (uint64_t)gridDim.x * blockDim.x / MSG_G;
-    const unsigned gl = lane_id() & (MSG_G - 1);
-    const uint32_t below = (1u << gl) - 1;  // this lane's predecessors in the group
-    for (uint64_t i = t / MSG_G; i < nmsg; i += groups) {
-        const uint64_t b = moff[i], e = moff[i + 1];
-        uint64_t po = coff_msg[i], pg = coff_msg[i] + nown[i];
-        if (gl == 0) split[i] = pg;
-        if (e < b || e > mtot) continue;  // flagged by k_msg_count; nothing was counted for it (uniform per group)
-        for (uint64_t p0 = b; p0 < e; p0 += MSG_G * MSG_E) {
-            MsgStep s;
-            s.load_mapped(mapped, p0, gl, e);
+__global__ void __launch_bounds__(SH_THREADS)
+    k_msg_write(uint32_t nl, uint32_t nmsg, uint64_t mtot, const uint64_t* __restrict__ moff,
+                const uint32_t* __restrict__ mbnd, const uint32_t* __restrict__ mapped,
+                const uint64_t* __restrict__ toff, uint64_t tiles, const uint64_t* __restrict__ split,
+                const uint64_t* __restrict__ gbeg, uint32_t* __restrict__ out, const uint32_t* __restrict__ err) {
+    constexpr int NW = SH_THREADS / KT_WAVE;
+    __shared__ uint32_t marks[SH_TILE];
+    __shared__ uint32_t wmax[NW];
+    __shared__ uint32_t bnd[2];
+    __shared__ uint32_t pre[KT_WAVE];  // owned << 16 | ghost entries of the tile's words before
+    if (messages_bad(err, bnd)) return;
+    const uint64_t tile0 = (uint64_t)blockIdx.x * SH_TILE;
+    const uint64_t tend = min(tile0 + SH_TILE, mtot);
+    uint32_t lo, hi;
+    __syncthreads();  // bnd has been read
+    tile_rows<SH_THREADS, SH_ITEMS>(moff, nmsg, tile0, tend, marks, bnd, wmax, lo, hi, mbnd);
+    const unsigned tid = threadIdx.x, wave = tid / KT_WAVE;
+    uint32_t c[SH_ITEMS];
 #pragma unroll
-            for (unsigned k = 0; k < MSG_E; ++k) {
-                // round k holds consecutive entries in lane order
-                const bool o = s.c[k] < nl, h = s.c[k] != 0xffffffffu && s.c[k] >= nl;
-                const uint32_t ob = group_bits(__ballot(o)), hb = group_bits(__ballot(h));
-                if (o) out[po + __popc(ob & below)] = s.c[k];
-                if (h) out[pg + __popc(hb & below)] = s.c[k];
-                po += __popc(ob);
-                pg += __popc(hb);
-            }
-        }
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const uint64_t p = tile0 + k * SH_THREADS + tid;
+        c[k] = p < tend ? mapped[p] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const uint32_t o = (uint32_t)__popcll(__ballot(c[k] < nl));
+        const uint32_t known = (uint32_t)__popcll(__ballot(c[k] != 0xffffffffu));
+        if (lane_id() == 0) pre[k * NW + wave] = o << 16 | (known - o);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const uint32_t n = pre[tid];
+        pre[tid] = wave_incl_sum(n) - n;
+    }
+    __syncthreads();
+    const uint64_t obase = toff[blockIdx.x], gbase = toff[tiles + blockIdx.x] - toff[tiles], lt = lanemask_lt();
+#pragma unroll
+    for (int k = 0; k < SH_ITEMS; ++k) {
+        const bool own = c[k] < nl, known = c[k] != 0xffffffffu;
+        const uint64_t ob = __ballot(own), gb = __ballot(known) & ~ob;
+        const uint32_t w = pre[k * NW + wave], i = lo + marks[k * SH_THREADS + tid];
+        if (!known) continue;
+        const uint64_t g0 = gbeg[i];
+        const uint64_t p = own ? obase + (w >> 16) + (uint32_t)__popcll(ob & lt) + g0
+                               : gbase + (w & 0xffffu) + (uint32_t)__popcll(gb & lt) + split[i] - g0;
+        out[p] = c[k];
     }
 }
 
@@ -370,9 +455,10 @@ struct ShardBufs {
     uint64_t* coff;
     uint32_t* cheads;
     uint64_t* cut;
-    uint64_t* mkept;
+    uint64_t* mgbeg;
     uint64_t* moff;
-    uint32_t* mnown;
+    uint64_t* mtoff;
+    uint32_t* mbnd;
     uint32_t* mtail;
     uint64_t* msplit;
     uint32_t* mheads2;
@@ -381,7 +467,6 @@ struct ShardBufs {
     uint64_t* tc_ws;
     uint64_t* pv;
     uint2* rs;
-    uint64_t* rs_cnt;
     uint32_t* tbnd;
     TcRoom room;
 };
@@ -409,24 +494,27 @@ uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t 
     B.coff = static_cast<uint64_t*>(cv.take((X + 1) * 8));
     B.cheads = static_cast<uint32_t*>(cv.take((nnz + 4) * 4));
     B.cut = static_cast<uint64_t*>(cv.take(std::max<uint64_t>(nloc, 1) * 8));
-    B.mkept = static_cast<uint64_t*>(cv.take(((uint64_t)in->n_msg + 1) * 8));
+    const uint64_t mtiles = (mtot + SH_TILE - 1) / SH_TILE;
+    B.mgbeg = static_cast<uint64_t*>(cv.take(std::max<uint64_t>(in->n_msg, 1) * 8));
     B.moff = static_cast<uint64_t*>(cv.take(((uint64_t)in->n_msg + 1) * 8));
-    B.mnown = static_cast<uint32_t*>(cv.take(std::max<uint64_t>(in->n_msg, 1) * 4));
+    B.mtoff = static_cast<uint64_t*>(cv.take((2 * mtiles + 1) * 8));
+    B.mbnd = static_cast<uint32_t*>(cv.take((2 * mtiles + 1) * 4));
     B.mtail = static_cast<uint32_t*>(cv.take(std::max<uint64_t>(in->n_msg, 1) * 4));
     B.msplit = static_cast<uint64_t*>(cv.take(std::max<uint64_t>(in->n_msg, 1) * 8));
-    B.mheads2 = static_cast<uint32_t*>(cv.take((mtot + 4) * 4));
+    // (the entry classes sit here until the entries are written)
+    static_assert(sizeof(MsgWord) <= 64 * sizeof(uint32_t), "words fit the entries' room");
+    B.mheads2 = static_cast<uint32_t*>(cv.take(std::max((mtot + 4) * 4, (mtot + 63) / 64 * sizeof(MsgWord))));
     B.mmapped = static_cast<uint32_t*>(cv.take(std::max<uint64_t>(mtot, 1) * 4));
     const uint64_t n_all = in->range_bounds[in->num_ranks];
     const uint64_t rs_words = (n_all + 31) / 32;
     B.scan_tmp = static_cast<uint64_t*>(
-        cv.take(scan_tmp_words(std::max(std::max<uint64_t>(X, in->n_msg), rs_words) + 1) * 8));
+        cv.take(scan_tmp_words(std::max<uint64_t>(X, 2 * mtiles) + 1) * 8));
     // both phases use it: the list of the larger set of tails, the parts of the longer walk
     B.room = rich ? tc_room(std::max(nnz, mtot), 0, want_pv ? X : 0) : TcRoom{};
     B.tc_ws = static_cast<uint64_t*>(
         cv.take(tc_ws_words((uint32_t)std::max<uint64_t>(X, in->n_msg), B.room, num_cus) * 8));
     B.pv = pv_dev ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(X, 1) * 8)) : nullptr;
     B.rs = static_cast<uint2*>(cv.take((rs_words + 1) * 8));
-    B.rs_cnt = static_cast<uint64_t*>(cv.take((rs_words + 1) * 8));
     B.tbnd = static_cast<uint32_t*>(cv.take((2 * ((nnz + SH_TILE - 1) / SH_TILE) + 1) * 4));
     return cv.used;
 }
@@ -434,7 +522,7 @@ uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t 
 }  // namespace
 
 // The body of kt_count_shard; the caller holds c->mu and has begun the call.
-int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) {
+int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, const ShardSizes* sizes) {
     int rc = KT_OK;
     if (!in || !out || !in->range_bounds || !in->offsets || in->num_ranks == 0 || in->rank >= in->num_ranks ||
         in->algorithm > KT_SHARD_DITRIC)
@@ -465,11 +553,16 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
         mtot = in->n_msg ? in->msg_offsets[in->n_msg] : 0;
         if (in->n_msg && in->msg_offsets[0] != 0) return c->fail(KT_EINVAL, "msg_offsets[0] != 0");
     } else {
-        rc = c->read_u64(in->offsets + nl, &nnz, "D2H nnz");
-        if (rc) return rc;
-        if (in->n_msg) {
-            rc = c->read_u64(in->msg_offsets + in->n_msg, &mtot, "D2H mtot");
+        if (sizes) {
+            nnz = sizes->slots;
+            mtot = sizes->entries;
+        } else {
+            const uint64_t* at[2] = {in->offsets + nl, in->n_msg ? in->msg_offsets + in->n_msg : in->offsets + nl};
+            uint64_t got[2];
+            rc = c->read_words(at, 2, got, "D2H shard sizes");
             if (rc) return rc;
+            nnz = got[0];
+            mtot = in->n_msg ? got[1] : 0;
         }
     }
     if ((nnz && !in->heads) || (ng && (!in->ghost_ids || !in->ghost_degree)) ||
@@ -517,29 +610,38 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
     (void)hipEventRecord(c->ev[EV_H2D], st);
     uint32_t* err = reinterpret_cast<uint32_t*>(B.small);
     uint64_t* nkeys = B.small + 1;
-    fill_u64(B.small, 64, 0, st);
     const uint64_t n_all = bd[P];
     ShardMap M{from, to, nl, ng, B.ghost_ids, B.rs, (uint32_t)std::min<uint64_t>(n_all, 0xffffffffull)};
     {
-        const uint64_t rs_words = (n_all + 31) / 32;
-        fill_u64(reinterpret_cast<uint64_t*>(B.rs), rs_words, 0, st);
-        if (ng)
-            k_ghost_bits<<<(unsigned)std::min<uint64_t>((ng + 255) / 256, 8192), 256, 0, st>>>(
-                ng, B.ghost_ids, M.n_all, reinterpret_cast<uint32_t*>(B.rs), err);
-        const unsigned gw = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((rs_words + 255) / 256, 16384));
-        k_rs_count<<<gw, 256, 0, st>>>(rs_words, B.rs, B.rs_cnt);
-        scan_u64(B.rs_cnt, B.rs_cnt, rs_words, B.scan_tmp, st);
-        k_rs_prefix<<<gw, 256, 0, st>>>(rs_words, B.rs_cnt, B.rs);
+        ClearList cl;
+        cl.add(B.small, 64);
+        cl.add(reinterpret_cast<uint64_t*>(B.rs), (n_all + 31) / 32);
+        cl.add(B.coff, X + 1);
+        clear(cl, st);
     }
     const int bits = std::max(1, bits_for(X));  // X itself is never a valid index: keys stay below 2^(2 bits)
     const bool cetric = in->algorithm == KT_SHARD_CETRIC;
-    k_shard_prepare<<<(unsigned)std::min<uint64_t>((X + 255) / 256, 8192), 256, 0, st>>>(M, nnz, B.off,
-                                                                                      B.ghost_degree, B.deg, err);
+    const uint64_t both = std::max<uint64_t>(X, in->n_msg);
+    k_shard_prepare<<<(unsigned)std::min<uint64_t>((both + 255) / 256, 8192), 256, 0, st>>>(
+        M, nnz, B.off, B.ghost_degree, B.deg, B.tbnd, B.rs, in->n_msg, mtot, B.msg_off, B.mbnd, err);
     const uint64_t tiles = (nnz + SH_TILE - 1) / SH_TILE;
-    if (tiles && nl) {
-        tile_bounds_launch(nl, nnz, SH_TILE, B.off, B.tbnd, st);
+    uint32_t* rank = reinterpret_cast<uint32_t*>(B.alt);
+    if (tiles && nl)
         k_shard_entries<<<(unsigned)tiles, SH_THREADS, 0, st>>>(M, nnz, B.off, B.tbnd, B.heads, B.deg, bits,
-                                                                cetric ? 1 : 0, B.keys, nkeys, err);
+                                                                cetric ? 1 : 0, B.keys, rank, B.coff, nkeys, err);
+    // messages (on a malformed shard the later passes do nothing)
+    if (in->n_msg) {
+        const uint64_t mt = (mtot + SH_TILE - 1) / SH_TILE;
+        MsgWord* words = reinterpret_cast<MsgWord*>(B.mheads2);
+        if (mt)
+            k_msg_map<<<(unsigned)mt, SH_THREADS, 0, st>>>(M, in->n_msg, mtot, B.msg_off, B.mbnd, B.msg_heads,
+                                                           B.mmapped, words, B.mtoff, err);
+        scan_u64(B.mtoff, B.mtoff, 2 * mt, B.scan_tmp, st);
+        k_msg_place<<<(unsigned)std::min<uint64_t>(((uint64_t)in->n_msg + 255) / 256, 8192), 256, 0, st>>>(
+            M, in->n_msg, mtot, mt, B.msg_src, B.msg_off, words, B.mtoff, B.moff, B.msplit, B.mgbeg, B.mtail, err);
+        if (mt)
+            k_msg_write<<<(unsigned)mt, SH_THREADS, 0, st>>>(nl, in->n_msg, mtot, B.msg_off, B.mbnd, B.mmapped,
+                                                             B.mtoff, mt, B.msplit, B.mgbeg, B.mheads2, err);
     }
     rc = c->hip_check(hipMemcpyAsync(c->host_small, B.small, 16, hipMemcpyDeviceToHost, st), "D2H flags");
     if (rc) return rc;
@@ -548,32 +650,35 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
     uint32_t flags = (uint32_t)c->host_small[0];
     const uint64_t Mk = c->host_small[1];
     if (flags & KT_ERR_MASK)
-        return c->fail(KT_EINVAL, "malformed shard:%s%s%s%s", (flags & KT_ERR_OFFSETS) ? " bad offsets" : "",
+        return c->fail(KT_EINVAL, "malformed shard:%s%s%s%s%s", (flags & KT_ERR_OFFSETS) ? " bad offsets" : "",
                        (flags & KT_ERR_GHOST) ? " ghost table" : "", (flags & KT_ERR_SELF_LOOP) ? " self-loop" : "",
-                       (flags & KT_ERR_DUPLICATE) ? " duplicate" : "");
-    radix_sort_u64(B.keys, B.alt, Mk, 2 * bits, B.radix_tmp, st);
-    fill_u64(B.coff, X + 1, 0, st);
-    if (Mk)
-        k_keys_csr<<<(unsigned)std::min<uint64_t>((Mk + 255) / 256, 16384), 256, 0, st>>>(Mk, bits, B.keys, B.coff,
-                                                                                         B.cheads, err);
+                       (flags & KT_ERR_DUPLICATE) ? " duplicate" : "",
+                       (flags & KT_ERR_MESSAGE) ? " bad message" : "");
+    // the lists: their offsets, then each entry to its rank's place and every
+    // list sorted by itself, or, with one longer than that sort takes, all keys
+    // by their bits.  (Five radix passes of five launches took 220 us for the
+    // 466,000 keys of an R-MAT CeTriC shard, place and sort 40.)
+    const bool over_wave = (flags & KT_FLAG_OVER_WAVE) != 0, over_group = (flags & KT_FLAG_OVER_GROUP) != 0;
     scan_u64(B.coff, B.coff, X, B.scan_tmp, st);
-    if (nl) k_cut_begin<<<(nl + 255) / 256, 256, 0, st>>>(nl, B.coff, B.cheads, B.cut);
-    // messages
-    if (in->n_msg) {
-        k_msg_count<<<(unsigned)std::min<uint64_t>(((uint64_t)in->n_msg * MSG_G + 255) / 256, 8192), 256, 0, st>>>(
-            M, in->n_msg, mtot, B.msg_src, B.msg_off, B.msg_heads, B.mkept, B.mnown, B.mtail, B.mmapped, err);
-        scan_u64(B.mkept, B.moff, in->n_msg, B.scan_tmp, st);
-        k_msg_write<<<(unsigned)std::min<uint64_t>(((uint64_t)in->n_msg * MSG_G + 255) / 256, 8192), 256, 0, st>>>(
-            M.nl, in->n_msg, mtot, B.msg_off, B.mmapped, B.moff, B.mnown, B.mheads2, B.msplit);
+    if (Mk) {
+        const unsigned g = (unsigned)std::min<uint64_t>((Mk + 255) / 256, 16384);
+        if (over_group) {
+            radix_sort_u64(B.keys, B.alt, Mk, 2 * bits, B.radix_tmp, st);
+            k_keys_csr<<<g, 256, 0, st>>>(Mk, bits, B.keys, B.cheads, err);
+        } else {
+            k_shard_place<<<g, 256, 0, st>>>(Mk, bits, B.keys, rank, B.coff, B.cheads);
+            segsort_launch((uint32_t)X, B.coff, B.cheads, err, over_wave ? segsort_max_len() : segsort_wave_len(),
+                           c->num_cus, st);
+        }
     }
+    if (nl) k_cut_begin<<<(nl + 255) / 256, 256, 0, st>>>(nl, B.coff, B.cheads, B.cut);
     rc = c->hip_check(hipMemcpyAsync(c->host_small, B.small, 8, hipMemcpyDeviceToHost, st), "D2H flags");
     if (rc) return rc;
     rc = c->hip_check(hipStreamSynchronize(st), "shard preprocessing");
     if (rc) return rc;
     flags = (uint32_t)c->host_small[0];
     if (flags & KT_ERR_MASK)
-        return c->fail(KT_EINVAL, "malformed shard:%s%s", (flags & KT_ERR_DUPLICATE) ? " duplicate edge" : "",
-                       (flags & KT_ERR_MESSAGE) ? " bad message" : "");
+        return c->fail(KT_EINVAL, "malformed shard:%s", (flags & KT_ERR_DUPLICATE) ? " duplicate edge" : "");
     (void)hipEventRecord(c->ev[EV_PREP], st);
     uint64_t* pv = want_pv ? (pv_dev ? out->per_vertex : B.pv) : nullptr;
     if (pv) fill_u64(pv, X, 0, st);
@@ -596,6 +701,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
             v.theads = B.cheads;
         }
         v.room = B.room;
+        v.longest = over_wave ? 0 : segsort_wave_len();
         TcOut o{pv, totals};
         rc = c->hip_check(tc_launch(v, o, c->prm, B.tc_ws, c->num_cus, st, c->ev[EV_TC0], c->ev[EV_TC1]),
                           "intersection launch");
@@ -628,6 +734,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out) 
         v.stat_off = B.msg_off;
         v.stat_skip_empty = cetric ? 1u : 0u;
         v.room = B.room;
+        v.longest = (flags & KT_FLAG_LONG_MESSAGE) ? 0 : segsort_wave_len();
         TcOut o{pv, totals + 1};
         // message tails have short owned parts: a whole workgroup on one of
         // them idles, so tails up to the largest wave table stay with one

@@ -42,40 +42,50 @@ __device__ __forceinline__ bool before(uint32_t da, uint32_t a, uint32_t db, uin
     return da < db || (da == db && a < b);
 }
 
-__device__ __forceinline__ void set_bit(uint32_t* bits, uint32_t u) {
-    const uint32_t w = u >> 5, b = 1u << (u & 31);
-    if (!(bits[w] & b)) atomicOr(&bits[w], b);  // a stale read only costs a redundant atomic
-}
-
+// Degrees (offsets validated), the rank's rebased offsets loff[0..nl], and the
+// rows of every tile's first and last slot: sbnd over the whole graph in tiles
+// of SYM_TILE, lbnd over the rank's slots in tiles of PD_TILE.
 __global__ void k_pd_degree(uint32_t n, uint64_t nnz, const uint64_t* __restrict__ off, uint32_t* __restrict__ deg,
-                            uint32_t* __restrict__ err) {
+                            uint32_t* __restrict__ sbnd, uint32_t from, uint32_t nl, uint64_t nnz_l,
+                            uint64_t* __restrict__ loff, uint32_t* __restrict__ lbnd, uint32_t* __restrict__ err) {
+    const uint64_t base = off[from];
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
-        if (v == 0 && (off[0] != 0 || off[n] != nnz)) atomicOr(err, KT_ERR_OFFSETS);
-        const uint64_t a = off[v], b = off[v + 1];
+    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= n; v += stride) {
+        const uint64_t a = off[v];
+        if (v >= from && v - from <= nl) loff[v - from] = a - base;
+        if (v == n) break;
+        const uint64_t b = off[v + 1];
+        if (v == 0 && (a != 0 || off[n] != nnz)) atomicOr(err, KT_ERR_OFFSETS);
         if (b < a || b - a > 0xffffffffull || b > nnz) {
             atomicOr(err, KT_ERR_OFFSETS);
             deg[v] = 0;
-        } else {
-            deg[v] = (uint32_t)(b - a);
+            continue;
         }
+        deg[v] = (uint32_t)(b - a);
+        note_tiles((uint32_t)v, a, b, nnz, SYM_TILE, sbnd);
+        if (v >= from && v - from < nl) note_tiles((uint32_t)(v - from), a - base, b - base, nnz_l, PD_TILE, lbnd);
     }
 }
 
 // Slots of the rank's rows [from, from + nl): loff = rebased offsets (loff[0]
 // = 0), lheads = the rows' heads, tbnd = rows of every tile's first and last
-// slot.
+// slot.  marks: two bytes per vertex the rank does not own, in id order: ghost,
+// sender.  Plain byte stores: every store to a byte writes the same value.  (With
+// a bit per vertex, set by atomics where a load saw it clear, the hubs' words
+// took the pass 155 us for 613,000 slots of an R-MAT graph: a load may see a
+// line from before, and atomics of all XCDs on one word take turns; the stores
+// take 24.)
 __global__ void __launch_bounds__(PD_THREADS)
     k_pd_mark(const uint64_t* __restrict__ loff, uint32_t nl, uint32_t from, uint32_t n, uint64_t nnz_l,
               const uint32_t* __restrict__ lheads, const uint32_t* __restrict__ tbnd, const uint32_t* __restrict__ deg,
-              uint32_t* __restrict__ gbits, uint32_t* __restrict__ sbits, uint32_t* __restrict__ err) {
+              uint16_t* __restrict__ marks2, uint32_t* __restrict__ err) {
     __shared__ uint32_t marks[PD_TILE];
     __shared__ uint32_t wmax[PD_THREADS / KT_WAVE];
     __shared__ uint32_t bnd[2];
     const uint64_t tile0 = (uint64_t)blockIdx.x * PD_TILE;
     const uint64_t tend = min(tile0 + PD_TILE, nnz_l);
     uint32_t lo, hi;
-    tile_rows<PD_THREADS, PD_ITEMS>(loff, nl, tile0, tend, marks, bnd, wmax, lo, hi, tbnd);
+    tile_rows<PD_THREADS, PD_ITEMS>(loff, nl, tile0, tend, marks, bnd, wmax, lo, hi, tbnd, err);
     const uint32_t to = from + nl;
     uint32_t us[PD_ITEMS];
 #pragma unroll
@@ -93,53 +103,80 @@ __global__ void __launch_bounds__(PD_THREADS)
             flags |= KT_ERR_HEAD_RANGE;
         } else if (u < from || u >= to) {
             const uint32_t x = from + lo + marks[i];
-            set_bit(gbits, u);
-            if (before(deg[u], u, deg[x], x)) set_bit(sbits, u);
+            uint16_t* m = marks2 + (u < from ? u : u - nl);
+            if (before(deg[u], u, deg[x], x))
+                *m = 0x0101;
+            else
+                *reinterpret_cast<uint8_t*>(m) = 1;
         }
     }
     or_flags(err, flags);
 }
 
-__global__ void k_pd_popc(uint64_t words, const uint32_t* __restrict__ gbits, const uint32_t* __restrict__ sbits,
-                          uint64_t* __restrict__ gcnt, uint64_t* __restrict__ scnt) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += stride) {
-        gcnt[w] = __popc(gbits[w]);
-        scnt[w] = __popc(sbits[w]);
-    }
+// Eight marks of a thread, 2048 of a block: bits 0 and 8 of each.
+constexpr int MK_ITEMS = 8;
+constexpr int MK_TILE = PD_THREADS * MK_ITEMS;
+
+// Ghosts and senders of every tile of marks.
+__global__ void __launch_bounds__(PD_THREADS)
+    k_pd_count(const uint4* __restrict__ marks, uint64_t* __restrict__ cnt) {
+    __shared__ uint32_t w[PD_THREADS / KT_WAVE];
+    const uint4 m = marks[(uint64_t)blockIdx.x * PD_THREADS + threadIdx.x];
+    const uint32_t g = __popc(m.x & 0x00ff00ffu) + __popc(m.y & 0x00ff00ffu) + __popc(m.z & 0x00ff00ffu) + __popc(m.w & 0x00ff00ffu);
+    const uint32_t s = __popc(m.x & 0xff00ff00u) + __popc(m.y & 0xff00ff00u) + __popc(m.z & 0xff00ff00u) + __popc(m.w & 0xff00ff00u);
+    const uint32_t t = wave_total_dpp(g << 16 | s);
+    if (lane_id() == 0) w[threadIdx.x / KT_WAVE] = t;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    uint32_t sum = 0;
+    for (unsigned i = 0; i < PD_THREADS / KT_WAVE; ++i) sum += w[i];
+    cnt[blockIdx.x] = sum >> 16;
+    cnt[gridDim.x + blockIdx.x] = sum & 0xffffu;
 }
 
-__global__ void k_pd_compact(uint64_t words, const uint32_t* __restrict__ gbits, const uint64_t* __restrict__ goff,
-                             const uint32_t* __restrict__ sbits, const uint64_t* __restrict__ soff,
-                             const uint64_t* __restrict__ off, uint32_t* __restrict__ ghost_ids,
-                             uint64_t* __restrict__ ghost_deg, uint32_t* __restrict__ msg_src,
-                             uint64_t* __restrict__ vlen) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += stride) {
-        uint32_t bits = gbits[w];
-        uint64_t p = goff[w];
-        while (bits) {
-            const uint32_t id = (uint32_t)(w * 32) + (__ffs(bits) - 1);
-            bits &= bits - 1;
-            ghost_ids[p] = id;
-            ghost_deg[p] = off[id + 1] - off[id];
-            ++p;
-        }
-        bits = sbits[w];
-        p = soff[w];
-        while (bits) {
-            const uint32_t id = (uint32_t)(w * 32) + (__ffs(bits) - 1);
-            bits &= bits - 1;
-            msg_src[p] = id;
-            vlen[p] = off[id + 1] - off[id];
-            ++p;
+// Ghosts and senders in id order, with their degrees; toff: scan of the tiles'
+// ghosts, then senders.  small[1..3]: ghosts, senders, the senders' degrees.
+__global__ void __launch_bounds__(PD_THREADS)
+    k_pd_compact(const uint4* __restrict__ marks, uint64_t tiles, const uint64_t* __restrict__ toff, uint32_t from,
+                 uint32_t nl, const uint32_t* __restrict__ deg, uint32_t* __restrict__ ghost_ids,
+                 uint64_t* __restrict__ ghost_deg, uint32_t* __restrict__ msg_src, uint64_t* __restrict__ vlen,
+                 uint64_t* __restrict__ small) {
+    __shared__ uint32_t w[PD_THREADS / KT_WAVE];
+    const uint64_t at = (uint64_t)blockIdx.x * PD_THREADS + threadIdx.x;
+    const uint4 m = marks[at];
+    const uint32_t q[4] = {m.x, m.y, m.z, m.w};
+    uint32_t mine = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mine += (uint32_t)__popc(q[k] & 0x00ff00ffu) << 16 | (uint32_t)__popc(q[k] & 0xff00ff00u);
+    const uint32_t incl = wave_incl_sum(mine);
+    if (lane_id() == KT_WAVE - 1) w[threadIdx.x / KT_WAVE] = incl;
+    __syncthreads();
+    uint32_t pre = incl - mine;
+    for (unsigned i = 0; i < threadIdx.x / KT_WAVE; ++i) pre += w[i];
+    uint64_t gp = toff[blockIdx.x] + (pre >> 16);
+    uint64_t sp = toff[tiles + blockIdx.x] - toff[tiles] + (pre & 0xffffu);
+    uint64_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < MK_ITEMS; ++k) {
+        const uint32_t mk = (q[k / 2] >> (16 * (k & 1))) & 0xffffu;
+        if (!mk) continue;
+        const uint64_t i = at * MK_ITEMS + k;
+        const uint32_t id = (uint32_t)(i < from ? i : i + nl);
+        const uint32_t d = deg[id];
+        ghost_ids[gp] = id;
+        ghost_deg[gp++] = d;
+        if (mk >> 8) {
+            msg_src[sp] = id;
+            vlen[sp++] = d;
+            sum += d;
         }
     }
-}
-
-__global__ void k_pd_rebase(uint32_t nl, const uint64_t* __restrict__ soff, uint64_t* __restrict__ loff) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= nl; i += stride) loff[i] = soff[i] - soff[0];
+    sum = wave_incl_sum(sum);
+    if (lane_id() == KT_WAVE - 1 && sum) atomic_add_u64(small + 3, sum);
+    if (at == 0) {
+        small[1] = toff[tiles];
+        small[2] = toff[2 * tiles] - toff[tiles];
+    }
 }
 
 // [lo, hi): the id range of the owner of a, the first rank r with a < bd[r+1]
@@ -169,7 +206,8 @@ struct SenderInfo {
 
 __global__ void k_pd_sinfo(uint32_t nmsg, const uint32_t* __restrict__ src, const uint64_t* __restrict__ voff,
                            const uint64_t* __restrict__ off, const uint32_t* __restrict__ deg,
-                           const uint64_t* __restrict__ bd, uint32_t P, int cetric, SenderInfo* __restrict__ si) {
+                           const uint64_t* __restrict__ bd, uint32_t P, int cetric, SenderInfo* __restrict__ si,
+                           uint64_t V, uint32_t* __restrict__ tbnd) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nmsg; i += gridDim.x * blockDim.x) {
         const uint32_t a = src[i];
         uint64_t lo = 0, hi = 0;
@@ -177,6 +215,7 @@ __global__ void k_pd_sinfo(uint32_t nmsg, const uint32_t* __restrict__ src, cons
         SenderInfo s;
         s.offa = off[a];
         s.vbeg = voff[i];
+        note_tiles(i, s.vbeg, voff[i + 1], V, PD_TILE, tbnd);
         s.a = a;
         s.da = deg[a];
         s.lo = (uint32_t)lo;
@@ -276,6 +315,7 @@ __global__ void __launch_bounds__(PD_THREADS)
         if (j < tend) {
             const uint32_t i = lo + marks[idx];
             if (j == si[i].vbeg) moff[i] = pos;
+            if (j + 1 == V) moff[nmsg] = pos + ((bits[k] >> lane_id()) & 1);
         }
         base += round;
     }
@@ -328,9 +368,8 @@ struct ProdBufs {
     uint64_t* small;
     uint64_t* bd;
     uint32_t* deg;
-    uint32_t* bits;  // ghost bits, then sender bits
-    uint64_t* gcnt;
-    uint64_t* scnt;
+    uint16_t* marks;  // two bytes per vertex outside the rank, whole tiles
+    uint64_t* mcnt;   // their tiles' ghosts, then senders, and the scan
     uint64_t* stmp;
     uint32_t* tbnd;
     uint64_t* tcnt;  // per-tile kept counts of the virtual slot space, then their scan
@@ -349,28 +388,36 @@ struct ProdBufs {
     uint64_t* symws;  // symmetry check of the whole graph
 };
 
+// Tiles of marks of the vertices outside the rank.
+uint64_t mark_tiles(uint32_t n, uint32_t nl) { return ((uint64_t)n - nl + MK_TILE - 1) / MK_TILE; }
+
 uint64_t prod_layout(void* base, uint32_t n, uint64_t nnz, uint32_t P, uint32_t nl, uint64_t ng_max, bool want_pv,
                      bool host_pv, bool host_in, ProdBufs& B) {
     Carver cv{base, 0};
-    const uint64_t W = ((uint64_t)n + 31) / 32;
+    const uint64_t mt = mark_tiles(n, nl);
     const uint64_t tiles = nnz / PD_TILE + 1;  // bounds the tiles of the slice and of the virtual slot space
     B.small = static_cast<uint64_t*>(cv.take(64 * 8));
     B.bd = static_cast<uint64_t*>(cv.take(((uint64_t)P + 1) * 8));
     B.deg = static_cast<uint32_t*>(cv.take((uint64_t)n * 4));
-    B.bits = static_cast<uint32_t*>(cv.take(2 * W * 4));
-    B.gcnt = static_cast<uint64_t*>(cv.take((W + 1) * 8));
-    B.scnt = static_cast<uint64_t*>(cv.take((W + 1) * 8));
-    B.stmp = static_cast<uint64_t*>(cv.take(scan_tmp_words(std::max(std::max<uint64_t>(W, ng_max), tiles) + 1) * 8));
+    B.mcnt = static_cast<uint64_t*>(cv.take((2 * mt + 1) * 8));
+    B.stmp = static_cast<uint64_t*>(cv.take(scan_tmp_words(std::max(std::max<uint64_t>(2 * mt, ng_max), tiles) + 1) * 8));
     B.tbnd = static_cast<uint32_t*>(cv.take(2 * tiles * 4));
     B.tcnt = static_cast<uint64_t*>(cv.take((tiles + 1) * 8));
-    B.vkeep = static_cast<uint64_t*>(cv.take(tiles * (PD_TILE / 64) * 8));
     B.loff = static_cast<uint64_t*>(cv.take(((uint64_t)nl + 1) * 8));
     B.ghost_ids = static_cast<uint32_t*>(cv.take(std::max<uint64_t>(ng_max, 1) * 4));
     B.ghost_deg = static_cast<uint64_t*>(cv.take(std::max<uint64_t>(ng_max, 1) * 8));
     B.msg_src = static_cast<uint32_t*>(cv.take(std::max<uint64_t>(ng_max, 1) * 4));
     B.voff = static_cast<uint64_t*>(cv.take((ng_max + 1) * 8));
+    // the marks are read for the last time before the rest of the messages'
+    // arrays are written
+    const uint64_t at = cv.used;
+    B.marks = static_cast<uint16_t*>(cv.take(mt * MK_TILE * 2));
+    const uint64_t after = cv.used;
+    cv.used = at;
+    B.vkeep = static_cast<uint64_t*>(cv.take(tiles * (PD_TILE / 64) * 8));
     B.moff = static_cast<uint64_t*>(cv.take((ng_max + 1) * 8));
     B.sinfo = static_cast<SenderInfo*>(cv.take(std::max<uint64_t>(ng_max, 1) * sizeof(SenderInfo)));
+    cv.used = std::max(cv.used, after);
     B.pvx = want_pv ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(nl + ng_max, 1) * 8)) : nullptr;
     B.gpv = host_pv ? static_cast<uint64_t*>(cv.take((uint64_t)n * 8)) : nullptr;
     B.hoff = host_in ? static_cast<uint64_t*>(cv.take(((uint64_t)n + 1) * 8)) : nullptr;
@@ -411,15 +458,12 @@ int count_shard_graph_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, con
         end = offsets[to];
     } else {
         const uint64_t* src[3] = {offsets + n, offsets + from, offsets + to};
-        for (int i = 0; i < 3; ++i) {
-            rc = c->hip_check(hipMemcpyAsync(c->host_small + i, src[i], 8, hipMemcpyDeviceToHost, st), "D2H sizes");
-            if (rc) return rc;
-        }
-        rc = c->hip_check(hipStreamSynchronize(st), "D2H sizes");
+        uint64_t got[3];
+        rc = c->read_words(src, 3, got, "D2H sizes");
         if (rc) return rc;
-        nnz = c->host_small[0];
-        base = c->host_small[1];
-        end = c->host_small[2];
+        nnz = got[0];
+        base = got[1];
+        end = got[2];
     }
     if (base > end || end > nnz || (nnz >> 40)) return c->fail(KT_EINVAL, "malformed CSR: bad offsets");
     if (nnz && !heads) return c->fail(KT_EINVAL, "null heads");
@@ -443,11 +487,15 @@ int count_shard_graph_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, con
     rc = c->hip_check(hipMemcpyAsync(B.bd, bd, ((uint64_t)P + 1) * 8, hipMemcpyHostToDevice, st), "H2D bounds");
     if (rc) return rc;
     uint32_t* err = reinterpret_cast<uint32_t*>(B.small);
-    const uint64_t W = ((uint64_t)n + 31) / 32;
-    fill_u64(B.small, 64, 0, st);
-    fill_u32(B.bits, 2 * W, 0, st);
-    fill_u64(B.voff, ng_max + 1, 0, st);
-    k_pd_degree<<<grid_for(n), 256, 0, st>>>(n, nnz, off, B.deg, err);
+    const uint64_t mt = mark_tiles(n, nl);
+    {
+        ClearList cl;
+        cl.add(B.small, 64);
+        cl.add(reinterpret_cast<uint64_t*>(B.marks), mt * MK_TILE / 4);
+        clear(cl, st);
+    }
+    k_pd_degree<<<grid_for((uint64_t)n + 1), 256, 0, st>>>(n, nnz, off, B.deg, sym_tile_bounds(nnz, B.symws), from, nl,
+                                                           nnz_l, B.loff, B.tbnd, err);
     // the whole graph must be symmetric, as every rank's view of it assumes
     // (one pass over all slots: pair checksums, self-loops, duplicates)
     const OrientCheck chk{{c->sym_key[0], c->sym_key[1]}};
@@ -455,25 +503,19 @@ int count_shard_graph_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, con
     // The kernels up to the first flag check stay in bounds whatever the
     // offsets hold: slots are bounded by the host-checked slice [base, end),
     // rows by tile_rows' clamping, ids by n.
-    k_pd_rebase<<<grid_for((uint64_t)nl + 1), 256, 0, st>>>(nl, off + from, B.loff);
     const uint64_t tiles_l = (nnz_l + PD_TILE - 1) / PD_TILE;
-    if (nl && tiles_l) {
-        tile_bounds_launch(nl, nnz_l, PD_TILE, B.loff, B.tbnd, st);
+    if (nl && tiles_l)
         k_pd_mark<<<(unsigned)tiles_l, PD_THREADS, 0, st>>>(B.loff, nl, from, n, nnz_l, hd + base, B.tbnd, B.deg,
-                                                            B.bits, B.bits + W, err);
+                                                            B.marks, err);
+    // ghosts and senders, in id order
+    if (mt) {
+        const uint4* marks = reinterpret_cast<const uint4*>(B.marks);
+        k_pd_count<<<(unsigned)mt, PD_THREADS, 0, st>>>(marks, B.mcnt);
+        scan_u64(B.mcnt, B.mcnt, 2 * mt, B.stmp, st);
+        k_pd_compact<<<(unsigned)mt, PD_THREADS, 0, st>>>(marks, mt, B.mcnt, from, nl, B.deg, B.ghost_ids, B.ghost_deg,
+                                                          B.msg_src, B.voff, B.small);
     }
-    // ghosts and senders, in id order; the senders' degrees are the lengths
-    // of the virtual lists (entries past the last sender stay zero)
-    k_pd_popc<<<grid_for(W), 256, 0, st>>>(W, B.bits, B.bits + W, B.gcnt, B.scnt);
-    scan_u64(B.gcnt, B.gcnt, W, B.stmp, st);
-    scan_u64(B.scnt, B.scnt, W, B.stmp, st);
-    k_pd_compact<<<grid_for(W), 256, 0, st>>>(W, B.bits, B.gcnt, B.bits + W, B.scnt, off, B.ghost_ids, B.ghost_deg,
-                                               B.msg_src, B.voff);
-    scan_u64(B.voff, B.voff, ng_max, B.stmp, st);
-    rc = c->hip_check(hipMemcpyAsync(B.small + 1, B.gcnt + W, 8, hipMemcpyDeviceToDevice, st), "D2D counts");
-    if (!rc) rc = c->hip_check(hipMemcpyAsync(B.small + 2, B.scnt + W, 8, hipMemcpyDeviceToDevice, st), "D2D counts");
-    if (!rc) rc = c->hip_check(hipMemcpyAsync(B.small + 3, B.voff + ng_max, 8, hipMemcpyDeviceToDevice, st), "D2D V");
-    if (!rc) rc = read_small(c, B.small, 4, "ghosts");
+    rc = read_small(c, B.small, 4, "ghosts");
     if (rc) return rc;
     uint32_t fl = (uint32_t)c->host_small[0];
     const uint64_t ng = c->host_small[1], nmsg = c->host_small[2], V = c->host_small[3];
@@ -488,18 +530,19 @@ int count_shard_graph_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, con
     uint32_t* mheads = nullptr;
     if (nmsg) {
         const uint64_t tiles_v = (V + PD_TILE - 1) / PD_TILE;
+        scan_u64(B.voff, B.voff, nmsg, B.stmp, st);  // the senders' full lists one after another
         k_pd_sinfo<<<grid_for(nmsg), 256, 0, st>>>((uint32_t)nmsg, B.msg_src, B.voff, off, B.deg, B.bd, P,
-                                                   cetric ? 1 : 0, B.sinfo);
-        tile_bounds_launch((uint32_t)nmsg, V, PD_TILE, B.voff, B.tbnd, st);
+                                                   cetric ? 1 : 0, B.sinfo, V, B.tbnd);
         k_pd_msgs<false><<<(unsigned)tiles_v, PD_THREADS, 0, st>>>(V, (uint32_t)nmsg, B.voff, B.tbnd, B.sinfo, hd,
                                                                    B.deg, n, B.vkeep, B.tcnt, nullptr, nullptr,
                                                                    nullptr, err);
         scan_u64(B.tcnt, B.tcnt, tiles_v, B.stmp, st);
-        rc = c->hip_check(hipMemcpyAsync(B.small + 1, B.tcnt + tiles_v, 8, hipMemcpyDeviceToDevice, st), "D2D total");
-        if (!rc) rc = read_small(c, B.small, 2, "message lengths");
+        const uint64_t* src[2] = {B.small, B.tcnt + tiles_v};
+        uint64_t got[2];
+        rc = c->read_words(src, 2, got, "message lengths");
         if (rc) return rc;
-        fl = (uint32_t)c->host_small[0];
-        mtot = c->host_small[1];
+        fl = (uint32_t)got[0];
+        mtot = got[1];
         if (fl & KT_ERR_MASK)
             return c->fail(KT_EINVAL, "malformed CSR:%s", (fl & KT_ERR_HEAD_RANGE) ? " head id >= n" : "");
         const bool unsorted = (fl & KT_FLAG_UNSORTED) != 0;
@@ -517,7 +560,6 @@ int count_shard_graph_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, con
         k_pd_msgs<true><<<(unsigned)tiles_v, PD_THREADS, 0, st>>>(V, (uint32_t)nmsg, B.voff, B.tbnd, B.sinfo, hd,
                                                                   B.deg, n, B.vkeep, nullptr, B.tcnt, mheads, B.moff,
                                                                   err);
-        fill_u64(B.moff + nmsg, 1, mtot, st);
         if (unsorted && mtot) {
             uint64_t* keys = static_cast<uint64_t*>(cv.take(mtot * 8));
             uint64_t* alt = static_cast<uint64_t*>(cv.take(mtot * 8));
@@ -548,9 +590,9 @@ int count_shard_graph_locked(kt_ctx* c, uint32_t n, const uint64_t* offsets, con
     if (want_pv) {
         in.flags |= KT_DEVICE_OUTPUT;
         o.per_vertex = B.pvx;
-        fill_u64(B.pvx, (uint64_t)nl + ng, 0, st);  // stays zero if the rank sees nothing
     }
-    rc = count_shard_locked(c, &in, &o);
+    const ShardSizes sizes{nnz_l, mtot};
+    rc = count_shard_locked(c, &in, &o, &sizes);
     if (rc) return rc;
     if (want_pv) {
         uint64_t* dst = pv_dev ? out->per_vertex : B.gpv;

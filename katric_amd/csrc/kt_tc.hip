@@ -1867,7 +1867,9 @@ static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const T
     }
     // huge and big tails are rare: one workgroup per CU; they exit at once
     // when there are none, and are not launched where none can be
-    auto longer = [&](uint64_t s) { return view.sym_slots == 0 || view.sym_slots > s * s; };
+    auto longer = [&](uint64_t s) {
+        return (view.sym_slots == 0 || view.sym_slots > s * s) && (view.longest == 0 || view.longest > s);
+    };
     if (longer(p.bsearch_min_deg))
         k_tc_huge<PLAIN, false><<<(unsigned)num_cus, TC_THREADS, 0, st>>>(V, out, p, q, list, row(ROW_HUGE));
     if (longer(p.group_max_deg)) {

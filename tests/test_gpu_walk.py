@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import katric_amd as K
+from katric_amd import shard as S
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -185,3 +186,30 @@ def test_scan_sizes(ctx, n, unsorted):
     _check(ctx, g, pv)
     o = ctx.orient(g)
     assert int(o.offsets[-1]) == len(e)
+
+
+@pytest.mark.parametrize("algo", [S.CETRIC, S.DITRIC])
+@pytest.mark.parametrize("longest", [16, 17, 1024, 1025, 4096, 4097])
+@pytest.mark.parametrize("lens", [(0, 4096, 0, 0, 1, 4095, 64, 65, 0), (3, 0, 4090, 3, 5000, 9001), (0, 0), (1,)])
+def test_shard_lists_and_messages(ctx, algo, longest, lens):
+    """Lists at the sort's size classes and messages at the edges of the entry
+    tiles: one rank, every ghost above every owned vertex in degree, so an owned
+    vertex' list is its ghosts and a message [a, list] closes a triangle for every
+    owned u in the list and every ghost of u in it."""
+    rng = np.random.default_rng(longest + len(lens))
+    nl, n = 40, 30000
+    ghosts = np.sort(rng.choice(np.arange(nl, n), 12000, replace=False))
+    rows = [np.sort(rng.choice(ghosts, longest if u == 7 else int(rng.integers(0, 60)), replace=False)) for u in range(nl)]
+    rows[11] = rows[11][:0]
+    msgs = [np.sort(rng.choice(n, k, replace=False)) for k in lens]
+    offsets = lambda lists: np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.uint64)
+    ids = lambda lists: np.concatenate(lists).astype(np.uint32)
+    sh = S.Shard(algorithm=algo, rank=0, bounds=np.array([0, nl, n], np.uint64), offsets=offsets(rows),
+                 heads=ids(rows), ghost_ids=ghosts.astype(np.uint32),
+                 ghost_degree=np.full(len(ghosts), 1 << 20, np.uint64),
+                 msg_src=rng.choice(ghosts, len(lens), replace=False).astype(np.uint32), msg_offsets=offsets(msgs),
+                 msg_heads=ids(msgs))
+    want = sum(len(np.intersect1d(rows[u], m)) for m in msgs for u in m[m < nl])
+    loc, t3, pv = S.count_shard(ctx, sh)
+    assert (loc, t3) == (0, want)
+    assert int(pv.sum()) == 3 * want
