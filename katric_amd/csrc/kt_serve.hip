@@ -3,9 +3,11 @@
 // A worker thread owns two device slots (own stream, own grow-only arena,
 // pinned result buffers).  Requests are admitted FIFO into the next batch
 // while the batch fits the slot's share of the HBM budget and the batch
-// limits; the batch's CSRs are uploaded into the slot (device-resident for
-// the batch's lifetime) and rebased into one disjoint-union CSR, then counted
-// by the batch pipeline.  While one slot computes, the other uploads and
+// limits; the batch's CSRs are gathered into one disjoint-union CSR in the slot
+// (device-resident for the batch's lifetime), by a kernel that reads page-locked
+// requests where they are and from copies of the others, then counted by the
+// batch pipeline.  Per-vertex counts for pageable memory leave the device as one
+// copy into the slot's page-locked buffer and are handed out from there.  While one slot computes, the other uploads and
 // launches the next batch, so requests arriving during a batch are admitted
 // as soon as a slot frees up, and their work overlaps on the device.
 //
@@ -33,8 +35,9 @@ static double now_ms() {
     return duration<double, std::milli>(steady_clock::now().time_since_epoch()).count();
 }
 
-// One request of a device batch: where its CSR was copied to in the batch
-// arena, its place in the batch, and its first work chunk.
+// One request of a device batch: its CSR as the device reads it (the request's
+// page-locked memory, or its copy at its place in the batch arena), its place in
+// the batch, and its first work chunk.
 struct GatherDesc {
     const uint64_t* off;
     const uint32_t* heads;
@@ -50,14 +53,17 @@ __host__ __device__ inline uint64_t gather_chunks(uint64_t n, uint64_t nnz) {
     return (n + GATHER_CHUNK - 1) / GATHER_CHUNK + (nnz + GATHER_CHUNK - 1) / GATHER_CHUNK;
 }
 
-// Rebases the copied CSRs in place into the batch's disjoint-union CSR in one
-// launch: off[vb_g + i] = off_g[i] + eb_g, heads[eb_g + k] = heads_g[k] + vb_g
-// (a head outside its own graph becomes an invalid id, flagged by the
-// orientation pass), off[N] = nnz.  Blocks take chunks of one request's
-// offsets or heads (every element is read and written by the same thread).
+// Writes the requests' CSRs into the batch's disjoint-union CSR in one launch:
+// off[vb_g + i] = off_g[i] + eb_g, heads[eb_g + k] = heads_g[k] + vb_g (a head
+// outside its own graph becomes an invalid id, flagged by the orientation pass),
+// off[N] = nnz.  Blocks take chunks of one request's offsets or heads, every
+// thread all its elements of a chunk at once: from page-locked memory the loads'
+// way over PCIe is what takes the time.  A copied CSR is rebased in place (every
+// element is read and written by the same thread).
 __global__ void __launch_bounds__(256) k_serve_gather(uint32_t G, const GatherDesc* __restrict__ d,
-                                                      uint64_t chunks, uint64_t* __restrict__ off,
-                                                      uint32_t* __restrict__ heads, uint64_t N, uint64_t nnz) {
+                                                      uint64_t chunks, uint64_t* off, uint32_t* heads, uint64_t N,
+                                                      uint64_t nnz) {
+    constexpr int E = GATHER_CHUNK / 256;
     for (uint64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
         uint32_t lo = 0, hi = G - 1;  // last request with c0 <= c
         while (lo < hi) {
@@ -71,17 +77,40 @@ __global__ void __launch_bounds__(256) k_serve_gather(uint32_t G, const GatherDe
         const uint64_t oc = (r.n + GATHER_CHUNK - 1) / GATHER_CHUNK;
         const uint64_t k = c - r.c0;
         if (k < oc) {
-            const uint64_t i0 = k * GATHER_CHUNK, i1 = min(r.n, i0 + GATHER_CHUNK);
-            for (uint64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) off[r.vb + i] = r.off[i] + r.eb;
+            const uint64_t i0 = k * GATHER_CHUNK + threadIdx.x;
+            uint64_t x[E];
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = i0 + j * 256 < r.n ? r.off[i0 + j * 256] : 0;
+#pragma unroll
+            for (int j = 0; j < E; ++j)
+                if (i0 + j * 256 < r.n) off[r.vb + i0 + j * 256] = x[j] + r.eb;
         } else {
-            const uint64_t e0 = (k - oc) * GATHER_CHUNK, e1 = min(r.nnz, e0 + GATHER_CHUNK);
-            for (uint64_t e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-                const uint32_t h = r.heads[e];
-                heads[r.eb + e] = (h < r.n) ? (uint32_t)(h + r.vb) : 0xffffffffu;
-            }
+            const uint64_t e0 = (k - oc) * GATHER_CHUNK + threadIdx.x;
+            uint32_t h[E];
+#pragma unroll
+            for (int j = 0; j < E; ++j) h[j] = e0 + j * 256 < r.nnz ? r.heads[e0 + j * 256] : 0;
+#pragma unroll
+            for (int j = 0; j < E; ++j)
+                if (e0 + j * 256 < r.nnz)
+                    heads[r.eb + e0 + j * 256] = (h[j] < r.n) ? (uint32_t)(h[j] + r.vb) : 0xffffffffu;
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) off[N] = nnz;
+}
+
+// The device's address of page-locked host memory p[0, bytes), or null (pageable
+// memory, or a range whose ends are not in one page-locked allocation).
+static const void* device_view(const void* p, uint64_t bytes) {
+    if (!bytes) return nullptr;
+    hipPointerAttribute_t a{}, z{};
+    const char* last = static_cast<const char*>(p) + bytes - 1;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&z, last) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (a.type != hipMemoryTypeHost || z.type != hipMemoryTypeHost || !a.devicePointer || !z.devicePointer) return nullptr;
+    if (static_cast<char*>(z.devicePointer) - static_cast<char*>(a.devicePointer) != (ptrdiff_t)(bytes - 1)) return nullptr;
+    return a.devicePointer;
 }
 
 struct ServeReq {
@@ -96,6 +125,7 @@ struct ServeReq {
     uint64_t total = 0;
     uint64_t batch_id = 0;
     uint32_t batch_graphs = 0;
+    bool staged = false;  // its per-vertex counts come through the slot's buffer
     bool isolate = false;
     bool cancelled = false;
     bool done = false;
@@ -110,6 +140,9 @@ struct ServeSlot {
     uint64_t* h_meta = nullptr;   // pinned: vbase (cap + 1), then the gather descriptors (cap)
     uint64_t* h_totals = nullptr; // pinned, cap
     uint64_t meta_cap = 0;
+    uint64_t* h_pv = nullptr;     // pinned, pv_cap: the batch's per-vertex counts
+    uint64_t pv_cap = 0;
+    bool staged = false;          // they are in h_pv when the batch is done
     std::vector<ServeReq*> reqs;
     bool busy = false;
     bool sorted = false;
@@ -179,7 +212,25 @@ static int slot_grow(ServeSlot& s, uint64_t bytes, uint32_t G) {
     return KT_OK;
 }
 
-// Uploads, rebases and enqueues one batch on the slot (worker thread, no lock).
+// Vertices whose counts are staged at most: 64 MiB of page-locked memory a slot.
+constexpr uint64_t STAGE_MAX = 1ull << 23;
+
+static bool stage_grow(ServeSlot& s, uint64_t n) {
+    if (n <= s.pv_cap) return true;
+    n = std::min(STAGE_MAX, std::max(n, 2 * s.pv_cap));
+    if (s.h_pv) (void)hipHostFree(s.h_pv);
+    s.h_pv = nullptr;
+    s.pv_cap = 0;
+    if (hipHostMalloc(reinterpret_cast<void**>(&s.h_pv), n * 8, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        s.h_pv = nullptr;
+        return false;
+    }
+    s.pv_cap = n;
+    return true;
+}
+
+// Gathers and enqueues one batch on the slot (worker thread, no lock).
 static int launch(ServeState* S, ServeSlot& sl, uint32_t sort) {
     const uint32_t G = (uint32_t)sl.reqs.size();
     uint64_t N = 0, nnz = 0;
@@ -221,15 +272,22 @@ static int launch(ServeState* S, ServeSlot& sl, uint32_t sort) {
         dg.vb = vb[g];
         dg.eb = e;
         dg.c0 = chunks;
-        // the request's arrays are copied into their place in the batch
-        // (copy engines: from page-locked memory these run beside the other
-        // slot's kernels) and rebased in place by k_serve_gather
-        if (r->n && hipMemcpyAsync(d_off + vb[g], r->off, (uint64_t)r->n * 8, hipMemcpyHostToDevice, st) != hipSuccess)
-            return KT_EHIP;
-        if (r->nnz && hipMemcpyAsync(d_heads + e, r->heads, r->nnz * 4, hipMemcpyHostToDevice, st) != hipSuccess)
-            return KT_EHIP;
-        dg.off = d_off + vb[g];
-        dg.heads = d_heads + e;
+        // k_serve_gather reads page-locked arrays itself (47 requests of 9,000
+        // vertices on average: 94 copies took 1.2 ms, the kernel takes 0.7);
+        // others are copied into their place in the batch and rebased there
+        dg.off = static_cast<const uint64_t*>(device_view(r->off, (uint64_t)r->n * 8));
+        dg.heads = static_cast<const uint32_t*>(device_view(r->heads, r->nnz * 4));
+        if (!dg.off) {
+            dg.off = d_off + vb[g];
+            if (r->n &&
+                hipMemcpyAsync(d_off + vb[g], r->off, (uint64_t)r->n * 8, hipMemcpyHostToDevice, st) != hipSuccess)
+                return KT_EHIP;
+        }
+        if (!dg.heads) {
+            dg.heads = d_heads + e;
+            if (r->nnz && hipMemcpyAsync(d_heads + e, r->heads, r->nnz * 4, hipMemcpyHostToDevice, st) != hipSuccess)
+                return KT_EHIP;
+        }
         chunks += gather_chunks(r->n, r->nnz);
         vb[g + 1] = vb[g] + r->n;
         e += r->nnz;
@@ -242,9 +300,24 @@ static int launch(ServeState* S, ServeSlot& sl, uint32_t sort) {
     if (batch_pipeline(st, S->num_cus, S->prm, B, G, N, nnz, B.pv, sl.h_totals, sl.h_small, sort, S->sym_key) !=
         hipSuccess)
         return KT_EHIP;
+    // per-vertex counts: a copy into pageable memory holds this thread until the
+    // batch is done, so a batch with several such requests takes one copy to the
+    // slot's buffer, which finish() hands out.  A single one is left to hold the
+    // thread: the requests that arrive meanwhile make one batch (staged too, a
+    // burst of 48 ran as three batches: 2.2 ms, with 1.6 ms in two)
+    sl.staged = false;
+    uint32_t pageable = 0;
     for (uint32_t g = 0; g < G; ++g) {
         ServeReq* r = sl.reqs[g];
-        if (r->pv_out && r->n &&
+        r->staged = r->pv_out && r->n && !device_view(r->pv_out, (uint64_t)r->n * 8);
+        pageable += r->staged;
+    }
+    if (pageable > 1 && N <= STAGE_MAX) sl.staged = stage_grow(sl, N);
+    if (sl.staged && hipMemcpyAsync(sl.h_pv, B.pv, N * 8, hipMemcpyDeviceToHost, st) != hipSuccess) return KT_EHIP;
+    for (uint32_t g = 0; g < G; ++g) {
+        ServeReq* r = sl.reqs[g];
+        r->staged = r->staged && sl.staged;
+        if (r->pv_out && r->n && !r->staged &&
             hipMemcpyAsync(r->pv_out, B.pv + vb[g], (uint64_t)r->n * 8, hipMemcpyDeviceToHost, st) != hipSuccess)
             return KT_EHIP;
     }
@@ -256,12 +329,21 @@ static int launch(ServeState* S, ServeSlot& sl, uint32_t sort) {
     return KT_OK;
 }
 
-// Completion of a slot's batch (worker thread, lock held by the caller).
-static void finish(ServeState* S, ServeSlot& sl) {
+// Completion of a slot's batch (worker thread, lock held by the caller and
+// released while counts are handed out).
+static void finish(ServeState* S, ServeSlot& sl, std::unique_lock<std::mutex>& lk) {
     const uint32_t fl = (uint32_t)sl.h_small[0];
     const uint64_t kept = sl.h_small[1];
     const uint32_t G = (uint32_t)sl.reqs.size();
     const bool bad = (fl & KT_ERR_MASK) || 2 * kept != sl.nnz;
+    if (sl.staged && !bad) {
+        lk.unlock();
+        for (uint32_t g = 0; g < G; ++g) {
+            ServeReq* r = sl.reqs[g];
+            if (r->staged) std::memcpy(r->pv_out, sl.h_pv + sl.h_meta[g], (uint64_t)r->n * 8);
+        }
+        lk.lock();
+    }
     if (bad && G > 1) {
         // isolate: every request of the batch runs alone, at the queue front
         for (int g = (int)G - 1; g >= 0; --g) {
@@ -337,7 +419,7 @@ static void worker_main(ServeState* S) {
                 if (rc != KT_OK) launch_failed(S, sl, rc);
                 continue;
             }
-            finish(S, sl);
+            finish(S, sl, lk);
         }
         ServeSlot* free_slot = nullptr;
         for (auto& sl : S->slots)
@@ -459,6 +541,7 @@ static int serve_stop_impl(kt_ctx* c) {
         if (sl.h_small) (void)hipHostFree(sl.h_small);
         if (sl.h_meta) (void)hipHostFree(sl.h_meta);
         if (sl.h_totals) (void)hipHostFree(sl.h_totals);
+        if (sl.h_pv) (void)hipHostFree(sl.h_pv);
         if (sl.ev) (void)hipEventDestroy(sl.ev);
         if (sl.stream) (void)hipStreamDestroy(sl.stream);
     }

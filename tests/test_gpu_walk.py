@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import katric_amd as K
+from katric_amd import serve as V
 from katric_amd import shard as S
 from oracle import oracle as O
 
@@ -213,3 +214,31 @@ def test_shard_lists_and_messages(ctx, algo, longest, lens):
     loc, t3, pv = S.count_shard(ctx, sh)
     assert (loc, t3) == (0, want)
     assert int(pv.sum()) == 3 * want
+
+
+def test_serve_reads_each_kind_of_memory(ctx):
+    """Requests with offsets, heads and counts each in pageable or page-locked
+    memory, at the edges of the gather's chunks, mixed in one burst."""
+    sizes = [1, 2, 255, 257, 4095, 4096, 4097, 8193]
+    cases, owners = [], []
+    for i in range(32):
+        n = sizes[i % len(sizes)]
+        g = K.gen_gnm(n, min(3 * n, n * (n - 1) // 2), seed=i)
+        view = V.Graph.__new__(V.Graph)
+        pinned, own = V.pinned_graph(g)
+        counts = V.PinnedArray(n, np.uint64)
+        owners += own + [counts]
+        view.n = n
+        view.offsets = pinned.offsets if i & 1 else g.offsets
+        view.heads = pinned.heads if i & 2 else g.heads
+        out = counts.array if i & 4 else np.zeros(n, np.uint64)
+        out[:] = 99
+        cases.append((view, out, *ctx.count(g)))
+    with K.Context(0) as sctx:
+        srv = V.Server(sctx)
+        tickets = [srv.submit(view, out) for view, out, _, _ in cases]
+        results = [srv.wait(t) for t in tickets]
+        srv.stop()
+    for r, (_, out, total, pv) in zip(results, cases):
+        assert (r.status, r.total) == (0, total)
+        np.testing.assert_array_equal(out, pv)
