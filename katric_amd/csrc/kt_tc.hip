@@ -550,10 +550,39 @@ struct PackLds {
     uint32_t ucnt[KT_WAVE];
 };
 
+// Bounds of a tail's S and R ranges and its counter length.
+struct TailBounds {
+    uint64_t sb, rb;
+    uint32_t ns, nr;  // lists hold distinct 32-bit ids
+    uint32_t nstat;
+};
+
+// The tails a wave has grabbed (in LDS: in registers they stay live through
+// the walk, and at 80 registers a wave that put 61 of them in scratch memory).
+template <uint32_t N>
+struct GrabLds {
+    static constexpr uint32_t MAX = N;
+    uint64_t sb[N], rb[N];
+    uint32_t x[N], ns[N], nr[N], nstat[N];
+    __device__ __forceinline__ TailBounds bounds(uint32_t j) const { return {sb[j], rb[j], ns[j], nr[j], nstat[j]}; }
+    __device__ __forceinline__ void put(uint32_t j, uint32_t tail, const TailBounds& b) {
+        sb[j] = b.sb;
+        rb[j] = b.rb;
+        x[j] = tail;
+        ns[j] = b.ns;
+        nr[j] = b.nr;
+        nstat[j] = b.nstat;
+    }
+};
+
+// 42 of the CU's 128 LDS granules of 1280 bytes at most: three workgroups fit
+// (a listing keeps its neighbours' ids beside it).
+template <bool LIST>
 struct Lds {
     uint32_t keys[GROUP_SLOTS];
     uint32_t cnt[GROUP_SLOTS];
     PackLds pk[TC_WAVES];
+    GrabLds<LIST ? 20 : 28> grab[TC_WAVES];
     uint32_t ovf[GROUP_SLOTS / 128];  // a bit per bucket (the team's table, or 4 words per wave table)
     uint64_t red[TC_WAVES];
     unsigned long long list_ctr[TC_WAVES];  // listing: triangles of the current tail written so far
@@ -635,6 +664,9 @@ __device__ __forceinline__ uint32_t table_insert(uint32_t* keys, uint32_t* ovf, 
 // of hits.  Each hit bumps the w-counter of its slot and calls
 // on_hit(e).  The four slot compares of a probe stay lane masks; hits are
 // counted per lane (one add), so the scalar unit only sees the branch masks.
+// Two buckets are read at a time: four held 16 registers, and what the walk
+// then kept in scratch memory cost more than the second read's latency (768
+// mixed graphs: 9.9 ms with four, 8.9 with two).
 // Lookups continue past a full home bucket only in a table where some key
 // went past its home bucket (moved, wave-uniform), and only from a bucket
 // with its `ovf` bit.
@@ -642,30 +674,36 @@ template <class OnHit>
 __device__ __forceinline__ uint32_t probe_ids(const uint32_t* keys, uint32_t* cnt, const uint32_t* ovf, uint32_t toff,
                                               uint32_t boff_mask, bool moved, const uint32_t (&w)[4], int lim,
                                               OnHit on_hit) {
-    uint32_t bo[4];
-    uint4 kk[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        bo[e] = bucket_off(w[e], boff_mask);
-        kk[e] = *bucket_at(keys, toff + bo[e]);
-    }
+    uint32_t bo[4], last[4];
     uint32_t nh = 0;
     bool hit[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const bool m0 = kk[e].x == w[e], m1 = kk[e].y == w[e], m2 = kk[e].z == w[e], m3 = kk[e].w == w[e];
-        hit[e] = e < lim && (m0 || m1 || m2 || m3);
-        nh += hit[e] ? 1u : 0u;
-        if (hit[e]) {
-            atomicAdd(at_byte(cnt, toff + bo[e]) + (m0 ? 0u : m1 ? 1u : m2 ? 2u : 3u), 1u);
-            on_hit(e);
+    for (int h = 0; h < 4; h += 2) {
+        uint4 kk[2];
+#pragma unroll
+        for (int e = h; e < h + 2; ++e) {
+            bo[e] = bucket_off(w[e], boff_mask);
+            kk[e - h] = *bucket_at(keys, toff + bo[e]);
         }
+#pragma unroll
+        for (int e = h; e < h + 2; ++e) {
+            const uint4 k = kk[e - h];
+            const bool m0 = k.x == w[e], m1 = k.y == w[e], m2 = k.z == w[e], m3 = k.w == w[e];
+            hit[e] = e < lim && (m0 || m1 || m2 || m3);
+            nh += hit[e] ? 1u : 0u;
+            if (hit[e]) {
+                atomicAdd(at_byte(cnt, toff + bo[e]) + (m0 ? 0u : m1 ? 1u : m2 ? 2u : 3u), 1u);
+                on_hit(e);
+            }
+            last[e] = k.w;
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (!moved) return nh;
     // a full home bucket without w: w may sit in a later bucket
     bool need[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) need[e] = e < lim && !hit[e] && kk[e].w != KT_EMPTY;
+    for (int e = 0; e < 4; ++e) need[e] = e < lim && !hit[e] && last[e] != KT_EMPTY;
     // one branch for the four ids, skipped as a whole when no lane needs it
     if (need[0] || need[1] || need[2] || need[3]) {
 #pragma unroll
@@ -746,22 +784,44 @@ struct Emitter {
     }
 };
 
-// Per-wave work counters: the reference's wedge_checks and
-// intersection_size, and the T-list ids this design streams through probes.
-// Kept per lane, summed over the wave once at the end.
+// Work counters: the reference's wedge_checks and intersection_size (wedge and
+// what the receivers add beside their lists), and the T-list ids this design
+// streams through probes.  Kept per lane in 32 bits (a register each through
+// the walk); sums that could leave them go to the workgroup's row at once.
 struct WorkStats {
-    uint64_t wedge_lane = 0, stream_lane = 0;
-    uint64_t recv_lane = 0;  // what the receivers add to intersection_size beside their lists
-    __device__ __forceinline__ uint64_t wedge() const { return uniform64(wave_sum(wedge_lane)); }
-    __device__ __forceinline__ uint64_t recv() const { return uniform64(wave_sum(recv_lane)); }
-    __device__ __forceinline__ uint64_t streamed() const { return uniform64(wave_sum(stream_lane)); }
+    uint32_t wedge_lane = 0, recv_lane = 0, stream_lane = 0;
+    uint64_t* row;
+    __device__ __forceinline__ explicit WorkStats(uint64_t* sums) : row(sums + (uint64_t)blockIdx.x * SUM_WORDS) {}
+    __device__ __forceinline__ void flush(uint64_t wedge, uint64_t recv, uint64_t stream) {
+        wedge = wave_sum(wedge);
+        recv = wave_sum(recv);
+        stream = wave_sum(stream);
+        if (lane_id() == 0) {
+            atomic_add_u64(&row[ST_WEDGE], wedge);
+            atomic_add_u64(&row[ST_ISZ], wedge + recv);
+            atomic_add_u64(&row[ST_STREAM], stream);
+        }
+    }
+    __device__ __forceinline__ void add(uint64_t wedge, uint32_t recv, uint64_t stream) {
+        const uint32_t high = (uint32_t)(wedge >> 32) | (uint32_t)(stream >> 32);
+        const uint32_t low = (uint32_t)wedge | recv | (uint32_t)stream | wedge_lane | recv_lane | stream_lane;
+        if (__builtin_amdgcn_ballot_w64((high | low >> 31) != 0)) {
+            flush(wedge + wedge_lane, (uint64_t)recv + recv_lane, stream + stream_lane);
+            wedge_lane = recv_lane = stream_lane = 0;
+            return;
+        }
+        wedge_lane += (uint32_t)wedge;
+        recv_lane += recv;
+        stream_lane += (uint32_t)stream;
+    }
 };
 
 // The workgroup's sums to its row (every wave calls it; `red` holds 4 words
 // per wave).
 template <int NW>
-__device__ __forceinline__ void flush_sums(uint64_t total, const WorkStats& wk, uint64_t* red, uint64_t* sums) {
-    const uint64_t streamed = wk.streamed(), wedge = wk.wedge(), recv = wk.recv();
+__device__ __forceinline__ void flush_sums(uint64_t total, const WorkStats& wk, uint64_t* red) {
+    const uint64_t streamed = wave_sum((uint64_t)wk.stream_lane), wedge = wave_sum((uint64_t)wk.wedge_lane),
+                   recv = wave_sum((uint64_t)wk.recv_lane);
     const unsigned wave = threadIdx.x / KT_WAVE;
     __syncthreads();
     if (lane_id() == 0) {
@@ -775,7 +835,7 @@ __device__ __forceinline__ void flush_sums(uint64_t total, const WorkStats& wk, 
         uint64_t t = 0;
         for (int i = 0; i < NW; ++i) t += red[4 * i + threadIdx.x];
         const int at[4] = {SUM_TOTAL, ST_WEDGE, ST_ISZ, ST_STREAM};
-        sums[(uint64_t)blockIdx.x * SUM_WORDS + at[threadIdx.x]] = t;
+        atomic_add_u64(&wk.row[at[threadIdx.x]], t);
     }
 }
 
@@ -938,13 +998,6 @@ __device__ __forceinline__ uint32_t walk_lists(const uint32_t* __restrict__ T, u
     return mine;
 }
 
-// Bounds of a tail's S and R ranges and its counter length.
-struct TailBounds {
-    uint64_t sb, rb;
-    uint32_t ns, nr;  // lists hold distinct 32-bit ids
-    uint32_t nstat;
-};
-
 template <bool PLAIN>
 __device__ __forceinline__ TailBounds tail_bounds(const View<PLAIN>& V, uint32_t x) {
     TailBounds t;
@@ -1041,9 +1094,7 @@ __device__ __forceinline__ void team_process(const View<PLAIN>& V, uint32_t x, c
         bool stc = false;
         if (lane < c) V.entry_bounds(rb + k + lane, u, kw, ns, b, e, stl, stc);
         const uint64_t len = e > b ? e - b : 0;
-        wk.wedge_lane += stl;
-        wk.recv_lane += stc ? nstat : 0u;
-        wk.stream_lane += len;
+        wk.add(stl, stc ? nstat : 0u, len);
         uint64_t hits;
         const uint32_t h = walk_lists<HASH, false, LIST>(V.t_heads(), b, len, u, 0, P, L.pk[wave], uid, hits);
         if (h && P.pv) atomic_add_u64(&P.pv[u], h);
@@ -1092,12 +1143,12 @@ __device__ __forceinline__ uint32_t pack_slots(uint32_t ns) {  // load 1/8 to 1/
     return 1u << max(ceil_log2(4ull * ns), 4u);
 }
 
-// Tails of lanes [j0, j0 + n) of a grab (tail xl with bounds bl; er / es / et
-// = its walk entries, set members and table slots below the pack's first).
-template <bool PLAIN>
-__device__ __forceinline__ void pack_process(const View<PLAIN>& V, uint32_t xl, const TailBounds& bl, uint32_t er,
-                                             uint32_t es, uint32_t et, uint32_t j0, uint32_t n, uint32_t nR,
-                                             uint32_t nS, PackLds& pk, uint32_t* keys, uint32_t* cnt, uint32_t* ovf,
+// Tails [j0, j0 + n) of a grab; lane j's walk entries, set members and table
+// slots start er, es and et after the pack's first.
+template <bool PLAIN, class GrabT>
+__device__ __forceinline__ void pack_process(const View<PLAIN>& V, const GrabT& gb, uint32_t er, uint32_t es,
+                                             uint32_t et, uint32_t j0, uint32_t n, uint32_t nR, uint32_t nS,
+                                             PackLds& pk, uint32_t* keys, uint32_t* cnt, uint32_t* ovf,
                                              const TcOut& out, uint64_t& my_total, WorkStats& wk) {
     const uint32_t lane = lane_id();
     // which tail a lane's entry / set member belongs to, from the bits at the
@@ -1113,13 +1164,13 @@ __device__ __forceinline__ void pack_process(const View<PLAIN>& V, uint32_t xl, 
     wave_sync();
     const uint64_t mr = (uint64_t)readlane32(word, 0) | ((uint64_t)readlane32(word, 1) << 32);
     const uint64_t ms = (uint64_t)readlane32(word, 2) | ((uint64_t)readlane32(word, 3) << 32);
+    // (at most the grab's last tail: lanes past the pack's entries read it)
     const uint32_t tr = j0 + rank_below(mr, 0), ts = j0 + rank_below(ms, 0);
-    const uint32_t tab = (4 * et << 16) | (((pack_slots(bl.ns) >> 2) - 1) << 4);
+    const uint32_t tab = (4 * et << 16) | (((pack_slots(gb.ns[min(lane, GrabT::MAX - 1)]) >> 2) - 1) << 4);
     // set members and walk entries
-    const uint64_t si = from_lane64(bl.sb - es, ts) + lane;
-    const uint64_t ri = from_lane64(bl.rb - er, tr) + lane;
+    const uint64_t si = gb.sb[ts] + (lane - from_lane(es, ts));
+    const uint64_t ri = gb.rb[tr] + (lane - from_lane(er, tr));
     const uint32_t stab = from_lane(tab, ts), rtab = from_lane(tab, tr);
-    const uint32_t rns = from_lane(bl.ns, tr), rstat = PLAIN ? rns : from_lane(bl.nstat, tr);
     uint32_t id = 0, u = 0, kw = 0;
     if (lane < nS) id = V.v.sheads[si];
     if (lane < nR) V.entry_head(ri, u, kw);
@@ -1135,27 +1186,25 @@ __device__ __forceinline__ void pack_process(const View<PLAIN>& V, uint32_t xl, 
     P.pv = out.per_vertex;
     uint64_t b = 0, e = 0, stl = 0;
     bool stc = false;
-    if (lane < nR) V.entry_bounds(ri, u, kw, rns, b, e, stl, stc);
+    if (lane < nR) V.entry_bounds(ri, u, kw, gb.ns[tr], b, e, stl, stc);
     const uint64_t len = e > b ? e - b : 0;
-    wk.wedge_lane += stl;
-    wk.recv_lane += stc ? rstat : 0u;
-    wk.stream_lane += len;
+    wk.add(stl, stc ? (PLAIN ? gb.ns[tr] : gb.nstat[tr]) : 0u, len);
     uint64_t hits;
     const uint32_t h = walk_lists<true, true, false>(V.t_heads(), b, len, u, rtab, P, pk, nullptr, hits);
     if (hits) {
         my_total += hits;
         if (P.pv) {
             if (h) atomic_add_u64(&P.pv[u], h);
-            const uint32_t sum = wave_scan_dpp(h);
-            const uint32_t last = from_lane(sum, er + bl.nr - 1), before = from_lane(sum, er - 1);
+            const uint32_t sum = wave_scan_dpp(h), j = min(lane, GrabT::MAX - 1);
+            const uint32_t last = from_lane(sum, er + gb.nr[j] - 1), before = from_lane(sum, er - 1);
             const uint32_t th = last - (lane > j0 ? before : 0u);
-            if (lane >= j0 && lane < j0 + n && th) atomic_add_u64(&P.pv[V.tail_pv(xl)], th);
+            if (lane >= j0 && lane < j0 + n && th) atomic_add_u64(&P.pv[V.tail_pv(gb.x[j])], th);
         }
     }
     if (lane < nS) {
         const uint32_t c = *at_byte(cnt, slot);
         if (c) {
-            if (P.pv) atomic_add_u64(&P.pv[id], c);
+            if (P.pv) atomic_add_u64(&P.pv[*at_byte(keys, slot)], c);
             *at_byte(cnt, slot) = 0;
         }
         *at_byte(keys, slot) = KT_EMPTY;
@@ -1209,13 +1258,13 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
                                                          const uint64_t* __restrict__ plist,
                                                          uint64_t* __restrict__ sums) {
     own_copy(out);
-    __shared__ Lds L;
+    __shared__ Lds<LIST> L;
     __shared__ uint32_t uids[LIST ? TC_THREADS : 1];  // a listing's neighbours, per wave
     const unsigned wave = threadIdx.x / KT_WAVE;
     const unsigned lane = lane_id();
     uint32_t* uid = uids + (LIST ? wave * KT_WAVE : 0);
     uint64_t my_total = 0;
-    WorkStats wk;
+    WorkStats wk(sums);
 
     // Every bucket's count and place in the list, read once.
     if (wave == 0) {
@@ -1296,7 +1345,8 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
             if (sg.cnt == 0) continue;
             const Shares sh(sg.cnt, parts || !by_vertex, sx,
                             parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : wave_parts);
-            const uint32_t most = pack ? min(max(prm.wave_grab, 1u), (uint32_t)KT_WAVE) : 2u;
+            const bool packs = !LIST && pack && !out.tail_count;
+            const uint32_t most = pack ? min(max(prm.wave_grab, 1u), L.grab[0].MAX) : 2u;
             const uint32_t grab = max(1u, min(most, sg.cnt / (4 * TC_WAVES * sh.blocks)));
             const uint32_t grabs = (sg.cnt + grab - 1) / grab;
             const uint32_t fixed = grabs <= 8 * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
@@ -1319,52 +1369,50 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
                     g = uniform(g);
                     if (g >= grabs) break;
                 }
-                // the grabbed tails (grab <= 64) and their bounds, loaded by
-                // one lane each before the first is processed: one round
-                // trip for the batch instead of two per tail
+                // the grabbed tails and their bounds, loaded by one lane each
+                // before the first is processed: one round trip for the batch
+                // instead of two per tail
                 const uint32_t i = g * grab;
                 const uint32_t ng = min(sg.cnt, i + grab) - i;
-                uint32_t xl = 0;
-                TailBounds bl{0, 0, 0, 0, 0};
+                auto& gb = L.grab[wave];
+                uint32_t nr = 0, ns = 0;
                 if (lane < ng) {
-                    if (parts) {
-                        const uint64_t xp = plist[sg.base + i + lane];
-                        xl = (uint32_t)xp;
-                        bl = part_bounds(V, xl, (uint32_t)(xp >> 32), prm.wave_split);
-                    } else {
-                        xl = list[sg.base + i + lane];
-                        bl = tail_bounds(V, xl);
-                    }
+                    const uint64_t xp = parts ? plist[sg.base + i + lane] : list[sg.base + i + lane];
+                    const TailBounds bl = parts ? part_bounds(V, (uint32_t)xp, (uint32_t)(xp >> 32), prm.wave_split)
+                                                : tail_bounds(V, (uint32_t)xp);
+                    gb.put(lane, (uint32_t)xp, bl);
+                    nr = bl.nr;
+                    ns = bl.ns;
                 }
-                // Consecutive small tails are taken together while their
-                // entries, set members and tables fit the wave.
-                const bool small = !LIST && !out.tail_count && pack && lane < ng;
-                const uint32_t sr = wave_scan_dpp(small ? bl.nr : 0u), ss = wave_scan_dpp(small ? bl.ns : 0u),
-                               st = wave_scan_dpp(small ? pack_slots(bl.ns) : 0u);
-                for (uint32_t j = 0; j < ng;) {
-                    const uint32_t br = j ? readlane32(sr, j - 1) : 0u, bs = j ? readlane32(ss, j - 1) : 0u,
-                                   bt = j ? readlane32(st, j - 1) : 0u;
-                    const bool fits = small && sr - br <= KT_WAVE && ss - bs <= KT_WAVE && st - bt <= WAVE_SLOTS;
-                    const uint64_t run = __builtin_amdgcn_ballot_w64(fits) >> j;
-                    if (run & 1) {
-                        const uint32_t n = run == ~0ull ? KT_WAVE : (uint32_t)__builtin_ctzll(~run);
-                        pack_process(V, xl, bl, sr - bl.nr - br, ss - bl.ns - bs, st - pack_slots(bl.ns) - bt, j, n,
-                                     readlane32(sr, j + n - 1) - br, readlane32(ss, j + n - 1) - bs, L.pk[wave], keys,
+                wave_sync();
+                if (packs) {
+                    // Consecutive small tails are taken together while their
+                    // entries, set members and tables fit the wave.
+                    const uint32_t rs = wave_scan_dpp(nr << 16 | ns), st = wave_scan_dpp(lane < ng ? pack_slots(ns) : 0u);
+                    for (uint32_t j = 0; j < ng;) {
+                        const uint32_t brs = j ? readlane32(rs, j - 1) : 0u, bt = j ? readlane32(st, j - 1) : 0u;
+                        const uint32_t in = rs - brs;  // (both halves ascend: no borrow from lane j on)
+                        const bool fits = lane < ng && (in >> 16) <= KT_WAVE && (in & 0xffffu) <= KT_WAVE &&
+                                          st - bt <= WAVE_SLOTS;
+                        const uint64_t run = __builtin_amdgcn_ballot_w64(fits) >> j;
+                        const uint32_t n = (uint32_t)__builtin_ctzll(~run);
+                        const uint32_t last = readlane32(in, j + n - 1), k = min(lane, gb.MAX - 1);
+                        pack_process(V, gb, (in >> 16) - gb.nr[k], (in & 0xffffu) - gb.ns[k],
+                                     st - pack_slots(gb.ns[k]) - bt, j, n, last >> 16, last & 0xffffu, L.pk[wave], keys,
                                      tcnt, wovf, out, my_total, wk);
                         j += n;
-                    } else {
-                        const TailBounds tb{readlane64(bl.sb, j), readlane64(bl.rb, j), readlane32(bl.ns, j),
-                                            readlane32(bl.nr, j), readlane32(bl.nstat, j)};
-                        team_process<1, WAVE_SLOTS / 2 / KT_WAVE, true, PLAIN, LIST>(
-                            V, readlane32(xl, j), tb, L, keys, tcnt, wovf, WAVE_SLOTS, prm.table_shift, KT_WAVE, out,
-                            my_total, wk, uid);
-                        ++j;
                     }
+                } else {
+                    for (uint32_t j = 0; j < ng; ++j)
+                        team_process<1, WAVE_SLOTS / 2 / KT_WAVE, true, PLAIN, LIST>(
+                            V, uniform(gb.x[j]), gb.bounds(j), L, keys, tcnt, wovf, WAVE_SLOTS, prm.table_shift, KT_WAVE,
+                            out, my_total, wk, uid);
                 }
+                wave_sync();  // the records are written again
             }
         }
     }
-    flush_sums<TC_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(L.keys), sums);
+    flush_sums<TC_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(L.keys));
 }
 
 // Tails whose S(x) exceeds the LDS table: 8-wave teams, binary-search probes
@@ -1375,11 +1423,11 @@ __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out
                                                          const uint32_t* __restrict__ list,
                                                          uint64_t* __restrict__ sums) {
     own_copy(out);
-    __shared__ Lds L;
+    __shared__ Lds<LIST> L;
     __shared__ uint32_t uids[LIST ? TC_THREADS : 1];
     uint32_t* uid = uids + (LIST ? threadIdx.x / KT_WAVE * KT_WAVE : 0);
     uint64_t my_total = 0;
-    WorkStats wk;
+    WorkStats wk(sums);
     const uint32_t cnt = q[Q_CNT + BUCKET_HUGE];
     if (cnt == 0) return;
     const uint32_t base = bucket_base(q, BUCKET_HUGE);
@@ -1397,7 +1445,7 @@ __global__ void __launch_bounds__(TC_THREADS) k_tc_huge(View<PLAIN> V, TcOut out
         team_process<TC_WAVES, 1, false, PLAIN, LIST>(V, x, tail_bounds(V, x), L, nullptr, nullptr, nullptr, 0, 0,
                                                             prm.team_chunk, out, my_total, wk, uid);
     }
-    flush_sums<TC_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(L.keys), sums);
+    flush_sums<TC_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(L.keys));
 }
 
 // Tails above the workgroup bin whose hash table fits one workgroup's LDS
@@ -1420,7 +1468,7 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
     if (threadIdx.x < BIG_SLOTS / 128) L.ovf[threadIdx.x] = 0;
     if (threadIdx.x == 0) L.full = 0;
     uint64_t my_total = 0;
-    WorkStats wk;
+    WorkStats wk(sums);
     const uint32_t cnt = q[Q_CNT + BUCKET_BIG];
     const uint32_t base = bucket_base(q, BUCKET_BIG);
     uint32_t* pull = &q[Q_PULL + Q_STRIDE * BUCKET_BIG];
@@ -1438,7 +1486,7 @@ __global__ void __launch_bounds__(BIG_THREADS) k_tc_big(View<PLAIN> V, TcOut out
                                                             big_table + BIG_SLOTS, L.ovf, BIG_SLOTS, prm.table_shift,
                                                             prm.team_chunk, out, my_total, wk, uid);
     }
-    flush_sums<BIG_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(big_table), sums);
+    flush_sums<BIG_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(big_table));
 }
 
 // ---------------------------------------------------------------------------
@@ -1588,7 +1636,7 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
     for (uint32_t i = tid; i < (2 * HUB_MAX + 16) / 4 + HUB_CNT; i += HUB_THREADS) hub_lds[i] = 0;
     __syncthreads();
     uint64_t my_total = 0;
-    WorkStats wk;
+    WorkStats wk(sums);
     const uint32_t fixed = parts <= 4 * gridDim.x ? parts : parts - parts / 4;
     uint32_t i = blockIdx.x;
     // the tail and bounds of the fixed share's next part, loaded a part ahead
@@ -1633,9 +1681,7 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
             bool stc = false;
             if (lane < c) V.entry_bounds(rb + k + lane, u, kw, ns, b, e, stl, stc);
             const uint64_t len = e > b ? e - b : 0;
-            wk.wedge_lane += stl;
-            wk.recv_lane += stc ? ns : 0u;
-            wk.stream_lane += len;
+            wk.add(stl, stc ? ns : 0u, len);
             uint64_t hits;
             const uint32_t h = walk_hub_lists(lists, b, len, tab, pk, hits);
             if (h && out.per_vertex) atomic_add_u64(&out.per_vertex[u], h);
@@ -1665,7 +1711,7 @@ __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_e
         __syncthreads();
         i = i < fixed ? i_nx : fixed;
     }
-    flush_sums<HUB_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(hub_lds), sums);
+    flush_sums<HUB_WAVES>(my_total, wk, reinterpret_cast<uint64_t*>(hub_lds));
 }
 
 // Adds up the per-XCD copies of the n per-vertex counts (n == 0: none) and,
