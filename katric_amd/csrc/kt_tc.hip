@@ -1304,7 +1304,7 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
         if (sg.cnt == 0) continue;
         const Shares sh(sg.cnt, parts || !by_vertex, sx, parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : team_parts);
         uint32_t* pull = &q[Q_PULL + Q_STRIDE * (parts ? BUCKET_TEAM_PARTS : CLASS_TEAM + (by_vertex ? (int)sx : 0))];
-        const uint32_t fixed = sg.cnt <= 4 * sh.blocks ? sg.cnt : sh.blocks;
+        const uint32_t fixed = !by_vertex || sg.cnt <= 4 * sh.blocks ? sg.cnt : sg.cnt - sg.cnt / 4;
         uint32_t i = sh.mine ? sh.first : fixed;
         while (true) {
             if (i >= fixed) {
@@ -1329,9 +1329,13 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
     }
     // wave phase: independent waves with private tables: the parts, the SOLO
     // tails (a few per grab: they are the long ones, and a grab that holds
-    // several ends late), then the PACK tails.  Grabs come from the
-    // workgroup's share, handed out by an LDS counter, and, where a wave gets
-    // many, the last quarter of a segment from its queue.
+    // several ends late), then the PACK tails.  Grabs are the workgroup's share,
+    // handed out by an LDS counter: with the last quarter of a segment taken from
+    // a queue, its word's atomics at 41 ns each were the time (G(n, m) n =
+    // 900,000, 3.6 M pairs 842 us by degree, 243 without; R-MAT scale 22 14.4 and
+    // 12.2 ms).  By vertex a queue per XCD also lets an XCD that is done help the
+    // others, which counts in long segments only (8192 mixed graphs, 290 grabs a
+    // wave, 82 ms with and 93 without; 768 of them, 31 grabs, 8.0 and 7.8).
     {
         uint32_t* keys = L.keys + wave * WAVE_SLOTS;
         uint32_t* tcnt = L.cnt + wave * WAVE_SLOTS;
@@ -1349,7 +1353,7 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
             const uint32_t most = pack ? min(max(prm.wave_grab, 1u), L.grab[0].MAX) : 2u;
             const uint32_t grab = max(1u, min(most, sg.cnt / (4 * TC_WAVES * sh.blocks)));
             const uint32_t grabs = (sg.cnt + grab - 1) / grab;
-            const uint32_t fixed = grabs <= 8 * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
+            const uint32_t fixed = !by_vertex || grabs <= 64 * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
             const int qi = parts ? cls : cls + (by_vertex ? (int)sx : 0);
             uint32_t* pull = &q[Q_PULL + Q_STRIDE * qi];
             bool own = sh.mine;
