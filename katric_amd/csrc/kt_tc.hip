@@ -403,7 +403,14 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
         return wave ? BUCKET_WAVE_PARTS : BUCKET_TEAM_PARTS;
     }
     const int cls = !wave ? CLASS_TEAM : s <= PACK_MAX && r <= PACK_MAX ? CLASS_PACK : CLASS_SOLO;
-    if (prm.order == TC_BY_VERTEX) return cls + (int)(((uint64_t)x * NXCD) / V.v.X);
+    // by vertex: the XCD whose eighth of the walk entries the tail starts in
+    // (an eighth of the vertices is a poor share where degrees drift with the
+    // id, as in a batch: 768 mixed graphs 8.6 ms, 8.2 with this)
+    if (prm.order == TC_BY_VERTEX) {
+        if (!PLAIN) return cls + (int)(((uint64_t)x * NXCD) / V.v.X);
+        const uint64_t all = V.min_side() ? V.v.in_off[V.v.X] : V.v.s_off[V.v.X];
+        return cls + min(NXCD - 1, (int)((float)rb * ((float)NXCD / (float)all)));
+    }
     return cls + (cls == CLASS_TEAM ? max(b - 4, 0) : cls == CLASS_SOLO ? min(b, 8) - 1 : b);
 }
 
@@ -1334,8 +1341,9 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
     // a queue, its word's atomics at 41 ns each were the time (G(n, m) n =
     // 900,000, 3.6 M pairs 842 us by degree, 243 without; R-MAT scale 22 14.4 and
     // 12.2 ms).  By vertex a queue per XCD also lets an XCD that is done help the
-    // others, which counts in long segments only (8192 mixed graphs, 290 grabs a
-    // wave, 82 ms with and 93 without; 768 of them, 31 grabs, 8.0 and 7.8).
+    // others, which counts in long segments only: 8192 mixed graphs (290 grabs a
+    // wave) 82 ms with and 93 without, 768 of them (31 and 34 grabs) 8.2 and 9.0,
+    // G(n, m) n = 900,000 (8 grabs) 372 and 245 us.
     {
         uint32_t* keys = L.keys + wave * WAVE_SLOTS;
         uint32_t* tcnt = L.cnt + wave * WAVE_SLOTS;
@@ -1353,7 +1361,7 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
             const uint32_t most = pack ? min(max(prm.wave_grab, 1u), L.grab[0].MAX) : 2u;
             const uint32_t grab = max(1u, min(most, sg.cnt / (4 * TC_WAVES * sh.blocks)));
             const uint32_t grabs = (sg.cnt + grab - 1) / grab;
-            const uint32_t fixed = !by_vertex || grabs <= 64 * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
+            const uint32_t fixed = !by_vertex || grabs <= (pack ? 24 : 16) * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
             const int qi = parts ? cls : cls + (by_vertex ? (int)sx : 0);
             uint32_t* pull = &q[Q_PULL + Q_STRIDE * qi];
             bool own = sh.mine;
