@@ -242,3 +242,16 @@ def test_serve_reads_each_kind_of_memory(ctx):
     for r, (_, out, total, pv) in zip(results, cases):
         assert (r.status, r.total) == (0, total)
         np.testing.assert_array_equal(out, pv)
+
+
+@pytest.mark.parametrize("order", [K.ORDER_DEGREE, K.ORDER_VERTEX])
+@pytest.mark.parametrize("n", [5, 1023, 1024, 1025, 4095, 4096, 4097])  # one block bins up to 4096 tails
+def test_bins_of_one_block(ctx, knobs, n, order):
+    knobs(order=order)
+    _check(ctx, *_wheel(n))
+    g = K.gen_gnm(n, min(8 * n, n * (n - 1) // 2), seed=n)
+    _, pv, want = O.run_shmem(g, threads=4)
+    _check(ctx, g, pv)
+    st = ctx.stats()
+    assert st["wedge_checks"] == want["wedge_checks"]
+    assert st["intersection_size_local"] == want["intersection_size_local"]
