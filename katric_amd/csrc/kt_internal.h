@@ -109,7 +109,7 @@ struct TcParams {
     uint32_t wave_split = 0xffffffffu;  // walk entries per part of a wave / workgroup tail (set by the launch)
     uint32_t team_split = 0xffffffffu;
     uint32_t hub_split = 0xffffffffu;
-    uint32_t wave_grab = 32;  // wave-bin tails a wave takes per queue access (1..64), vertex order
+    uint32_t wave_grab = 32;  // packed tails a wave takes per grab (at most what its LDS holds: 28)
     uint32_t bsearch_min_deg = 8192;  // |S(x)| above this: binary-search probes in global memory (<= 8192)
     uint32_t pseudo2core = 0; // skip tails with |S(x)| < 2 and count them (Config::pseudo2core)
     uint32_t min_side = 1;    // plain counting: intersect every edge from the side with the shorter T list

@@ -511,6 +511,9 @@ uint64_t shard_layout(void* base, const kt_shard_in* in, uint64_t nnz, uint64_t 
         cv.take(scan_tmp_words(std::max<uint64_t>(X, 2 * mtiles) + 1) * 8));
     // both phases use it: the list of the larger set of tails, the parts of the longer walk
     B.room = rich ? tc_room(std::max(nnz, mtot), 0, want_pv ? X : 0) : TcRoom{};
+    // hub lists for CeTriC's local phase, a plain view with at most nnz entries
+    // (scale 21 / 2 ranks: count 6.6 ms without, 5.7 with)
+    if (rich && in->algorithm == KT_SHARD_CETRIC) B.room.hub_slots = tc_room(nnz, nnz, 0).hub_slots;
     B.tc_ws = static_cast<uint64_t*>(
         cv.take(tc_ws_words((uint32_t)std::max<uint64_t>(X, in->n_msg), B.room, num_cus) * 8));
     B.pv = pv_dev ? static_cast<uint64_t*>(cv.take(std::max<uint64_t>(X, 1) * 8)) : nullptr;
@@ -690,7 +693,8 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, 
         v.sheads = B.cheads;
         v.s_off = B.coff;
         if (cetric) {
-            v.X = (uint32_t)X;  // plain view over owned + ghost tails
+            v.X = (uint32_t)X;  // plain view over owned + ghost tails, by global degrees
+            v.deg = B.deg;
         } else {
             v.X = nl;
             v.r_beg = B.coff;
@@ -741,9 +745,10 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, 
         // wave (measured on RMAT-22 and RMAT-26 / 16 ranks); the workgroup
         // teams on the remaining (large) message tails share their receivers
         // 4 (CeTriC) or 2 (DiTriC) at a time, since a few long lists per
-        // message make coarser grabs leave waves idle at the end (RMAT-26 /
-        // 16: CeTriC contracted phase 64.6 ms with 8 per grab, 58.4 ms with 4;
-        // DiTriC count 76.7 / 70.3 / 68.9 ms with 8 / 4 / 2)
+        // message make coarser grabs leave waves idle at the end on large
+        // shards (with one list per step, RMAT-26 / 16: CeTriC contracted phase
+        // 64.6 ms with 8 per grab, 58.4 with 4; with the present walk no
+        // difference from 4 to 64 at scale 20 / 16)
         TcParams pm = c->prm;
         pm.wave_max_deg = std::max<uint32_t>(pm.wave_max_deg, 256u);
         pm.team_chunk = std::min<uint32_t>(pm.team_chunk, cetric ? 4u : 2u);

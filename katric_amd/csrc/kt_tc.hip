@@ -18,8 +18,8 @@
 //     privatised -- per-slot LDS counters for w, a count per list for u, a
 //     team sum for x -- and flushed with one global atomic per non-zero counter;
 //   * tails are bucketed by ceil(log2 |S(x)|), largest first; walks longer than
-//     a team's share are split into parts (split_rule); workgroups take fixed
-//     shares first and pull the rest from queues (Shares);
+//     a team's share are split into parts (split_rule); the workgroups' shares
+//     are fixed in advance (Shares), with queues only where they pay;
 //   * tails above the workgroup bin go to 16-wave teams whose table fills a
 //     workgroup's LDS (16384 slots, |S| <= 8192); only larger S(x) are probed
 //     by binary search in the sorted S(x) in global memory.
@@ -1293,7 +1293,10 @@ struct Shares {
     }
 };
 
-// 80 VGPRs and 43 KB of LDS: three workgroups per CU, 6 waves per SIMD.
+// 80 VGPRs and 51.6 KB of LDS: three workgroups per CU, 6 waves per SIMD.  Bound
+// by the chain of dependent loads that every pack or chunk of 64 entries starts
+// with, and by VALU (73 % busy at R-MAT scale 22, where it takes 2.7 ms; 768
+// mixed graphs 6.1 ms).
 template <bool PLAIN, bool LIST>
 __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) k_tc_main(View<PLAIN> V, TcOut out, TcParams prm,
                                                          uint32_t* __restrict__ q,
@@ -1661,9 +1664,13 @@ __device__ __forceinline__ uint32_t walk_hub_lists(const uint16_t* __restrict__ 
     return mine;
 }
 
-// Workgroup tails that are hubs, part by part: 16-wave teams, two workgroups
+// Workgroup tails that are hubs, part by part: 12-wave teams, two workgroups
 // per CU, each with a table of one entry per hub in dynamic LDS.  The table is
-// empty between parts (the thread that set an entry clears it).
+// empty between parts (the thread that set an entry clears it).  Bound by LDS
+// reads (57 % busy, half of it bank conflicts) and VALU (65 %) of 24 waves a CU:
+// R-MAT scale 22 4.8 to 5.0 ms (8 waves a workgroup 5.3, 16 with room for 29,696
+// hubs 4.9 and 0.4 more in k_tc_main).  The last quarter of the parts comes from
+// a queue: without one 9.2 ms in place of 8.4 for the whole count phase.
 __global__ void __launch_bounds__(HUB_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6)))
     k_tc_hub(View<true> V, TcOut out, TcParams prm, uint32_t* __restrict__ q, const uint64_t* __restrict__ plist,
              const uint16_t* __restrict__ lists, uint64_t* __restrict__ sums) {

@@ -255,3 +255,18 @@ def test_bins_of_one_block(ctx, knobs, n, order):
     st = ctx.stats()
     assert st["wedge_checks"] == want["wedge_checks"]
     assert st["intersection_size_local"] == want["intersection_size_local"]
+
+
+@pytest.mark.parametrize("rank", [0, 1])
+def test_shard_hubs(ctx, knobs, rank):
+    """CeTriC's local phase above 2^22 slots: hub lists over owned and ghost tails."""
+    knobs(wave_max_deg=32)
+    g = K.gen_rmat(18, 24, seed=9)
+    sh = S.make_shard(g, 2, rank, S.CETRIC)
+    assert len(sh.heads) >= 1 << 22
+    loc, t3, pv = S.count_shard(ctx, sh)
+    oloc, ot3, opv, _ = O.rank_sim(g, 2, rank, S.CETRIC, threads=4)
+    assert (loc, t3) == (oloc, ot3)
+    full = np.zeros(g.n, np.uint64)
+    full[sh.vertex_ids()] = pv
+    np.testing.assert_array_equal(full, opv)
