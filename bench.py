@@ -38,16 +38,17 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 
-# HBM bytes per k_tc_main launch, measured with two rocprofv3 --pmc runs of
+# HBM bytes per intersection, measured with two rocprofv3 --pmc runs of
 # this workload under its autotuned knobs (FETCH_SIZE, then WRITE_SIZE, KiB
 # per dispatch).  A plain 1 GiB device copy reads FETCH_SIZE = 524,308 KiB and
 # WRITE_SIZE = 1,048,576 KiB on MI355X, so FETCH_SIZE is scaled by 2.000 and
-# WRITE_SIZE by 1.000.  RMAT-22 ef16 seed 1 (min-side walk):
-# 34,703,157 KiB x 2.000 + 3,177,102 KiB = 74.33 GB.
+# WRITE_SIZE by 1.000.  RMAT-22 ef16 seed 1 (min-side walk), KiB of
+# k_hub_lists, k_tc_hub and k_tc_main: (129,510 + 15,626,000 + 7,638,900) x 2.000
+# + 143,230 + 1,832,800 + 778,000 = 50.73 GB.
 # Shard (RMAT-26 ef16 seed 1, 16 ranks, rank 0, CeTriC), the count phase's
-# intersection launches (k_tc_main + k_tc_big, local and contracted, binning
-# and k_tc_huge): FETCH_SIZE 292,888,269 KiB x 2.000 + WRITE_SIZE 15,960,809 KiB = 616.18 GB.
-MEASURED_TRAFFIC = {("plain", 22, 16, 1): 74.33e9, ("shard-cetric", 26, 16, 1, 16, 0): 616.18e9}
+# k_hub_lists, k_tc_hub, k_tc_main and k_tc_big launches, local and contracted:
+# FETCH_SIZE 257,986,013 KiB x 2.000 + WRITE_SIZE 12,359,441 KiB = 541.01 GB.
+MEASURED_TRAFFIC = {("plain", 22, 16, 1): 50.73e9, ("shard-cetric", 26, 16, 1, 16, 0): 541.01e9}
 
 
 
@@ -695,7 +696,7 @@ def run_plain(args):
     dg.free()
     d_pv.free()
 
-    # roofline of k_tc_main on the bytes this design must move (unit = one
+    # roofline of the intersection on the bytes this design must move (unit = one
     # oriented edge: 4 B per streamed T-list id -- streamed_ids in all -- plus
     # 4 B of S(x) per kept slot, 20 B per walk entry and 16 B per vertex); the
     # reference's intersection_size_local figure, which charges both lists
@@ -730,7 +731,7 @@ def run_plain(args):
             "pipeline_reference_bytes_GBs": pipeline_gbs,
         },
         "roofline": {
-            "kernel": "k_tc_main (intersection)",
+            "kernel": "k_tc_hub + k_tc_main (intersection)",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
