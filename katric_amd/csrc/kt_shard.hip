@@ -64,8 +64,8 @@ struct ShardMap {
 // Ghost ids ascend, so the first ghost of a table word owns it: it reads the up
 // to 31 ids after its own, and its index is the word's prefix.  Words without a
 // ghost stay zero.  (The bits were set by atomics and counted, scanned and
-// spread by four more launches: six in all, 85 us for 77,000 ghosts among 2^18
-// ids in the CeTriC shard of an R-MAT graph; this one takes 8.)  Only
+// spread by six more launches, 37 us for 246,000 ghosts among 2^20 ids in the
+// CeTriC shard of an R-MAT graph; this one takes 8 with all it does.)  Only
 // strictly ascending ids are taken, so every index below is in range.
 __global__ void k_shard_prepare(ShardMap M, uint64_t nnz, const uint64_t* __restrict__ off,
                                 const uint64_t* __restrict__ ghost_degree, uint32_t* __restrict__ deg,
@@ -256,8 +256,9 @@ __global__ void k_cut_begin(uint32_t nl, const uint64_t* __restrict__ coff, cons
 // message order.  A count pass gives every 64 entries' bits and every tile's
 // totals; a thread per message then ranks its b and e, and a write pass places
 // the entries.  Short and long messages take the same time (8 lanes per message
-// took 126 + 44 us for the 241,000 messages of an R-MAT CeTriC shard, most of it
-// one long message's steps; the three passes take 60).
+// took 126 + 44 us for the 241,000 messages, 12 M ids, of an R-MAT CeTriC shard, the
+// three passes take 111 + 8 + 34, the first at the rate of its gathers; 63 + 29 and
+// 44 + 5 + 19 us for 6 M ids of a DiTriC shard).
 struct MsgWord {
     uint64_t own, ghost;      // entry classes of 64 entries
     uint32_t pre_own, pre_ghost;  // those of the tile's words before
@@ -659,8 +660,8 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, 
                        (flags & KT_ERR_MESSAGE) ? " bad message" : "");
     // the lists: their offsets, then each entry to its rank's place and every
     // list sorted by itself, or, with one longer than that sort takes, all keys
-    // by their bits.  (Five radix passes of five launches took 220 us for the
-    // 466,000 keys of an R-MAT CeTriC shard, place and sort 40.)
+    // by their bits.  (Five radix passes of five launches took 215 us for the
+    // 1.9 M keys of an R-MAT CeTriC shard, place and sort 57.)
     const bool over_wave = (flags & KT_FLAG_OVER_WAVE) != 0, over_group = (flags & KT_FLAG_OVER_GROUP) != 0;
     scan_u64(B.coff, B.coff, X, B.scan_tmp, st);
     if (Mk) {
