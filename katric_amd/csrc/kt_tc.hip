@@ -30,6 +30,7 @@
 // handed to this kernel carries 4 ids of padding.
 #include <algorithm>
 
+#include "kt_bins.h"
 #include "kt_device.h"
 #include "kt_internal.h"
 
@@ -40,33 +41,14 @@ constexpr int TC_WAVES = TC_THREADS / KT_WAVE;           // 8
 constexpr uint32_t GROUP_SLOTS = 4096;                   // shared table of the 8-wave team
 constexpr uint32_t WAVE_SLOTS = GROUP_SLOTS / TC_WAVES;  // private table of a 1-wave team (512)
 constexpr uint32_t MIN_LOGS = 6;
-// Work-queue buckets: three classes of eight.  Class PACK holds the tails that
-// a wave takes several at a time, SOLO the other wave tails, TEAM the
-// workgroup tails; the eight are size steps (by degree) or the contiguous
-// eighths of the tail range, one per XCD, each in vertex order (by vertex).
-// Then the tails beyond any LDS table (binary search, k_tc_huge) and those
-// above the workgroup bin whose table still fits a workgroup's whole LDS
-// (k_tc_big), and, in a list of their own, the parts of tails whose walk is
-// too long for one team (split_rule): entries (part << 32 | tail), taken by
-// workgroup teams and by waves before everything else.
-constexpr int CLASS_PACK = 0, CLASS_SOLO = 8, CLASS_TEAM = 16;
-constexpr int BUCKET_HUGE = 24;
-constexpr int BUCKET_BIG = 25;
-constexpr int NLIST = 26;  // buckets whose tails share the u32 list
-constexpr int BUCKET_TEAM_PARTS = 26;
-constexpr int BUCKET_WAVE_PARTS = 27;
-// Parts of the workgroup tails that k_tc_hub takes (every such tail, whole or
-// split).
-constexpr int BUCKET_HUB_PARTS = 28;
-constexpr int NBUCKET = 29;
-// Tails of class PACK: at most 64 ids in S(x) and 64 walk entries.
-constexpr uint32_t PACK_MAX = KT_WAVE;
 // k_tc_big: one 1024-thread workgroup per CU with a 16384-slot table (128 KB
 // of LDS for keys and counters), for |S| <= 8192
 constexpr int BIG_THREADS = 1024;
 constexpr int BIG_WAVES = BIG_THREADS / KT_WAVE;
 constexpr uint32_t BIG_SLOTS = 16384;
 constexpr int NXCD = 8;  // MI355X: workgroup i runs on XCD i % 8
+static_assert(NXCD == CLASS_STEPS, "a class' buckets are size steps or XCDs");
+static_assert(PACK_MAX == KT_WAVE, "a tail of class PACK fits a wave by itself");
 
 // work-queue header (u32 words at the start of the workspace); every counter
 // that waves update concurrently sits on its own 128-byte line so that the
@@ -179,8 +161,6 @@ struct View {
     __device__ __forceinline__ bool gated() const { return v.gate && (*v.gate & v.gate_bits); }
     __device__ __forceinline__ bool stat_skip_empty() const { return !PLAIN && v.stat_skip_empty; }
 };
-
-__device__ __forceinline__ uint32_t ceil_log2(uint64_t x) { return x <= 1 ? 0 : 64 - __clzll(x - 1); }
 
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
@@ -386,32 +366,20 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
     s = se - sb;
     r = re - rb;
     if (s == 0 || r == 0 || ((PLAIN || prm.pseudo2core) && s < 2)) return -1;
-    if (s > prm.bsearch_min_deg) return BUCKET_HUGE;
-    if (s > prm.group_max_deg) return BUCKET_BIG;
-    int b = (int)ceil_log2(s);  // size step, 0..11
-    // a min-side walk covers the whole input row: a long row goes to a
-    // bigger bucket (a workgroup team beyond 512 entries), whatever |S(x)|
-    if (V.min_side()) b = max(b, min((int)ceil_log2(r) - 2, (int)ceil_log2(prm.group_max_deg)));
-    const bool wave = b <= (int)ceil_log2(prm.wave_max_deg);
-    if (!wave && hub_min && deg_bin(V.v.deg[x]) >= *hub_min) {
-        parts = (uint32_t)((r + prm.hub_split - 1) / prm.hub_split);
-        return BUCKET_HUB_PARTS;
-    }
-    const uint32_t split = wave ? prm.wave_split : prm.team_split;
-    if (r > split) {
-        parts = (uint32_t)((r + split - 1) / split);
-        return wave ? BUCKET_WAVE_PARTS : BUCKET_TEAM_PARTS;
-    }
-    const int cls = !wave ? CLASS_TEAM : s <= PACK_MAX && r <= PACK_MAX ? CLASS_PACK : CLASS_SOLO;
+    const BinRule rule{prm.wave_max_deg, prm.group_max_deg, prm.bsearch_min_deg, prm.wave_split,
+                       prm.team_split,   prm.hub_split,     V.min_side()};
+    const TailBin t = tail_bin(s, r, rule, [&]() { return hub_min && deg_bin(V.v.deg[x]) >= *hub_min; });
+    parts = t.parts;
+    if (t.bucket >= BUCKET_HUGE) return t.bucket;
     // by vertex: the XCD whose eighth of the walk entries the tail starts in
     // (an eighth of the vertices is a poor share where degrees drift with the
     // id, as in a batch: 768 mixed graphs 8.6 ms, 8.2 with this)
     if (prm.order == TC_BY_VERTEX) {
-        if (!PLAIN) return cls + (int)(((uint64_t)x * NXCD) / V.v.X);
+        if (!PLAIN) return t.bucket + (int)(((uint64_t)x * NXCD) / V.v.X);
         const uint64_t all = V.min_side() ? V.v.in_off[V.v.X] : V.v.s_off[V.v.X];
-        return cls + min(NXCD - 1, (int)((float)rb * ((float)NXCD / (float)all)));
+        return t.bucket + min(NXCD - 1, (int)((float)rb * ((float)NXCD / (float)all)));
     }
-    return cls + (cls == CLASS_TEAM ? max(b - 4, 0) : cls == CLASS_SOLO ? min(b, 8) - 1 : b);
+    return t.bucket + t.step;
 }
 
 // Bucket regions in one list, the highest bucket first, so that by degree the
@@ -1436,29 +1404,34 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
                     ns = bl.ns;
                 }
                 wave_sync();
+                uint32_t j = 0;
                 if (packs) {
                     // Consecutive small tails are taken together while their
-                    // entries, set members and tables fit the wave.
-                    const uint32_t rs = wave_scan_dpp(nr << 16 | ns), st = wave_scan_dpp(lane < ng ? pack_slots(ns) : 0u);
-                    for (uint32_t j = 0; j < ng;) {
+                    // entries, set members and tables fit the wave.  (Every tail
+                    // of the class fits by itself; the sums are of capped sizes
+                    // and the loop ends at one that does not, so that no bin
+                    // rule could make it spin.)
+                    const uint32_t rs = wave_scan_dpp(min(nr, 2 * PACK_MAX) << 16 | min(ns, 2 * PACK_MAX)),
+                                   st = wave_scan_dpp(lane < ng ? pack_slots(ns) : 0u);
+                    while (j < ng) {
                         const uint32_t brs = j ? readlane32(rs, j - 1) : 0u, bt = j ? readlane32(st, j - 1) : 0u;
                         const uint32_t in = rs - brs;  // (both halves ascend: no borrow from lane j on)
                         const bool fits = lane < ng && (in >> 16) <= KT_WAVE && (in & 0xffffu) <= KT_WAVE &&
                                           st - bt <= WAVE_SLOTS;
                         const uint64_t run = __builtin_amdgcn_ballot_w64(fits) >> j;
                         const uint32_t n = (uint32_t)__builtin_ctzll(~run);
+                        if (n == 0) break;
                         const uint32_t last = readlane32(in, j + n - 1), k = min(lane, gb.MAX - 1);
                         pack_process(V, gb, (in >> 16) - gb.nr[k], (in & 0xffffu) - gb.ns[k],
                                      st - pack_slots(gb.ns[k]) - bt, j, n, last >> 16, last & 0xffffu, L.pk[wave], keys,
                                      tcnt, wovf, out, my_total, wk);
                         j += n;
                     }
-                } else {
-                    for (uint32_t j = 0; j < ng; ++j)
-                        team_process<1, WAVE_SLOTS / 2 / KT_WAVE, true, PLAIN, LIST>(
-                            V, uniform(gb.x[j]), gb.bounds(j), L, keys, tcnt, wovf, WAVE_SLOTS, prm.table_shift, KT_WAVE,
-                            out, my_total, wk, uid);
                 }
+                for (; j < ng; ++j)
+                    team_process<1, WAVE_SLOTS / 2 / KT_WAVE, true, PLAIN, LIST>(
+                        V, uniform(gb.x[j]), gb.bounds(j), L, keys, tcnt, wovf, WAVE_SLOTS, prm.table_shift, KT_WAVE,
+                        out, my_total, wk, uid);
                 wave_sync();  // the records are written again
             }
         }

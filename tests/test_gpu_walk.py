@@ -270,3 +270,59 @@ def test_shard_hubs(ctx, knobs, rank):
     full = np.zeros(g.n, np.uint64)
     full[sh.vertex_ids()] = pv
     np.testing.assert_array_equal(full, opv)
+
+
+def _few_ghost_messages(algo, pad, seed):
+    """A shard whose messages hold 1 to 3 known ghosts and 63 to 2000 owned ids, and one message of `pad` unknown
+    ids (the length of walks that are split goes with the received entries): (shard, triangles, per-vertex counts)."""
+    rng = np.random.default_rng(seed)
+    nl, ng = 4096, 200
+    n = nl + 2000 + pad
+    ghosts = np.sort(rng.choice(np.arange(nl, nl + 1000), ng, replace=False))
+    adj = rng.random((nl, ng)) < 0.1
+    rows = [ghosts[a] for a in adj]
+    src, msgs, pv = [], [], np.zeros(nl + ng, np.uint64)
+    for r in (63, 64, 65, 128, 129, 2000):
+        for k in (1, 2, 3, 1):
+            own = np.sort(rng.choice(nl, r, replace=False))
+            sender, *known = rng.choice(ng, k + 1, replace=False)
+            known = np.sort(known)
+            src.append(sender)
+            msgs.append(np.concatenate([own, ghosts[known]]))
+            hit = adj[np.ix_(own, known)].astype(np.uint64)
+            pv[own] += hit.sum(1)
+            pv[nl + known] += hit.sum(0)
+            pv[nl + sender] += hit.sum()
+    src.append(0)
+    msgs.append(np.arange(nl + 2000, n))
+    offsets = lambda lists: np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.uint64)
+    ids = lambda lists: np.concatenate(lists).astype(np.uint32)
+    sh = S.Shard(algorithm=algo, rank=0, bounds=np.array([0, nl, n], np.uint64), offsets=offsets(rows),
+                 heads=ids(rows), ghost_ids=ghosts.astype(np.uint32), ghost_degree=np.full(ng, 1 << 20, np.uint64),
+                 msg_src=ghosts[src].astype(np.uint32), msg_offsets=offsets(msgs), msg_heads=ids(msgs))
+    return sh, int(pv.sum()) // 3, pv
+
+
+@pytest.mark.parametrize("order", [K.ORDER_DEGREE, K.ORDER_VERTEX])
+@pytest.mark.parametrize("algo", [S.CETRIC, S.DITRIC])
+@pytest.mark.parametrize("pad", [0, 900_000, 7_000_000])  # walks split at 16 entries, at 128, not at all
+def test_few_ghost_messages(ctx, knobs, order, algo, pad):
+    knobs(order=order)
+    sh, want, pv = _few_ghost_messages(algo, pad, seed=pad)
+    loc, t3, got = S.count_shard(ctx, sh)
+    assert (loc, t3) == (0, want)
+    np.testing.assert_array_equal(got, pv)
+
+
+@pytest.mark.parametrize("order", [K.ORDER_DEGREE, K.ORDER_VERTEX])
+def test_few_ghost_messages_under_a_tight_budget(order):
+    sh, want, pv = _few_ghost_messages(S.CETRIC, 0, seed=1)
+    with K.Context(0) as free:
+        S.count_shard(free, sh)
+        rich = free.device_bytes()
+    with K.Context(0, hbm_budget_bytes=rich - 64 * len(pv)) as tight:
+        tight.set_params(order=order)
+        loc, t3, got = S.count_shard(tight, sh)
+        assert tight.device_bytes() <= rich - 64 * len(pv)
+    assert (loc, t3) == (0, want)
+    np.testing.assert_array_equal(got, pv)
