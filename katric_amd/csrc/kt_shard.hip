@@ -549,7 +549,8 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, 
     const bool want_pv = out->per_vertex != nullptr;
     const bool pv_dev = want_pv && (in->flags & KT_DEVICE_OUTPUT);
     if (nl == 0 && ng == 0) return KT_OK;
-    // sizes
+    // sizes (read by a kernel from device arrays)
+    if (in->n_msg && (!in->msg_src || !in->msg_offsets)) return c->fail(KT_EINVAL, "null shard array");
     uint64_t nnz = 0, mtot = 0;
     if (host_in) {
         if (in->offsets[0] != 0) return c->fail(KT_EINVAL, "offsets[0] != 0");
@@ -570,7 +571,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, 
         }
     }
     if ((nnz && !in->heads) || (ng && (!in->ghost_ids || !in->ghost_degree)) ||
-        (in->n_msg && (!in->msg_src || !in->msg_offsets || (mtot && !in->msg_heads))))
+        (mtot && !in->msg_heads))
         return c->fail(KT_EINVAL, "null shard array");
     ShardBufs B;
     // the intersection's optional room is left out where only it does not fit

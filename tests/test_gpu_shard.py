@@ -1,5 +1,7 @@
 """Parity of the HIP shard path (kt_count_shard) with the oracle's P-rank
 simulation, per rank, for CeTriC (cetric-x) and DiTriC (patric)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,20 @@ def test_shard_bad_message(ctx):
         S.count_shard(ctx, sh)
     assert e.value.status == K.KT_EINVAL
     check_rank(ctx, g, 4, 1, S.CETRIC)
+
+
+@pytest.mark.parametrize("device", [False, True])
+@pytest.mark.parametrize("missing", ["heads", "ghost_ids", "ghost_degree", "msg_src", "msg_offsets", "msg_heads"])
+def test_shard_null_array(ctx, missing, device):
+    sh = S.make_shard(K.gen_rmat(10, 8, seed=2), 4, 1)
+    names = ("offsets", "heads", "ghost_ids", "ghost_degree", "msg_src", "msg_offsets", "msg_heads")
+    bufs = S.upload_shard(ctx, sh).bufs if device else None
+    ptr = {k: bufs[k].ptr if device else getattr(sh, k).ctypes.data for k in names}
+    ptr[missing] = None
+    si = S.KtShardIn(algorithm=sh.algorithm, rank=1, num_ranks=4, flags=K.KT_DEVICE_INPUT if device else 0,
+                     range_bounds=sh.bounds.ctypes.data, n_ghost=len(sh.ghost_ids), n_msg=len(sh.msg_src), **ptr)
+    assert len(sh.msg_src) and len(sh.ghost_ids)
+    out = S.KtShardOut(0, 0, None)
+    with pytest.raises(K.KatricError) as e:
+        ctx.check(S.lib().kt_count_shard(ctx.handle, C.byref(si), C.byref(out)), "kt_count_shard")
+    assert e.value.status == K.KT_EINVAL
