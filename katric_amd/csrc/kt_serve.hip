@@ -27,6 +27,7 @@
 #include "../../include/katric_serve.h"
 #include "kt_ctx.h"
 #include "kt_device.h"
+#include "kt_pinned.h"
 
 namespace kt {
 
@@ -98,19 +99,20 @@ __global__ void __launch_bounds__(256) k_serve_gather(uint32_t G, const GatherDe
     if (blockIdx.x == 0 && threadIdx.x == 0) off[N] = nnz;
 }
 
-// The device's address of page-locked host memory p[0, bytes), or null (pageable
-// memory, or a range whose ends are not in one page-locked allocation).
+// The device's address of host memory p[0, bytes) that is page-locked as a
+// whole, or null.
 static const void* device_view(const void* p, uint64_t bytes) {
-    if (!bytes) return nullptr;
-    hipPointerAttribute_t a{}, z{};
-    const char* last = static_cast<const char*>(p) + bytes - 1;
-    if (hipPointerGetAttributes(&a, p) != hipSuccess || hipPointerGetAttributes(&z, last) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (a.type != hipMemoryTypeHost || z.type != hipMemoryTypeHost || !a.devicePointer || !z.devicePointer) return nullptr;
-    if (static_cast<char*>(z.devicePointer) - static_cast<char*>(a.devicePointer) != (ptrdiff_t)(bytes - 1)) return nullptr;
-    return a.devicePointer;
+    return pinned_view(p, bytes, [](const void* q) {
+        hipPointerAttribute_t a{};
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipPointerGetAttributes(&a, q) != hipSuccess || a.type != hipMemoryTypeHost ||
+            hipMemGetAddressRange(&base, &size, const_cast<void*>(q)) != hipSuccess) {
+            (void)hipGetLastError();
+            return PinnedAt{nullptr, nullptr, 0};
+        }
+        return PinnedAt{static_cast<const char*>(a.devicePointer), static_cast<const char*>(base), size};
+    });
 }
 
 struct ServeReq {
