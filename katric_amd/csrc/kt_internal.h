@@ -186,6 +186,9 @@ struct TcView {
     uint32_t gate_bits = 0;
     bool cleared = false;  // the caller cleared tc_clear's ranges
     uint64_t longest = 0;  // no list S is longer (0: not known)
+    // by vertex: plain tails go to the XCDs in stripes of this many (0: in
+    // eighths of the walk entries)
+    uint32_t stripe = 0;
     // host words (page-locked; nullable) that receive the gate word, *kept, the
     // total and the four work counters at the end; with them, per_vertex is
     // assigned (room.pv_n set) and left alone when the gate is closed

@@ -697,6 +697,7 @@ int kt::count_shard_locked(kt_ctx* c, const kt_shard_in* in, kt_shard_out* out, 
         if (cetric) {
             v.X = (uint32_t)X;  // plain view over owned + ghost tails, by global degrees
             v.deg = B.deg;
+            v.stripe = 1024;
         } else {
             v.X = nl;
             v.r_beg = B.coff;

@@ -373,9 +373,14 @@ __device__ __forceinline__ int tail_bucket(const View<PLAIN>& V, const TcParams&
     if (t.bucket >= BUCKET_HUGE) return t.bucket;
     // by vertex: the XCD whose eighth of the walk entries the tail starts in
     // (an eighth of the vertices is a poor share where degrees drift with the
-    // id, as in a batch: 768 mixed graphs 8.6 ms, 8.2 with this)
+    // id, as in a batch: 768 mixed graphs 8.6 ms, 8.2 with this).  The entries
+    // say little about the work where the lists that they stream differ with the
+    // id: of a CeTriC shard's combined tails, owned first and then ghosts, one
+    // eighth had twice the mean (R-MAT scale 26, rank 0 of 16: local phase 70.8 ms,
+    // 49.2 in stripes of 128 to 8192; scale 20 / 16 0.48 and 0.35)
     if (prm.order == TC_BY_VERTEX) {
         if (!PLAIN) return t.bucket + (int)(((uint64_t)x * NXCD) / V.v.X);
+        if (V.v.stripe) return t.bucket + (int)(x / V.v.stripe % NXCD);
         const uint64_t all = V.min_side() ? V.v.in_off[V.v.X] : V.v.s_off[V.v.X];
         return t.bucket + min(NXCD - 1, (int)((float)rb * ((float)NXCD / (float)all)));
     }

@@ -326,3 +326,19 @@ def test_few_ghost_messages_under_a_tight_budget(order):
         assert tight.device_bytes() <= rich - 64 * len(pv)
     assert (loc, t3) == (0, want)
     np.testing.assert_array_equal(got, pv)
+
+
+@pytest.mark.parametrize("algo", [S.CETRIC, S.DITRIC])
+@pytest.mark.parametrize("n", [1023, 8191, 8193, 100_003])  # the stripes of tails that go to one XCD: 1024
+def test_shard_by_vertex(ctx, knobs, n, algo):
+    knobs(order=K.ORDER_VERTEX)
+    g = K.gen_rmat(17, 12, seed=n, n=n)
+    bounds = np.array([0, n // 5, n], np.uint64)
+    for rank in (0, 1):
+        sh = S.make_shard(g, 2, rank, algo, bounds=bounds)
+        loc, t3, pv = S.count_shard(ctx, sh)
+        oloc, ot3, opv, _ = O.rank_sim(g, 2, rank, algo, bounds=bounds, threads=4)
+        assert (loc, t3) == (oloc, ot3)
+        full = np.zeros(g.n, np.uint64)
+        full[sh.vertex_ids()] = pv
+        np.testing.assert_array_equal(full, opv)
