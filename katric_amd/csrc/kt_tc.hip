@@ -957,18 +957,20 @@ __device__ __forceinline__ uint32_t walk_lists(const uint32_t* __restrict__ T, u
             int lim = 0;
             Ids4 q;
             // (s == steps, loaded but not probed: every lane takes the step's
-            // first block, which is in list `base`, or the last block there is)
+            // first block, which is in list `base`, or the last block there is;
+            // without a branch, as the loop waits longest for its own issue)
+            const uint32_t last = min(w0 + steps * KT_WAVE, blocks - 1);
             auto load = [&](uint32_t s) {
-                const bool over = s == steps;
-                const int l0 = over ? 0 : (int)(2 * s);
-                ends = over ? 0 : (uint64_t)readlane32(bits, l0) | ((uint64_t)readlane32(bits, l0 + 1) << 32);
+                const uint64_t on = s == steps ? 0 : ~0ull;
+                const uint32_t l0 = 2 * s % KT_WAVE;
+                ends = ((uint64_t)readlane32(bits, (int)l0) | ((uint64_t)readlane32(bits, (int)l0 + 1) << 32)) & on;
                 rk = rank_below(ends, base);
                 base += (uint32_t)__popcll(ends);
                 const uint4 r = pk.rec[rk];
-                const uint32_t p = w0 + s * KT_WAVE + (over ? 0 : lane);
-                lim = (int)r.z - (int)(4 * p);
+                const uint32_t p = w0 + s * KT_WAVE + lane;
+                lim = (int)r.z - (int)(4 * p);  // past the last block: its list's, and not above zero
                 tt = r.w;
-                q = load_ids4(T + ((((uint64_t)r.y << 32) | r.x) + 4ull * min(p, blocks - 1)));
+                q = load_ids4(T + ((((uint64_t)r.y << 32) | r.x) + 4ull * min(p, last)));
             };
             load(0);
             for (uint32_t s = 0; s < steps; ++s) {
@@ -976,7 +978,7 @@ __device__ __forceinline__ uint32_t walk_lists(const uint32_t* __restrict__ T, u
                 const uint64_t c_ends = ends;
                 const uint32_t c_rk = rk;
                 const uint32_t c_off = TAILS ? tt >> 16 : 0u, c_mask = TAILS ? tt & 0xffffu : P.boff;
-                const int c_lim = s * KT_WAVE + w0 + lane < blocks ? lim : 0;
+                const int c_lim = lim;
                 load(s + 1);
                 uint32_t nh = 0;
                 if (HASH) {
@@ -1370,8 +1372,13 @@ __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu
             const Shares sh(sg.cnt, parts || !by_vertex, sx,
                             parts ? 0 : by_vertex ? sx * (gridDim.x / NXCD) : wave_parts);
             const bool packs = !LIST && pack && !out.tail_count;
+            // SOLO tails: two while a wave gets at least four grabs, from 32 grabs a
+            // wave on up to eight (one round trip for the bounds of all: R-MAT
+            // scale 26, rank 0 of 16, DiTriC's distributed phase 64.6 -> 64.0 ms
+            // with 4, 8 or 16; no change at scale 22 and for batches)
             const uint32_t most = pack ? min(max(prm.wave_grab, 1u), L.grab[0].MAX) : 2u;
-            const uint32_t grab = max(1u, min(most, sg.cnt / (4 * TC_WAVES * sh.blocks)));
+            const uint32_t per_wave = sg.cnt / (TC_WAVES * sh.blocks);
+            const uint32_t grab = max(max(1u, min(most, per_wave / 4)), pack ? 0u : min(8u, per_wave / 32));
             const uint32_t grabs = (sg.cnt + grab - 1) / grab;
             const uint32_t fixed = !by_vertex || grabs <= (pack ? 24 : 16) * TC_WAVES * sh.blocks ? grabs : grabs - grabs / 4;
             const int qi = parts ? cls : cls + (by_vertex ? (int)sx : 0);

@@ -342,3 +342,18 @@ def test_shard_by_vertex(ctx, knobs, n, algo):
         full = np.zeros(g.n, np.uint64)
         full[sh.vertex_ids()] = pv
         np.testing.assert_array_equal(full, opv)
+
+
+@pytest.mark.parametrize("order", [K.ORDER_DEGREE, K.ORDER_VERTEX])
+@pytest.mark.parametrize("n", [150_000, 700_003, 1_700_001])  # 2, 3 and 8 long tails per grab by degree
+def test_many_long_tails(ctx, knobs, n, order):
+    # a ring where everyone knows the k nearest on both sides: 66 walk entries a tail
+    k = 33
+    knobs(order=order, min_side=1)
+    near = np.concatenate([np.arange(-k, 0), np.arange(1, k + 1)])
+    heads = ((np.arange(n)[:, None] + near) % n).astype(np.uint32)
+    ends = np.r_[:k, n - k:n]
+    heads[ends] = np.sort(heads[ends], 1)
+    g = K.Graph(n, np.arange(n + 1, dtype=np.uint64) * (2 * k), heads.reshape(-1))
+    per = sum(1 for a in near for b in near if a < b and b - a <= k)
+    _check(ctx, g, np.full(n, per, np.uint64))
