@@ -357,3 +357,12 @@ def test_many_long_tails(ctx, knobs, n, order):
     g = K.Graph(n, np.arange(n + 1, dtype=np.uint64) * (2 * k), heads.reshape(-1))
     per = sum(1 for a in near for b in near if a < b and b - a <= k)
     _check(ctx, g, np.full(n, per, np.uint64))
+
+
+@pytest.mark.parametrize("algo", [S.CETRIC, S.DITRIC])
+def test_messages_beyond_the_cache(ctx, knobs, algo):
+    knobs(order=K.ORDER_DEGREE)
+    sh, want, pv = _few_ghost_messages(algo, 1 << 26, seed=3)  # taken by vertex from there on
+    loc, t3, got = S.count_shard(ctx, sh)
+    assert (loc, t3) == (0, want)
+    np.testing.assert_array_equal(got, pv)
