@@ -223,8 +223,15 @@ static HubWs hub_ws(uint64_t* ws, uint32_t X) {
 // than HUB_MAX vertices are in it or above -- or none, where the hubs' rows
 // hold less than a quarter of the `entries`: numbering them and writing the
 // lists (0.5 ms for 106 M oriented slots of 768 mixed graphs, where hubs hold a
-// sixth) then costs more than k_tc_hub gains.
+// sixth) then costs more than k_tc_hub gains.  The combined tails of a shard
+// (rows: their lists' offsets) have the whole graph's degrees, which say nothing
+// about the rank's entries: of these, the lists of the hubs that k_tc_hub would
+// take (longer than wave_max) have to hold a sixth.  R-MAT, count phase without
+// and with hubs: scale 22 / 2 (0.24 of the entries) 14.4 and 12.9 ms, / 4 (0.18)
+// 10.5 and 10.3, / 8 (0.13) 6.88 and 6.91, / 16 (0.12) 4.41 and 4.48, scale 26 / 16
+// 105.1 and 106.4.
 __global__ void __launch_bounds__(HUB_HIST_THREADS) k_hub_hist(uint32_t X, const uint32_t* __restrict__ deg,
+                                                               const uint64_t* __restrict__ rows, uint32_t wave_max,
                                                                uint64_t entries, HubWs h) {
     __shared__ uint32_t bins[DEG_BINS];
     __shared__ unsigned long long sums[DEG_BINS];
@@ -239,7 +246,8 @@ __global__ void __launch_bounds__(HUB_HIST_THREADS) k_hub_hist(uint32_t X, const
         const uint32_t d = deg[x];
         if (d >= 8) {
             atomicAdd(&bins[deg_bin(d)], 1u);
-            atomicAdd(&sums[deg_bin(d)], (unsigned long long)d);
+            const uint64_t len = rows ? rows[x + 1] - rows[x] : d;
+            if (!rows || len > wave_max) atomicAdd(&sums[deg_bin(d)], (unsigned long long)len);
         }
     }
     __syncthreads();
@@ -284,7 +292,7 @@ __global__ void __launch_bounds__(HUB_HIST_THREADS) k_hub_hist(uint32_t X, const
     if (threadIdx.x == 0) {
         sum = 0;
         for (int w = 0; w < HUB_HIST_THREADS / KT_WAVE; ++w) sum += wsum[w];
-        *h.min_bin = 4 * sum >= entries ? pick : DEG_BINS;
+        *h.min_bin = (rows ? 6 * sum >= rows[X] : 4 * sum >= entries) ? pick : DEG_BINS;
     }
 }
 
@@ -1909,7 +1917,8 @@ static hipError_t launch_impl(const TcView& view, const TcOut& user_out, const T
             hub = hub_ws(room, view.X);
             // few blocks: each adds up to a thousand bins to the global ones
             k_hub_hist<<<std::clamp<unsigned>(view.X / (32 * HUB_HIST_THREADS), 1, HUB_BLOCKS), HUB_HIST_THREADS, 0,
-                         st>>>(view.X, view.deg, view.room.entries, hub);
+                         st>>>(view.X, view.deg, view.sym_slots ? nullptr : view.s_off, p.wave_max_deg, view.room.entries,
+                               hub);
         }
     }
     room += hub_ws_words(view.X, view.room.hub_slots);

@@ -366,3 +366,20 @@ def test_messages_beyond_the_cache(ctx, knobs, algo):
     loc, t3, got = S.count_shard(ctx, sh)
     assert (loc, t3) == (0, want)
     np.testing.assert_array_equal(got, pv)
+
+
+@pytest.mark.parametrize("wave_max_deg", [2, 64])  # the hubs' lists that k_tc_hub would take: all, none
+def test_shard_hub_rule(ctx, knobs, wave_max_deg):
+    """Above 2^22 slots, global degrees far above a rank's list lengths."""
+    knobs(wave_max_deg=wave_max_deg)
+    n = 70_000
+    g = K.gen_gnm(n, 9_000_000, seed=4)
+    bounds = np.array([0, n // 4, n], np.uint64)
+    sh = S.make_shard(g, 2, 0, S.CETRIC, bounds=bounds)
+    assert len(sh.heads) >= 1 << 22
+    loc, t3, pv = S.count_shard(ctx, sh)
+    oloc, ot3, opv, _ = O.rank_sim(g, 2, 0, S.CETRIC, bounds=bounds, threads=4)
+    assert (loc, t3) == (oloc, ot3)
+    full = np.zeros(n, np.uint64)
+    full[sh.vertex_ids()] = pv
+    np.testing.assert_array_equal(full, opv)
