@@ -3,6 +3,8 @@
 Closed forms (cliques, wheels) for the edges of packs, parts, list blocks and
 windows; the oracle for a skewed graph whose workgroup tails are partly hubs.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -383,3 +385,42 @@ def test_shard_hub_rule(ctx, knobs, wave_max_deg):
     full = np.zeros(n, np.uint64)
     full[sh.vertex_ids()] = pv
     np.testing.assert_array_equal(full, opv)
+
+
+@pytest.mark.parametrize("lens", [
+    [(255, 256), (1, 1), (0, 0), (257, 255), (0, 3)],     # tiles of one id per thread: 256 ids
+    [(2047, 9)], [(2048, 9)], [(2049, 9)],                # sums of 2048 ids: one, one, two
+    [(0, 700)], [(700, 0)],
+    [(1, 1)] * 300 + [(0, 0)] * 400 + [(64, 64)] * 9,     # more pairs than a tile has ids
+    [(32768, 32768)], [(32768, 32769)],                   # 2^16 ids in all: the larger tiles from there on
+])
+@pytest.mark.parametrize("device", [False, True])
+def test_intersect_few_ids(ctx, lens, device):
+    rng = np.random.default_rng(len(lens))
+    pairs = [tuple(np.sort(rng.choice(2 * (la + lb) + 1, n, replace=False)).astype(np.uint32) for n in (la, lb))
+             for la, lb in lens]
+    want = [np.intersect1d(a, b) for a, b in pairs]
+    if not device:
+        counts, matches = ctx.intersect(pairs)
+    else:
+        arrays = []
+        for side in (0, 1):
+            arrays.append(np.concatenate([[0], np.cumsum([len(p[side]) for p in pairs])]).astype(np.uint64))
+            arrays.append(np.concatenate([p[side] for p in pairs]).astype(np.uint32))
+        bufs = [ctx.alloc(max(a.nbytes, 8)) for a in arrays]
+        for b, a in zip(bufs, arrays):
+            if a.size:
+                b.upload(a)
+        cap = sum(len(w) for w in want)
+        out = [ctx.alloc(8 * len(pairs)), ctx.alloc(4 * cap + 8)]
+        total = C.c_uint64()
+        ctx.check(K._ffi.lib().kt_intersect(ctx.handle, len(pairs), *[b.ptr for b in bufs],
+                                            K.KT_DEVICE_INPUT | K.KT_DEVICE_OUTPUT, out[0].ptr, out[1].ptr, cap,
+                                            C.byref(total)), "kt_intersect")
+        assert total.value == cap
+        counts = out[0].download(np.uint64, len(pairs))
+        matches = np.split(out[1].download(np.uint32, cap) if cap else np.zeros(0, np.uint32),
+                           np.cumsum([len(w) for w in want])[:-1])
+    assert counts.tolist() == [len(w) for w in want]
+    for m, w in zip(matches, want):
+        np.testing.assert_array_equal(m, w)
