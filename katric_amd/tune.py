@@ -1,17 +1,17 @@
 """Autotuner for the intersection knobs (kt_params).
 
-The knobs -- wave/workgroup bin thresholds, how a team walks its T lists
-(streamed or grouped), from which side each edge is intersected (min_side),
-queue order (degree or vertex), persistent workgroups per CU -- move work between
-kernels and code paths and never change a count.  Their best setting depends
+The knobs -- wave/workgroup bin thresholds, from which side each edge is
+intersected (min_side), queue order (degree or vertex), persistent workgroups
+per CU, and the list-walk hint, of which every value takes the same walk -- move
+work between kernels and code paths and never change a count.  Their best setting depends
 on the degree profile of the input, so the tuner
 
   * reduces an input to a *graph class*: log2 buckets of the vertex count,
     of the average degree and of the largest degree (for a batch: of the
     graph count, the average degree and the largest degree);
-  * times every candidate setting on the device (HIP events inside the
-    library: binning + intersection + everything after orientation), keeping
-    the fastest by median over a few repetitions;
+  * times every candidate setting that the device tells apart (HIP events
+    inside the library: binning + intersection + everything after orientation),
+    keeping the fastest by median over a few repetitions;
   * stores the winner per class in a JSON table.
 
 The table shipped in the package (tuned_params.json) was measured on MI355X;
@@ -81,6 +81,12 @@ def candidates(stage: dict, base: Dict[str, int]) -> List[Dict[str, int]]:
     return out
 
 
+def effective(p: Dict[str, int]) -> Dict[str, int]:
+    """The setting that the device runs for `p`: one walk whatever the hint
+    says, and at most the three workgroups per CU that fit."""
+    return dict(p, strategy=0, grid_per_cu=min(p["grid_per_cu"], 3))
+
+
 def load_table(path: Optional[str] = None) -> Dict[str, dict]:
     table: Dict[str, dict] = {}
     for p in ([PACKAGE_TABLE, user_table_path()] if path is None else [path]):
@@ -137,12 +143,14 @@ def tune(ctx, run: Callable[[], float], reps: int = 3, key: Optional[str] = None
     """Times `run` (one counting call on `ctx` returning its device
     milliseconds) stage by stage: each stage tries every combination of its
     knobs on top of the best setting so far and keeps the fastest (median of
-    `reps` runs after one warm-up run).  Returns {"params", "ms",
+    `reps` runs after one warm-up run); settings that the device runs alike are
+    timed once, so that noise does not choose among them.  Returns {"params", "ms",
     "default_ms", "trials"} and installs the winner on `ctx`; with `save`,
     stores it under `key` in the user table (or `path`)."""
     saved = ctx.params()
-    best = dict(DEFAULTS)
+    best = effective(DEFAULTS)
     trials = 0
+    timed = [best]
 
     def measure(p):
         ctx.set_params(**p)
@@ -152,7 +160,10 @@ def tune(ctx, run: Callable[[], float], reps: int = 3, key: Optional[str] = None
     try:
         default_ms = best_ms = measure(best)
         for stage in (stages or STAGES):
-            for p in candidates(stage, best):
+            for p in map(effective, candidates(stage, best)):
+                if p in timed:
+                    continue
+                timed.append(p)
                 ms = measure(p)
                 trials += 1
                 if log:

@@ -39,3 +39,33 @@ def test_package_table_is_valid():
     for key, entry in T.load_table(T.PACKAGE_TABLE).items():
         assert key.split("/")[0] in ("plain", "batch")
         assert set(entry["params"]) == set(T.DEFAULTS)
+
+
+class _FakeContext:
+    """Records the settings that are timed; `ms` is the time of the current one."""
+
+    def __init__(self, cost):
+        self.cost, self.now, self.timed = cost, dict(T.DEFAULTS), []
+
+    def params(self):
+        return dict(self.now)
+
+    def set_params(self, **p):
+        self.now = dict(p)
+
+    def run(self):
+        if not self.timed or self.timed[-1] != self.now:
+            self.timed.append(dict(self.now))
+        return self.cost(self.now, len(self.timed))
+
+
+def test_settings_that_run_alike_are_timed_once():
+    # every later measurement looks faster: repeats of one setting would win
+    ctx = _FakeContext(lambda p, k: 10.0 - 0.01 * k)
+    e = T.tune(ctx, ctx.run, reps=2)
+    alike = [tuple(sorted(T.effective(p).items())) for p in ctx.timed]
+    assert len(alike) == len(set(alike)) == e["trials"] + 1
+    assert e["params"] == T.effective(e["params"]) == ctx.now
+    ctx = _FakeContext(lambda p, k: 1.0 if p["order"] == 1 and p["wave_max_deg"] == 64 else 2.0 - p["order"] / 2)
+    assert T.tune(ctx, ctx.run)["params"] == dict(T.effective(T.DEFAULTS), order=1, wave_max_deg=64,
+                                                  group_max_deg=1024, grid_per_cu=2)
