@@ -587,15 +587,23 @@ def run_batch(args):
     print(json.dumps(result), flush=True)
 
 
-def design_bytes(streamed, m, n, entries):
-    """HBM bytes the hash-probe intersection must move per launch: every
-    streamed T-list id once (4 B; the library's streamed_ids, close to the
-    reference's wedge_checks when every oriented edge is intersected from its
-    first vertex and far smaller with min_side), every S(x) once when its
-    table is built (4m), per walk entry the neighbour id and the bounds of
-    its T list (4 + 16 B; entries = 2m for the min-side walk over whole input
-    rows, m otherwise), and the tail offsets and per-vertex counts (16n)."""
-    return 4 * streamed + 4 * m + 20 * entries + 16 * n
+def id_bytes(nnz):
+    """Bytes of a streamed id: from 2^22 input slots on the hub tails of a
+    skewed graph stream lists of 2 bytes per id (85 % of all streamed ids at
+    RMAT-22), the other tails 4; every id is counted at the smaller size."""
+    return 2 if nnz >= 1 << 22 else 4
+
+
+def design_bytes(streamed, m, n, entries, per_id):
+    """Lower bound on the HBM bytes the intersection moves per launch: every
+    streamed T-list id once (per_id bytes; the library's streamed_ids, close
+    to the reference's wedge_checks when every oriented edge is intersected
+    from its first vertex and far smaller with min_side), every S(x) once when
+    its table is built (per_id * m), per walk entry the neighbour id and the
+    bounds of its T list (4 + 16 B; entries = 2m for the min-side walk over
+    whole input rows, m otherwise), and the tail offsets and per-vertex counts
+    (16n)."""
+    return per_id * (streamed + m) + 20 * entries + 16 * n
 
 
 def unsorted_leg(args, ctx, g, total):
@@ -696,12 +704,13 @@ def run_plain(args):
     dg.free()
     d_pv.free()
 
-    # roofline of the intersection on the bytes this design must move (unit = one
-    # oriented edge: 4 B per streamed T-list id -- streamed_ids in all -- plus
-    # 4 B of S(x) per kept slot, 20 B per walk entry and 16 B per vertex); the
+    # roofline of the intersection on the bytes this design must move at least
+    # (unit = one oriented edge: id_bytes per streamed T-list id -- streamed_ids
+    # in all -- and per kept slot, 20 B per walk entry and 16 B per vertex); the
     # reference's intersection_size_local figure, which charges both lists
     # per edge (B_count = 4W + 4m + 8(n+1) + 8n), is reported beside it
-    b_design = design_bytes(streamed, m, n, entries)
+    per_id = id_bytes(nnz)
+    b_design = design_bytes(streamed, m, n, entries, per_id)
     b_count = 4 * W + 4 * m + 8 * (n + 1) + 8 * n
     b_pre = 16 * (n + 1) + 12 * m
     k_ms = float(np.mean(kern_ms))
@@ -741,7 +750,7 @@ def run_plain(args):
             "traffic": None if args.params else MEASURED_TRAFFIC.get(("plain", args.scale, args.edge_factor, args.seed)),
             "kernel_ms": k_ms,
             "bytes_per_launch": b_design,
-            "bytes": "4 * streamed_ids + 4 * m + 20 * walk_entries + 16 * n",
+            "bytes": f"{per_id} * (streamed_ids + m) + 20 * walk_entries + 16 * n",
             "algorithmic_effective_GBs": b_count / (k_ms * 1e-3) / 1e9,
             "algorithmic_bytes": "4 * W + 4 * m + 8 * (n + 1) + 8 * n, W = intersection_size_local",
         },

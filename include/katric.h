@@ -80,11 +80,12 @@ typedef struct {
     float d2h_ms;       /* device -> host copies of the outputs */
 } kt_timing;
 
-/* Intersection strategy knobs (bin thresholds and list walk); the package's
- * autotuner (katric_amd.tune) chooses them per graph class.  Counts never
- * depend on them. */
-/* List-walk hints; accepted for callers that set them.  Every value takes the
- * same walk: the T lists of up to 64 neighbours are streamed as one sequence
+/* Intersection knobs (bin thresholds, order of the tails, walk side); the
+ * package's autotuner (katric_amd.tune) chooses them per graph class.  Counts
+ * never depend on them.
+ *
+ * List-walk hints, accepted for callers that set them: every value takes the
+ * same walk, the T lists of up to 64 neighbours are streamed as one sequence
  * of 16-byte blocks, one block per lane, so that short and long lists fill a
  * wave alike. */
 #define KT_STRATEGY_STREAMED 0u
@@ -93,8 +94,8 @@ typedef struct {
 #define KT_STRATEGY_GROUPED32 3u
 #define KT_STRATEGY_GROUPED4 4u
 #define KT_STRATEGY_GROUPED2 5u
-#define KT_ORDER_DEGREE 0u      /* work queues by degree bucket, largest first */
-#define KT_ORDER_VERTEX 1u      /* work queues by vertex id (locality across a batch's graphs) */
+#define KT_ORDER_DEGREE 0u      /* tails by size step, largest first */
+#define KT_ORDER_VERTEX 1u      /* tails by vertex id (locality across a batch's graphs) */
 typedef struct {
     uint32_t wave_max_deg;  /* |N+(v)| <= this: one wave per tail, LDS hash (<= 256) */
     uint32_t group_max_deg; /* |N+(v)| <= this: one workgroup per tail, LDS hash (<= 2048) */

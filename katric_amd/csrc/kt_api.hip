@@ -227,7 +227,7 @@ extern "C" int kt_create(kt_ctx** out, int device, uint64_t hbm_budget_bytes) {
     c->prm.group_max_deg = 2048;
     c->prm.team_chunk = 8;
     c->prm.grid_per_cu = 4;
-    c->prm.strategy = TC_STREAMED;
+    c->prm.strategy = KT_STRATEGY_STREAMED;
     c->prm.order = TC_BY_DEGREE;
     trace("context on device %d: %d CUs, stream %p", device, c->num_cus, (void*)c->stream);
     *out = c;

@@ -68,11 +68,11 @@ struct kt_ctx {
     // Grows aux[i] to at least `bytes` (its contents are dropped).
     int reserve_aux(int i, uint64_t bytes);
     void release_aux();
-    // One device word, read in order after the work queued on `stream`.
-    int read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what);
-    // Up to four of them with one launch and one wait.
-    int read_words(const uint64_t* const* dev, int count, uint64_t* out, const char* what);
+    // Device words, read in order after the work queued on `stream`: one, two,
+    // or up to four with one launch and one wait.
     int read_u64(const uint64_t* dev, uint64_t* out, const char* what);
+    int read_2u64(const uint64_t* a, const uint64_t* b, uint64_t out[2], const char* what);
+    int read_words(const uint64_t* const* dev, int count, uint64_t* out, const char* what);
     void destroy_extensions();
 };
 

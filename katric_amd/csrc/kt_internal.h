@@ -82,7 +82,6 @@ void segsort_launch(uint32_t n, const uint64_t* ooff, uint32_t* oheads, uint32_t
 // fill kernels (kt_util.hip); used instead of hipMemsetAsync so that every
 // pipeline stays capturable in a HIP graph.
 void fill_u64(uint64_t* p, uint64_t count, uint64_t value, hipStream_t st);
-void fill_u32(uint32_t* p, uint64_t count, uint32_t value, hipStream_t st);
 // Several ranges of words zeroed by one launch.
 struct ClearList {
     uint64_t* p[6];
@@ -102,7 +101,7 @@ struct TcParams {
     uint32_t group_max_deg;   // d+(v) <= this: one workgroup (8 waves) per tail vertex (LDS hash)
     uint32_t team_chunk;      // neighbours per work grab inside a workgroup team (1..64)
     uint32_t grid_per_cu;     // persistent workgroups per CU (at most three fit)
-    uint32_t strategy;        // TC_STREAMED or TC_GROUPED*
+    uint32_t strategy;        // list-walk hint of kt_params: every value takes the same walk
     uint32_t order;           // TC_BY_DEGREE or TC_BY_VERTEX (work-queue order)
     uint32_t table_shift = 3; // hash tables hold >= 2^table_shift slots per key where they fit (8: smaller
                               // tables to clear and flush per tail; 16 gave the same RMAT-22 time, batches 1 % slower)
@@ -115,20 +114,10 @@ struct TcParams {
     uint32_t min_side = 1;    // plain counting: intersect every edge from the side with the shorter T list
 };
 
-// List-walk hints of kt_params: every value takes the same walk, which fills
-// a wave whatever the lists' lengths are (walk_lists in kt_tc.hip).
-enum : uint32_t {
-    TC_STREAMED = 0,
-    TC_GROUPED16 = 1,
-    TC_GROUPED8 = 2,
-    TC_GROUPED32 = 3,
-    TC_GROUPED4 = 4,
-    TC_GROUPED2 = 5
-};
-// Order of the work queues: tails by degree bucket, largest first, in 13
-// buckets (TC_BY_DEGREE), or by vertex id in two classes -- workgroup tails,
-// then wave tails (TC_BY_VERTEX: tails of one graph of a batch, and their
-// data, stay together in time and cache).
+// Order of the tails inside each of the three classes of kt_bins.h: by size
+// step, largest first (TC_BY_DEGREE), or by vertex id, every XCD its share
+// (TC_BY_VERTEX: tails of one graph of a batch, and their data, stay together
+// in time and cache).
 enum : uint32_t { TC_BY_DEGREE = 0, TC_BY_VERTEX = 1 };
 
 // Optional parts of the launch workspace; without them (all zero) every tail

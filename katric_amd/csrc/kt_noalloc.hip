@@ -18,7 +18,7 @@
 
 namespace kt {
 
-// a little more than promised: the intersection's queue and sums (150 KB) come
+// a little more than promised: the intersection's queue and sums (90 KB) come
 // on top of what the limit in the header counts
 constexpr uint64_t NOALLOC_BYTES = KT_NOALLOC_SCRATCH_BYTES + (256ull << 10);
 constexpr int MAX_DEVICES = 64;

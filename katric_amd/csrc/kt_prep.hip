@@ -365,7 +365,7 @@ __global__ void __launch_bounds__(OR_THREADS)
     block_excl_sum(s0, lw, &stot);
     if (tid == 0) {
         tile_cnt[blockIdx.x] = tot;
-        sym_part[blockIdx.x] = stot;  // the tile's checksum, summed by k_sym_final
+        sym_part[blockIdx.x] = stot;  // the tile's checksum, summed by k_scan_one
     }
 }
 
@@ -1061,8 +1061,6 @@ uint64_t orient_ws_words(uint32_t n, uint64_t nnz) {
            orient_scan_words(n, tiles) + ((uint64_t)n + 15) / 16 + tiles;
 }
 
-// Rows of the first and last slot of every `tile`-slot tile of a CSR whose
-// offsets start at 0 (bnd: 2 entries per tile), for tile_rows.
 // Degrees, validation flags, keep bitmask, d+ per row and its scan into ooff
 // (ooff[n] = kept total), per-tile kept counts and their scan.
 void orient_count_launch(uint32_t n, uint64_t nnz, const uint64_t* off, const uint32_t* heads, uint32_t* deg,

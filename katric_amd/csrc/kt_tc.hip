@@ -175,7 +175,7 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
 // they are hubs too: S(x) of a hub fits a table indexed by hub number, in
 // which a lookup is one 2-byte LDS read (k_tc_hub).
 // ---------------------------------------------------------------------------
-constexpr uint32_t HUB_MAX = 32000;            // 2-byte entries: 58 KB of LDS, two workgroups per CU
+constexpr uint32_t HUB_MAX = 32000;            // 2-byte entries: 64,000 bytes of LDS, two workgroups per CU
 constexpr uint32_t HUB_NONE = 2 * HUB_MAX;     // hub-list entry of any other id: its table entry stays empty
 constexpr uint32_t DEG_BINS = 1024;
 constexpr int HUB_BLOCKS = 256, HUB_HIST_THREADS = 256, HUB_NUMBER_THREADS = 256;
@@ -410,7 +410,7 @@ __device__ __forceinline__ uint32_t bucket_base(const uint32_t* q, int b, int cn
 // Grid-stride over tails; per-block bucket counts in LDS, one global atomic
 // per bucket per block.  ONE: one block, which knows every tail's place from its
 // own counts, so it writes the list too (a call on a small graph is a chain of
-// launches of 3 to 15 us each: n = 1200 115 -> 111 us with this one in place of
+// launches of 3 to 15 us each: n = 1531 115 -> 111 us with this one in place of
 // two).
 constexpr int BIN_THREADS = 1024;
 constexpr uint32_t BIN_ONE = 4;  // tails per thread of that block
@@ -1864,6 +1864,9 @@ TcRoom tc_room(uint64_t entries, uint64_t slots, uint64_t pv_n) {
     // below, the launches for the hubs cost what they gain (R-MAT n = 65,521 with
     // 1.8 M entries: 206 us without, 213 us with)
     if (entries >= (1ull << 22)) r.hub_slots = slots;
+    // (beyond, clearing and adding up 128 bytes per vertex costs more than the
+    // copies save: G(n, m) n = 5 M, 15 M pairs 1.51 ms without, 1.62 with; R-MAT
+    // scale 23 with 4 and 16 pairs per vertex 4.15 and 4.44, 22.6 and 23.0)
     if (pv_n <= (1ull << 22)) r.pv_n = pv_n;
     return r;
 }

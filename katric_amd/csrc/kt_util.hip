@@ -11,12 +11,6 @@ __global__ void k_fill_u64(uint64_t* __restrict__ p, uint64_t count, uint64_t va
         p[i] = value;
 }
 
-__global__ void k_fill_u32(uint32_t* __restrict__ p, uint64_t count, uint32_t value) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = value;
-}
-
 __global__ void __launch_bounds__(256) k_clear(ClearList c) {
     const uint64_t n = c.n[blockIdx.y];
     uint64_t* p = c.p[blockIdx.y];
@@ -41,11 +35,6 @@ static unsigned fill_grid(uint64_t count) {
 void fill_u64(uint64_t* p, uint64_t count, uint64_t value, hipStream_t st) {
     if (count == 0) return;
     k_fill_u64<<<fill_grid(count), 256, 0, st>>>(p, count, value);
-}
-
-void fill_u32(uint32_t* p, uint64_t count, uint32_t value, hipStream_t st) {
-    if (count == 0) return;
-    k_fill_u32<<<fill_grid(count), 256, 0, st>>>(p, count, value);
 }
 
 }  // namespace kt
