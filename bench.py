@@ -43,12 +43,12 @@ HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 # per dispatch).  A plain 1 GiB device copy reads FETCH_SIZE = 524,308 KiB and
 # WRITE_SIZE = 1,048,576 KiB on MI355X, so FETCH_SIZE is scaled by 2.000 and
 # WRITE_SIZE by 1.000.  RMAT-22 ef16 seed 1 (min-side walk), KiB of
-# k_hub_lists, k_tc_hub and k_tc_main: (129,510 + 15,626,000 + 7,638,900) x 2.000
-# + 143,230 + 1,832,800 + 778,000 = 50.73 GB.
+# k_hub_lists, k_tc_hub and k_tc_main: (129,512 + 15,628,472 + 7,637,287) x 2.000
+# + 143,368 + 1,832,787 + 620,301 = 50.57 GB.
 # Shard (RMAT-26 ef16 seed 1, 16 ranks, rank 0, CeTriC), the count phase's
-# k_hub_lists, k_tc_hub, k_tc_main and k_tc_big launches, local and contracted:
-# FETCH_SIZE 257,986,013 KiB x 2.000 + WRITE_SIZE 12,359,441 KiB = 541.01 GB.
-MEASURED_TRAFFIC = {("plain", 22, 16, 1): 50.73e9, ("shard-cetric", 26, 16, 1, 16, 0): 541.01e9}
+# k_tc_main and k_tc_big launches, local and contracted:
+# FETCH_SIZE 257,925,265 KiB x 2.000 + WRITE_SIZE 11,769,024 KiB = 540.28 GB.
+MEASURED_TRAFFIC = {("plain", 22, 16, 1): 50.57e9, ("shard-cetric", 26, 16, 1, 16, 0): 540.28e9}
 
 
 

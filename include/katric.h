@@ -85,7 +85,7 @@ typedef struct {
  * never depend on them.
  *
  * List-walk hints, accepted for callers that set them: every value takes the
- * same walk, the T lists of up to 64 neighbours are streamed as one sequence
+ * same walk: the T lists of up to 64 neighbours are streamed as one sequence
  * of 16-byte blocks, one block per lane, so that short and long lists fill a
  * wave alike. */
 #define KT_STRATEGY_STREAMED 0u

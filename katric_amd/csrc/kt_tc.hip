@@ -1278,8 +1278,10 @@ struct Shares {
 
 // 80 VGPRs and 51.6 KB of LDS: three workgroups per CU, 6 waves per SIMD.  Bound
 // by the chain of dependent loads that every pack or chunk of 64 entries starts
-// with, and by VALU (73 % busy at R-MAT scale 22, where it takes 2.7 ms; 768
-// mixed graphs 6.1 ms).
+// with, and by VALU (72 % busy at R-MAT scale 22, where it takes 2.7 ms; 768
+// mixed graphs 6.0 ms).  On a large shard's long lists VALU and latency, which its
+// 24 waves a CU hide less of than 32 would (R-MAT scale 26, rank 0 of 16: local
+// phase 47 ms, contracted phase 56).
 template <bool PLAIN, bool LIST>
 __global__ void __launch_bounds__(TC_THREADS) __attribute__((amdgpu_waves_per_eu(6, 6))) k_tc_main(View<PLAIN> V, TcOut out, TcParams prm,
                                                          uint32_t* __restrict__ q,
@@ -1660,7 +1662,7 @@ __device__ __forceinline__ uint32_t walk_hub_lists(const uint16_t* __restrict__ 
 // Workgroup tails that are hubs, part by part: 12-wave teams, two workgroups
 // per CU, each with a table of one entry per hub in dynamic LDS.  The table is
 // empty between parts (the thread that set an entry clears it).  Bound by LDS
-// reads (57 % busy, half of it bank conflicts) and VALU (65 %) of 24 waves a CU:
+// reads (56 % busy, half of it bank conflicts) and VALU (64 %) of 24 waves a CU:
 // R-MAT scale 22 4.8 to 5.0 ms (8 waves a workgroup 5.3, 16 with room for 29,696
 // hubs 4.9 and 0.4 more in k_tc_main).  The last quarter of the parts comes from
 // a queue: without one 9.2 ms in place of 8.4 for the whole count phase.
